@@ -321,21 +321,11 @@ static int group_rows(hivf_index* h, const int32_t* label, const uint32_t* key2,
 int gpu_lloyd_round(hivf_index* h, const float4* xa, const float* xsum, int64_t ldx, int64_t n, float* cent_host,
                     DevBuf<float>& dcent) {
     hipStream_t s = h->stream;
-    // assignment: nearest centroid of every row (coarse kernel, one probe)
-    HIP_TRY(h, h->d_cd.ensure((size_t)n));
-    HIP_TRY(h, h->d_probes.ensure((size_t)n));
-    CoarseArgs c;
-    c.q = xa;
-    c.nq = (int)n;
-    c.nquad = h->nquad;
-    c.cent = h->d_cent.p;
-    c.nlist = (int)h->nlist;
-    c.P = 1;
-    c.out_d = h->d_cd.p;
-    c.out_l = h->d_probes.p;
-    HIP_TRY(h, launch_coarse(c, h->metric, s));
+    // assignment: nearest centroid of every row
+    int rc = run_assign(h, xa, n, false, s);
+    if (rc) return rc;
     Grouping G;
-    int rc = group_rows(h, h->d_probes.p, nullptr, n, G, s);
+    rc = group_rows(h, h->d_probes.p, nullptr, n, G, s);
     if (rc) return rc;
     const size_t cb = (size_t)h->nlist * h->d * sizeof(float);
     HIP_TRY(h, dcent.ensure((size_t)h->nlist * h->d));
@@ -451,20 +441,12 @@ int gpu_add(hivf_index* h, int64_t n) {
     Grouping G;
     DevBuf<uint32_t> key;
     if (n > 0) {
-        CoarseArgs c;
-        c.q = h->d_q.p;
-        c.nq = (int)n;
-        c.nquad = h->nquad;
-        c.cent = h->d_cent.p;
-        c.nlist = (int)nlist;
-        c.P = 1;
-        c.out_d = h->d_cd.p;
-        c.out_l = h->d_probes.p;
-        HIP_TRY(h, launch_coarse(c, h->metric, s));
+        int rc = run_assign(h, h->d_q.p, n, true, s);
+        if (rc) return rc;
         HIP_TRY(h, key.ensure((size_t)n));
         hipLaunchKernelGGL(dist_key_kernel, dim3(grid_of(n, 256)), dim3(256), 0, s, h->d_cd.p, n,
                            h->metric == HIVF_METRIC_L2 ? 1 : 0, key.p);
-        int rc = group_rows(h, h->d_probes.p, key.p, n, G, s);
+        rc = group_rows(h, h->d_probes.p, key.p, n, G, s);
         if (rc) return rc;
     }
     std::vector<int64_t> list_off(nlist + 1, 0);

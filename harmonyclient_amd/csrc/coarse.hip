@@ -20,6 +20,7 @@
 //       exact, ties included.
 #include <climits>
 #include <cmath>
+#include <type_traits>
 
 #include "bf16.hpp"
 #include "index_impl.hpp"
@@ -704,6 +705,230 @@ __global__ __launch_bounds__(kNT) void coarse_pick_wave_kernel(CoarsePickArgs a,
     }
 }
 
+// ---- row assignment (one probe): training and add ----------------------
+//
+// Nearest centroid of every row, as the per-query kernel with P = 1 (lowest
+// id among exact ties), from the same approximate ranks as the search's coarse
+// step.  Per row the scan keeps the two centroids with the smallest lower
+// bounds rank - E and the third smallest lower bound.  U, an upper bound of
+// the first one's exact rank, bounds the nearest centroid's: every centroid
+// whose lower bound is <= U can be the nearest, the others cannot.  With the
+// third bound above U at most two centroids qualify; both are rescored with
+// the exact chain.  The other rows (and any whose norms could overflow) go
+// through hard[] to the per-query kernel.
+//
+// What bounds it: the MFMA chain (6 products per 16 dims) and about 13 vector
+// operations per (row, centroid).  A workgroup holds 256 (d <= 128) rows'
+// BF16 pieces in registers as B operands for the whole scan and streams the
+// centroid shadow through LDS, 8 dim chunks of a 32-centroid tile at a time
+// (24 KB, double buffered, read by all four waves), so the vector memory path
+// carries a quarter of what each wave reading the shadow itself would take.
+// Measured: 500k x 128 rows, 1024 centroids 0.82 ms (0.96 PFLOP/s issued, of
+// 1.18 that a large BF16 product reaches) against 13.4 ms for one workgroup
+// per row streaming every centroid; 131k x 96, 512 centroids 0.097 ms
+// against 1.54; a few rows in a thousand are handed over (5 us).
+struct AssignArgs {
+    const float4* x;      // rows [n x nquad]
+    int64_t n;
+    int nquad, nkc;
+    const uint16_t* cbf;  // centroid shadow
+    const float* cn;      // centroid squared norms (0 on padding)
+    const float4* crow;   // FP32 centroids, row-major [nlist x nquad]
+    int nlist;
+    float coef;
+    float cn_max;         // largest centroid norm (inf when one is not finite)
+    int need_dist;        // the exact distance is wanted for every row
+    float* out_d;         // [n]
+    int32_t* out_l;       // [n]
+    int32_t* hard;        // rows for the per-query kernel, count in *nhard
+    uint32_t* nhard;
+};
+
+constexpr int kStageKc = 8;                           // 16-dim chunks of a stage
+constexpr int kStageFrags = 3 * kStageKc;             // 1 KiB fragments of a stage
+constexpr int kStageRegs = kStageFrags * 64 / kNT;    // 16-byte loads per thread and stage
+
+// NS stages of 8 dim chunks per tile (d <= 128 NS), QG groups of 32 rows per wave.
+template <int METRIC, int NS, int QG>
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(NS <= 2 ? 2 : 1)))
+void assign_kernel(AssignArgs a) {
+    __shared__ bf16x8 sa[2][kStageFrags * 64];
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, half = lane >> 5, slot = lane & 31;
+    const int64_t r0 = ((int64_t)blockIdx.x * (kNT / 64) + tid / 64) * 32 * QG;
+    const int nkc = a.nkc;
+    // the rows' two BF16 pieces (B operands) and squared norms (FP64 sums)
+    bf16x8 hr[QG][NS * kStageKc], lr[QG][NS * kStageKc];
+    float qn[QG];
+#pragma unroll
+    for (int g = 0; g < QG; ++g) {
+        const int64_t r = r0 + g * 32 + slot;
+        const float4* xp = a.x + (r < a.n ? r : a.n - 1) * a.nquad;
+        double s = 0.0;
+#pragma unroll
+        for (int kc = 0; kc < NS * kStageKc; ++kc) {
+            bf16x8 h = {}, l = {};
+            if (kc < nkc) {
+                const int j = kc * 4 + half * 2;
+                const float4 u = j < a.nquad ? xp[j] : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float4 v = j + 1 < a.nquad ? xp[j + 1] : make_float4(0.f, 0.f, 0.f, 0.f);
+                const float e[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+                uint16_t hb[8], lb[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    hb[i] = f2bf(e[i]);
+                    lb[i] = f2bf(e[i] - bf2f(hb[i]));
+                    s += (double)e[i] * (double)e[i];
+                }
+                h = *reinterpret_cast<const bf16x8*>(hb);
+                l = *reinterpret_cast<const bf16x8*>(lb);
+            }
+            hr[g][kc] = h;
+            lr[g][kc] = l;
+        }
+        s += __shfl_xor(s, 32);
+        qn[g] = (float)s;
+    }
+    float l1[QG], l2[QG], l3[QG];
+    int c1[QG], c2[QG];
+#pragma unroll
+    for (int g = 0; g < QG; ++g) {
+        l1[g] = l2[g] = l3[g] = INFINITY;
+        c1[g] = c2[g] = -1;
+    }
+    auto insert = [&](int g, float v, int c) {
+        const bool b1 = v < l1[g], b2 = v < l2[g];
+        c2[g] = b1 ? c1[g] : (b2 ? c : c2[g]);
+        c1[g] = b1 ? c : c1[g];
+        l3[g] = __builtin_amdgcn_fmed3f(l2[g], l3[g], v);
+        l2[g] = __builtin_amdgcn_fmed3f(l1[g], l2[g], v);
+        l1[g] = fminf(l1[g], v);
+    };
+    const int tiles = (a.nlist + 31) / 32;
+    const int total = tiles * NS;  // stages: stage u = dim chunks (u % NS) * 8 .. of tile u / NS
+    const bf16x8* cb = reinterpret_cast<const bf16x8*>(a.cbf);
+    bf16x8 pre[kStageRegs];
+    auto fetch = [&](int u) {  // (chunks past nkc read chunk nkc - 1; they are not used)
+        const int T = u / NS, k0 = (u % NS) * kStageKc;
+#pragma unroll
+        for (int i = 0; i < kStageRegs; ++i) {
+            const int e = i * kNT + tid, f = e >> 6, p = f / kStageKc, kc = min(k0 + f % kStageKc, nkc - 1);
+            pre[i] = cb[((size_t)(T * 3 + p) * nkc + kc) * 64 + (e & 63)];
+        }
+    };
+    auto put = [&](int b) {
+#pragma unroll
+        for (int i = 0; i < kStageRegs; ++i) sa[b][i * kNT + tid] = pre[i];
+    };
+    fetch(0);
+    put(0);
+    if (total > 1) fetch(1);
+    __syncthreads();
+    int u = 0;
+    for (int T = 0; T < tiles; ++T) {
+        floatx16 acc[QG];
+#pragma unroll
+        for (int g = 0; g < QG; ++g) acc[g] = floatx16{};
+        float4 cv[4];
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4)
+            cv[r4] = *reinterpret_cast<const float4*>(a.cn + (size_t)T * 32 + r4 * 8 + half * 4);
+#pragma unroll
+        for (int ks = 0; ks < NS; ++ks, ++u) {
+            const bf16x8* A = sa[u & 1] + lane;
+#pragma unroll
+            for (int kc = 0; kc < kStageKc; ++kc) {
+                if (ks * kStageKc + kc < nkc) {
+                    const bf16x8 a0 = A[(size_t)kc * 64], a1 = A[(size_t)(kStageKc + kc) * 64],
+                                 a2 = A[(size_t)(2 * kStageKc + kc) * 64];
+                    auto mm = [&](const bf16x8& av, const bf16x8 (&b)[QG][NS * kStageKc]) {
+#pragma unroll
+                        for (int g = 0; g < QG; ++g)
+                            acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b[g][ks * kStageKc + kc], acc[g], 0, 0, 0);
+                    };
+                    mm(a2, lr);
+                    mm(a1, lr);
+                    mm(a0, lr);
+                    mm(a2, hr);
+                    mm(a1, hr);
+                    mm(a0, hr);
+                }
+            }
+            // the next stage into the other buffer (its last readers passed
+            // the previous barrier), the one after it into registers
+            if (u + 1 < total) {
+                put((u + 1) & 1);
+                if (u + 2 < total) fetch(u + 2);
+            }
+            __syncthreads();
+        }
+        const bool tail = T * 32 + 32 > a.nlist;
+#pragma unroll
+        for (int r4 = 0; r4 < 4; ++r4) {
+            const float cn[4] = {cv[r4].x, cv[r4].y, cv[r4].z, cv[r4].w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int c = T * 32 + r4 * 8 + half * 4 + e;
+#pragma unroll
+                for (int g = 0; g < QG; ++g) {
+                    const float dot = acc[g][r4 * 4 + e], s = qn[g] + cn[e];
+                    const float rank = METRIC == kL2 ? s - 2.0f * dot : -dot;
+                    float lb = rank - (a.coef * s + kEabs);
+                    if (tail && c >= a.nlist) lb = INFINITY;
+                    insert(g, lb, c);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int g = 0; g < QG; ++g) {
+        // the other half's three, then one view of the row for both halves
+        const float o1 = __shfl_xor(l1[g], 32), o2 = __shfl_xor(l2[g], 32), o3 = __shfl_xor(l3[g], 32);
+        const int oc1 = __shfl_xor(c1[g], 32), oc2 = __shfl_xor(c2[g], 32);
+        insert(g, o1, oc1);
+        insert(g, o2, oc2);
+        insert(g, o3, -1);
+        const int k1 = __shfl(c1[g], slot), k2 = __shfl(c2[g], slot);
+        const float b1 = __shfl(l1[g], slot), b2 = __shfl(l2[g], slot), b3 = __shfl(l3[g], slot);
+        const int64_t r = r0 + g * 32 + slot;
+        const bool live = r < a.n;
+        // U: the first one's upper bound (lower bound + 2 E), widened past
+        // the rounding of the three operations
+        const float s1 = qn[g] + a.cn[max(k1, 0)];
+        const float U = b1 + 2.0f * (a.coef * s1 + kEabs) + 0x1p-20f * s1;
+        // norms this large could overflow a rank; NaN compares false
+        const bool sane = qn[g] + a.cn_max < 1e37f;
+        const bool hard = !sane || k1 < 0 || b3 <= U;
+        const bool two = b2 <= U;
+        uint64_t key = ~0ull;
+        const int c = half ? k2 : k1;
+        if (live && !hard && (two || (half == 0 && a.need_dist))) {
+            const float4* xp = a.x + r * a.nquad;
+            const float4* cp = a.crow + (size_t)c * a.nquad;
+            float acc = 0.0f;
+#pragma unroll 8
+            for (int j = 0; j < a.nquad; ++j) acc = accum<METRIC>(acc, xp[j], cp[j]);
+            const float rk = rank_of<METRIC>(acc);
+            if (rk < FLT_MAX) key = make_key(rk, (uint32_t)c);
+        }
+        const uint32_t ohi = __shfl_xor((uint32_t)(key >> 32), 32), olo = __shfl_xor((uint32_t)key, 32);
+        const uint64_t ok = ((uint64_t)ohi << 32) | olo;
+        if (live && half == 0) {
+            if (hard) {
+                a.hard[atomicAdd(a.nhard, 1u)] = (int32_t)r;
+            } else if (two || a.need_dist) {
+                const uint64_t best = key < ok ? key : ok;
+                a.out_l[r] = best == ~0ull ? -1 : (int32_t)(uint32_t)best;
+                a.out_d[r] = best == ~0ull ? sentinel<METRIC>() : dist_of_rank(METRIC, key_rank(best));
+            } else {
+                a.out_l[r] = k1;
+            }
+        }
+    }
+}
+
+__global__ void zero_word_kernel(uint32_t* p) { *p = 0u; }
+
 }  // namespace
 
 // Bound on |approximate rank - exact chain rank| per unit of
@@ -725,6 +950,82 @@ float coarse_coef(int64_t d) {
     return (float)(c * 1.01);
 }
 
+// The 3-piece BF16 centroid shadow of the current centroids.
+static int ensure_cent_shadow(hivf_index* h, hipStream_t s) {
+    CoarseState& C = h->coarse;
+    if (C.valid) return HIVF_OK;
+    const int nkc = (int)((h->d + 15) / 16);
+    const int64_t tiles32 = 2 * ((h->nlist + kTileRows - 1) / kTileRows);
+    const int64_t total = tiles32 * 3 * nkc * 64;
+    HIP_TRY(h, C.cbf.ensure((size_t)total * 8));
+    hipLaunchKernelGGL(cent_split_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, h->d_cent.p,
+                       h->nquad, tiles32, nkc, C.cbf.p);
+    HIP_TRY(h, hipGetLastError());
+    C.valid = true;
+    return HIVF_OK;
+}
+
+int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStream_t s) {
+    CoarseState& C = h->coarse;
+    HIP_TRY(h, h->d_cd.ensure((size_t)n));
+    HIP_TRY(h, h->d_probes.ensure((size_t)n));
+    CoarseArgs c;
+    c.q = x;
+    c.nq = (int)n;
+    c.nquad = h->nquad;
+    c.cent = h->d_cent.p;
+    c.nlist = (int)h->nlist;
+    c.P = 1;
+    c.out_d = h->d_cd.p;
+    c.out_l = h->d_probes.p;
+    const int nkc = (int)((h->d + 15) / 16);
+    if (nkc > 32) {  // (the per-query kernel takes any d)
+        HIP_TRY(h, launch_coarse(c, h->metric, s));
+        return HIVF_OK;
+    }
+    const int rc = ensure_cent_shadow(h, s);
+    if (rc) return rc;
+    HIP_TRY(h, C.hard.ensure((size_t)n));
+    HIP_TRY(h, C.nhard.ensure(1));
+    hipLaunchKernelGGL(zero_word_kernel, dim3(1), dim3(1), 0, s, C.nhard.p);
+    AssignArgs a;
+    a.x = x;
+    a.n = n;
+    a.nquad = h->nquad;
+    a.nkc = nkc;
+    a.cbf = C.cbf.p;
+    a.cn = h->d_cent_norm.p;
+    a.crow = h->d_cent_rows.p;
+    a.nlist = (int)h->nlist;
+    a.coef = coarse_coef(h->d);
+    a.cn_max = h->cent_norm_max;
+    a.need_dist = need_dist ? 1 : 0;
+    a.out_d = h->d_cd.p;
+    a.out_l = h->d_probes.p;
+    a.hard = C.hard.p;
+    a.nhard = C.nhard.p;
+    auto launch = [&](auto metric) {
+        constexpr int M = decltype(metric)::value;
+        const int64_t rows = nkc <= kStageKc ? 256 : 128;  // per workgroup
+        const dim3 grid((unsigned)((n + rows - 1) / rows));
+        if (nkc <= kStageKc)
+            hipLaunchKernelGGL((assign_kernel<M, 1, 2>), grid, dim3(kNT), 0, s, a);
+        else if (nkc <= 2 * kStageKc)
+            hipLaunchKernelGGL((assign_kernel<M, 2, 1>), grid, dim3(kNT), 0, s, a);
+        else
+            hipLaunchKernelGGL((assign_kernel<M, 4, 1>), grid, dim3(kNT), 0, s, a);
+    };
+    if (h->metric == HIVF_METRIC_L2)
+        launch(std::integral_constant<int, kL2>{});
+    else
+        launch(std::integral_constant<int, kIP>{});
+    HIP_TRY(h, hipGetLastError());
+    c.qlist = C.hard.p;
+    c.qcount = C.nhard.p;
+    HIP_TRY(h, launch_coarse(c, h->metric, s));
+    return HIVF_OK;
+}
+
 // nprobe nearest centroids of n staged queries into h->d_cd / h->d_probes.
 // Returns HIVF_EUNSUPPORTED (nothing launched) where the MFMA form does not
 // apply (d > 512), so the caller runs the per-query kernel.
@@ -735,14 +1036,8 @@ int run_coarse_mfma(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStr
     const int64_t tiles32 = 2 * ((h->nlist + kTileRows - 1) / kTileRows);
     const int64_t ldo = tiles32 * 32;
     CoarseState& C = h->coarse;
-    if (!C.valid) {
-        HIP_TRY(h, C.cbf.ensure((size_t)tiles32 * 3 * nkc * 64 * 8));
-        const int64_t total = tiles32 * 3 * nkc * 64;
-        hipLaunchKernelGGL(cent_split_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, h->d_cent.p,
-                           h->nquad, tiles32, nkc, C.cbf.p);
-        HIP_TRY(h, hipGetLastError());
-        C.valid = true;
-    }
+    const int rc = ensure_cent_shadow(h, s);
+    if (rc) return rc;
     const int64_t chunk = std::max<int64_t>(32, std::min<int64_t>((n + 31) / 32 * 32, kMaxRankFloats / ldo / 32 * 32));
     HIP_TRY(h, C.qh.ensure((size_t)n * dpad16));
     HIP_TRY(h, C.ql.ensure((size_t)n * dpad16));

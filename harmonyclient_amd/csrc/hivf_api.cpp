@@ -253,6 +253,9 @@ int upload_centroids(hivf_index* h, const float* c) {
         for (int64_t j = 0; j < h->d; ++j) acc += (double)c[i * h->d + j] * (double)c[i * h->d + j];
         cn[i] = (float)acc;
     }
+    h->cent_norm_max = 0.0f;
+    for (int64_t i = 0; i < h->nlist; ++i)
+        h->cent_norm_max = std::isfinite(cn[i]) ? std::max(h->cent_norm_max, cn[i]) : INFINITY;
     HIP_TRY(h, h->d_cent_norm.ensure(cn.size()));
     HIP_TRY(h, hipMemcpy(h->d_cent_norm.p, cn.data(), cn.size() * sizeof(float), hipMemcpyHostToDevice));
     h->coarse.valid = false;

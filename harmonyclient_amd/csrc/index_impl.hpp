@@ -95,6 +95,7 @@ struct hivf_index {
     hivf::DevBuf<float4> d_cent;      // centroid tiles
     hivf::DevBuf<float4> d_cent_rows; // centroids row-major [nlist x nquad], zero-padded
     hivf::DevBuf<float> d_cent_norm;  // [tiles * 64] FP64-computed squared norms (0 on padding)
+    float cent_norm_max = 0.0f;       // largest centroid norm (inf when one is not finite)
     hivf::CoarseState coarse;
     hivf::DevBuf<float4> d_codes;
     hivf::DevBuf<uint32_t> d_ids;
@@ -215,6 +216,9 @@ int run_coarse_mfma(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStr
 // per-query kernel for P = 1 and d > 512.
 int run_coarse(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStream_t s,
                const PrepArgs* prep = nullptr, bool* prep_done = nullptr);
+// Nearest centroid of n padded device rows (coarse.hip): labels into
+// d_probes (-1: none) and, with need_dist, every distance into d_cd.
+int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStream_t s);
 // Index build on the GPU (build.hip).  One Lloyd round: assign the rows xa
 // (padded device rows), then set every centroid with rows to the FP64 mean
 // of its rows of xsum (row stride ldx floats) in row order; cent_host holds

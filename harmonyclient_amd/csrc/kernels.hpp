@@ -75,6 +75,8 @@ struct CoarseArgs {
     int P;                  // probes to keep
     float* out_d;           // [nq x P]
     int32_t* out_l;         // [nq x P], -1 = none
+    const int32_t* qlist = nullptr;    // optional: only these queries (count in *qcount)
+    const uint32_t* qcount = nullptr;
 };
 
 hipError_t launch_coarse(const CoarseArgs& a, int metric, hipStream_t s);

@@ -241,10 +241,9 @@ __global__ __launch_bounds__(kNT) void scan_kernel(ScanArgs a) {
 }
 
 template <int METRIC>
-__global__ __launch_bounds__(kNT) void coarse_kernel(CoarseArgs a) {
+__device__ void coarse_one(const CoarseArgs& a, const int qi) {
     __shared__ LdsTopK<kNT, kBuf> top;
     extern __shared__ float4 qs[];
-    const int qi = blockIdx.x;
     const int tid = threadIdx.x;
     const int wave = tid / kWave;
     const int lane = tid % kWave;
@@ -285,6 +284,20 @@ __global__ __launch_bounds__(kNT) void coarse_kernel(CoarseArgs a) {
     }
 }
 
+// One workgroup per query, or, with a query list, a grid that walks the list.
+template <int METRIC>
+__global__ __launch_bounds__(kNT) void coarse_kernel(CoarseArgs a) {
+    if (a.qlist) {
+        const uint32_t nl = *a.qcount;
+        for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
+            __syncthreads();  // the previous query's LDS reads are done
+            coarse_one<METRIC>(a, a.qlist[i]);
+        }
+        return;
+    }
+    coarse_one<METRIC>(a, blockIdx.x);
+}
+
 template <int MODE>
 hipError_t launch_scan_mode(const ScanArgs& a, int metric, hipStream_t s) {
     size_t lds = (size_t)a.lists.nquad * sizeof(float4);
@@ -310,10 +323,11 @@ hipError_t launch_scan(const ScanArgs& a, int mode, int metric, hipStream_t s) {
 hipError_t launch_coarse(const CoarseArgs& a, int metric, hipStream_t s) {
     if (a.nq <= 0) return hipSuccess;
     size_t lds = (size_t)a.nquad * sizeof(float4);
+    const dim3 grid((unsigned)(a.qlist ? std::min(a.nq, kListGrid) : a.nq));
     if (metric == kL2)
-        hipLaunchKernelGGL((coarse_kernel<kL2>), dim3(a.nq), dim3(kNT), lds, s, a);
+        hipLaunchKernelGGL((coarse_kernel<kL2>), grid, dim3(kNT), lds, s, a);
     else
-        hipLaunchKernelGGL((coarse_kernel<kIP>), dim3(a.nq), dim3(kNT), lds, s, a);
+        hipLaunchKernelGGL((coarse_kernel<kIP>), grid, dim3(kNT), lds, s, a);
     return hipGetLastError();
 }
 
