@@ -58,6 +58,22 @@ struct DevBuf {
     }
 };
 
+// Pinned host memory that large uploads of pageable rows go through
+// (upload_rows in hivf_api.cpp): one slot per copying thread and turn, made on
+// the first such upload, kept with the handle.
+struct PinnedRing {
+    static constexpr int kThreads = 6, kTurns = 2;
+    static constexpr size_t kSlot = 4u << 20;
+    char* p = nullptr;
+    hipEvent_t done[kThreads][kTurns] = {};
+    PinnedRing() = default;
+    PinnedRing(const PinnedRing&) = delete;
+    PinnedRing& operator=(const PinnedRing&) = delete;
+    ~PinnedRing() { release(); }
+    bool ensure();
+    void release();
+};
+
 // State of the MFMA coarse quantizer: the 3-piece BF16 centroid shadow and
 // per-search scratch.
 struct CoarseState {
@@ -106,6 +122,7 @@ struct hivf_index {
     // search scratch
     hivf::DevBuf<float4> d_q;
     hivf::DevBuf<float> d_stage;  // unpadded host queries on their way to d_q
+    hivf::PinnedRing ring;        // large uploads of rows
     hivf::DevBuf<float> d_cd;
     hivf::DevBuf<int32_t> d_probes;
     hivf::DevBuf<int32_t> d_npq;

@@ -30,6 +30,7 @@ def _rows(kind, n, d, nlist, seed):
     ("int", 5000, 128, 100), ("int", 257, 1, 33), ("real", 255, 17, 1), ("real", 4097, 128, 65),
     ("real", 1000, 129, 40), ("real", 1000, 200, 32), ("dup", 1500, 24, 31), ("near", 700, 64, 50),
     ("real", 600, 420, 97), ("int", 1, 96, 5), ("real", 300, 512, 20), ("real", 200, 516, 20),
+    ("int", 250_000, 17, 24),  # an upload in pinned chunks, rows padded on the way
 ])
 def test_add_assignment(metric, kind, n, d, nlist):
     print(f"[case] add {kind} n={n} d={d} nlist={nlist} metric={metric}", flush=True)
