@@ -247,6 +247,48 @@ __global__ __launch_bounds__(64) void centroid_mean_kernel(const float* __restri
     if (j < d) cent[(size_t)l * d + j] = (float)(acc / (double)(m1 - m0));
 }
 
+// The search's forms of the centroids, one thread per (row, quad): tiles (as
+// the list arena) and padded rows; clears the largest norm.
+__global__ void cent_layout_kernel(const float* __restrict__ raw, int64_t nlist, int d, int nquad, int64_t tiles,
+                                   float4* __restrict__ cent, float4* __restrict__ rows,
+                                   uint32_t* __restrict__ cmax) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *cmax = 0u;
+    if (i >= tiles * kTileRows * nquad) return;
+    const int64_t r = i / nquad;
+    const int j = (int)(i % nquad);
+    float v[4] = {0.f, 0.f, 0.f, 0.f};
+    if (r < nlist)
+        for (int c = 0; c < 4; ++c)
+            if (j * 4 + c < d) v[c] = raw[r * d + j * 4 + c];
+    const float4 q = make_float4(v[0], v[1], v[2], v[3]);
+    cent[((r / kTileRows) * nquad + j) * kTileRows + r % kTileRows] = q;
+    if (r < nlist) rows[r * nquad + j] = q;
+}
+
+// Squared norms, FP64 sums in dim order rounded once (0 on padding rows), and
+// the bits of the largest (those of inf when one is not finite).
+__global__ __launch_bounds__(64) void cent_norm_kernel(const float* __restrict__ raw, int64_t nlist, int d,
+                                                       float* __restrict__ norm, uint32_t* __restrict__ cmax) {
+    const int64_t r = (int64_t)blockIdx.x * 64 + threadIdx.x;
+    double s = 0.0;
+    if (r < nlist) {
+        const float* p = raw + r * d;
+        int j = 0;
+        for (; j + 16 <= d; j += 16) {
+            float v[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) v[t] = p[j + t];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) s += (double)v[t] * (double)v[t];
+        }
+        for (; j < d; ++j) s += (double)p[j] * (double)p[j];
+    }
+    const float f = (float)s;
+    norm[r] = f;
+    atomicMax(cmax, f <= FLT_MAX ? __float_as_uint(f) : 0x7F800000u);
+}
+
 // The tiled list arena from rows in list order: one thread per (tile, lane).
 __global__ __launch_bounds__(256) void fill_arena_kernel(const float4* __restrict__ x, int nquad, int d,
                                                          const int32_t* __restrict__ order,
@@ -365,22 +407,39 @@ static int group_rows(hivf_index* h, const int32_t* label, const uint32_t* key2,
     return HIVF_OK;
 }
 
-int gpu_lloyd_round(hivf_index* h, const float4* xa, const float* xsum, int64_t ldx, int64_t n, float* cent_host,
-                    DevBuf<float>& dcent) {
-    hipStream_t s = h->stream;
-    // assignment: nearest centroid of every row
-    int rc = run_assign(h, xa, n, false, s);
-    if (rc) return rc;
-    Grouping G;
-    rc = group_rows(h, h->d_probes.p, nullptr, n, G, s);
-    if (rc) return rc;
-    const size_t cb = (size_t)h->nlist * h->d * sizeof(float);
-    HIP_TRY(h, dcent.ensure((size_t)h->nlist * h->d));
-    HIP_TRY(h, hipMemcpyAsync(dcent.p, cent_host, cb, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(centroid_mean_kernel, dim3((unsigned)h->nlist, (unsigned)((h->d + 63) / 64)), dim3(64), 0, s, xsum, ldx, (int)h->d,
-                       G.order, G.off.p, dcent.p);
+int layout_centroids(hivf_index* h, hipStream_t s) {
+    const int64_t tiles = (h->nlist + kTileRows - 1) / kTileRows;
+    HIP_TRY(h, h->d_cent.ensure((size_t)tiles * h->nquad * kTileRows));
+    HIP_TRY(h, h->d_cent_rows.ensure((size_t)h->nlist * h->nquad));
+    HIP_TRY(h, h->d_cent_norm.ensure((size_t)tiles * kTileRows));
+    HIP_TRY(h, h->d_cent_max.ensure(1));
+    hipLaunchKernelGGL(cent_layout_kernel, dim3(grid_of(tiles * kTileRows * h->nquad, 256)), dim3(256), 0, s,
+                       h->d_cent_raw.p, h->nlist, (int)h->d, h->nquad, tiles, h->d_cent.p, h->d_cent_rows.p,
+                       h->d_cent_max.p);
+    hipLaunchKernelGGL(cent_norm_kernel, dim3((unsigned)tiles), dim3(kTileRows), 0, s, h->d_cent_raw.p, h->nlist,
+                       (int)h->d, h->d_cent_norm.p, h->d_cent_max.p);
     HIP_TRY(h, hipGetLastError());
-    HIP_TRY(h, hipMemcpyAsync(cent_host, dcent.p, cb, hipMemcpyDeviceToHost, s));
+    h->coarse.valid = false;
+    return HIVF_OK;
+}
+
+int gpu_lloyd(hivf_index* h, const float4* xa, const float* xsum, int64_t ldx, int64_t n, int niter,
+              float* cent_host) {
+    hipStream_t s = h->stream;
+    Grouping G;
+    for (int it = 0; it < niter; ++it) {
+        int rc = run_assign(h, xa, n, false, s);
+        if (rc) return rc;
+        rc = group_rows(h, h->d_probes.p, nullptr, n, G, s);
+        if (rc) return rc;
+        hipLaunchKernelGGL(centroid_mean_kernel, dim3((unsigned)h->nlist, (unsigned)((h->d + 63) / 64)), dim3(64), 0, s,
+                           xsum, ldx, (int)h->d, G.order, G.off.p, h->d_cent_raw.p);
+        HIP_TRY(h, hipGetLastError());
+        rc = layout_centroids(h, s);
+        if (rc) return rc;
+    }
+    HIP_TRY(h, hipMemcpyAsync(cent_host, h->d_cent_raw.p, (size_t)h->nlist * h->d * sizeof(float),
+                              hipMemcpyDeviceToHost, s));
     HIP_TRY(h, hipStreamSynchronize(s));
     return HIVF_OK;
 }

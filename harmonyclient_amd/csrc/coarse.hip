@@ -736,7 +736,7 @@ struct AssignArgs {
     const float4* crow;   // FP32 centroids, row-major [nlist x nquad]
     int nlist;
     float coef;
-    float cn_max;         // largest centroid norm (inf when one is not finite)
+    const uint32_t* cn_max; // bits of the largest centroid norm (inf when one is not finite)
     int need_dist;        // the exact distance is wanted for every row
     float* out_d;         // [n]
     int32_t* out_l;       // [n]
@@ -897,7 +897,7 @@ void assign_kernel(AssignArgs a) {
         const float s1 = qn[g] + a.cn[max(k1, 0)];
         const float U = b1 + 2.0f * (a.coef * s1 + kEabs) + 0x1p-20f * s1;
         // norms this large could overflow a rank; NaN compares false
-        const bool sane = qn[g] + a.cn_max < 1e37f;
+        const bool sane = qn[g] + __uint_as_float(*a.cn_max) < 1e37f;
         const bool hard = !sane || k1 < 0 || b3 <= U;
         const bool two = b2 <= U;
         uint64_t key = ~0ull;
@@ -998,7 +998,7 @@ int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStr
     a.crow = h->d_cent_rows.p;
     a.nlist = (int)h->nlist;
     a.coef = coarse_coef(h->d);
-    a.cn_max = h->cent_norm_max;
+    a.cn_max = h->d_cent_max.p;
     a.need_dist = need_dist ? 1 : 0;
     a.out_d = h->d_cd.p;
     a.out_l = h->d_probes.p;

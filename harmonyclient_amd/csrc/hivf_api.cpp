@@ -262,32 +262,12 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
 
 int upload_centroids(hivf_index* h, const float* c) {
     h->cent.assign(c, c + h->nlist * h->d);
-    int64_t tiles = (h->nlist + kTileRows - 1) / kTileRows;
-    std::vector<float> t((size_t)tiles * h->nquad * kTileRows * 4, 0.0f);
-    for (int64_t tt = 0; tt < tiles; ++tt) {
-        int64_t rows = std::min<int64_t>(kTileRows, h->nlist - tt * kTileRows);
-        tile_rows(c + tt * kTileRows * h->d, rows, h->d, h->nquad,
-                  t.data() + (size_t)tt * h->nquad * kTileRows * 4);
-    }
-    HIP_TRY(h, h->d_cent.ensure(t.size() / 4));
-    HIP_TRY(h, hipMemcpy(h->d_cent.p, t.data(), t.size() * sizeof(float), hipMemcpyHostToDevice));
-    std::vector<float> rows((size_t)h->nlist * h->nquad * 4, 0.0f);
-    for (int64_t i = 0; i < h->nlist; ++i)
-        std::memcpy(rows.data() + (size_t)i * h->nquad * 4, c + i * h->d, sizeof(float) * h->d);
-    HIP_TRY(h, h->d_cent_rows.ensure(rows.size() / 4));
-    HIP_TRY(h, hipMemcpy(h->d_cent_rows.p, rows.data(), rows.size() * sizeof(float), hipMemcpyHostToDevice));
-    std::vector<float> cn((size_t)tiles * kTileRows, 0.0f);
-    for (int64_t i = 0; i < h->nlist; ++i) {
-        double acc = 0.0;
-        for (int64_t j = 0; j < h->d; ++j) acc += (double)c[i * h->d + j] * (double)c[i * h->d + j];
-        cn[i] = (float)acc;
-    }
-    h->cent_norm_max = 0.0f;
-    for (int64_t i = 0; i < h->nlist; ++i)
-        h->cent_norm_max = std::isfinite(cn[i]) ? std::max(h->cent_norm_max, cn[i]) : INFINITY;
-    HIP_TRY(h, h->d_cent_norm.ensure(cn.size()));
-    HIP_TRY(h, hipMemcpy(h->d_cent_norm.p, cn.data(), cn.size() * sizeof(float), hipMemcpyHostToDevice));
-    h->coarse.valid = false;
+    HIP_TRY(h, h->d_cent_raw.ensure((size_t)h->nlist * h->d));
+    HIP_TRY(h, hipMemcpyAsync(h->d_cent_raw.p, h->cent.data(), h->cent.size() * sizeof(float), hipMemcpyHostToDevice,
+                              h->stream));
+    int rc = layout_centroids(h, h->stream);
+    if (rc) return rc;
+    HIP_TRY(h, hipStreamSynchronize(h->stream));
     h->have_centroids = true;
     h->batched.invalidate();
     h->drop_graph();
@@ -681,13 +661,12 @@ int hivf_index_train(hivf_index* h, int64_t n, const float* x, const float* init
         if (rc) return rc;
         xa = dxn.p;
     }
-    DevBuf<float> dcent;
-    for (int it = 0; it < niter; ++it) {
-        rc = gpu_lloyd_round(h, xa, reinterpret_cast<const float*>(dx.p), h->d_pad, n, cent.data(), dcent);
-        if (rc) return rc;
-        rc = upload_centroids(h, cent.data());
-        if (rc) return rc;
-    }
+    // the rounds stay on the device; the host copy follows the last one
+    rc = gpu_lloyd(h, xa, reinterpret_cast<const float*>(dx.p), h->d_pad, n, niter, cent.data());
+    if (rc) return rc;
+    h->cent = cent;
+    h->batched.invalidate();
+    h->drop_graph();
     if (h->metric == HIVF_METRIC_IP) {  // src/Index.cpp:409-421
         for (int64_t c = 0; c < nlist; ++c) {
             float s = 0.0f;

@@ -111,7 +111,8 @@ struct hivf_index {
     hivf::DevBuf<float4> d_cent;      // centroid tiles
     hivf::DevBuf<float4> d_cent_rows; // centroids row-major [nlist x nquad], zero-padded
     hivf::DevBuf<float> d_cent_norm;  // [tiles * 64] FP64-computed squared norms (0 on padding)
-    float cent_norm_max = 0.0f;       // largest centroid norm (inf when one is not finite)
+    hivf::DevBuf<float> d_cent_raw;   // [nlist x d] as given (or trained)
+    hivf::DevBuf<uint32_t> d_cent_max; // bits of the largest norm (inf when one is not finite)
     hivf::CoarseState coarse;
     hivf::DevBuf<float4> d_codes;
     hivf::DevBuf<uint32_t> d_ids;
@@ -236,12 +237,15 @@ int run_coarse(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStream_t
 // Nearest centroid of n padded device rows (coarse.hip): labels into
 // d_probes (-1: none) and, with need_dist, every distance into d_cd.
 int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStream_t s);
-// Index build on the GPU (build.hip).  One Lloyd round: assign the rows xa
+// Index build on the GPU (build.hip).  The search's forms of the centroids
+// in d_cent_raw: tiles, padded rows, norms.
+int layout_centroids(hivf_index* h, hipStream_t s);
+// niter Lloyd rounds from the centroids in d_cent_raw: assign the rows xa
 // (padded device rows), then set every centroid with rows to the FP64 mean
-// of its rows of xsum (row stride ldx floats) in row order; cent_host holds
-// the centroids before and after.
-int gpu_lloyd_round(hivf_index* h, const float4* xa, const float* xsum, int64_t ldx, int64_t n, float* cent_host,
-                    DevBuf<float>& dcent);
+// of its rows of xsum (row stride ldx floats) in row order; cent_host gets
+// the centroids after the last round.
+int gpu_lloyd(hivf_index* h, const float4* xa, const float* xsum, int64_t ldx, int64_t n, int niter,
+              float* cent_host);
 // Unit-norm copies of n padded device rows (zero rows stay zero).
 int normalize_rows(hivf_index* h, const float4* x, int64_t n, float4* y);
 // Index::add of the n rows staged in d_q: lists, their order, the arena.
