@@ -13,8 +13,9 @@
 // any query with fewer than k survivors at or below it.
 //
 // Training runs on the GPU with the kernels below: a tiled FP32 GEMM with
-// bias / ReLU / mask epilogues (forward and both backward products), column
-// sums for bias gradients, the pinball-loss gradient and Adam.  Every
+// bias / ReLU / mask epilogues (forward, and the backward to the hidden
+// layers), the weight and bias gradients summed per chunk of rows and then
+// over the chunks, the pinball-loss gradient and Adam.  Every
 // reduction runs in a fixed order, so training is deterministic.
 #include <algorithm>
 #include <cfloat>
@@ -59,11 +60,15 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
     float acc[4][4] = {};
     for (int k0 = 0; k0 < g.K; k0 += 16) {
-        for (int e = threadIdx.x; e < 1024; e += 256) {
-            int kk = e / 64, r = e % 64;
-            int m = m0 + r, k = k0 + kk, n = n0 + r;
-            As[kk][r] = (m < g.M && k < g.K) ? (g.transA ? g.A[(size_t)k * g.lda + m] : g.A[(size_t)m * g.lda + k]) : 0.0f;
-            Bs[kk][r] = (n < g.N && k < g.K) ? (g.transB ? g.B[(size_t)n * g.ldb + k] : g.B[(size_t)k * g.ldb + n]) : 0.0f;
+        // consecutive threads along the operand's contiguous index
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int e = t * 256 + threadIdx.x;
+            const int ka = g.transA ? e / 64 : e % 16, ra = g.transA ? e % 64 : e / 16;
+            const int kb = g.transB ? e % 16 : e / 64, rb = g.transB ? e / 16 : e % 64;
+            const int m = m0 + ra, n = n0 + rb;
+            As[ka][ra] = (m < g.M && k0 + ka < g.K) ? g.A[g.transA ? (size_t)(k0 + ka) * g.lda + m : (size_t)m * g.lda + k0 + ka] : 0.0f;
+            Bs[kb][rb] = (n < g.N && k0 + kb < g.K) ? g.B[g.transB ? (size_t)n * g.ldb + k0 + kb : (size_t)(k0 + kb) * g.ldb + n] : 0.0f;
         }
         __syncthreads();
 #pragma unroll
@@ -97,18 +102,110 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     }
 }
 
-// out[c] = sum_r X[r * ld + c], rows in a fixed order.
-__global__ __launch_bounds__(256) void colsum_kernel(const float* __restrict__ X, int rows, int cols, int ld,
-                                                     float* __restrict__ out) {
-    __shared__ float part[4][64];
-    const int c = blockIdx.x * 64 + threadIdx.x % 64;
-    const int w = threadIdx.x / 64;
+// dZ2 = (dy w3^T) * [H2 > 0], one thread per element.
+__global__ void dz2_kernel(const float* __restrict__ dy, const float* __restrict__ w3, const float* __restrict__ H2,
+                           int64_t n, int hid, float* __restrict__ dZ2) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    dZ2[i] = H2[i] > 0.0f ? dy[i / hid] * w3[i % hid] : 0.0f;
+}
+
+// Gradients of the parameters, summed over one chunk of rows per blockIdx.x
+// into the chunk's row of `part` (parameter layout); grad_sum_kernel adds the
+// chunks in order.  The sums over the rows are what the whole backward is bound by:
+// as products with K = rows they filled 2 to 4 workgroups (1.6 ms each for
+// 8192 rows), and the bias sums one or two.  Cut into chunks they fill the
+// chip, and each FP32 chain is a chunk long instead of all rows: a gradient
+// over 8192 rows at 128 hidden units 5.47 -> 0.23 ms, its error against 64
+// bits 2.5e-6 -> 1.5e-7 of the gradient's norm.  blockIdx.y:
+// the 64 x 64 tiles of W2's gradient (the first row of tiles also sums b2's),
+// then W1's (and b1's), then 64-column pieces of w3's (the first also b3's).
+struct WgradArgs {
+    const float *Xs, *H1, *H2, *dZ1, *dZ2, *dy;
+    int rows, chunk, in, hid;
+    int64_t off_W1, off_b1, off_W2, off_b2, off_w3, off_b3, n_trained;
+    float* part;
+};
+
+__global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
+    __shared__ __align__(16) float As[16][68];
+    __shared__ __align__(16) float Bs[16][68];
+    const int tid = threadIdx.x, tx = tid % 16, ty = tid / 16;
+    const int r0 = blockIdx.x * a.chunk, r1 = min(a.rows, r0 + a.chunk);
+    float* out = a.part + (size_t)blockIdx.x * a.n_trained;
+    const int ht = (a.hid + 63) / 64, it = (a.in + 63) / 64;
+    int job = blockIdx.y;
+    if (job >= ht * ht + it * ht) {  // w3: H2^T dy; rows split over the four waves
+        job -= ht * ht + it * ht;
+        const int c = job * 64 + tid % 64, w = tid / 64;
+        float s = 0.0f, sy = 0.0f;
+        if (c < a.hid)
+            for (int r = r0 + w; r < r1; r += 4) {
+                s = __builtin_fmaf(a.H2[(size_t)r * a.hid + c], a.dy[r], s);
+                sy += a.dy[r];
+            }
+        As[w][tid % 64] = s;
+        Bs[w][tid % 64] = sy;
+        __syncthreads();
+        if (w == 0 && c < a.hid) {
+            out[a.off_w3 + c] = (As[0][tid] + As[1][tid]) + (As[2][tid] + As[3][tid]);
+            if (c == 0) out[a.off_b3] = (Bs[0][0] + Bs[1][0]) + (Bs[2][0] + Bs[3][0]);
+        }
+        return;
+    }
+    const bool second = job < ht * ht;
+    if (!second) job -= ht * ht;
+    const int m0 = (job / ht) * 64, n0 = (job % ht) * 64;
+    const float* A = second ? a.H1 : a.Xs;
+    const float* B = second ? a.dZ2 : a.dZ1;
+    const int M = second ? a.hid : a.in;
+    float acc[4][4] = {}, bias[4] = {};
+    for (int k0 = r0; k0 < r1; k0 += 16) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int e = t * 256 + tid, kk = e / 64, c = e % 64, k = k0 + kk;
+            As[kk][c] = (m0 + c < M && k < r1) ? A[(size_t)k * M + m0 + c] : 0.0f;
+            Bs[kk][c] = (n0 + c < a.hid && k < r1) ? B[(size_t)k * a.hid + n0 + c] : 0.0f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int kk = 0; kk < 16; ++kk) {
+            const float4 av = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
+            const float4 bv = *reinterpret_cast<const float4*>(&Bs[kk][tx * 4]);
+            const float x[4] = {av.x, av.y, av.z, av.w}, y[4] = {bv.x, bv.y, bv.z, bv.w};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bias[j] += y[j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(x[i], y[j], acc[i][j]);
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int n = n0 + tx * 4 + j;
+        if (n >= a.hid) continue;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int m = m0 + ty * 4 + i;
+            if (m < M) out[(second ? a.off_W2 : a.off_W1) + (size_t)m * a.hid + n] = acc[i][j];
+        }
+        if (m0 == 0 && ty == 0) out[(second ? a.off_b2 : a.off_b1) + n] = bias[j];
+    }
+}
+
+// G[i] = the chunks' partials in order (zero for the untrained parameters).
+__global__ void grad_sum_kernel(const float* __restrict__ part, int chunks, int64_t n_trained, int64_t n_params,
+                                float* __restrict__ G) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n_params) return;
     float s = 0.0f;
-    if (c < cols)
-        for (int r = w; r < rows; r += 4) s += X[(size_t)r * ld + c];
-    part[w][threadIdx.x % 64] = s;
-    __syncthreads();
-    if (w == 0 && c < cols) out[c] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
+    if (i < n_trained) {
+#pragma unroll 8
+        for (int c = 0; c < chunks; ++c) s += part[(size_t)c * n_trained + i];
+    }
+    G[i] = s;
 }
 
 // Raw features from the sorted coarse distances (stride P) and the query's
@@ -339,18 +436,13 @@ __global__ __launch_bounds__(256) void tau_mlp_kernel(FusedArgs a) {
     }
 }
 
-__global__ void fill_zero_kernel(float* p, int64_t n) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0.0f;
-}
-
 }  // namespace
 
 // ---- model --------------------------------------------------------------
 }  // namespace hivf
 
 hivf_tau_model::~hivf_tau_model() {
-    for (float** p : {&params, &grads, &m1, &m2, &work})
+    for (float** p : {&params, &grads, &m1, &m2, &work, &part, &io})
         if (*p) hivf::dev_free(*p);
     if (stream) (void)hipStreamDestroy(stream);
 }
@@ -386,30 +478,50 @@ hipError_t hivf_tau_model::forward(hipStream_t s, const float* Xs, int rows, flo
     hipError_t e;
     if ((e = gemm(s, Xs, in, 0, W1, hid, 0, H1, hid, rows, hid, in, b1, 1, nullptr, 0)) != hipSuccess) return e;
     if ((e = gemm(s, H1, hid, 0, W2, hid, 0, H2, hid, rows, hid, hid, b2, 1, nullptr, 0)) != hipSuccess) return e;
+    if (!yhat) return hipSuccess;  // (the backward alone needs no output)
     return gemm(s, H2, hid, 0, w3, 1, 0, yhat, 1, rows, 1, hid, b3, 0, nullptr, 0);
 }
 
-// Gradient of sum_i dy[i] yhat[i] w.r.t. the trained parameters into G.
+// Gradient of sum_i dy[i] yhat[i] w.r.t. the trained parameters into G (all
+// n_params of it; zeros for the untrained ones).
 hipError_t hivf_tau_model::backward(hipStream_t s, const float* Xs, int rows, const float* H1, const float* H2,
-                              const float* dy, float* dZ2, float* dZ1, float* G) const {
+                              const float* dy, float* dZ2, float* dZ1, float* G) {
     using namespace hivf;
-    const float *W2 = params + off_W2, *w3 = params + off_w3;
+    // chunks of at least 32 rows, at most 64 of them and 16 M partials: 8192
+    // rows 128 each (448 workgroups at 128 hidden units), 1024 rows 32
+    const int64_t most = std::max<int64_t>(1, std::min<int64_t>(64, ((int64_t)16 << 20) / n_trained));
+    const int64_t chunk = std::max<int64_t>(32, ((rows + most - 1) / most + 15) / 16 * 16);
+    const int64_t chunks = (rows + chunk - 1) / chunk;
     hipError_t e;
-    // layer 3: dw3 = H2^T dy, db3 = sum dy
-    if ((e = gemm(s, H2, hid, 1, dy, 1, 0, G + off_w3, 1, hid, 1, rows, nullptr, 0, nullptr, 0)) != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(colsum_kernel, dim3(1), dim3(256), 0, s, dy, rows, 1, 1, G + off_b3);
-    // dZ2 = (dy w3^T) * [H2 > 0]
-    if ((e = gemm(s, dy, 1, 0, w3, 1, 1, dZ2, hid, rows, hid, 1, nullptr, 0, H2, hid)) != hipSuccess) return e;
-    if ((e = gemm(s, H1, hid, 1, dZ2, hid, 0, G + off_W2, hid, hid, hid, rows, nullptr, 0, nullptr, 0)) != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(colsum_kernel, dim3(blocks(hid, 64)), dim3(256), 0, s, dZ2, rows, hid, hid, G + off_b2);
+    if (chunks * n_trained > part_floats) {
+        if (part) hivf::dev_free(part);
+        part = nullptr;
+        part_floats = 0;
+        if ((e = hipMalloc(&part, chunks * n_trained * sizeof(float))) != hipSuccess) return e;
+        part_floats = chunks * n_trained;
+    }
+    const float *W2 = params + off_W2, *w3 = params + off_w3;
+    const int64_t nz = (int64_t)rows * hid;
+    hipLaunchKernelGGL(dz2_kernel, dim3(blocks(nz)), dim3(256), 0, s, dy, w3, H2, nz, hid, dZ2);
     // dZ1 = (dZ2 W2^T) * [H1 > 0]
     if ((e = gemm(s, dZ2, hid, 0, W2, hid, 1, dZ1, hid, rows, hid, hid, nullptr, 0, H1, hid)) != hipSuccess) return e;
-    if ((e = gemm(s, Xs, in, 1, dZ1, hid, 0, G + off_W1, hid, in, hid, rows, nullptr, 0, nullptr, 0)) != hipSuccess)
-        return e;
-    hipLaunchKernelGGL(colsum_kernel, dim3(blocks(hid, 64)), dim3(256), 0, s, dZ1, rows, hid, hid, G + off_b1);
+    const WgradArgs wa{Xs, H1, H2, dZ1, dZ2, dy, rows, (int)chunk, in, hid, off_W1, off_b1, off_W2, off_b2, off_w3,
+                       off_b3, n_trained, part};
+    const unsigned ht = blocks(hid, 64), it = blocks(in, 64);
+    hipLaunchKernelGGL(wgrad_kernel, dim3((unsigned)chunks, ht * ht + it * ht + ht), dim3(256), 0, s, wa);
+    hipLaunchKernelGGL(grad_sum_kernel, dim3(blocks(n_params)), dim3(256), 0, s, part, (int)chunks, n_trained, n_params,
+                       G);
     return hipGetLastError();
+}
+
+hipError_t hivf_tau_model::ensure_io(int64_t floats) {
+    if (floats <= io_floats) return hipSuccess;
+    if (io) hivf::dev_free(io);
+    io = nullptr;
+    io_floats = 0;
+    const hipError_t e = hipMalloc(&io, floats * sizeof(float));
+    if (e == hipSuccess) io_floats = floats;
+    return e;
 }
 
 void hivf_tau_model::layout() {
@@ -553,59 +665,45 @@ int hivf_tau_model_forward(hivf_tau_model* m, int64_t n, const float* x, float* 
     HIVF_API_BEGIN
     if (!m || n < 0 || (n > 0 && (!x || !y))) return HIVF_EINVAL;
     if (n == 0) return HIVF_OK;
-    float *dx = nullptr, *dy = nullptr;
-    int rc = HIVF_OK;
-    if (hipMalloc(&dx, n * m->in * sizeof(float)) != hipSuccess || hipMalloc(&dy, n * sizeof(float)) != hipSuccess ||
-        hipMemcpy(dx, x, n * m->in * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-        m->ensure_work(n) != hipSuccess) {
-        rc = HIVF_EHIP;
-    } else {
-        float* Xs = m->work;
-        float* H1 = Xs + n * m->in;
-        float* H2 = H1 + n * m->hid;
-        hipLaunchKernelGGL(gather_std_kernel, dim3(blocks(n * m->in)), dim3(256), 0, m->stream, dx, nullptr, nullptr,
-                           (int)n, m->in, m->params + m->off_mu, m->params + m->off_sd, Xs, nullptr);
-        if (m->forward(m->stream, Xs, (int)n, H1, H2, dy, m->params) != hipSuccess ||
-            hipStreamSynchronize(m->stream) != hipSuccess ||
-            hipMemcpy(y, dy, n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
-            rc = HIVF_EHIP;
-    }
-    if (dx) hivf::dev_free(dx);
-    if (dy) hivf::dev_free(dy);
-    return rc;
+    if (m->ensure_work(n) != hipSuccess || m->ensure_io(n * (m->in + 1)) != hipSuccess) return HIVF_EHIP;
+    hipStream_t s = m->stream;
+    float *dx = m->io, *dy = dx + n * m->in;
+    float* Xs = m->work;
+    float* H1 = Xs + n * m->in;
+    float* H2 = H1 + n * m->hid;
+    if (hipMemcpyAsync(dx, x, n * m->in * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess) return HIVF_EHIP;
+    hipLaunchKernelGGL(gather_std_kernel, dim3(blocks(n * m->in)), dim3(256), 0, s, dx, nullptr, nullptr, (int)n,
+                       m->in, m->params + m->off_mu, m->params + m->off_sd, Xs, nullptr);
+    if (m->forward(s, Xs, (int)n, H1, H2, dy, m->params) != hipSuccess ||
+        hipMemcpyAsync(y, dy, n * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return HIVF_EHIP;
+    return HIVF_OK;
     HIVF_API_END(nullptr)
 }
 
 int hivf_tau_model_grad(hivf_tau_model* m, int64_t n, const float* x, const float* dyh, float* grad) {
     HIVF_API_BEGIN
     if (!m || n < 1 || !x || !dyh || !grad) return HIVF_EINVAL;
-    float *dx = nullptr, *ddy = nullptr;
-    int rc = HIVF_OK;
-    if (hipMalloc(&dx, n * m->in * sizeof(float)) != hipSuccess || hipMalloc(&ddy, n * sizeof(float)) != hipSuccess ||
-        hipMemcpy(dx, x, n * m->in * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(ddy, dyh, n * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-        m->ensure_work(n) != hipSuccess) {
-        rc = HIVF_EHIP;
-    } else {
-        float* Xs = m->work;
-        float* H1 = Xs + n * m->in;
-        float* H2 = H1 + n * m->hid;
-        float* yh = H2 + n * m->hid;
-        float* dZ2 = yh + n;
-        float* dZ1 = dZ2 + n * m->hid;
-        hipLaunchKernelGGL(gather_std_kernel, dim3(blocks(n * m->in)), dim3(256), 0, m->stream, dx, nullptr, nullptr,
-                           (int)n, m->in, m->params + m->off_mu, m->params + m->off_sd, Xs, nullptr);
-        std::vector<float> zero(m->n_params, 0.0f);
-        if (hipMemcpy(m->grads, zero.data(), m->n_params * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
-            m->forward(m->stream, Xs, (int)n, H1, H2, yh, m->params) != hipSuccess ||
-            m->backward(m->stream, Xs, (int)n, H1, H2, ddy, dZ2, dZ1, m->grads) != hipSuccess ||
-            hipStreamSynchronize(m->stream) != hipSuccess ||
-            hipMemcpy(grad, m->grads, m->n_params * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess)
-            rc = HIVF_EHIP;
-    }
-    if (dx) hivf::dev_free(dx);
-    if (ddy) hivf::dev_free(ddy);
-    return rc;
+    if (m->ensure_work(n) != hipSuccess || m->ensure_io(n * (m->in + 1)) != hipSuccess) return HIVF_EHIP;
+    hipStream_t s = m->stream;
+    float *dx = m->io, *ddy = dx + n * m->in;
+    float* Xs = m->work;
+    float* H1 = Xs + n * m->in;
+    float* H2 = H1 + n * m->hid;
+    float* dZ2 = H2 + n * m->hid;
+    float* dZ1 = dZ2 + n * m->hid;
+    if (hipMemcpyAsync(dx, x, n * m->in * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess ||
+        hipMemcpyAsync(ddy, dyh, n * sizeof(float), hipMemcpyHostToDevice, s) != hipSuccess)
+        return HIVF_EHIP;
+    hipLaunchKernelGGL(gather_std_kernel, dim3(blocks(n * m->in)), dim3(256), 0, s, dx, nullptr, nullptr, (int)n,
+                       m->in, m->params + m->off_mu, m->params + m->off_sd, Xs, nullptr);
+    if (m->forward(s, Xs, (int)n, H1, H2, nullptr, m->params) != hipSuccess ||
+        m->backward(s, Xs, (int)n, H1, H2, ddy, dZ2, dZ1, m->grads) != hipSuccess ||
+        hipMemcpyAsync(grad, m->grads, m->n_params * sizeof(float), hipMemcpyDeviceToHost, s) != hipSuccess ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return HIVF_EHIP;
+    return HIVF_OK;
     HIVF_API_END(nullptr)
 }
 
@@ -688,7 +786,6 @@ int hivf_tau_model_train(hivf_tau_model* m, int64_t n, const float* x, const flo
             const int rows = (int)std::min<size_t>(B, perm.size() - b0);
             hipLaunchKernelGGL(gather_std_kernel, dim3(blocks((int64_t)rows * in)), dim3(256), 0, s, dX, dY,
                                didx + b0, rows, in, m->params + m->off_mu, m->params + m->off_sd, dXb, dyb);
-            hipLaunchKernelGGL(fill_zero_kernel, dim3(blocks(m->n_params)), dim3(256), 0, s, m->grads, m->n_params);
             if (m->forward(s, dXb, rows, H1, H2, yh, m->params) != hipSuccess) {
                 cleanup();
                 return HIVF_EHIP;

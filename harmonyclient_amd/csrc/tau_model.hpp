@@ -17,16 +17,21 @@ struct hivf_tau_model {
     float* m2 = nullptr;
     float* work = nullptr;  // activations
     int64_t work_floats = 0;
+    float* part = nullptr;  // per-chunk partial gradients
+    int64_t part_floats = 0;
+    float* io = nullptr;    // inputs and outputs of host calls
+    int64_t io_floats = 0;
     float host_offset = 0.0f;
     float host_scale = 1.0f;  // distance scale s of the target log1p(D_k / s)
     hipStream_t stream = nullptr;
 
     void layout();
     hipError_t ensure_work(int64_t rows);
+    hipError_t ensure_io(int64_t floats);
     hipError_t forward(hipStream_t s, const float* Xs, int rows, float* H1, float* H2, float* yhat,
                        const float* P) const;
     hipError_t backward(hipStream_t s, const float* Xs, int rows, const float* H1, const float* H2, const float* dy,
-                        float* dZ2, float* dZ1, float* G) const;
+                        float* dZ2, float* dZ1, float* G);
     hipError_t predict(hipStream_t s, const float* F, int64_t n, float* tau, const float* P);
     ~hivf_tau_model();
 };
