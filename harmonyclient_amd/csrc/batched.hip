@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <climits>
 #include <cstring>
+#include <type_traits>
 
 #include "bf16.hpp"
 #include "index_impl.hpp"
@@ -1549,6 +1550,7 @@ struct SelArgs {
     const float4* q;            // padded queries
     int nquad;
     int k;
+    int metric;                 // of the keys' ranks (IP: the exact FP32 scans only)
     float* out_d;
     int64_t* out_i;
     int32_t* fallback;          // [nq] flags
@@ -1686,10 +1688,10 @@ __device__ void select_one(const SelArgs& a, const int qi) {
     }
     const int cnt = top.cnt;
     for (int i = tid; i < a.k; i += kNT) {
-        float dv = FLT_MAX;
+        float dv = a.metric == kL2 ? FLT_MAX : -FLT_MAX;
         int64_t iv = -1;
         if (i < cnt) {
-            dv = key_rank(top.buf[i]);
+            dv = dist_of_rank(a.metric, key_rank(top.buf[i]));
             iv = (int64_t)(uint32_t)top.buf[i];
         }
         a.out_d[(size_t)qi * a.k + i] = dv;
@@ -1902,10 +1904,10 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
         return;
     }
     for (int i = lane; i < a.k; i += 64) {
-        float dv = FLT_MAX;
+        float dv = a.metric == kL2 ? FLT_MAX : -FLT_MAX;
         int64_t iv = -1;
         if ((uint32_t)i < nc) {
-            dv = key_rank(kk[i]);
+            dv = dist_of_rank(a.metric, key_rank(kk[i]));
             iv = (int64_t)(uint32_t)kk[i];
         }
         a.out_d[(size_t)qi * a.k + i] = dv;
@@ -2104,9 +2106,82 @@ float margin_coef(int64_t d) {
                    1.01);
 }
 
+// Buffers of the planning (carved from the scratch) and its work-item bound.
+struct PlanBufs {
+    int nlist;
+    uint32_t *lcnt, *lcur, *lend, *qoff, *hwg, *ioff, *lnear, *meta;
+    int32_t* lq;
+    float* lqd;
+    BatchItem* items;
+    int64_t max_items;
+};
+
+// Words of a planning workgroup's per-(class, list) counts buffer.
+size_t plan_hwg_bytes(int64_t nlist, int64_t entries) {
+    return nlist * 2 <= kWgSlots ? (size_t)((entries + kPlanEntries - 1) / kPlanEntries + 1) * kWgSlots * 4 : 0;
+}
+
+// Inverts the pass's probes into work items of qc queries and rt 32-row tiles
+// (queries with lcnt cleared before).  nint: queries whose qint flags decide
+// *all_int.
+hipError_t launch_plan(const PlanBufs& b, const int32_t* probes, const float* cd, const int32_t* list_size, PairSet ps,
+                       PairFilter pf, uint32_t qc, uint32_t rt, const int32_t* qint, int nint, uint32_t* all_int,
+                       unsigned long long* cand, hipStream_t s) {
+    const int nlist = b.nlist;
+    const int64_t np = (int64_t)ps.nq * ps.P;
+    const unsigned gnp = (unsigned)((np + 255) / 256);
+    const bool lds = nlist <= kLdsLists;
+    const unsigned gpe = (unsigned)((np + kPlanEntries - 1) / kPlanEntries);
+    const int wgc = nlist * 8 <= kWgSlots ? 8 : nlist * 4 <= kWgSlots ? 4 : nlist * 2 <= kWgSlots ? 2 : 0;
+    const ItemArgs ia{b.lcnt, wgc ? b.lnear : nullptr, b.qoff, b.ioff, b.meta, list_size, nlist, qc, rt,
+                      b.max_items, b.items};
+    const unsigned iwg = (unsigned)((b.max_items + 255) / 256);
+    if (wgc) {
+        const unsigned nwg = std::max(1u, gpe);
+        const dim3 g1(nwg), gs((unsigned)((nlist + 63) / 64)), gf(nwg + iwg);
+        auto classes = [&](auto c) {
+            constexpr int C = decltype(c)::value;
+            hipLaunchKernelGGL(count_wg_kernel<C>, g1, dim3(256), 0, s, probes, ps, list_size, nlist, pf, b.hwg, cand);
+            hipLaunchKernelGGL(wg_scan_kernel<C>, gs, dim3(1024), 0, s, b.hwg, (int)nwg, nlist, b.lcnt, b.lnear);
+            hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, b.lcnt, b.lnear, list_size, nlist, qc, rt,
+                               b.qoff, b.lcur, b.lend, b.ioff, b.meta, qint, nint, all_int);
+            hipLaunchKernelGGL(fill_wg_kernel<C>, gf, dim3(256), 0, s, probes, cd, ps, nlist, pf, b.hwg, b.qoff, b.lq,
+                               b.lqd, nwg, ia);
+        };
+        if (wgc == 8)
+            classes(std::integral_constant<int, 8>{});
+        else if (wgc == 4)
+            classes(std::integral_constant<int, 4>{});
+        else
+            classes(std::integral_constant<int, 2>{});
+        return hipGetLastError();
+    }
+    if (lds)
+        hipLaunchKernelGGL(count_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, probes, ps, list_size, nlist,
+                           pf, b.lcnt, cand);
+    else
+        hipLaunchKernelGGL(count_kernel, dim3(gnp), dim3(256), 0, s, probes, ps.nq, ps.P, ps.npq, ps.active, list_size,
+                           pf, b.lcnt, cand);
+    hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, b.lcnt, (const uint32_t*)nullptr, list_size, nlist, qc,
+                       rt, b.qoff, b.lcur, b.lend, b.ioff, b.meta, qint, nint, all_int);
+    if (lds)
+        hipLaunchKernelGGL(fill_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, probes, cd, ps, nlist, pf,
+                           b.lcur, b.lend, b.lq, b.lqd);
+    else
+        hipLaunchKernelGGL(fill_kernel, dim3(gnp), dim3(256), 0, s, probes, cd, ps.nq, ps.P, ps.npq, ps.active, pf,
+                           b.lcur, b.lend, b.lq, b.lqd);
+    hipLaunchKernelGGL(items_par_kernel, dim3(iwg), dim3(256), 0, s, ia);
+    return hipGetLastError();
+}
+
 size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 }  // namespace
+}  // namespace hivf
+
+#include "flat.hpp"
+
+namespace hivf {
 
 void BatchedState::release() {
     if (bf16) hivf::dev_free(bf16);
@@ -2250,8 +2325,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                  o_qaug = take((size_t)n * 16), o_qn = take(n * 4), o_qint = take(n * 4),
                  o_lcnt = take(nlist * 4), o_lcur = take(nlist * 4), o_lend = take(nlist * 4),
                  o_qoff = take((nlist + 1) * 4), o_lqd = take((size_t)n * P * 4),
-                 o_hwg = take(nlist * 2 <= kWgSlots  // the atomic-free planning's counts
-                                  ? (size_t)((n * P + kPlanEntries - 1) / kPlanEntries + 1) * kWgSlots * 4 : 0),
+                 o_hwg = take(plan_hwg_bytes(nlist, n * P)),
                  o_ioff = take((nlist + 1) * 8), o_lnear = take(nlist * 4), o_meta = take(kMetaWords * 4), o_lq = take((size_t)n * P * 4),
                  o_items = take((size_t)max_items * sizeof(BatchItem)), o_scnt = take(n * 4),
                  o_sbuf = take((size_t)n * cap * 8), o_fb = take(n * 4), o_tau = take(n * 4),
@@ -2298,8 +2372,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     float* tau2 = (float*)at(o_tau2);
     float* rtau2 = (float*)at(o_rtau2);
     int32_t* fb2 = (int32_t*)at(o_fb2);
-    const int64_t np = n * P;
-    const unsigned gnp = (unsigned)((np + 255) / 256);
+    const PlanBufs pl{(int)nlist, lcnt, lcur, lend, qoff, hwg, ioff, lnear, meta, lq, lqd, items, max_items};
     // the BF16 scans are exact for integer queries and lists when d <= 129
     const int exact_bf16 = (h->lists_uint8 && h->d <= 129) ? 1 : 0;
     // the queries each rescue pass handles, as lists the selections append
@@ -2376,6 +2449,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.q = q;
         sa.nquad = h->nquad;
         sa.k = (int)k;
+        sa.metric = kL2;
         sa.out_d = D;
         sa.out_i = I;
         sa.fallback = fb_out;
@@ -2409,59 +2483,8 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         pf.cd = h->d_cd.p;
         pf.tau = tau_in;
         pf.lbound = static_cast<const float2*>(B.lbound);
-        const bool lds = nlist <= kLdsLists;
-        const unsigned gpe = (unsigned)((np + kPlanEntries - 1) / kPlanEntries);
-        PairSet ps{npq, active, qlist, qcount, (int)n, P};
-        const int wgc = nlist * 8 <= kWgSlots ? 8 : nlist * 4 <= kWgSlots ? 4 : nlist * 2 <= kWgSlots ? 2 : 0;
-        const ItemArgs ia{lcnt, wgc ? lnear : nullptr, qoff, ioff, meta, h->d_size.p, (int)nlist, qc, (uint32_t)rt,
-                          max_items, items};
-        const unsigned iwg = (unsigned)((max_items + 255) / 256);
-        if (wgc) {
-            const unsigned nwg = std::max(1u, gpe);
-            const dim3 g1(nwg), gs((unsigned)((nlist + 63) / 64));
-            if (wgc == 8) {
-                hipLaunchKernelGGL(count_wg_kernel<8>, g1, dim3(256), 0, s, h->d_probes.p, ps, h->d_size.p,
-                                   (int)nlist, pf, hwg, cand);
-                hipLaunchKernelGGL(wg_scan_kernel<8>, gs, dim3(1024), 0, s, hwg, (int)nwg, (int)nlist, lcnt, lnear);
-            } else if (wgc == 4) {
-                hipLaunchKernelGGL(count_wg_kernel<4>, g1, dim3(256), 0, s, h->d_probes.p, ps, h->d_size.p,
-                                   (int)nlist, pf, hwg, cand);
-                hipLaunchKernelGGL(wg_scan_kernel<4>, gs, dim3(1024), 0, s, hwg, (int)nwg, (int)nlist, lcnt, lnear);
-            } else {
-                hipLaunchKernelGGL(count_wg_kernel<2>, g1, dim3(256), 0, s, h->d_probes.p, ps, h->d_size.p,
-                                   (int)nlist, pf, hwg, cand);
-                hipLaunchKernelGGL(wg_scan_kernel<2>, gs, dim3(1024), 0, s, hwg, (int)nwg, (int)nlist, lcnt, lnear);
-            }
-            hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, lcnt, lnear, h->d_size.p, (int)nlist, qc,
-                               (uint32_t)rt, qoff, lcur, lend, ioff, meta, qint, (int)n, all_int);
-            const dim3 gf(nwg + iwg);
-            if (wgc == 8)
-                hipLaunchKernelGGL(fill_wg_kernel<8>, gf, dim3(256), 0, s, h->d_probes.p, h->d_cd.p, ps, (int)nlist,
-                                   pf, hwg, qoff, lq, lqd, nwg, ia);
-            else if (wgc == 4)
-                hipLaunchKernelGGL(fill_wg_kernel<4>, gf, dim3(256), 0, s, h->d_probes.p, h->d_cd.p, ps, (int)nlist,
-                                   pf, hwg, qoff, lq, lqd, nwg, ia);
-            else
-                hipLaunchKernelGGL(fill_wg_kernel<2>, gf, dim3(256), 0, s, h->d_probes.p, h->d_cd.p, ps, (int)nlist,
-                                   pf, hwg, qoff, lq, lqd, nwg, ia);
-        } else {
-        if (lds)
-            hipLaunchKernelGGL(count_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, h->d_probes.p, ps,
-                               h->d_size.p, (int)nlist, pf, lcnt, cand);
-        else
-            hipLaunchKernelGGL(count_kernel, dim3(gnp), dim3(256), 0, s, h->d_probes.p, (int)n, P, npq, active,
-                               h->d_size.p, pf, lcnt, cand);
-        hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, lcnt, (const uint32_t*)nullptr, h->d_size.p,
-                           (int)nlist, qc, (uint32_t)rt, qoff, lcur, lend, ioff, meta, qint, (int)n, all_int);
-        if (lds)
-            hipLaunchKernelGGL(fill_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, h->d_probes.p, h->d_cd.p,
-                               ps, (int)nlist, pf, lcur, lend, lq, lqd);
-        else
-            hipLaunchKernelGGL(fill_kernel, dim3(gnp), dim3(256), 0, s, h->d_probes.p, h->d_cd.p, (int)n, P, npq,
-                               active, pf, lcur, lend, lq, lqd);
-        }
-        if (!wgc) hipLaunchKernelGGL(items_par_kernel, dim3(iwg), dim3(256), 0, s, ia);
-        HIP_TRY(h, hipGetLastError());
+        HIP_TRY(h, launch_plan(pl, h->d_probes.p, h->d_cd.p, h->d_size.p, PairSet{npq, active, qlist, qcount, (int)n, P}, pf,
+                               qc, (uint32_t)rt, qint, (int)n, all_int, cand, s));
         if (timing && first) HIP_TRY(h, hipEventRecord(h->ev[6], s));
         BatchArgs ba;
         ba.items = items;
@@ -2652,6 +2675,190 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         st->blocks_total = (int64_t)c[1];    // 32-row tiles of the first pass's work items
         st->blocks_skipped = (int64_t)c[2];  // of which skipped by the radius bound
         st->candidates = (int64_t)c[0];
+    }
+    return HIVF_OK;
+}
+
+
+// Whether a batch repays the exact FP32 scans' launches (bound, plan,
+// selection).  The per-query kernel takes a workgroup 64 x 4 rows at a time
+// through a query's lists: one query of 100 tiles 224 us against 59, of 20
+// tiles 71 against 46, of 6 tiles (one list) 19 against 34; 16 queries of 6
+// tiles 65 against 47.
+static bool flat_pays(int64_t n, int P, double tiles_per_list) {
+    return P * tiles_per_list >= 12.0 || (double)n * P * tiles_per_list >= 90.0;
+}
+// Whether its queries share lists enough for the list-major form (else a
+// workgroup per query and list): 6 per list and tiles enough to fill the
+// chip.  1024 queries of 32 lists in 1024 (1.5 tiles each) 233 us against 292,
+// 512 of them 221 against 181; 256 queries of 20 lists in 400 (7.8 tiles) 270
+// against 401, 64 of them 238 against 182.
+static bool flat_shared(int64_t n, int P, int64_t nlist, double tiles_per_list) {
+    return n * P >= 6 * nlist && (double)n * P * tiles_per_list >= 40000.0;
+}
+
+// Batches of plain and pruned searches by the exact FP32 scans (flat.hpp).
+// HIVF_EUNSUPPORTED, with nothing launched: the per-query kernel serves them.
+int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
+             const hivf_search_params& p, float* D, int64_t* I, unsigned long long* stats, hipEvent_t tau_done,
+             hipStream_t s) {
+    const int64_t nlist = h->nlist;
+    int block_dims, nblocks;
+    const bool pruned = p.algo == HIVF_ALGO_PRUNED;
+    pruning_blocks(h->d, pruned ? p.dim_block : 0, &block_dims, &nblocks);
+    if (!pruned) {  // (four checks of whole quads; their place does not change the result)
+        block_dims = std::max(h->nquad / 4, 1) * 4;
+        nblocks = h->nquad >= 8 ? 4 : 1;
+    }
+    const double tiles_per_list = (double)h->tiles / (double)nlist;
+    if (!flat_pays(n, P, tiles_per_list)) return HIVF_EUNSUPPORTED;
+    const bool shared = flat_shared(n, P, nlist, tiles_per_list);
+    // survivors kept per query (a query with more is rescanned by the
+    // per-query kernel), and the queries of a chunk, so that their buffers
+    // stay within 512 MB
+    const uint32_t cap = (uint32_t)std::max<int64_t>(8192, 16 * k);
+    const int64_t chunk = std::min<int64_t>(n, ((int64_t)64 << 20) / cap);
+    int64_t max_t32 = 1;
+    for (int64_t l = 0; l < nlist; ++l)
+        max_t32 = std::max<int64_t>(max_t32, 2 * (h->tile_off[l + 1] - h->tile_off[l]));
+    const int64_t rtn = near_tiles(kFlatTiles);
+    const int64_t max_items = shared ? (chunk * P / kFlatItem + nlist) * ((max_t32 + rtn - 1) / rtn) : 0;
+    if (chunk * P >= INT32_MAX || max_items >= INT32_MAX) return HIVF_EUNSUPPORTED;
+    size_t off = 0;
+    auto take = [&](size_t bytes) {
+        size_t o = off;
+        off = align256(off + bytes);
+        return o;
+    };
+    const size_t entries = shared ? (size_t)chunk * P : 0;
+    const size_t o_sbuf = take((size_t)chunk * cap * 8), o_scnt = take(chunk * 4), o_fb = take(chunk * 4),
+                 o_fbl = take(chunk * 4), o_hard = take(chunk * 4), o_tau = take(chunk * 4), o_rtau = take(chunk * 4),
+                 o_fbc = take(16), o_allint = take(4), o_lcnt = take(nlist * 4), o_lcur = take(nlist * 4),
+                 o_lend = take(nlist * 4), o_qoff = take((nlist + 1) * 4), o_ioff = take((nlist + 1) * 8),
+                 o_lnear = take(nlist * 4), o_meta = take(kMetaWords * 4), o_lq = take(entries * 4),
+                 o_lqd = take(entries * 4), o_hwg = take(shared ? plan_hwg_bytes(nlist, (int64_t)entries) : 0),
+                 o_items = take((size_t)max_items * sizeof(BatchItem));
+    BatchedState& B = h->batched;
+    if (off > B.scratch_bytes) {
+        if (B.scratch) hivf::dev_free(B.scratch);
+        B.scratch = nullptr;
+        B.scratch_bytes = 0;
+        if (hipMalloc(&B.scratch, off) != hipSuccess) {  // no room for the buffers
+            (void)hipGetLastError();
+            B.scratch = nullptr;
+            return HIVF_EUNSUPPORTED;
+        }
+        B.scratch_bytes = off;
+    }
+    auto at = [&](size_t o) { return static_cast<void*>(static_cast<char*>(B.scratch) + o); };
+    uint32_t* scnt = (uint32_t*)at(o_scnt);
+    int32_t* fb = (int32_t*)at(o_fb);
+    uint32_t* lcnt = (uint32_t*)at(o_lcnt);
+    uint32_t* fbc = (uint32_t*)at(o_fbc);
+    uint32_t* all_int = (uint32_t*)at(o_allint);
+    float* tau = (float*)at(o_tau);
+    const PlanBufs pl{(int)nlist, lcnt, (uint32_t*)at(o_lcur), (uint32_t*)at(o_lend), (uint32_t*)at(o_qoff),
+                      (uint32_t*)at(o_hwg), (uint32_t*)at(o_ioff), (uint32_t*)at(o_lnear), (uint32_t*)at(o_meta),
+                      (int32_t*)at(o_lq), (float*)at(o_lqd), (BatchItem*)at(o_items), max_items};
+    // the warm-up's lists: enough that they hold twice k rows at the mean list
+    // size, and no fewer than asked for
+    const double mean_rows = std::max(1.0, (double)h->ntotal / (double)nlist);
+    const int warm_lists = (int)std::min<double>(std::max({10.0, (double)p.warmup_lists, 2.0 * (double)k / mean_rows}), 1024.0);
+    const int warm_rows = (int)std::max<int64_t>(k, p.warmup_list_size);
+    for (int64_t q0 = 0; q0 < n; q0 += chunk) {
+        const int64_t m = std::min(chunk, n - q0);
+        const int32_t* probes = h->d_probes.p + q0 * P;
+        const int32_t* npqc = npq ? npq + q0 : nullptr;
+        hipLaunchKernelGGL(flat_clear_kernel, dim3((unsigned)((std::max(m, nlist) + 255) / 256)), dim3(256), 0, s, scnt,
+                           fb, (int)m, lcnt, (int)nlist, fbc, all_int);
+        ScanArgs w{};
+        w.lists = h->lists();
+        w.q = q + q0 * h->nquad;
+        w.nq = (int)m;
+        w.probes = probes;
+        w.probe_stride = P;
+        w.nprobe_q = npqc;
+        w.nprobe = P;
+        w.k = (int)k;
+        w.block_dims = (int)h->d;
+        w.nblocks = 1;
+        w.row_limit = warm_rows;
+        w.warm_lists = warm_lists;
+        w.out_tau = tau;
+        HIP_TRY(h, launch_scan(w, kScanWarmup, h->metric, s));
+        if (tau_done && q0 == 0) HIP_TRY(h, hipEventRecord(tau_done, s));
+        FlatArgs a{};
+        a.lists = h->lists();
+        a.q = w.q;
+        a.tau = tau;
+        a.scnt = scnt;
+        a.sbuf = (uint64_t*)at(o_sbuf);
+        a.cap = cap;
+        a.block_dims = block_dims;
+        a.nblocks = nblocks;
+        a.rows_scanned = stats;
+        a.skips = pruned && stats ? stats + 2 : nullptr;
+        const bool l2 = h->metric == HIVF_METRIC_L2;
+        if (shared) {
+            PairFilter pf{};  // (no radius intervals here: every pair is scanned)
+            HIP_TRY(h, launch_plan(pl, probes, h->d_cd.p + q0 * P, h->d_size.p, PairSet{npqc, nullptr, nullptr, nullptr, (int)m, P},
+                                   pf, kFlatItem, kFlatTiles, fb, 0, all_int, stats, s));
+            a.items = pl.items;
+            a.meta = pl.meta;
+            a.lq = pl.lq;
+            a.max_items = (uint32_t)max_items;
+            const dim3 grid((unsigned)(h->cus * 6));
+            if (l2) hipLaunchKernelGGL(flat_scan_kernel<kL2>, grid, dim3(kNT), 0, s, a);
+            else hipLaunchKernelGGL(flat_scan_kernel<kIP>, grid, dim3(kNT), 0, s, a);
+        } else {
+            a.probes = probes;
+            a.npq = npqc;
+            a.P = P;
+            // a workgroup's waves take two tiles each at a time
+            a.parts = (int)std::min<int64_t>(std::max<int64_t>(1, (int64_t)(tiles_per_list / 8.0 + 0.75)), 64);
+            const dim3 grid((unsigned)(m * P * a.parts));
+            if (l2) hipLaunchKernelGGL(flat_pair_kernel<kL2>, grid, dim3(kNT), 0, s, a);
+            else hipLaunchKernelGGL(flat_pair_kernel<kIP>, grid, dim3(kNT), 0, s, a);
+        }
+        HIP_TRY(h, hipGetLastError());
+        SelArgs sa{};
+        sa.scnt = scnt;
+        sa.sbuf = a.sbuf;
+        sa.cap = cap;
+        sa.qint = fb;  // (read, not used: every key is exact)
+        sa.all_int = all_int;
+        sa.keys_exact = 1;
+        sa.tau = tau;
+        sa.ids = h->d_ids.p;
+        sa.codes = h->d_codes.p;
+        sa.q = w.q;
+        sa.nquad = h->nquad;
+        sa.k = (int)k;
+        sa.metric = h->metric;
+        sa.out_d = D + q0 * k;
+        sa.out_i = I + q0 * k;
+        sa.fallback = fb;
+        sa.rescan_tau = (float*)at(o_rtau);
+        sa.flist = (int32_t*)at(o_fbl);
+        sa.fcount = fbc;
+        sa.lcnt = lcnt;
+        sa.nlist = 0;  // (cleared with the chunk's counters)
+        int32_t* hard = (int32_t*)at(o_hard);
+        hipLaunchKernelGGL(select_wave_kernel, dim3((unsigned)((m + 3) / 4)), dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
+        sa.qlist = hard;
+        sa.qcount = fbc + 2;
+        hipLaunchKernelGGL(select_kernel, dim3((unsigned)std::min<int64_t>(m, 1024)), dim3(kNT), 0, s, sa);
+        HIP_TRY(h, hipGetLastError());
+        // survivors past the buffer: the query's lists scanned by the per-query kernel
+        ScanArgs f = w;
+        f.row_limit = INT_MAX;
+        f.warm_lists = INT_MAX;
+        f.out_tau = nullptr;
+        f.out_d = sa.out_d;
+        f.out_i = sa.out_i;
+        f.qlist = sa.flist;
+        f.qcount = fbc;
+        HIP_TRY(h, launch_scan(f, kScanPlain, h->metric, s));
     }
     return HIVF_OK;
 }

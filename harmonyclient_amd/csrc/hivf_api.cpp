@@ -462,6 +462,32 @@ int run_search(hivf_index* h, const float4* q, int64_t n, int64_t k, float* D, i
     return run_search_core(h, q, n, k, D, I, p, P, npq, st, s);
 }
 
+// The per-query kernels: one workgroup per query scans its probed lists.
+int per_query_scan(hivf_index* h, const float4* q, int64_t n, int64_t k, float* D, int64_t* I,
+                   const hivf_search_params& p, int64_t P, const int32_t* npq, bool timing, hipStream_t s) {
+    ScanArgs a = base_scan_args(h, q, n, P, k);
+    a.nprobe_q = npq;
+    a.out_d = D;
+    a.out_i = I;
+    a.stats = timing ? h->d_stats.p : nullptr;
+    const float* tau = nullptr;
+    if (p.algo == HIVF_ALGO_PRUNED && p.tau_source == HIVF_TAU_WARMUP) {
+        HIP_TRY(h, h->d_tau.ensure(n));
+        ScanArgs w = base_scan_args(h, q, n, P, k);
+        w.nprobe_q = npq;
+        w.row_limit = p.warmup_list_size > 0 ? p.warmup_list_size : (int)k;  // src/query.cpp:847
+        w.warm_lists = p.warmup_lists > 0 ? p.warmup_lists : 10;             // src/query.cpp:845
+        w.out_tau = h->d_tau.p;
+        HIP_TRY(h, launch_scan(w, kScanWarmup, h->metric, s));
+        tau = h->d_tau.p;
+    }
+    if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
+    a.tau = tau;
+    set_blocks(h, p, &a);
+    HIP_TRY(h, launch_scan(a, p.algo == HIVF_ALGO_PRUNED ? kScanPruned : kScanPlain, h->metric, s));
+    return HIVF_OK;
+}
+
 int run_search_core(hivf_index* h, const float4* q, int64_t n, int64_t k, float* D, int64_t* I,
                     const hivf_search_params& p, int64_t P, const int32_t* npq, hivf_search_stats* st,
                     hipStream_t s) {
@@ -481,28 +507,16 @@ int run_search_core(hivf_index* h, const float4* q, int64_t n, int64_t k, float*
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[1], s));
 
-    ScanArgs a = base_scan_args(h, q, n, P, k);
-    a.nprobe_q = npq;
-    a.out_d = D;
-    a.out_i = I;
-    a.stats = timing ? h->d_stats.p : nullptr;
-    const float* tau = nullptr;
-    if (p.algo == HIVF_ALGO_PRUNED && p.tau_source == HIVF_TAU_WARMUP) {
-        HIP_TRY(h, h->d_tau.ensure(n));
-        ScanArgs w = base_scan_args(h, q, n, P, k);
-        w.nprobe_q = npq;
-        w.row_limit = p.warmup_list_size > 0 ? p.warmup_list_size : (int)k;  // src/query.cpp:847
-        w.warm_lists = p.warmup_lists > 0 ? p.warmup_lists : 10;             // src/query.cpp:845
-        w.out_tau = h->d_tau.p;
-        HIP_TRY(h, launch_scan(w, kScanWarmup, h->metric, s));
-        tau = h->d_tau.p;
-    } else if (p.algo == HIVF_ALGO_PRUNED && p.tau_source == HIVF_TAU_LEARNED) {
+    if (p.algo == HIVF_ALGO_PRUNED && p.tau_source == HIVF_TAU_LEARNED)
         return h->fail(HIVF_EUNSUPPORTED, "the learned bound is used by the batched scan");
+    int bdims, nblocks;
+    pruning_blocks(h->d, p.dim_block, &bdims, &nblocks);
+    if (p.algo != HIVF_ALGO_PRUNED) nblocks = 1;
+    rc = run_flat(h, q, n, k, (int)P, npq, p, D, I, timing ? h->d_stats.p : nullptr, timing ? h->ev[2] : nullptr, s);
+    if (rc == HIVF_EUNSUPPORTED) {
+        rc = per_query_scan(h, q, n, k, D, I, p, P, npq, timing, s);
     }
-    if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
-    a.tau = tau;
-    set_blocks(h, p, &a);
-    HIP_TRY(h, launch_scan(a, p.algo == HIVF_ALGO_PRUNED ? kScanPruned : kScanPlain, h->metric, s));
+    if (rc) return rc;
     if (timing) {
         HIP_TRY(h, hipEventRecord(h->ev[3], s));
         HIP_TRY(h, hipEventSynchronize(h->ev[3]));
@@ -514,8 +528,8 @@ int run_search_core(hivf_index* h, const float4* q, int64_t n, int64_t k, float*
         st->scan_ms = elapsed(h->ev[2], h->ev[3]);
         st->total_ms = elapsed(h->ev[0], h->ev[3]);
         st->candidates = (int64_t)c[0];
-        st->blocks_total = (int64_t)c[1];
-        st->blocks_skipped = (int64_t)c[2];
+        st->blocks_total = st->candidates * nblocks;
+        st->blocks_skipped = nblocks > 1 ? (int64_t)c[2] : 0;
         st->scan_launches = 1;
     }
     return HIVF_OK;

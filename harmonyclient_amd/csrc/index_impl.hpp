@@ -225,6 +225,12 @@ int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_
 int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
                 const hivf_search_params& p, float* D, int64_t* I, hivf_search_stats* st,
                 hipStream_t s, bool timing);
+// Plain or pruned search of n staged queries whose probes are in d_probes, by
+// the batch's exact FP32 scans (batched.hip); stats: d_stats or null; tau_done:
+// recorded after the first bound, or null.
+int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
+             const hivf_search_params& p, float* D, int64_t* I, unsigned long long* stats, hipEvent_t tau_done,
+             hipStream_t s);
 struct PrepArgs;  // prep.hpp
 // MFMA coarse quantizer (coarse.hip); HIVF_EUNSUPPORTED when d > 512.  With
 // prep, its query-preparation launch also runs the batched search's.
