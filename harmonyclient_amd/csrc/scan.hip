@@ -79,20 +79,97 @@ __device__ inline float accum_dims(float acc, const float4* qs, const float4* tp
     return acc;
 }
 
-// Tiles of probe j of a query (rows capped at row_limit).
-__device__ inline int probe_tiles(const ScanArgs& a, const int32_t* probes, int j) {
-    int l = probes[j];
-    if (l < 0) return 0;
-    int rows = a.lists.list_size[l];
-    if (rows > a.row_limit) rows = a.row_limit;
-    return (rows + kTileRows - 1) / kTileRows;
+// The probes' lists, kProbeChunk at a time, staged in LDS: first arena tile,
+// rows (capped at row_limit) and tiles before each.
+constexpr int kProbeChunk = kNT;
+struct ProbeMap {
+    int tile0[kProbeChunk];
+    int rows[kProbeChunk];
+    int before[kProbeChunk + 1];
+    int wsum[kNW];
+};
+
+// Stages probes [j0, j0 + m) (m <= kProbeChunk); all threads, ends with a
+// barrier.  Their tiles number pm.before[m].
+__device__ inline void stage_probes(const ScanArgs& a, const int32_t* probes, int j0, int m, ProbeMap& pm) {
+    const int tid = threadIdx.x, lane = tid % kWave, wave = tid / kWave;
+    int rows = 0, tile0 = 0;
+    if (tid < m) {
+        const int l = probes[j0 + tid];
+        if (l >= 0) {
+            rows = min(a.lists.list_size[l], a.row_limit);
+            tile0 = a.lists.list_tile_off[l];
+        }
+    }
+    const int nt = (rows + kTileRows - 1) / kTileRows;
+    int incl = nt;
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int v = __shfl_up(incl, off);
+        if (lane >= off) incl += v;
+    }
+    if (lane == kWave - 1) pm.wsum[wave] = incl;
+    pm.tile0[tid] = tile0;
+    pm.rows[tid] = rows;
+    __syncthreads();
+    int base = 0;
+    for (int w = 0; w < wave; ++w) base += pm.wsum[w];
+    pm.before[tid + 1] = base + incl;
+    if (tid == 0) pm.before[0] = 0;
+    __syncthreads();
 }
 
-// One query, by the whole workgroup.
+// The kth smallest (1-based) of n <= 1024 keys' ranks, by one wave: the keys
+// stay in registers and the rank's bits are fixed from the highest that
+// differs down, one count per bit.  (A bitonic sort of the 1000-odd rows of a
+// warm-up scan is 55 stages with a barrier each.)
+__device__ inline uint32_t wave_kth_rank(const uint64_t* keys, int n, int kth, int lane) {
+    constexpr int kSlots = 16;
+    uint32_t v[kSlots];
+    uint32_t all_or = 0, all_and = ~0u;
+#pragma unroll
+    for (int t = 0; t < kSlots; ++t) {
+        const int i = t * kWave + lane;
+        v[t] = i < n ? (uint32_t)(keys[i] >> 32) : ~0u;
+        if (i < n) {
+            all_or |= v[t];
+            all_and &= v[t];
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        all_or |= __shfl_xor(all_or, off);
+        all_and &= __shfl_xor(all_and, off);
+    }
+    const uint32_t diff = all_or ^ all_and;
+    // res: the bits fixed so far (those above the highest difference are common)
+    const int top = diff ? 31 - __builtin_clz(diff) : -1;
+    uint32_t res = top < 31 ? all_and & ~((2u << max(top, 0)) - 1u) : 0u;
+    if (top < 0) return all_and;
+    for (int b = top; b >= 0; --b) {
+        const uint32_t test = res | (1u << b);  // ranks below it: the b-th bit clear under the prefix, or smaller
+        int c = 0;
+#pragma unroll
+        for (int t = 0; t < kSlots; ++t) c += __popcll(__ballot(v[t] < test));
+        if (c < kth) res = test;
+    }
+    return res;
+}
+
+// Tiles a wave takes between two barriers of the workgroup: the top-k's
+// buffer holds k <= 1024 kept keys and 4 x 256 more.  (The pruned scan takes
+// one: its bound follows the running k-th.)
+constexpr int kRoundTiles = 4;
+static_assert(kMaxK + kRoundTiles * kNT <= kBuf, "a round's keys fit beside the kept ones");
+
+// One query, by the whole workgroup.  The probes' sizes come from LDS (a chain
+// of two dependent loads per list otherwise), a warm-up scan ends in a bit
+// search for its k-th rank instead of a sort: warm-up of 2000 queries over 10
+// lists x 100 rows of 128 dims 103 -> 65 us, of 4096 on skewed lists 221 -> 172, of
+// 2000 with 420 dims 190 -> 163 (the rows come from L2 at 17 to 21 TB/s).  More
+// than 8 row loads in flight per wave is slower (16: 305 us at 420 dims).
 template <int MODE, int METRIC>
 __device__ void scan_one(const ScanArgs& a, const int qi) {
     __shared__ LdsTopK<kNT, kBuf> top;
-    __shared__ int s_tiles;
+    __shared__ ProbeMap pm;
     __shared__ unsigned long long s_stats[3];
     extern __shared__ float4 qs[];
 
@@ -106,84 +183,62 @@ __device__ void scan_one(const ScanArgs& a, const int qi) {
     if (MODE == kScanWarmup && P > a.warm_lists) P = a.warm_lists;  // src/Index.cpp:1008-1011
 
     top.init();
-    if (tid == 0) {
-        s_tiles = 0;
-        s_stats[0] = s_stats[1] = s_stats[2] = 0;
-    }
+    if (tid == 0) s_stats[0] = s_stats[1] = s_stats[2] = 0;
     load_query(qs, a.q + (size_t)qi * nquad, nquad);
-    __syncthreads();
-    {
-        int t = 0;
-        for (int j = tid; j < P; j += kNT) t += probe_tiles(a, probes, j);
-        if (t) atomicAdd(&s_tiles, t);
-    }
-    __syncthreads();
-    const int total = s_tiles;
-    const int rounds = (total + kNW - 1) / kNW;
-
-    // wave cursor: probe j, tile t within that list, for global tile `wave`
-    int j = 0, t = wave;
-    int nt_j = P > 0 ? probe_tiles(a, probes, 0) : 0;
-    while (j < P && t >= nt_j) {
-        t -= nt_j;
-        ++j;
-        nt_j = j < P ? probe_tiles(a, probes, j) : 0;
-    }
 
     const float tau_q = (MODE == kScanPruned && a.tau) ? a.tau[qi] : FLT_MAX;
     const int nblocks = MODE == kScanPruned ? a.nblocks : 1;
     unsigned long long my_cand = 0, my_skip = 0;
     uint64_t thr = top.thr;
 
-    for (int r = 0; r < rounds; ++r) {
-        if (j < P) {
-            const int l = probes[j];
-            int rows = a.lists.list_size[l];
-            if (rows > a.row_limit) rows = a.row_limit;
-            const int tile = a.lists.list_tile_off[l] + t;
-            const bool valid = lane < rows - t * kTileRows;
-            const float4* tp = a.lists.codes + (size_t)tile * nquad * kWave + lane;
-            float acc = 0.0f;
-            bool keep = valid;
-            if constexpr (MODE == kScanPruned) {
-                const float bound = fminf(tau_q, key_rank(thr));
-                for (int b = 0; b < nblocks; ++b) {
-                    if (__ballot(keep) == 0) break;
-                    if (keep) {
-                        const int d0 = b * a.block_dims;
-                        const int d1 = b < nblocks - 1 ? d0 + a.block_dims : 4 * nquad;
-                        acc = accum_dims<METRIC>(acc, qs, tp, d0, d1);
-                        if (b < nblocks - 1 && acc > bound) {
-                            keep = false;
-                            my_skip += nblocks - 1 - b;
+    constexpr int kRound = MODE == kScanPruned ? 1 : kRoundTiles;
+    for (int j0 = 0; j0 < P; j0 += kProbeChunk) {
+        stage_probes(a, probes, j0, min(kProbeChunk, P - j0), pm);
+        const int m = min(kProbeChunk, P - j0);
+        const int total = pm.before[m];
+        int j = 0;  // this wave's probe: before[j] <= its tile < before[j + 1]
+        for (int g0 = 0; g0 < total; g0 += kNW * kRound) {
+            for (int u = 0; u < kRound; ++u) {
+                const int g = g0 + u * kNW + wave;
+                if (g >= total) break;
+                while (pm.before[j + 1] <= g) ++j;
+                const int t = __builtin_amdgcn_readfirstlane(g - pm.before[j]);
+                const int tile = __builtin_amdgcn_readfirstlane(pm.tile0[j]) + t;
+                const bool valid = lane < pm.rows[j] - t * kTileRows;
+                const float4* tp = a.lists.codes + (size_t)tile * nquad * kWave + lane;
+                const uint32_t id = a.lists.ids[(size_t)tile * kWave + lane];
+                float acc = 0.0f;
+                bool keep = valid;
+                if constexpr (MODE == kScanPruned) {
+                    const float bound = fminf(tau_q, key_rank(thr));
+                    for (int b = 0; b < nblocks; ++b) {
+                        if (__ballot(keep) == 0) break;
+                        if (keep) {
+                            const int d0 = b * a.block_dims;
+                            const int d1 = b < nblocks - 1 ? d0 + a.block_dims : 4 * nquad;
+                            acc = accum_dims<METRIC>(acc, qs, tp, d0, d1);
+                            if (b < nblocks - 1 && acc > bound) {
+                                keep = false;
+                                my_skip += nblocks - 1 - b;
+                            }
                         }
                     }
-                }
-            } else {
-                if (valid) {
+                } else {
+                    if (valid) {
 #pragma unroll 8
-                    for (int jj = 0; jj < nquad; ++jj)
-                        acc = accum<METRIC>(acc, qs[jj], tp[(size_t)jj * kWave]);
+                        for (int jj = 0; jj < nquad; ++jj)
+                            acc = accum<METRIC>(acc, qs[jj], tp[(size_t)jj * kWave]);
+                    }
                 }
+                if (valid) my_cand++;
+                if (keep) top.offer(make_key(rank_of<METRIC>(acc), id), thr);
             }
-            if (valid) my_cand++;
-            if (keep) {
-                uint32_t id = a.lists.ids[(size_t)tile * kWave + lane];
-                top.offer(make_key(rank_of<METRIC>(acc), id), thr);
-            }
-            // advance this wave's cursor by kNW tiles
-            t += kNW;
-            while (j < P && t >= nt_j) {
-                t -= nt_j;
-                ++j;
-                nt_j = j < P ? probe_tiles(a, probes, j) : 0;
-            }
+            __syncthreads();
+            top.maybe_compact(a.k, kNT * kRound);
+            thr = top.thr;
         }
-        __syncthreads();
-        top.maybe_compact(a.k, kNT);
-        thr = top.thr;
+        __syncthreads();  // the map's last reads are done
     }
-    top.finish(a.k);
 
     if (a.stats) {
         if (my_cand) atomicAdd(&s_stats[0], my_cand);
@@ -197,16 +252,17 @@ __device__ void scan_one(const ScanArgs& a, const int qi) {
     }
 
     if constexpr (MODE == kScanWarmup) {
-        if (tid == 0) {
+        // only the k-th rank is wanted, of the keys kept so far
+        if (top.cnt > 1024) top.finish(a.k);
+        if (wave == 0) {
+            const int cnt = top.cnt;
             float v = sentinel<METRIC>();
-            if (top.cnt >= a.k) {
-                float rk = key_rank(top.buf[a.k - 1]);
-                v = dist_of_rank(METRIC, rk);
-            }
+            if (cnt >= a.k) v = dist_of_rank(METRIC, ord2f(wave_kth_rank(top.buf, cnt, a.k, lane)));
             if (a.tau_cap) v = fminf(v, a.tau_cap[qi]);
-            a.out_tau[qi] = v;
+            if (lane == 0) a.out_tau[qi] = v;
         }
     } else {
+        top.finish(a.k);
         const int cnt = top.cnt;
         for (int i = tid; i < a.k; i += kNT) {
             float dv = sentinel<METRIC>();
