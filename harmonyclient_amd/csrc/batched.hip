@@ -23,6 +23,7 @@
 // below its k-th distance, is rescanned by the exact per-query kernel.
 #include <algorithm>
 #include <climits>
+#include <cmath>
 #include <cstring>
 #include <type_traits>
 
@@ -1537,7 +1538,9 @@ struct SelArgs {
     const int32_t* qint;
     const float* qnorm;         // [nq] squared query norms (as the BF16 scan used them)
     const float* norms;         // [rows] squared row norms
-    float mcoef;                // BF16 margin coefficient (margin_coef)
+    float mcoef;                // margin of inexact keys: mcoef (||q||^2 + ||x||^2) + mabs
+    float mabs;
+    float qn_max;               // APPROX: a query whose norm is not below it is flagged for the exact rescan
     int exact_ok;               // BF16 keys exact for integer queries
     int i8;                     // the int8 scan ran when *all_int
     const uint32_t* all_int;
@@ -1597,7 +1600,7 @@ __device__ void select_one(const SelArgs& a, const int qi) {
             thr = top.thr;
         }
     } else {
-        // A BF16 key's distance v is within E = mcoef (||q||^2 + ||x||^2) of
+        // A key's rank v is within E = mcoef (||q||^2 + ||x||^2) + mabs of
         // the FP32 chain's (the margin the scan admitted the row with).
         // Pass 1: U = the k-th smallest upper bound v + E.  At least k rows
         // have chain distance <= U, so a row with v - E > U is beyond the
@@ -1611,7 +1614,7 @@ __device__ void select_one(const SelArgs& a, const int qi) {
                 ++real;
                 const uint32_t pos = (uint32_t)key;
                 const float sn = qn + a.norms[pos];
-                top.offer(make_key(__builtin_fmaf(a.mcoef, sn, key_rank(key)), pos), thr);
+                top.offer(make_key(key_rank(key) + __builtin_fmaf(a.mcoef, sn, a.mabs), pos), thr);
             }
             __syncthreads();
             top.maybe_compact(a.k, kNT);
@@ -1628,7 +1631,7 @@ __device__ void select_one(const SelArgs& a, const int qi) {
             if (key != kNoKey) {
                 const uint32_t pos = (uint32_t)key;
                 const float sn = qn + a.norms[pos];
-                if (__builtin_fmaf(-a.mcoef, sn, key_rank(key)) <= U) pend[atomicAdd(&s_np, 1u)] = pos;
+                if (key_rank(key) - __builtin_fmaf(a.mcoef, sn, a.mabs) <= U) pend[atomicAdd(&s_np, 1u)] = pos;
             }
             __syncthreads();
             const uint32_t c = s_np;  // < 2 kNT
@@ -1640,14 +1643,13 @@ __device__ void select_one(const SelArgs& a, const int qi) {
                         const uint32_t pos = pend[j];
                         const float4* tp = a.codes + (size_t)(pos / 64) * a.nquad * 64 + (pos % 64);
                         float acc = 0.0f;
-                        for (int jj = 0; jj < a.nquad; ++jj) {
-                            const float4 x = tp[(size_t)jj * 64];
-                            const float4 qq = qs[jj];
-                            float t;
-                            t = qq.x - x.x; acc = __builtin_fmaf(t, t, acc);
-                            t = qq.y - x.y; acc = __builtin_fmaf(t, t, acc);
-                            t = qq.z - x.z; acc = __builtin_fmaf(t, t, acc);
-                            t = qq.w - x.w; acc = __builtin_fmaf(t, t, acc);
+                        if (a.metric == kL2) {
+#pragma unroll 4
+                            for (int jj = 0; jj < a.nquad; ++jj) acc = accum<kL2>(acc, qs[jj], tp[(size_t)jj * 64]);
+                        } else {
+#pragma unroll 4
+                            for (int jj = 0; jj < a.nquad; ++jj) acc = accum<kIP>(acc, qs[jj], tp[(size_t)jj * 64]);
+                            acc = rank_of<kIP>(acc);
                         }
                         top.offer(make_key(acc, ids[pos]), thr);
                     }
@@ -1723,8 +1725,9 @@ __global__ __launch_bounds__(kNT) void select_kernel(SelArgs a) {
 // the top k), re-keys those candidates with their ids and sorts them in LDS.
 // The keys are read once per pass (they are in L2 from the scan).  The
 // result -- and the flags, rescan bounds and counts -- are those of
-// select_one.  Every other query (not exact, more than kSelSort candidates,
-// k above kSelSort / 2) goes to the workgroup form through hard[] / *nhard.
+// select_one.  Approximate keys take select_wave_inexact.  Every other query
+// (more than kSelSort candidates, k above kSelSort / 2, more than 1024
+// approximate keys) goes to the workgroup form through hard[] / *nhard.
 constexpr int kSelSort = 512;   // candidates one wave sorts in LDS
 constexpr int kSelThin = 128;   // more admissible keys than this (and k): thinned by the histograms first
 
@@ -1915,6 +1918,145 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
     }
 }
 
+// The wave form for keys that hold approximate ranks (at most 64
+// kSelRegSlots survivors, k <= kSelSort / 2): U, an upper bound of the k-th
+// smallest upper bound v + E, is the upper edge of its bin in a 1024-bin
+// histogram (widened past the binning's rounding); every survivor with
+// v - E <= U can be among the top k and is rescored with the exact chain, a
+// candidate per lane, the query's components as scalar operands.  The
+// workgroup form reads all survivors twice and compacts them with LDS sorts.
+template <int METRIC>
+__device__ float chain_of(const float4* q, const float4* tp, int nquad) {
+    typedef const __attribute__((address_space(4))) float4* UniformQuads;
+    const UniformQuads qu = (UniformQuads)q;
+    float acc = 0.0f;
+#pragma unroll 8
+    for (int j = 0; j < nquad; ++j) {
+        const float4 qv = {qu[j].x, qu[j].y, qu[j].z, qu[j].w};
+        acc = accum<METRIC>(acc, qv, tp[(size_t)j * 64]);
+    }
+    return rank_of<METRIC>(acc);
+}
+
+__device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool overflow, uint64_t* kk, int lane,
+                                    int32_t* hard, uint32_t* nhard, float tau, bool ids8,
+                                    uint64_t (&kr)[kSelRegSlots]) {
+    const uint64_t* sb = a.sbuf + (size_t)qi * a.cap;
+    float xn[kSelRegSlots];
+#pragma unroll
+    for (int t = kSelSpecSlots; t < kSelRegSlots; ++t) {
+        const uint32_t i = (uint32_t)t * 64 + lane;
+        if ((uint32_t)t * 64 < n) kr[t] = sb[i < n ? i : 0];
+    }
+#pragma unroll
+    for (int t = 0; t < kSelRegSlots; ++t) {
+        const uint32_t i = (uint32_t)t * 64 + lane;
+        if (i >= n) kr[t] = kNoKey;
+        if ((uint32_t)t * 64 < n) xn[t] = a.norms[kr[t] != kNoKey ? (uint32_t)kr[t] : 0u];
+    }
+    const float qn = a.qnorm[qi];
+    float mn = INFINITY, mx = -INFINITY;
+    uint32_t fin = 0, real = 0;
+    auto each = [&](auto&& f) {  // f(slot, v, E) over this lane's survivors
+#pragma unroll
+        for (int t = 0; t < kSelRegSlots; ++t)
+            if ((uint32_t)t * 64 < n && kr[t] != kNoKey)
+                f(t, key_rank(kr[t]), __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs));
+    };
+    each([&](int, float v, float e) {
+        const float u = v + e;
+        ++real;
+        if (u < FLT_MAX) {
+            mn = fminf(mn, u);
+            mx = fmaxf(mx, u);
+            ++fin;
+        }
+    });
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    for (int off = 32; off > 0; off >>= 1) {
+        fin += __shfl_xor(fin, off);
+        real += __shfl_xor(real, off);
+    }
+    float U = INFINITY;  // fewer than k: every survivor is a candidate
+    if (fin >= (uint32_t)a.k) {
+        uint32_t* h1k = reinterpret_cast<uint32_t*>(kk);
+        wave_clear1024(h1k, lane);
+        __builtin_amdgcn_wave_barrier();
+        const float w = (mx - mn) * (1.0f / 1024.0f);
+        const float inv = w > 0.0f ? 1.0f / w : 0.0f;
+        each([&](int, float v, float e) {
+            if (v + e < FLT_MAX) atomicAdd(&h1k[lin_bin1024(v + e, mn, inv)], 1u);
+        });
+        __builtin_amdgcn_wave_barrier();
+        const int b = wave_find_bin1024(h1k, (uint32_t)a.k, lane);
+        float edge = mx;
+        if (inv > 0.0f && b < 1023) edge = mn + (float)(b + 1) * w;
+        U = fminf(mx, edge + 0x1p-16f * (fabsf(mn) + fabsf(mx) + w));
+        __builtin_amdgcn_wave_barrier();  // the histogram's reads are done before the compaction's writes
+    }
+    // the candidates' rows (ballot compaction)
+    uint32_t* cid = reinterpret_cast<uint32_t*>(kk);
+    uint32_t nc = 0;
+#pragma unroll
+    for (int t = 0; t < kSelRegSlots; ++t) {
+        if ((uint32_t)t * 64 >= n) continue;
+        const bool take = kr[t] != kNoKey && !(key_rank(kr[t]) - __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs) > U);
+        const uint64_t mk = __ballot(take);
+        const uint32_t pos = nc + lanes_below(mk);
+        nc += (uint32_t)__popcll(mk);
+        if (take && pos < (uint32_t)kSelSort) cid[pos] = (uint32_t)kr[t];
+    }
+    if (nc > (uint32_t)kSelSort) {
+        if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
+        return;
+    }
+    if (lane == 0) a.scnt[qi] = 0;  // read by every lane at the start
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t* ids = ids8 ? a.ids8 : a.ids;
+    uint32_t n2 = 64;
+    while (n2 < nc) n2 <<= 1;
+    // groups of 64 from the last: a group's keys overwrite only rows of
+    // groups already read
+    for (int g = (int)(n2 / 64) - 1; g >= 0; --g) {
+        const uint32_t i = (uint32_t)g * 64 + lane;
+        const bool on = i < nc;
+        const uint32_t pos = on ? cid[i] : 0u;
+        __builtin_amdgcn_wave_barrier();
+        uint64_t key = ~0ull;
+        if (on) {
+            const uint32_t id = ids[pos];
+            const float4* tp = a.codes + (size_t)(pos / 64) * a.nquad * 64 + (pos % 64);
+            const float4* q = a.q + (size_t)qi * a.nquad;
+            const float r = a.metric == kL2 ? chain_of<kL2>(q, tp, a.nquad) : chain_of<kIP>(q, tp, a.nquad);
+            if (r < FLT_MAX) key = make_key(r, id);  // the heap's strict admission
+        }
+        kk[i] = key;
+        __builtin_amdgcn_wave_barrier();
+    }
+    wave_sort(kk, n2, lane);
+    if (lane == 0 && a.stats) atomicAdd(&a.stats[3], (unsigned long long)real);
+    const uint64_t kth = (uint32_t)a.k <= n2 ? kk[a.k - 1] : ~0ull;
+    const bool full = kth < key_limit();
+    if (overflow || (a.check_tau && !(full && key_rank(kth) <= tau))) {
+        if (lane == 0) {
+            a.fallback[qi] = 1;
+            a.rescan_tau[qi] = full ? key_rank(kth) : FLT_MAX;
+            a.flist[atomicAdd(a.fcount, 1u)] = qi;
+            if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
+            if (a.stats && overflow && a.fb_slot == 4) atomicAdd(&a.stats[6], 1ull);  // first pass
+        }
+        return;
+    }
+    for (int i = lane; i < a.k; i += 64) {
+        const uint64_t key = (uint32_t)i < n2 ? kk[i] : ~0ull;
+        const bool ok = key < key_limit();
+        a.out_d[(size_t)qi * a.k + i] = ok ? dist_of_rank(a.metric, key_rank(key)) : a.metric == kL2 ? FLT_MAX : -FLT_MAX;
+        a.out_i[(size_t)qi * a.k + i] = ok ? (int64_t)(uint32_t)key : -1;
+    }
+}
+
+template <bool APPROX>
 __device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t* kk, int lane, int32_t* hard,
                                 uint32_t* nhard) {
     // everything the selection reads first, loaded together: the count,
@@ -1932,18 +2074,32 @@ __device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t
     const uint32_t n = overflow ? a.cap : total;
     const bool ids8 = a.i8 && all_int;
     const bool exact = a.keys_exact || ids8 || (a.exact_ok && qint);
-    if (!exact || a.k > kSelSort / 2) {
+    if (APPROX && !(a.qnorm[qi] < a.qn_max)) {  // (NaN too)
+        if (lane == 0) {
+            a.fallback[qi] = 1;
+            a.rescan_tau[qi] = FLT_MAX;
+            a.flist[atomicAdd(a.fcount, 1u)] = qi;
+        }
+        return;
+    }
+    if (a.k > kSelSort / 2 || (!exact && !(APPROX && n <= 64u * kSelRegSlots))) {
         if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
         return;
     }
-    if (n <= 64u * kSelRegSlots)
+    if (APPROX && !exact)
+        select_wave_inexact(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
+    else if (n <= 64u * kSelRegSlots)
         select_wave_one<true>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
     else
         select_wave_one<false>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
 }
 
 // One wave per query: all queries (nq, or those flagged in `active`), or a
-// walk over the query list.
+// walk over the query list.  APPROX: approximate keys are selected here too
+// (those of the split scans, whose error bound leaves little more than k to
+// rescore; the BF16 shadow's leaves most survivors, which the workgroup form
+// rescores faster: 2000 queries of 420 dims 0.29 ms against 0.41).
+template <bool APPROX>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void select_wave_kernel(SelArgs a, int nq, int32_t* hard, uint32_t* nhard) {
     constexpr int kW = kNT / 64;
     __shared__ uint32_t hist[kW][256];
@@ -1955,13 +2111,13 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
         const uint32_t nl = *a.qcount;
         for (uint32_t w = blockIdx.x * kW + wv; w < nl; w += gridDim.x * kW) {
             __builtin_amdgcn_wave_barrier();  // the previous query's LDS reads are done
-            select_wave_any(a, a.qlist[w], hist[wv], keys[wv], lane, hard, nhard);
+            select_wave_any<APPROX>(a, __builtin_amdgcn_readfirstlane(a.qlist[w]), hist[wv], keys[wv], lane, hard, nhard);
         }
         return;
     }
-    const int qi = blockIdx.x * kW + wv;
+    const int qi = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kW + wv);
     if (qi >= nq || (a.active && !a.active[qi])) return;
-    select_wave_any(a, qi, hist[wv], keys[wv], lane, hard, nhard);
+    select_wave_any<APPROX>(a, qi, hist[wv], keys[wv], lane, hard, nhard);
 }
 
 
@@ -2180,6 +2336,7 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 }  // namespace hivf
 
 #include "flat.hpp"
+#include "split.hpp"
 
 namespace hivf {
 
@@ -2437,6 +2594,8 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.qnorm = qnorm;
         sa.norms = h->d_norms.p;
         sa.mcoef = margin_coef(h->d);
+        sa.mabs = 0.0f;
+        sa.qn_max = INFINITY;
         sa.exact_ok = exact_bf16;
         sa.i8 = i8;
         sa.all_int = all_int;
@@ -2462,7 +2621,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.nlist = (int)nlist;
         uint32_t* nhard = fbc + (first ? 2 : 3);
         const int64_t wgs = (n + 3) / 4;
-        hipLaunchKernelGGL(select_wave_kernel, dim3((unsigned)(qlist ? std::min<int64_t>(wgs, 1024) : wgs)),
+        hipLaunchKernelGGL(select_wave_kernel<false>, dim3((unsigned)(qlist ? std::min<int64_t>(wgs, 1024) : wgs)),
                            dim3(kNT), 0, s, sa, (int)n, shard, nhard);
         sa.active = nullptr;
         sa.qlist = shard;
@@ -2688,13 +2847,19 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 static bool flat_pays(int64_t n, int P, double tiles_per_list) {
     return P * tiles_per_list >= 12.0 || (double)n * P * tiles_per_list >= 90.0;
 }
-// Whether its queries share lists enough for the list-major form (else a
-// workgroup per query and list): 6 per list and tiles enough to fill the
-// chip.  1024 queries of 32 lists in 1024 (1.5 tiles each) 233 us against 292,
-// 512 of them 221 against 181; 256 queries of 20 lists in 400 (7.8 tiles) 270
-// against 401, 64 of them 238 against 182.
-static bool flat_shared(int64_t n, int P, int64_t nlist, double tiles_per_list) {
-    return n * P >= 6 * nlist && (double)n * P * tiles_per_list >= 40000.0;
+// Whether its queries share lists enough for a list-major form (else a
+// workgroup per query and list, which reads every pair's rows through the
+// caches).  The split scan and its plan repay themselves from about 500 MB of
+// such reads on: 256 queries of 16 lists in 512 (6.1 tiles, 128 dims) 148 us
+// against 179, 128 of them 141 against 127; 512 of 32 lists in 1024 (1.5 tiles,
+// 96 dims) 153 against 166, 256 of them 151 against 119; past 128 dims from 1 GB:
+// 128 of 20 lists (7.8 tiles, 201 dims) 245 against 255, 64 of them 243 against
+// 178.  The FP32 scan from about 40,000 tiles: 256 queries of 20 lists 270
+// against 401, 512 of 32 lists of 1.5 tiles 221 against 181.
+static bool flat_shared(int64_t n, int P, int64_t nlist, double tiles_per_list, int64_t d, bool split) {
+    const double pair_tiles = (double)n * P * tiles_per_list;
+    if (!split) return n * P >= 6 * nlist && pair_tiles >= 40000.0;
+    return n * P >= 2 * nlist && pair_tiles * (double)d >= (d <= 128 ? 2.2e6 : 4.0e6);
 }
 
 // Batches of plain and pruned searches by the exact FP32 scans (flat.hpp).
@@ -2712,18 +2877,32 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     }
     const double tiles_per_list = (double)h->tiles / (double)nlist;
     if (!flat_pays(n, P, tiles_per_list)) return HIVF_EUNSUPPORTED;
-    const bool shared = flat_shared(n, P, nlist, tiles_per_list);
+    const int nkc = (int)((h->d + 15) / 16);
+    const bool small_d = nkc <= 8;
+    // the split scan, unless norms could overflow its ranks or the caller
+    // wants the pruning's statistics, which the FP32 scan counts
+    const bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
+    const bool shared = flat_shared(n, P, nlist, tiles_per_list, h->d, can_split);
+    const bool split = shared && can_split;
+    const uint32_t qc = split ? kSplitItem : kFlatItem;
+    // (fewer tiles per item do not pay even where the items are few: 256
+    // queries of 16 lists 157 us at 2 tiles, 148 at 8)
+    const uint32_t rt = !split ? kFlatTiles : small_d ? kSplitTiles : kSplitWgTiles;
     // survivors kept per query (a query with more is rescanned by the
     // per-query kernel), and the queries of a chunk, so that their buffers
     // stay within 512 MB
-    const uint32_t cap = (uint32_t)std::max<int64_t>(8192, 16 * k);
+    const uint32_t cap = (uint32_t)std::max<int64_t>(16384, 16 * k);
     const int64_t chunk = std::min<int64_t>(n, ((int64_t)64 << 20) / cap);
     int64_t max_t32 = 1;
     for (int64_t l = 0; l < nlist; ++l)
         max_t32 = std::max<int64_t>(max_t32, 2 * (h->tile_off[l + 1] - h->tile_off[l]));
-    const int64_t rtn = near_tiles(kFlatTiles);
-    const int64_t max_items = shared ? (chunk * P / kFlatItem + nlist) * ((max_t32 + rtn - 1) / rtn) : 0;
+    const int64_t rtn = near_tiles(rt);
+    const int64_t max_items = shared ? (chunk * P / qc + nlist) * ((max_t32 + rtn - 1) / rtn) : 0;
     if (chunk * P >= INT32_MAX || max_items >= INT32_MAX) return HIVF_EUNSUPPORTED;
+    if (split && P == 1) {  // (otherwise the coarse step split the queries)
+        const int rc = split_queries(h, q, n, s, nullptr);
+        if (rc) return rc;
+    }
     size_t off = 0;
     auto take = [&](size_t bytes) {
         size_t o = off;
@@ -2761,10 +2940,13 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
                       (uint32_t*)at(o_hwg), (uint32_t*)at(o_ioff), (uint32_t*)at(o_lnear), (uint32_t*)at(o_meta),
                       (int32_t*)at(o_lq), (float*)at(o_lqd), (BatchItem*)at(o_items), max_items};
     // the warm-up's lists: enough that they hold twice k rows at the mean list
-    // size, and no fewer than asked for
+    // size, and no fewer than asked for; k rows of each (a whole tile at
+    // least).  Fewer lists with more rows bound most queries better and a few
+    // much worse: 1000 queries (k 100) keep 617 rows on average and 5.4 k at
+    // most from 10 x 100, 398 and 13 k from 3 x 300
     const double mean_rows = std::max(1.0, (double)h->ntotal / (double)nlist);
     const int warm_lists = (int)std::min<double>(std::max({10.0, (double)p.warmup_lists, 2.0 * (double)k / mean_rows}), 1024.0);
-    const int warm_rows = (int)std::max<int64_t>(k, p.warmup_list_size);
+    const int warm_rows = (int)std::max<int64_t>({k, (int64_t)p.warmup_list_size, (int64_t)kTileRows});
     for (int64_t q0 = 0; q0 < n; q0 += chunk) {
         const int64_t m = std::min(chunk, n - q0);
         const int32_t* probes = h->d_probes.p + q0 * P;
@@ -2799,10 +2981,33 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         a.rows_scanned = stats;
         a.skips = pruned && stats ? stats + 2 : nullptr;
         const bool l2 = h->metric == HIVF_METRIC_L2;
+        CoarseState& C = h->coarse;
+        const int64_t dpad16 = (int64_t)nkc * 16;
         if (shared) {
             PairFilter pf{};  // (no radius intervals here: every pair is scanned)
             HIP_TRY(h, launch_plan(pl, probes, h->d_cd.p + q0 * P, h->d_size.p, PairSet{npqc, nullptr, nullptr, nullptr, (int)m, P},
-                                   pf, kFlatItem, kFlatTiles, fb, 0, all_int, stats, s));
+                                   pf, qc, rt, fb, 0, all_int, stats, s));
+        }
+        if (split) {
+            SplitArgs b;
+            b.lists = a.lists;
+            b.norms = h->d_norms.p;
+            b.qh = C.qh.p + q0 * dpad16;
+            b.ql = C.ql.p + q0 * dpad16;
+            b.qn = C.qn.p + q0;
+            b.tau = tau;
+            b.items = pl.items;
+            b.meta = pl.meta;
+            b.lq = pl.lq;
+            b.max_items = (uint32_t)max_items;
+            b.scnt = scnt;
+            b.sbuf = a.sbuf;
+            b.cap = cap;
+            b.nkc = nkc;
+            b.dpad16 = (int)dpad16;
+            b.coef = split_coef(h->d);
+            launch_split(b, l2, !h->lists_uint8, h->cus, s);
+        } else if (shared) {
             a.items = pl.items;
             a.meta = pl.meta;
             a.lq = pl.lq;
@@ -2825,9 +3030,17 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         sa.scnt = scnt;
         sa.sbuf = a.sbuf;
         sa.cap = cap;
-        sa.qint = fb;  // (read, not used: every key is exact)
+        sa.qint = split ? C.qint.p + q0 : fb;  // (fb: read, not used)
         sa.all_int = all_int;
-        sa.keys_exact = 1;
+        // (the FP32 scans' keys are final; the split scan's are where every
+        // product and sum is an integer below 2^24)
+        sa.keys_exact = split ? 0 : 1;
+        sa.exact_ok = h->lists_uint8 && h->d <= 129 ? 1 : 0;
+        sa.qnorm = C.qn.p + q0;
+        sa.norms = h->d_norms.p;
+        sa.mcoef = split_coef(h->d);
+        sa.mabs = kSplitAbs;
+        sa.qn_max = 1e37f;
         sa.tau = tau;
         sa.ids = h->d_ids.p;
         sa.codes = h->d_codes.p;
@@ -2844,10 +3057,13 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         sa.lcnt = lcnt;
         sa.nlist = 0;  // (cleared with the chunk's counters)
         int32_t* hard = (int32_t*)at(o_hard);
-        hipLaunchKernelGGL(select_wave_kernel, dim3((unsigned)((m + 3) / 4)), dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
+        const dim3 sgrid((unsigned)((m + 3) / 4));
+        if (split) hipLaunchKernelGGL(select_wave_kernel<true>, sgrid, dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
+        else hipLaunchKernelGGL(select_wave_kernel<false>, sgrid, dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
         sa.qlist = hard;
         sa.qcount = fbc + 2;
-        hipLaunchKernelGGL(select_kernel, dim3((unsigned)std::min<int64_t>(m, 1024)), dim3(kNT), 0, s, sa);
+        hipLaunchKernelGGL(select_kernel, dim3((unsigned)std::min<int64_t>(m, 1024)), dim3(kNT),
+                           split ? h->nquad * sizeof(float4) : 0, s, sa);
         HIP_TRY(h, hipGetLastError());
         // survivors past the buffer: the query's lists scanned by the per-query kernel
         ScanArgs f = w;

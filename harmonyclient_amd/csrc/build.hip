@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void fill_arena_kernel(const float4* __restric
                                                          const int32_t* __restrict__ tile_off,
                                                          const int32_t* __restrict__ tile_list, int64_t tiles,
                                                          float4* __restrict__ codes, uint32_t* __restrict__ ids,
-                                                         float* __restrict__ norms, uint32_t* __restrict__ not_u8) {
+                                                         float* __restrict__ norms, uint32_t* __restrict__ flags) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g >= tiles * kTileRows) return;
     const int64_t T = g / kTileRows;
@@ -326,8 +326,11 @@ __global__ __launch_bounds__(256) void fill_arena_kernel(const float4* __restric
         }
     }
     ids[g] = (uint32_t)row;
-    norms[g] = (float)s;
-    if (!u8) atomicOr(not_u8, 1u);
+    const float nr = (float)s;
+    norms[g] = nr;
+    // bit 0: a value that is no integer in [0, 255]; bit 1: a norm past 1e37
+    const uint32_t f = (u8 ? 0u : 1u) | (nr < 1e37f ? 0u : 2u);
+    if (f) atomicOr(flags, f);
 }
 
 // Row i divided by its norm (the FP32 FMA chain over the d dims, then a
@@ -585,7 +588,7 @@ int gpu_add(hivf_index* h, int64_t n) {
     HIP_TRY(h, hipMemcpyAsync(h->d_tile_off.p, tile_off.data(), (nlist + 1) * sizeof(int32_t), hipMemcpyHostToDevice,
                               s));
     HIP_TRY(h, hipMemcpyAsync(h->d_size.p, size.data(), nlist * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    uint32_t not_u8 = 0;
+    uint32_t flags = 0;
     if (tiles > 0) {
         DevBuf<int32_t> dtl;
         DevBuf<uint32_t> flag;
@@ -597,10 +600,11 @@ int gpu_add(hivf_index* h, int64_t n) {
                            nquad, (int)h->d, G.order, G.off.p, h->d_tile_off.p, dtl.p, tiles, h->d_codes.p,
                            h->d_ids.p, h->d_norms.p, flag.p);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, hipMemcpyAsync(&not_u8, flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipMemcpyAsync(&flags, flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     }
     HIP_TRY(h, hipStreamSynchronize(s));  // host vectors and local buffers
-    h->lists_uint8 = not_u8 == 0;
+    h->lists_uint8 = (flags & 1u) == 0;
+    h->lists_sane = (flags & 2u) == 0;
     h->list_off = list_off;
     h->tile_off = tile_off;
     h->ntotal = list_off[nlist];

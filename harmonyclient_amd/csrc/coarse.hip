@@ -75,18 +75,21 @@ __global__ void cent_split_kernel(const float4* __restrict__ cent, int nquad, in
 // Per query (one wave): qh = bf16(q), ql = bf16(q - qh), row-major
 // [n x dpad16], and the squared norm accumulated in FP64.
 __global__ void coarse_prep_kernel(const float* __restrict__ q, int d, int ld, int dpad16, uint16_t* __restrict__ qh,
-                                   uint16_t* __restrict__ ql, float* __restrict__ qn, PrepArgs pa, int with_prep) {
+                                   uint16_t* __restrict__ ql, float* __restrict__ qn, int32_t* __restrict__ qint, PrepArgs pa,
+                                   int with_prep) {
     const int64_t qi = blockIdx.x;
     const int lane = threadIdx.x;
     float qv[kQRegs];  // (one round of loads for both preparations)
     query_regs(q, qi, ld, d, lane, qv);
     if (with_prep) prep_query(pa, (int)qi, lane, qv);
     double s = 0.0;
+    int ok = 1;
     auto one = [&](int c, float v) {
         const uint16_t h = f2bf(v);
         qh[qi * dpad16 + c] = h;
         ql[qi * dpad16 + c] = f2bf(v - bf2f(h));
         s += (double)v * (double)v;
+        ok &= (v == rintf(v)) && v >= 0.0f && v <= 255.0f;
     };
     if (dpad16 <= 64 * kQRegs) {
 #pragma unroll
@@ -96,7 +99,11 @@ __global__ void coarse_prep_kernel(const float* __restrict__ q, int d, int ld, i
         for (int c = lane; c < dpad16; c += 64) one(c, c < d ? q[qi * ld + c] : 0.0f);
     }
     for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off);
-    if (lane == 0) qn[qi] = (float)s;
+    const bool all = __ballot(!ok) == 0;
+    if (lane == 0) {
+        qn[qi] = (float)s;
+        qint[qi] = all ? 1 : 0;
+    }
 }
 
 struct CoarseDotArgs {
@@ -965,6 +972,20 @@ static int ensure_cent_shadow(hivf_index* h, hipStream_t s) {
     return HIVF_OK;
 }
 
+int split_queries(hivf_index* h, const float4* q, int64_t n, hipStream_t s, const PrepArgs* prep) {
+    CoarseState& C = h->coarse;
+    const int64_t dpad16 = (h->d + 15) / 16 * 16;
+    HIP_TRY(h, C.qh.ensure((size_t)n * dpad16));
+    HIP_TRY(h, C.ql.ensure((size_t)n * dpad16));
+    HIP_TRY(h, C.qn.ensure((size_t)n));
+    HIP_TRY(h, C.qint.ensure((size_t)n));
+    hipLaunchKernelGGL(coarse_prep_kernel, dim3((unsigned)n), dim3(64), 0, s, reinterpret_cast<const float*>(q),
+                       (int)h->d, (int)h->d_pad, (int)dpad16, C.qh.p, C.ql.p, C.qn.p, C.qint.p,
+                       prep ? *prep : PrepArgs{}, prep ? 1 : 0);
+    HIP_TRY(h, hipGetLastError());
+    return HIVF_OK;
+}
+
 int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStream_t s) {
     CoarseState& C = h->coarse;
     HIP_TRY(h, h->d_cd.ensure((size_t)n));
@@ -1039,17 +1060,15 @@ int run_coarse_mfma(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStr
     const int rc = ensure_cent_shadow(h, s);
     if (rc) return rc;
     const int64_t chunk = std::max<int64_t>(32, std::min<int64_t>((n + 31) / 32 * 32, kMaxRankFloats / ldo / 32 * 32));
-    HIP_TRY(h, C.qh.ensure((size_t)n * dpad16));
-    HIP_TRY(h, C.ql.ensure((size_t)n * dpad16));
-    HIP_TRY(h, C.qn.ensure((size_t)n));
     HIP_TRY(h, C.rank.ensure((size_t)chunk * ldo));
     HIP_TRY(h, C.hard.ensure((size_t)chunk));
     HIP_TRY(h, C.nhard.ensure(1));
     HIP_TRY(h, h->d_cd.ensure((size_t)n * P));
     HIP_TRY(h, h->d_probes.ensure((size_t)n * P));
-    hipLaunchKernelGGL(coarse_prep_kernel, dim3((unsigned)n), dim3(64), 0, s, reinterpret_cast<const float*>(q),
-                       (int)h->d, (int)h->d_pad, (int)dpad16, C.qh.p, C.ql.p, C.qn.p, prep ? *prep : PrepArgs{},
-                       prep ? 1 : 0);
+    {
+        const int rc2 = split_queries(h, q, n, s, prep);
+        if (rc2) return rc2;
+    }
     const float coef = coarse_coef(h->d);
     const int groups = (int)((tiles32 + kTilesPerTask - 1) / kTilesPerTask);
     for (int64_t q0 = 0; q0 < n; q0 += chunk) {

@@ -28,6 +28,7 @@ __host__ __device__ inline uint32_t f2ord(float f) {
     uint32_t u;
     __builtin_memcpy(&u, &f, 4);
 #endif
+    if (f != f) u = 0x7FC00000u;  // NaN ranks last whatever its sign (a subtraction may flip it)
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 

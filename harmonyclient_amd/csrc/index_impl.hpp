@@ -81,6 +81,7 @@ struct CoarseState {
     DevBuf<uint16_t> cbf;
     DevBuf<uint16_t> qh, ql;
     DevBuf<float> qn, rank;
+    DevBuf<int32_t> qint;   // the query holds integers in [0, 255]
     DevBuf<int32_t> hard;   // queries the one-wave pick hands to the workgroup pick
     DevBuf<uint32_t> nhard;
 };
@@ -102,6 +103,7 @@ struct hivf_index {
     bool have_centroids = false;
     bool have_lists = false;
     bool lists_uint8 = false;  // every list value is an integer in [0, 255]
+    bool lists_sane = false;   // every row's squared norm is below 1e37
 
     // list arena (device) and its host-side shape
     std::vector<int64_t> list_off;  // [nlist + 1] rows
@@ -236,6 +238,9 @@ struct PrepArgs;  // prep.hpp
 // prep, its query-preparation launch also runs the batched search's.
 int run_coarse_mfma(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStream_t s,
                     const PrepArgs* prep = nullptr);
+// The BF16 pieces, norms and integer flags of n staged queries, into the
+// coarse state (coarse.hip); with prep, the batched search's preparation too.
+int split_queries(hivf_index* h, const float4* q, int64_t n, hipStream_t s, const PrepArgs* prep);
 // Top-P centroids of n staged queries (hivf_api.cpp): the MFMA form, or the
 // per-query kernel for P = 1 and d > 512.
 int run_coarse(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStream_t s,

@@ -1,5 +1,5 @@
-"""Plain and pruned searches of a batch (the exact FP32 scans with their bound,
-plan and selection) against the oracle, over the forms those searches accept:
+"""Plain and pruned searches of a batch (the exact FP32 scans and the split
+MFMA scan, with their bound, plan and selection) against the oracle, over the forms those searches accept:
 both metrics, odd dimensions, a query alone and queries that share lists,
 per-query probe counts, k past the candidates, rows with many equal distances
 (more survivors than a query's buffer holds), empty lists.  Ids and distances
@@ -69,6 +69,56 @@ def test_plain_batches(kind, rows, d, nlist, metric, n, P, k):
                 nb = -(-d // min(blk, d)) if blk else (4 if d >= 4 else 1)
                 assert st.candidates == ost.candidates and st.blocks_total == nb * st.candidates
                 assert 0 <= st.blocks_skipped <= (nb - 1) * st.candidates
+
+
+@pytest.mark.parametrize("kind,rows,d,nlist,metric,n,P,k", [
+    # sizes of the split scan: a wave's 64 and 128 dims, its last whole and
+    # partial chunks, the workgroup form with odd and even chunk groups
+    ("int", 30000, 64, 16, 1, 2500, 12, 20), ("real", 30000, 65, 16, 1, 2500, 12, 20), ("real", 30000, 113, 16, 1, 1300, 16, 130),
+    ("unit", 30000, 128, 16, 0, 1300, 16, 50), ("int", 30000, 129, 16, 1, 1300, 16, 10), ("real", 16000, 240, 12, 1, 1600, 12, 256),
+    ("unit", 12000, 300, 12, 0, 2000, 12, 30), ("real", 9000, 512, 12, 1, 1900, 12, 100), ("int", 20000, 250, 9, 0, 1500, 9, 7),
+    ("dup", 33000, 130, 7, 1, 1100, 7, 12), ("dup", 33000, 40, 7, 0, 4100, 7, 300), ("int", 150, 128, 3, 1, 60000, 3, 4),
+])
+def test_split_batches_device(kind, rows, d, nlist, metric, n, P, k):
+    """The device entry point without statistics (plain, and pruned for L2)."""
+    import torch
+    print(f"[case] split {kind} rows={rows} d={d} nlist={nlist} metric={metric} n={n} P={P} k={k}", flush=True)
+    idx, ix = _index(kind, rows, d, nlist, metric)
+    xq = _data(kind, n, d, max(nlist // 2, 1), 78)
+    OD, OI, _ = ix.search(xq, P, k)
+    q = torch.from_numpy(xq).cuda()
+    for algo in (hx.ALGO_PLAIN, hx.ALGO_PRUNED)[:1 + metric]:
+        D = torch.full((n, k), -7.0, device="cuda")
+        I = torch.full((n, k), -7, dtype=torch.int64, device="cuda")
+        torch.cuda.synchronize()
+        idx.search_device(n, q.data_ptr(), k, D.data_ptr(), I.data_ptr(), hx.make_params(nprobe=P, algo=algo), stats=False)
+        torch.cuda.synchronize()
+        _same(D.cpu().numpy(), I.cpu().numpy(), OD, OI)
+
+
+def test_split_margin_and_non_finite_queries():
+    """Rows whose distances differ by less than the split ranks resolve (large
+    common offset), queries with inf, NaN and overflowing norms among them."""
+    import torch
+    print("[case] split: offset 4096 +- 1e-2, non-finite queries", flush=True)
+    r = np.random.default_rng(5)
+    rows, d, n, P, k = 30000, 100, 2000, 12, 40
+    xb = (4096.0 + 1e-2 * r.normal(0, 1, (rows, d))).astype(np.float32)
+    cent = xb[:16].copy()
+    ix = oracle.Index.build(1, xb, cent)
+    idx = hx.Index(d, 16, 1)
+    idx.set_centroids(cent)
+    idx.add(rows, xb)
+    xq = (4096.0 + 1e-2 * r.normal(0, 1, (n, d))).astype(np.float32)
+    xq[3, 5], xq[70, 0], xq[71] = np.nan, np.inf, 1e19
+    OD, OI, _ = ix.search(xq, P, k)
+    q = torch.from_numpy(xq).cuda()
+    D = torch.empty(n, k, device="cuda")
+    I = torch.empty(n, k, dtype=torch.int64, device="cuda")
+    torch.cuda.synchronize()
+    idx.search_device(n, q.data_ptr(), k, D.data_ptr(), I.data_ptr(), hx.make_params(nprobe=P), stats=False)
+    torch.cuda.synchronize()
+    _same(D.cpu().numpy(), I.cpu().numpy(), OD, OI)
 
 
 @pytest.mark.parametrize("metric", [1, 0])
