@@ -14,7 +14,9 @@
 //     every product, sum and norm is an integer below 2^24, so the MFMA
 //     distance is the exact distance, bit-identical to the FP32 FMA chain;
 //   - otherwise a row survives when  dist - E <= tau  with E a proven bound
-//     of the BF16 error (margin_coef below), and the survivors that can
+//     of the shadow's error (margin_coef below; real-valued lists are kept in
+//     FP16 at a power-of-two scale, an eighth of BF16's rounding: 250k x 420,
+//     2000 queries at nprobe 50: 290 us of selection became 240), and the survivors that can
 //     reach the top-k (lower bound <= the k-th smallest upper bound) are
 //     rescored with the exact FP32 FMA chain from the original vectors.
 // Every row of the true top-k has exact distance <= D_k <= tau, so it
@@ -44,14 +46,20 @@ constexpr int kNT = 256;
 
 
 
-// BF16 shadow of the FP32 tile arena in MFMA operand order:
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
+
+__device__ inline uint16_t f2h(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }  // RNE
+
+// 16-bit shadow of the FP32 tile arena in MFMA operand order: FP16 of the
+// scaled values (f16_scale > 0, real-valued lists), else BF16:
 // [32-row tile T][16-dim chunk kc][lane][8 bf16], lane l holding row l % 32,
 // dims kc*16 + (l / 32) * 8 .. +7; `stride` chunks per tile.  With `aug`, the
 // extra chunk kc = nkc of a row holds [n_hi, n_mid, n_lo, 1, 1, 1, 0, 0] in
 // its first half (n = the row's squared norm split by split3) and zeros in
 // the second, so one more MFMA adds ||x||^2 + ||q||^2 to -2 q.x.
 __global__ void build_bf16_kernel(const float4* __restrict__ codes, const float* __restrict__ norms, int nquad,
-                                  int64_t tiles32, int nkc, int stride, uint16_t* __restrict__ out) {
+                                  int64_t tiles32, int nkc, int stride, float f16_scale,
+                                  uint16_t* __restrict__ out) {
     int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid >= tiles32 * stride * 64) return;
     int lane = (int)(gid % 64);
@@ -65,10 +73,8 @@ __global__ void build_bf16_kernel(const float4* __restrict__ codes, const float*
         for (int h = 0; h < 2; ++h) {
             int qd = c0 / 4 + h;
             float4 f = qd < nquad ? codes[(t64 * nquad + qd) * 64 + r64] : make_float4(0.f, 0.f, 0.f, 0.f);
-            v[h * 4 + 0] = f2bf(f.x);
-            v[h * 4 + 1] = f2bf(f.y);
-            v[h * 4 + 2] = f2bf(f.z);
-            v[h * 4 + 3] = f2bf(f.w);
+            const float e[4] = {f.x, f.y, f.z, f.w};
+            for (int i = 0; i < 4; ++i) v[h * 4 + i] = f16_scale > 0.0f ? f2h(e[i] * f16_scale) : f2bf(e[i]);
         }
     } else if (lane < 32) {
         split3(norms[T * 32 + lane], v);
@@ -980,7 +986,9 @@ struct BatchArgs {
     int aug;                   // the arena carries the norm chunk (stride nkc + 1)
     int dpad16;
     int exact_ok;              // lists integer in [0,255] and d <= 129
-    float mcoef;               // margin coefficient for non-exact queries
+    float mcoef;               // margin of non-exact queries: mcoef (||q||^2 + ||x||^2) + mabs
+    float mabs;
+    float dot_scale;           // -2 / (the FP16 shadow's scale squared); -2 for BF16
     const uint32_t* all_int;   // every query of the batch integer-valued in [0, 255]
     uint32_t max_items;        // capacity of the item table
     uint32_t* scnt;            // [nq] survivors per query
@@ -1030,7 +1038,16 @@ __device__ inline int batch_kind(const BatchArgs& a) {
 // MFMA chain over -2q and the norm chunk yields the exact distance, and the
 // epilogue is one compare per distance.  General form: ||q||^2 + ||x||^2 -
 // 2 q.x with the error margin.
-template <int NKC, int QG, bool FAST>
+// F16: the shadow and the queries' fragments are FP16 of the scaled values.
+template <bool F16>
+__device__ __forceinline__ floatx16 mfma16(const bf16x8& x, const bf16x8& y, const floatx16& c) {
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, x), __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+}
+
+template <int NKC, int QG, bool FAST, bool F16>
 __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
     // exactly one of the scan kernels works on a batch; none when there is
     // no work (a rescue pass with nothing flagged)
@@ -1094,6 +1111,7 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
             __builtin_amdgcn_wave_barrier();
         };
         constexpr bool fast = FAST;
+        const float ds = F16 ? a.dot_scale : -2.0f;
         float qn[QG], marg[QG];
         bf16x8 b[QG][NKC];
         bf16x8 bx[QG];
@@ -1102,6 +1120,7 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
             const bool live = qid[g] >= 0;
             qn[g] = (!FAST && live) ? a.qnorm[qid[g]] : 0.0f;
             marg[g] = (!FAST && live && !(a.exact_ok && a.qint[qid[g]])) ? a.mcoef : 0.0f;
+            if (F16) tau[g] += a.mabs;
             const uint16_t* base = fast ? a.qbf2 : a.qbf;
             const bf16x8* src = reinterpret_cast<const bf16x8*>(base + (size_t)max(qid[g], 0) * a.dpad16 + half * 8);
             bf16x8 z = {};
@@ -1109,10 +1128,19 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
             for (int kc = 0; kc < NKC; ++kc) b[g][kc] = (live && kc < a.nkc) ? src[kc * 2] : z;
             bx[g] = (fast && live && half == 0) ? *reinterpret_cast<const bf16x8*>(a.qaug + (size_t)qid[g] * 8) : z;
         }
-        // A fragments (list rows) of the first tile; the next tile's are
-        // loaded while the current tile's epilogue runs
+        // A fragments (list rows) and norms of the first tile; each chunk's
+        // next fragment is loaded as its current one goes into the products,
+        // the norms before any (loaded behind them, their wait covered the whole
+        // next tile: memory returns in order)
         bf16x8 av[NKC];
         bf16x8 ax;
+        float4 xv[4];
+        auto norms = [&](int64_t G) {
+#pragma unroll
+            for (int rq = 0; rq < 4; ++rq)
+                xv[rq] = *reinterpret_cast<const float4*>(a.norms + G * 32 + rq * 8 + half * 4);
+        };
+        if constexpr (!FAST) norms(G0 + w.t0);
         {
             const bf16x8* xa = reinterpret_cast<const bf16x8*>(a.xbf) + (G0 + w.t0) * stride * 64 + lane;
             bf16x8 z = {};
@@ -1125,29 +1153,35 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
             floatx16 acc[QG];
 #pragma unroll
             for (int g = 0; g < QG; ++g) acc[g] = floatx16{};
+            float xn[16];
+            if constexpr (!FAST) {
+#pragma unroll
+                for (int rq = 0; rq < 4; ++rq) {
+                    xn[rq * 4 + 0] = xv[rq].x;
+                    xn[rq * 4 + 1] = xv[rq].y;
+                    xn[rq * 4 + 2] = xv[rq].z;
+                    xn[rq * 4 + 3] = xv[rq].w;
+                }
+                norms(min(G + 1, G0 + te - 1));
+            }
+            // (the next tile, or the last again)
+            const bf16x8* xa = reinterpret_cast<const bf16x8*>(a.xbf) + min(G + 1, G0 + te - 1) * stride * 64 + lane;
 #pragma unroll
             for (int kc = 0; kc < NKC; ++kc) {
                 if (kc < a.nkc) {
 #pragma unroll
-                    for (int g = 0; g < QG; ++g)
-                        acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[kc], b[g][kc], acc[g], 0, 0, 0);
+                    for (int g = 0; g < QG; ++g) acc[g] = mfma16<F16>(av[kc], b[g][kc], acc[g]);
+                    av[kc] = xa[kc * 64];
                 }
             }
             if (fast) {
 #pragma unroll
                 for (int g = 0; g < QG; ++g)
                     acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ax, bx[g], acc[g], 0, 0, 0);
-            }
-            if (T + 1 < te) {
-                const bf16x8* xa = reinterpret_cast<const bf16x8*>(a.xbf) + (G + 1) * stride * 64 + lane;
-#pragma unroll
-                for (int kc = 0; kc < NKC; ++kc)
-                    if (kc < a.nkc) av[kc] = xa[kc * 64];
-                if (fast) ax = xa[a.nkc * 64];
+                ax = xa[a.nkc * 64];
             }
             // rows of this lane that exist (only the list's last tile is partial)
             const uint32_t rows_ok = tile_rows_ok(nrows - T * 32, half);
-            float xn[16];
             uint64_t m = 0;
             if constexpr (FAST) {
                 // acc is the exact distance: reject the tile with one min per
@@ -1170,20 +1204,12 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
                 }
             } else {
 #pragma unroll
-                for (int rq = 0; rq < 4; ++rq) {
-                    float4 v = *reinterpret_cast<const float4*>(a.norms + G * 32 + rq * 8 + half * 4);
-                    xn[rq * 4 + 0] = v.x;
-                    xn[rq * 4 + 1] = v.y;
-                    xn[rq * 4 + 2] = v.z;
-                    xn[rq * 4 + 3] = v.w;
-                }
-#pragma unroll
                 for (int g = 0; g < QG; ++g) {
                     uint32_t mg = 0;
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const float sn = qn[g] + xn[r];
-                        const float dist = __builtin_fmaf(-2.0f, acc[g][r], sn);
+                        const float dist = __builtin_fmaf(ds, acc[g][r], sn);
                         const float lo = __builtin_fmaf(-marg[g], sn, dist);
                         mg |= (lo <= tau[g] ? 1u : 0u) << r;
                     }
@@ -1203,7 +1229,7 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
                 for (int r = 0; r < 16; ++r) {
                     if ((m16 >> r) & 1u) {
                         const int row = (r >> 2) * 8 + half * 4 + (r & 3);
-                        const float dist = fast ? acc[0][r] : __builtin_fmaf(-2.0f, acc[0][r], qn[0] + xn[r]);
+                        const float dist = fast ? acc[0][r] : __builtin_fmaf(ds, acc[0][r], qn[0] + xn[r]);
                         sk[__builtin_popcount(m16 & ((1u << r) - 1u))] = make_key(dist, (uint32_t)(G * 32 + row));
                     }
                 }
@@ -1226,7 +1252,7 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
                         if (sl < a.cap) {
                             const int row = (r >> 2) * 8 + half * 4 + (r & 3);
                             const float dist =
-                                fast ? acc[g][r] : __builtin_fmaf(-2.0f, acc[g][r], qn[g] + xn[r]);
+                                fast ? acc[g][r] : __builtin_fmaf(ds, acc[g][r], qn[g] + xn[r]);
                             dst[sl] = make_key(dist, (uint32_t)(G * 32 + row));
                         }
                         ++sl;
@@ -1240,10 +1266,10 @@ __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
     }
 }
 
-template <int NKC, int QG, bool FAST>
+template <int NKC, int QG, bool FAST, bool F16 = false>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(FAST && QG == 1 && NKC == 8 ? 4 : 1)))
 void batched_scan_kernel(BatchArgs a) {
-    batched_scan_body<NKC, QG, FAST>(a);
+    batched_scan_body<NKC, QG, FAST, F16>(a);
 }
 
 // Int8 form of the scan for integer data.  With x' = x - 128 and q' = q -
@@ -1270,7 +1296,7 @@ void batched_scan_i8_kernel(BatchArgs a) {
         if constexpr (kI8RunsBf16<NKC8, QG>) {
             BatchArgs ab = a;
             ab.rbound = a.rbound_bf16;
-            batched_scan_body<8, 2, false>(ab);
+            batched_scan_body<8, 2, false, false>(ab);
         }
         return;
     }
@@ -1518,7 +1544,7 @@ void batched_scan_i8_kernel(BatchArgs a) {
 // (cus * the occupancy of kNT-thread workgroups), cached per variant.
 template <typename K>
 dim3 resident_grid(K kernel, int variant, int cus, dim3 want) {
-    static int per_cu[3] = {0, 0, 0};
+    static int per_cu[9] = {};
     if (per_cu[variant] == 0) {
         int n = 0;
         per_cu[variant] =
@@ -1726,8 +1752,8 @@ __global__ __launch_bounds__(kNT) void select_kernel(SelArgs a) {
 // The keys are read once per pass (they are in L2 from the scan).  The
 // result -- and the flags, rescan bounds and counts -- are those of
 // select_one.  Approximate keys take select_wave_inexact.  Every other query
-// (more than kSelSort candidates, k above kSelSort / 2, more than 1024
-// approximate keys) goes to the workgroup form through hard[] / *nhard.
+// (more than kSelSort candidates, k above kSelSort / 2) goes to the
+// workgroup form through hard[] / *nhard.
 constexpr int kSelSort = 512;   // candidates one wave sorts in LDS
 constexpr int kSelThin = 128;   // more admissible keys than this (and k): thinned by the histograms first
 
@@ -1918,19 +1944,21 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
     }
 }
 
-// The wave form for keys that hold approximate ranks (at most 64
-// kSelRegSlots survivors, k <= kSelSort / 2): U, an upper bound of the k-th
-// smallest upper bound v + E, is the upper edge of its bin in a 1024-bin
-// histogram (widened past the binning's rounding); every survivor with
-// v - E <= U can be among the top k and is rescored with the exact chain, a
-// candidate per lane, the query's components as scalar operands.  The
-// workgroup form reads all survivors twice and compacts them with LDS sorts.
+// The wave form for keys that hold approximate ranks (k <= kSelSort / 2; up to
+// 64 kSelRegSlots survivors in registers, more are read once per pass): U, an
+// upper bound of the k-th smallest upper bound v + E, is the upper edge of its
+// bin in a 1024-bin histogram (widened past the binning's rounding); every
+// survivor with v - E <= U can be among the top k and is rescored with the
+// exact chain, a candidate per lane, the query's components as scalar
+// operands, 16 loads of its row in flight (8: 4000 queries of 96 dims 172 us,
+// 16: 136).  The workgroup form reads all survivors twice and compacts them
+// with LDS sorts.
 template <int METRIC>
 __device__ float chain_of(const float4* q, const float4* tp, int nquad) {
     typedef const __attribute__((address_space(4))) float4* UniformQuads;
     const UniformQuads qu = (UniformQuads)q;
     float acc = 0.0f;
-#pragma unroll 8
+#pragma unroll 16
     for (int j = 0; j < nquad; ++j) {
         const float4 qv = {qu[j].x, qu[j].y, qu[j].z, qu[j].w};
         acc = accum<METRIC>(acc, qv, tp[(size_t)j * 64]);
@@ -1938,33 +1966,56 @@ __device__ float chain_of(const float4* q, const float4* tp, int nquad) {
     return rank_of<METRIC>(acc);
 }
 
+template <bool REG>
 __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool overflow, uint64_t* kk, int lane,
                                     int32_t* hard, uint32_t* nhard, float tau, bool ids8,
                                     uint64_t (&kr)[kSelRegSlots]) {
     const uint64_t* sb = a.sbuf + (size_t)qi * a.cap;
-    float xn[kSelRegSlots];
-#pragma unroll
-    for (int t = kSelSpecSlots; t < kSelRegSlots; ++t) {
-        const uint32_t i = (uint32_t)t * 64 + lane;
-        if ((uint32_t)t * 64 < n) kr[t] = sb[i < n ? i : 0];
-    }
-#pragma unroll
-    for (int t = 0; t < kSelRegSlots; ++t) {
-        const uint32_t i = (uint32_t)t * 64 + lane;
-        if (i >= n) kr[t] = kNoKey;
-        if ((uint32_t)t * 64 < n) xn[t] = a.norms[kr[t] != kNoKey ? (uint32_t)kr[t] : 0u];
-    }
     const float qn = a.qnorm[qi];
+    float xn[REG ? kSelRegSlots : 1];
+    if constexpr (REG) {
+#pragma unroll
+        for (int t = kSelSpecSlots; t < kSelRegSlots; ++t) {
+            const uint32_t i = (uint32_t)t * 64 + lane;
+            if ((uint32_t)t * 64 < n) kr[t] = sb[i < n ? i : 0];
+        }
+#pragma unroll
+        for (int t = 0; t < kSelRegSlots; ++t) {
+            const uint32_t i = (uint32_t)t * 64 + lane;
+            if (i >= n) kr[t] = kNoKey;
+            if ((uint32_t)t * 64 < n) xn[t] = a.norms[kr[t] != kNoKey ? (uint32_t)kr[t] : 0u];
+        }
+    }
     float mn = INFINITY, mx = -INFINITY;
     uint32_t fin = 0, real = 0;
-    auto each = [&](auto&& f) {  // f(slot, v, E) over this lane's survivors
+    // f(key, v, E) over this lane's survivors, a group of 64 at a time (every
+    // lane calls it; a lane without one passes kNoKey)
+    auto each = [&](auto&& f) {
+        if constexpr (REG) {
 #pragma unroll
-        for (int t = 0; t < kSelRegSlots; ++t)
-            if ((uint32_t)t * 64 < n && kr[t] != kNoKey)
-                f(t, key_rank(kr[t]), __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs));
+            for (int t = 0; t < kSelRegSlots; ++t)
+                if ((uint32_t)t * 64 < n) f(kr[t], key_rank(kr[t]), __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs));
+        } else {
+            constexpr int kB = 4;  // groups whose keys and norms are in flight together
+            for (uint32_t b0 = 0; b0 < n; b0 += 64 * kB) {
+                uint64_t k[kB];
+                float x[kB];
+#pragma unroll
+                for (int t = 0; t < kB; ++t) {
+                    const uint32_t i = b0 + t * 64 + lane;
+                    k[t] = sb[i < n ? i : 0];
+                    if (i >= n) k[t] = kNoKey;
+                }
+#pragma unroll
+                for (int t = 0; t < kB; ++t) x[t] = a.norms[k[t] != kNoKey ? (uint32_t)k[t] : 0u];
+#pragma unroll
+                for (int t = 0; t < kB; ++t) f(k[t], key_rank(k[t]), __builtin_fmaf(a.mcoef, qn + x[t], a.mabs));
+            }
+        }
     };
-    each([&](int, float v, float e) {
+    each([&](uint64_t key, float v, float e) {
         const float u = v + e;
+        if (key == kNoKey) return;
         ++real;
         if (u < FLT_MAX) {
             mn = fminf(mn, u);
@@ -1985,8 +2036,8 @@ __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool o
         __builtin_amdgcn_wave_barrier();
         const float w = (mx - mn) * (1.0f / 1024.0f);
         const float inv = w > 0.0f ? 1.0f / w : 0.0f;
-        each([&](int, float v, float e) {
-            if (v + e < FLT_MAX) atomicAdd(&h1k[lin_bin1024(v + e, mn, inv)], 1u);
+        each([&](uint64_t key, float v, float e) {
+            if (key != kNoKey && v + e < FLT_MAX) atomicAdd(&h1k[lin_bin1024(v + e, mn, inv)], 1u);
         });
         __builtin_amdgcn_wave_barrier();
         const int b = wave_find_bin1024(h1k, (uint32_t)a.k, lane);
@@ -1998,15 +2049,13 @@ __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool o
     // the candidates' rows (ballot compaction)
     uint32_t* cid = reinterpret_cast<uint32_t*>(kk);
     uint32_t nc = 0;
-#pragma unroll
-    for (int t = 0; t < kSelRegSlots; ++t) {
-        if ((uint32_t)t * 64 >= n) continue;
-        const bool take = kr[t] != kNoKey && !(key_rank(kr[t]) - __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs) > U);
+    each([&](uint64_t key, float v, float e) {
+        const bool take = key != kNoKey && !(v - e > U);
         const uint64_t mk = __ballot(take);
         const uint32_t pos = nc + lanes_below(mk);
         nc += (uint32_t)__popcll(mk);
-        if (take && pos < (uint32_t)kSelSort) cid[pos] = (uint32_t)kr[t];
-    }
+        if (take && pos < (uint32_t)kSelSort) cid[pos] = (uint32_t)key;
+    });
     if (nc > (uint32_t)kSelSort) {
         if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
         return;
@@ -2079,16 +2128,21 @@ __device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t
             a.fallback[qi] = 1;
             a.rescan_tau[qi] = FLT_MAX;
             a.flist[atomicAdd(a.fcount, 1u)] = qi;
+            a.scnt[qi] = 0;
+            if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
         }
         return;
     }
-    if (a.k > kSelSort / 2 || (!exact && !(APPROX && n <= 64u * kSelRegSlots))) {
+    if (a.k > kSelSort / 2 || (!exact && !APPROX)) {
         if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
         return;
     }
-    if (APPROX && !exact)
-        select_wave_inexact(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
-    else if (n <= 64u * kSelRegSlots)
+    if (APPROX && !exact) {
+        if (n <= 64u * kSelRegSlots)
+            select_wave_inexact<true>(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
+        else
+            select_wave_inexact<false>(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
+    } else if (n <= 64u * kSelRegSlots)
         select_wave_one<true>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
     else
         select_wave_one<false>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
@@ -2096,9 +2150,11 @@ __device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t
 
 // One wave per query: all queries (nq, or those flagged in `active`), or a
 // walk over the query list.  APPROX: approximate keys are selected here too
-// (those of the split scans, whose error bound leaves little more than k to
-// rescore; the BF16 shadow's leaves most survivors, which the workgroup form
-// rescores faster: 2000 queries of 420 dims 0.29 ms against 0.41).
+// (those of the split scans and of the FP16 shadow, whose error bounds leave
+// few more than k rows to rescore; the BF16 shadow's leaves most survivors,
+// which the workgroup form rescores faster: 2000 queries of 420 dims 0.29 ms
+// against 0.41).  A query whose scaled values could overflow FP16 has no
+// bound on its error: it goes to the exact rescan.
 template <bool APPROX>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void select_wave_kernel(SelArgs a, int nq, int32_t* hard, uint32_t* nhard) {
     constexpr int kW = kNT / 64;
@@ -2262,6 +2318,23 @@ float margin_coef(int64_t d) {
                    1.01);
 }
 
+// The same for the FP16 shadow (u = 2^-11).  Values below FP16's normal range
+// are off by delta = 2^-14 / scale at most (all of them, should the matrix
+// cores flush them): that adds at most delta
+// sqrt(d) (||q|| + ||x||) + d delta^2 to |q.x - q~.x~|, and delta sqrt(d) sqrt(2
+// s) <= 2^-15 s + d delta^2 2^14 (s = ||q||^2 + ||x||^2) splits it into a
+// relative and an absolute part, both doubled for -2 q.x.
+float margin_coef_f16(int64_t d) {
+    const double u = 1.0 / 2048.0, e = 1.0 / 16777216.0;
+    auto gamma = [&](double m) { return m * e / (1.0 - m * e); };
+    return (float)(((2 * u + u * u) + 2 * gamma((double)d) * (1 + u) * (1 + u) + 8 * e + 2 * gamma(d + 2.0) +
+                    2 * std::ldexp(1.0, -15)) * 1.01);
+}
+float margin_abs_f16(int64_t d, float scale) {
+    const double delta = std::ldexp(1.0, -14) / scale;
+    return (float)(1.01 * 2 * (double)d * delta * delta * (16384.0 + 1.0)) + 1e-30f;
+}
+
 // Buffers of the planning (carved from the scratch) and its work-item bound.
 struct PlanBufs {
     int nlist;
@@ -2368,9 +2441,16 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     if (nkc > 32) return h->fail(HIVF_EUNSUPPORTED, "batched scan: d <= 512");
     if (n * P >= INT32_MAX) return h->fail(HIVF_EUNSUPPORTED, "batched scan: queries x nprobe < 2^31");
     const int64_t tiles32 = h->tiles * 2;
+    // Real-valued lists hold their shadow in FP16, scaled by a power of two so
+    // that the largest value lies in [2^13, 2^14): three bits more than BF16,
+    // so the margin is an eighth and little more than k survivors of a query
+    // need rescoring.  (Values whose squares leave FP32's range keep BF16.)
+    const bool f16 = !h->lists_uint8 && h->lists_sane && (h->lists_absmax == 0.0f ||
+                     (h->lists_absmax >= 0x1p-40f && h->lists_absmax < 0x1p50f));
     if (!B.valid) {
         B.release();
         B.nkc = nkc;
+        B.f16_scale = !f16 ? 0.0f : h->lists_absmax > 0.0f ? std::ldexp(1.0f, 13 - std::ilogb(h->lists_absmax)) : 1.0f;
         // integer lists: the int8 arena (d <= 256, distances below 2^24);
         // otherwise the BF16 norm chunk where it is exact (d <= 129)
         B.i8 = (h->lists_uint8 && h->d <= 256) ? 1 : 0;
@@ -2381,7 +2461,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         int64_t total = tiles32 * stride * 64;
         if (total > 0)
             hipLaunchKernelGGL(build_bf16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s,
-                               h->d_codes.p, h->d_norms.p, h->nquad, tiles32, nkc, stride,
+                               h->d_codes.p, h->d_norms.p, h->nquad, tiles32, nkc, stride, B.f16_scale,
                                static_cast<uint16_t*>(B.bf16));
         HIP_TRY(h, hipGetLastError());
         // tile radius intervals (list of every 32-row tile from the host's
@@ -2443,6 +2523,10 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         B.cus = prop.multiProcessorCount;
         B.valid = true;
     }
+    const float mcoef = f16 ? margin_coef_f16(h->d) : margin_coef(h->d);
+    const float mabs = f16 ? margin_abs_f16(h->d, B.f16_scale) : 0.0f;
+    // (a query's scaled values stay finite in FP16 below this norm)
+    const float qn_max = f16 ? std::min(1e37f, (60000.0f / B.f16_scale) * (60000.0f / B.f16_scale)) : INFINITY;
     // the int8 scan serves integer lists unless the caller asks for the BF16
     // shadow (HIVF_PREC_BF16); results are the same either way
     const int i8 = (B.i8 && p.precision != HIVF_PREC_BF16) ? 1 : 0;
@@ -2458,7 +2542,17 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     if (qg == 3) qg = 2;
     if (i8) qg = B.nkc8 == 4 ? std::min(qg, 2) : 1;  // the int8 kernel takes 32 or (d <= 128) 64 queries per item
     int rt = p.batch_rows > 0 ? std::max(1, p.batch_rows / 32) : h->tune.item_tiles;
+    // Rows per item: the caller's or the tuned size as it is; the default is at
+    // most 1024, cut (cut_rt) where the (query, list) pairs are too few to fill
+    // the chip or to even out its last items.  Measured at 1024, 512, 256 and
+    // 128 rows, whole search: FP16 shadow 37 queries x 24 probes 157, 143,
+    // 135, 130 us; 300 x 16 (d = 200) 239, 213, 210, 212; 4000 x 32 433, 423,
+    // 430, 448; 2000 x 50 (d = 420) 1024, 1020, 1052, 1141.  Int8 shadow 37 x
+    // 24 132, 127, 120, 112; 1000 x 32 337, 271, 254, 261; 4000 x 32 433, 387,
+    // 377, 403; 10k x 64 (its scan) 430, 408, 459 at 256.
+    const bool cut_rt = rt <= 0;
     if (rt <= 0) rt = 32;
+    const int rt_items = !cut_rt ? rt : n * P <= 2048 ? 4 : n * P <= 65536 ? 8 : 16;
     int waves = p.batch_waves > 0 ? p.batch_waves : h->tune.waves_per_cu;
     if (waves <= 0) waves = 16;
     const uint32_t qc = 32u * qg;
@@ -2468,7 +2562,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     for (int64_t l = 0; l < nlist; ++l)
         max_t32 = std::max<int64_t>(max_t32, 2 * (h->tile_off[l + 1] - h->tile_off[l]));
     // (near-query items hold rt / kNearSplit tiles: bound every item by that)
-    const int64_t rtn = std::max(1, rt / (int)kNearSplit);
+    const int64_t rtn = std::max(1, rt_items / (int)kNearSplit);
     const int64_t max_items = (n * P / qc + nlist) * ((max_t32 + rtn - 1) / rtn);
 
     // scratch layout
@@ -2543,7 +2637,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         // the coarse step, whose query-preparation launch also prepares the
         // queries for the scan (else prep_kernel does)
         PrepArgs pa{reinterpret_cast<const float*>(q), (int)h->d, (int)h->d_pad, (int)dpad16, dpad32, qbf, qbf2,
-                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, fb, fb2, scnt, fbc, lcnt, (int)nlist};
+                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, fb, fb2, scnt, fbc, lcnt, (int)nlist, B.f16_scale};
         bool prepped = false;
         const int rc0 = run_coarse(h, q, n, P, s, &pa, &prepped);
         if (rc0) return rc0;
@@ -2593,9 +2687,10 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.qint = qint;
         sa.qnorm = qnorm;
         sa.norms = h->d_norms.p;
-        sa.mcoef = margin_coef(h->d);
-        sa.mabs = 0.0f;
-        sa.qn_max = INFINITY;
+        sa.mcoef = mcoef;
+        sa.mabs = mabs;
+        // (a query flagged for its norm goes through the exact rescans)
+        sa.qn_max = first ? qn_max : INFINITY;
         sa.exact_ok = exact_bf16;
         sa.i8 = i8;
         sa.all_int = all_int;
@@ -2621,8 +2716,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.nlist = (int)nlist;
         uint32_t* nhard = fbc + (first ? 2 : 3);
         const int64_t wgs = (n + 3) / 4;
-        hipLaunchKernelGGL(select_wave_kernel<false>, dim3((unsigned)(qlist ? std::min<int64_t>(wgs, 1024) : wgs)),
-                           dim3(kNT), 0, s, sa, (int)n, shard, nhard);
+        const dim3 sgrid((unsigned)(qlist ? std::min<int64_t>(wgs, 1024) : wgs));
+        if (f16) hipLaunchKernelGGL(select_wave_kernel<true>, sgrid, dim3(kNT), 0, s, sa, (int)n, shard, nhard);
+        else hipLaunchKernelGGL(select_wave_kernel<false>, sgrid, dim3(kNT), 0, s, sa, (int)n, shard, nhard);
         sa.active = nullptr;
         sa.qlist = shard;
         sa.qcount = nhard;
@@ -2674,7 +2770,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         ba.tstat = cand ? h->d_stats.p + 1 : nullptr;  // blocks_total, blocks_skipped (first pass)
         ba.rbound = static_cast<const float2*>(B.rbound);
         ba.rbound_bf16 = ba.rbound;
-        ba.mcoef = margin_coef(h->d);
+        ba.mcoef = mcoef;
+        ba.mabs = mabs;
+        ba.dot_scale = f16 ? -2.0f / (B.f16_scale * B.f16_scale) : -2.0f;
         ba.all_int = all_int;
         ba.max_items = (uint32_t)std::min<int64_t>(max_items, UINT32_MAX);
         ba.scnt = scnt;
@@ -2701,7 +2799,26 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                 hipLaunchKernelGGL((batched_scan_i8_kernel<8, 1>),
                                    resident_grid((batched_scan_i8_kernel<8, 1>), 2, B.cus, grid), dim3(kNT), 0, s, b8);
         }
-        if (nkc <= 8) {
+        if (f16) {
+            if (nkc <= 8 && qg == 4)
+                hipLaunchKernelGGL((batched_scan_kernel<8, 4, false, true>),
+                                   resident_grid((batched_scan_kernel<8, 4, false, true>), 3, B.cus, grid), dim3(kNT), 0, s, ba);
+            else if (nkc <= 8 && qg == 2)
+                hipLaunchKernelGGL((batched_scan_kernel<8, 2, false, true>),
+                                   resident_grid((batched_scan_kernel<8, 2, false, true>), 4, B.cus, grid), dim3(kNT), 0, s, ba);
+            else if (nkc <= 8)
+                hipLaunchKernelGGL((batched_scan_kernel<8, 1, false, true>),
+                                   resident_grid((batched_scan_kernel<8, 1, false, true>), 5, B.cus, grid), dim3(kNT), 0, s, ba);
+            else if (nkc <= 16 && qg == 2)
+                hipLaunchKernelGGL((batched_scan_kernel<16, 2, false, true>),
+                                   resident_grid((batched_scan_kernel<16, 2, false, true>), 6, B.cus, grid), dim3(kNT), 0, s, ba);
+            else if (nkc <= 16)
+                hipLaunchKernelGGL((batched_scan_kernel<16, 1, false, true>),
+                                   resident_grid((batched_scan_kernel<16, 1, false, true>), 7, B.cus, grid), dim3(kNT), 0, s, ba);
+            else
+                hipLaunchKernelGGL((batched_scan_kernel<32, 1, false, true>),
+                                   resident_grid((batched_scan_kernel<32, 1, false, true>), 8, B.cus, grid), dim3(kNT), 0, s, ba);
+        } else if (nkc <= 8) {
             if (qg == 4) {
                 if (B.aug) hipLaunchKernelGGL((batched_scan_kernel<8, 4, true>), grid, dim3(kNT), 0, s, ba);
                 hipLaunchKernelGGL((batched_scan_kernel<8, 4, false>), grid, dim3(kNT), 0, s, ba);
@@ -2739,7 +2856,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     int rc = learned ? run_tau_model(h, q, n, P, npq, tau, s) : warmup(tau, nullptr, nullptr, nullptr);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
-    rc = pass(nullptr, nullptr, nullptr, tau, fb, rtau, learned, 4, true, rt);
+    rc = pass(nullptr, nullptr, nullptr, tau, fb, rtau, learned, 4, true, rt_items);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[4], s));
     // Under the learned bound, flagged queries are few (the model is trained
@@ -2989,7 +3106,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
                                    pf, qc, rt, fb, 0, all_int, stats, s));
         }
         if (split) {
-            SplitArgs b;
+            SplitArgs b{};
             b.lists = a.lists;
             b.norms = h->d_norms.p;
             b.qh = C.qh.p + q0 * dpad16;

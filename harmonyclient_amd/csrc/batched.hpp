@@ -24,7 +24,8 @@ struct BatchedState {
     bool valid = false;     // bf16 arena matches the current lists
     int nkc = 0;            // 16-dim chunks of the padded dimension
     int aug = 0;            // the arena carries the norm chunk per row
-    void* bf16 = nullptr;   // [tiles32 x (nkc + aug) x 64 lanes x 8] bf16
+    float f16_scale = 0.0f; // the shadow holds FP16 of the values times this (0: BF16)
+    void* bf16 = nullptr;   // [tiles32 x (nkc + aug) x 64 lanes x 8] bf16 or fp16
     size_t bf16_bytes = 0;
 
     // int8 arena of integer lists (d <= 256): operands and row norms

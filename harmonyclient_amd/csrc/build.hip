@@ -298,39 +298,50 @@ __global__ __launch_bounds__(256) void fill_arena_kernel(const float4* __restric
                                                          float4* __restrict__ codes, uint32_t* __restrict__ ids,
                                                          float* __restrict__ norms, uint32_t* __restrict__ flags) {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= tiles * kTileRows) return;
-    const int64_t T = g / kTileRows;
+    const int64_t T = g / kTileRows;  // (a tile is one wave: its lanes stay together)
+    if (T >= tiles) return;
     const int r = (int)(g % kTileRows);
     const int l = tile_list[T];
     const int64_t rr = (T - tile_off[l]) * kTileRows + r;
     const int64_t n_l = list_off[l + 1] - list_off[l];
     float4* dst = codes + (size_t)T * nquad * kTileRows + r;
+    uint32_t f = 0;
+    float mx = 0.0f;
     if (rr >= n_l) {
         for (int j = 0; j < nquad; ++j) dst[(size_t)j * kTileRows] = make_float4(0.f, 0.f, 0.f, 0.f);
         ids[g] = kNoId;
         norms[g] = 0.0f;
-        return;
-    }
-    const int32_t row = order[list_off[l] + rr];
-    const float4* src = x + (size_t)row * nquad;
-    double s = 0.0;
-    bool u8 = true;
-    for (int j = 0; j < nquad; ++j) {
-        const float4 v = src[j];
-        dst[(size_t)j * kTileRows] = v;
-        const float c[4] = {v.x, v.y, v.z, v.w};
-        for (int i = 0; i < 4; ++i) {
-            if (4 * j + i >= d) break;
-            s += (double)c[i] * (double)c[i];
-            u8 = u8 && c[i] >= 0.0f && c[i] <= 255.0f && c[i] == rintf(c[i]);
+    } else {
+        const int32_t row = order[list_off[l] + rr];
+        const float4* src = x + (size_t)row * nquad;
+        double s = 0.0;
+        bool u8 = true;
+#pragma unroll 4
+        for (int j = 0; j < nquad; ++j) {
+            const float4 v = src[j];
+            dst[(size_t)j * kTileRows] = v;
+            const float c[4] = {v.x, v.y, v.z, v.w};
+            for (int i = 0; i < 4; ++i) {
+                if (4 * j + i >= d) break;
+                s += (double)c[i] * (double)c[i];
+                mx = fmaxf(mx, fabsf(c[i]));
+                u8 = u8 && c[i] >= 0.0f && c[i] <= 255.0f && c[i] == rintf(c[i]);
+            }
         }
+        ids[g] = (uint32_t)row;
+        const float nr = (float)s;
+        norms[g] = nr;
+        f = (u8 ? 0u : 1u) | (nr < 1e37f ? 0u : 2u);
     }
-    ids[g] = (uint32_t)row;
-    const float nr = (float)s;
-    norms[g] = nr;
-    // bit 0: a value that is no integer in [0, 255]; bit 1: a norm past 1e37
-    const uint32_t f = (u8 ? 0u : 1u) | (nr < 1e37f ? 0u : 2u);
-    if (f) atomicOr(flags, f);
+    // bit 0: a value that is no integer in [0, 255]; bit 1: a norm past 1e37;
+    // flags[1]: bits of the largest magnitude.  One atomic per wave, and none
+    // where it would change nothing (one per row queued up on the line).
+    const uint32_t fw = (__ballot(f & 1u) ? 1u : 0u) | (__ballot(f & 2u) ? 2u : 0u);
+    mx = wave_max(mx);
+    if (r == 0) {
+        if (fw & ~flags[0]) atomicOr(flags, fw);
+        if (__float_as_uint(mx) > flags[1]) atomicMax(flags + 1, __float_as_uint(mx));
+    }
 }
 
 // Row i divided by its norm (the FP32 FMA chain over the d dims, then a
@@ -580,7 +591,7 @@ int gpu_add(hivf_index* h, int64_t n) {
     for (int64_t l = 0; l < nlist; ++l)
         for (int32_t t = tile_off[l]; t < tile_off[l + 1]; ++t) tile_list[t] = (int32_t)l;
     const int nquad = h->nquad;
-    HIP_TRY(h, h->d_codes.ensure((size_t)std::max<int64_t>(tiles, 1) * nquad * kTileRows));
+    HIP_TRY(h, h->d_codes.ensure((size_t)std::max<int64_t>(tiles, 1) * nquad * kTileRows + kArenaTail));
     HIP_TRY(h, h->d_ids.ensure((size_t)std::max<int64_t>(tiles, 1) * kTileRows));
     HIP_TRY(h, h->d_norms.ensure((size_t)std::max<int64_t>(tiles, 1) * kTileRows));
     HIP_TRY(h, h->d_tile_off.ensure(nlist + 1));
@@ -588,23 +599,27 @@ int gpu_add(hivf_index* h, int64_t n) {
     HIP_TRY(h, hipMemcpyAsync(h->d_tile_off.p, tile_off.data(), (nlist + 1) * sizeof(int32_t), hipMemcpyHostToDevice,
                               s));
     HIP_TRY(h, hipMemcpyAsync(h->d_size.p, size.data(), nlist * sizeof(int32_t), hipMemcpyHostToDevice, s));
-    uint32_t flags = 0;
+    uint32_t flags[2] = {0, 0};
     if (tiles > 0) {
         DevBuf<int32_t> dtl;
         DevBuf<uint32_t> flag;
         HIP_TRY(h, dtl.ensure((size_t)tiles));
-        HIP_TRY(h, flag.ensure(1));
+        HIP_TRY(h, flag.ensure(2));
         HIP_TRY(h, hipMemcpyAsync(dtl.p, tile_list.data(), tiles * sizeof(int32_t), hipMemcpyHostToDevice, s));
-        hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, flag.p, 1);
+        hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(64), 0, s, flag.p, 2);
+        hipLaunchKernelGGL(zero_u32_kernel, dim3(grid_of(kArenaTail * 4, 256)), dim3(256), 0, s,
+                           reinterpret_cast<uint32_t*>(h->d_codes.p + (size_t)tiles * nquad * kTileRows),
+                           kArenaTail * 4);
         hipLaunchKernelGGL(fill_arena_kernel, dim3(grid_of(tiles * kTileRows, 256)), dim3(256), 0, s, h->d_q.p,
                            nquad, (int)h->d, G.order, G.off.p, h->d_tile_off.p, dtl.p, tiles, h->d_codes.p,
                            h->d_ids.p, h->d_norms.p, flag.p);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, hipMemcpyAsync(&flags, flag.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipMemcpyAsync(flags, flag.p, sizeof(flags), hipMemcpyDeviceToHost, s));
     }
     HIP_TRY(h, hipStreamSynchronize(s));  // host vectors and local buffers
-    h->lists_uint8 = (flags & 1u) == 0;
-    h->lists_sane = (flags & 2u) == 0;
+    h->lists_uint8 = (flags[0] & 1u) == 0;
+    h->lists_sane = (flags[0] & 2u) == 0;
+    std::memcpy(&h->lists_absmax, flags + 1, sizeof(float));
     h->list_off = list_off;
     h->tile_off = tile_off;
     h->ntotal = list_off[nlist];

@@ -11,6 +11,9 @@ namespace hivf {
 constexpr int kWave = 64;        // CDNA wavefront width
 constexpr int kTileRows = 64;    // list rows per tile: one row per lane
 constexpr int kMaxK = 1024;      // largest k of the per-query scans
+// Zeroed float4s past the list arena: the split scans read whole 16-dim chunks,
+// up to 3 quads past a tile's last.
+constexpr int kArenaTail = 3 * kTileRows;
 constexpr uint32_t kNoId = 0xFFFFFFFFu;
 
 // A result entry packed into one 64-bit word: order-preserving bits of the

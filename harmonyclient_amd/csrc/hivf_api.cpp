@@ -209,7 +209,7 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
     std::vector<uint32_t> ids;
     std::vector<float> norms;
     try {
-        codes.assign(std::max<size_t>(tiles * tile_floats, 4), 0.0f);
+        codes.assign(std::max<size_t>(tiles * tile_floats, 4) + (size_t)kArenaTail * 4, 0.0f);
         ids.assign(std::max<int64_t>(tiles * kTileRows, 1), kNoId);
         norms.assign(std::max<int64_t>(tiles * kTileRows, 1), 0.0f);
     } catch (const std::bad_alloc&) {
@@ -217,6 +217,7 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
     }
     int bad = 0;
     std::vector<char> small(nlist, 1), sane(nlist, 1);
+    std::vector<float> amax(nlist, 0.0f);
     parallel_for(nlist, [&](int64_t l) {
         int64_t n_l = size[l];
         float* base = codes.data() + (size_t)tile_off[l] * tile_floats;
@@ -231,6 +232,7 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
             double s = 0.0;  // norms in FP64, rounded once
             for (int64_t c = 0; c < h->d; ++c) {
                 s += (double)src[c] * (double)src[c];
+                amax[l] = std::max(amax[l], std::fabs(src[c]));
                 if (!(src[c] >= 0.0f && src[c] <= 255.0f && src[c] == std::rint(src[c]))) small[l] = 0;
             }
             norms[slot] = (float)s;
@@ -250,6 +252,7 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
     HIP_TRY(h, hipMemcpy(h->d_norms.p, norms.data(), norms.size() * sizeof(float), hipMemcpyHostToDevice));
     HIP_TRY(h, hipMemcpy(h->d_tile_off.p, tile_off.data(), (nlist + 1) * sizeof(int32_t), hipMemcpyHostToDevice));
     HIP_TRY(h, hipMemcpy(h->d_size.p, size.data(), nlist * sizeof(int32_t), hipMemcpyHostToDevice));
+    h->lists_absmax = amax.empty() ? 0.0f : *std::max_element(amax.begin(), amax.end());
     h->lists_sane = std::all_of(sane.begin(), sane.end(), [](char c) { return c != 0; });
     h->lists_uint8 = std::all_of(small.begin(), small.end(), [](char c) { return c != 0; });
     h->list_off = list_off;

@@ -104,6 +104,7 @@ struct hivf_index {
     bool have_lists = false;
     bool lists_uint8 = false;  // every list value is an integer in [0, 255]
     bool lists_sane = false;   // every row's squared norm is below 1e37
+    float lists_absmax = 0.0f; // largest magnitude of a list value (when sane)
 
     // list arena (device) and its host-side shape
     std::vector<int64_t> list_off;  // [nlist + 1] rows

@@ -33,6 +33,7 @@ struct PrepArgs {
     uint32_t* fbc;   // [4]
     uint32_t* lcnt;  // [nlist]
     int nlist;
+    float f16_scale;  // > 0: qbf holds FP16 of q times this (the FP16 shadow's queries)
 };
 
 // A query's first kQRegs * 64 components (0 past d), one round of loads:
@@ -55,7 +56,8 @@ __device__ inline void prep_query(const PrepArgs& a, const int qi, const int lan
     double s = 0.0;
     int ok = 1;
     auto one = [&](int c, float v) {
-        a.qbf[(size_t)qi * a.dpad16 + c] = f2bf(v);
+        a.qbf[(size_t)qi * a.dpad16 + c] =
+            a.f16_scale > 0.0f ? __builtin_bit_cast(uint16_t, (_Float16)(v * a.f16_scale)) : f2bf(v);
         a.qbf2[(size_t)qi * a.dpad16 + c] = f2bf(-2.0f * v);  // = -2 bf16(v) exactly
         s += (double)v * (double)v;
         ok &= (v == rintf(v)) && v >= 0.0f && v <= 255.0f;

@@ -127,20 +127,22 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
         float4 raw[NKC][2];
         float4 xv[4];
         // a tile's rows (lane: row slot, quads 4 kc + 2 half and the next) and
-        // norms; chunks and quads past the row's end read its last quad, and
-        // the queries' pieces are zero there
+        // norms; quads past the row's end are the next tile's (or the arena's
+        // zeroed tail), finite values that meet zeros of the queries' pieces
         auto load = [&](int T) {
-            const int g = T0 + T;
-            const float4* p = a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32 + slot;
+            const int g = __builtin_amdgcn_readfirstlane(T0 + T);
+            const float4* p = a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32;
+            const uint32_t lo = half * 128 + slot;
 #pragma unroll
             for (int kc = 0; kc < NKC; ++kc) {
-                const int j = kc * 4 + half * 2;
-                raw[kc][0] = p[(size_t)min(j, nquad - 1) * 64];
-                raw[kc][1] = p[(size_t)min(j + 1, nquad - 1) * 64];
+                if (kc < nkc) {
+                    raw[kc][0] = (p + kc * 256)[lo];
+                    raw[kc][1] = (p + kc * 256 + 64)[lo];
+                }
             }
+            const float* np = a.norms + (size_t)g * 32;
 #pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4)
-                xv[r4] = *reinterpret_cast<const float4*>(a.norms + (size_t)g * 32 + r4 * 8 + half * 4);
+            for (int r4 = 0; r4 < 4; ++r4) xv[r4] = *reinterpret_cast<const float4*>(np + r4 * 8 + half * 4);
         };
         load(w.t0);
         bf16x8 bh[NKC], bl[NKC];
@@ -191,6 +193,7 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
             }
 #pragma unroll
             for (int kc = 0; kc < NKC; ++kc) {
+                if (kc >= nkc) break;
                 bf16x8 h, l;
                 split8<XLO>(raw[kc][0], raw[kc][1], h, l);
                 if constexpr (XLO) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, bh[kc], acc, 0, 0, 0);
@@ -273,13 +276,16 @@ __global__ __launch_bounds__(kSplitWgNT) __attribute__((amdgpu_waves_per_eu(4)))
                 ch -= nch;
                 T += kW;
             }
-            const int g = T0 + min(T, te - 1);
-            const float4* p = a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32 + slot;
+            const int g = __builtin_amdgcn_readfirstlane(T0 + min(T, te - 1));
+            const float4* p = a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32;
+            const uint32_t lo = half * 128 + slot;
 #pragma unroll
             for (int c = 0; c < kC; ++c) {
-                const int j = (ch * kC + c) * 4 + half * 2;
-                raw[c][0] = p[(size_t)min(j, nquad - 1) * 64];
-                raw[c][1] = p[(size_t)min(j + 1, nquad - 1) * 64];
+                const int kc = ch * kC + c;
+                if (kc < nkc) {
+                    raw[c][0] = (p + kc * 256)[lo];
+                    raw[c][1] = (p + kc * 256 + 64)[lo];
+                }
             }
         };
         if (w.t0 + wv < te) load(ra, w.t0 + wv, 0);

@@ -73,7 +73,8 @@ typedef struct {
     int32_t survivor_cap;            /* batched: candidates kept per query before its exact rescan; 0 = 16384;
                                         rounded up to an even count */
     int32_t batch_queries;           /* batched: queries per work item (32, 64, 128); 0 = tuned/default */
-    int32_t batch_rows;              /* batched: list rows per work item (multiple of 32); 0 = tuned/default */
+    int32_t batch_rows;              /* batched: list rows per work item (multiple of 32); 0 = tuned/default
+                                        (default: at most 1024, fewer for small batches) */
     int32_t batch_waves;             /* batched: resident waves per CU of the persistent launch; 0 = tuned/default */
     int32_t use_graph;               /* search_device only, no stats: capture the search in a hipGraph on the
                                         first call of a shape and replay it on later calls with the same
@@ -99,7 +100,7 @@ typedef struct {
     int64_t fallback_queries; /* batched scan: queries its first pass could not finish (rescanned) */
     int64_t scan_launches; /* launches of the dominant kernel in this search */
     int64_t exact_rescans; /* batched scan: queries left to the per-query exact scan */
-    int64_t batch_queries; /* batched scan: tile shape used (queries, rows, waves per CU) */
+    int64_t batch_queries; /* batched scan: tile shape used (queries, most rows, waves per CU) */
     int64_t batch_rows;
     int64_t batch_waves;
     double plan_ms;        /* batched scan: probe inversion and work-item planning */
