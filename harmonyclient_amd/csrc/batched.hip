@@ -43,6 +43,9 @@ namespace {
 // A work item is (list, up to 32 * QG queries, up to item_tiles 32-row
 // tiles); QG is the kernel variant's number of 32-query MFMA column groups.
 constexpr int kNT = 256;
+// a search's counters: the two rescue lists', the two hard lists', then the
+// per-query part counts of the exact rescan
+constexpr int kFbcWords = 4 + kListSlots;
 
 
 
@@ -2581,7 +2584,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                  o_items = take((size_t)max_items * sizeof(BatchItem)), o_scnt = take(n * 4),
                  o_sbuf = take((size_t)n * cap * 8), o_fb = take(n * 4), o_tau = take(n * 4),
                  o_rtau = take(n * 4), o_tau2 = take(n * 4), o_rtau2 = take(n * 4), o_fb2 = take(n * 4),
-                 o_fbl = take(n * 4), o_fbl2 = take(n * 4), o_fbc = take(16), o_shard = take(n * 4),
+                 o_fbl = take(n * 4), o_fbl2 = take(n * 4), o_fbc = take(kFbcWords * 4), o_part = take(part_keys_bytes(k)), o_shard = take(n * 4),
                  o_allint = take(4), o_q8 = take(i8 ? (size_t)n * B.nkc8 * 32 : 0),
                  o_qn8 = take(i8 ? (size_t)n * 4 : 0);
     if (off > B.scratch_bytes) {
@@ -2637,7 +2640,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         // the coarse step, whose query-preparation launch also prepares the
         // queries for the scan (else prep_kernel does)
         PrepArgs pa{reinterpret_cast<const float*>(q), (int)h->d, (int)h->d_pad, (int)dpad16, dpad32, qbf, qbf2,
-                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, fb, fb2, scnt, fbc, lcnt, (int)nlist, B.f16_scale};
+                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, fb, fb2, scnt, fbc, kFbcWords, lcnt, (int)nlist, B.f16_scale};
         bool prepped = false;
         const int rc0 = run_coarse(h, q, n, P, s, &pa, &prepped);
         if (rc0) return rc0;
@@ -2862,12 +2865,12 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     // Under the learned bound, flagged queries are few (the model is trained
     // and its offset tuned for a small miss rate): where one query's exact
     // rescan is small (at most 2^24 list elements at the mean list size:
-    // 1M x 128 at nprobe 128) they go straight to the exact per-query rescan below, one launch, where the
-    // pair-parallel pass and its selection would cost three launches in every
-    // search that flags none.  Larger probe sets (a miss over 10M rows at
-    // nprobe 256 would hold one workgroup for milliseconds), and every
-    // warm-up-bound search (overflowing survivor buffers can flag many
-    // queries), take pass 2 first.
+    // 1M x 128 at nprobe 128) they go straight to the exact per-query rescan
+    // below, one launch, where the pair-parallel pass and its selection would
+    // cost three launches in every search that flags none.  Larger probe sets
+    // (the pair-parallel pass reads an integer list's int8 rows, a quarter of
+    // the rescan's bytes), and every warm-up-bound search (overflowing
+    // survivor buffers can flag many queries), take pass 2 first.
     const double rescan_elems = (double)h->ntotal / (double)std::max<int64_t>(1, nlist) * (double)P * (double)h->d;
     const bool pair_rescue = !learned || rescan_elems > (double)(1 << 24);
     // pass 2: the flagged queries, each (query, probed list, tile group) a
@@ -2923,6 +2926,8 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     f.out_i = I;
     f.qlist = pair_rescue ? fbl2 : fbl;
     f.qcount = pair_rescue ? fbc + 1 : fbc;
+    f.part_keys = (uint64_t*)at(o_part);
+    f.part_cnt = fbc + 4;
     HIP_TRY(h, launch_scan(f, kScanPruned, h->metric, s));
     if (timing) {
         HIP_TRY(h, hipEventRecord(h->ev[5], s));
@@ -3029,7 +3034,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     const size_t entries = shared ? (size_t)chunk * P : 0;
     const size_t o_sbuf = take((size_t)chunk * cap * 8), o_scnt = take(chunk * 4), o_fb = take(chunk * 4),
                  o_fbl = take(chunk * 4), o_hard = take(chunk * 4), o_tau = take(chunk * 4), o_rtau = take(chunk * 4),
-                 o_fbc = take(16), o_allint = take(4), o_lcnt = take(nlist * 4), o_lcur = take(nlist * 4),
+                 o_fbc = take(kFbcWords * 4), o_part = take(part_keys_bytes(k)), o_allint = take(4), o_lcnt = take(nlist * 4), o_lcur = take(nlist * 4),
                  o_lend = take(nlist * 4), o_qoff = take((nlist + 1) * 4), o_ioff = take((nlist + 1) * 8),
                  o_lnear = take(nlist * 4), o_meta = take(kMetaWords * 4), o_lq = take(entries * 4),
                  o_lqd = take(entries * 4), o_hwg = take(shared ? plan_hwg_bytes(nlist, (int64_t)entries) : 0),
@@ -3068,8 +3073,8 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         const int64_t m = std::min(chunk, n - q0);
         const int32_t* probes = h->d_probes.p + q0 * P;
         const int32_t* npqc = npq ? npq + q0 : nullptr;
-        hipLaunchKernelGGL(flat_clear_kernel, dim3((unsigned)((std::max(m, nlist) + 255) / 256)), dim3(256), 0, s, scnt,
-                           fb, (int)m, lcnt, (int)nlist, fbc, all_int);
+        hipLaunchKernelGGL(flat_clear_kernel, dim3((unsigned)((std::max<int64_t>(std::max(m, nlist), kFbcWords) + 255) / 256)),
+                           dim3(256), 0, s, scnt, fb, (int)m, lcnt, (int)nlist, fbc, kFbcWords, all_int);
         ScanArgs w{};
         w.lists = h->lists();
         w.q = q + q0 * h->nquad;
@@ -3191,6 +3196,8 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         f.out_i = sa.out_i;
         f.qlist = sa.flist;
         f.qcount = fbc;
+        f.part_keys = (uint64_t*)at(o_part);
+        f.part_cnt = fbc + 4;
         HIP_TRY(h, launch_scan(f, kScanPlain, h->metric, s));
     }
     return HIVF_OK;

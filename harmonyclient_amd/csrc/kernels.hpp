@@ -44,7 +44,19 @@ struct ScanArgs {
     const int32_t* only;      // optional [nq] flags: scan only the flagged queries
     const int32_t* qlist;     // optional: scan only these queries (count in *qcount)
     const uint32_t* qcount;
+    // optional, with qlist: short lists' queries are split over several
+    // workgroups, whose top k meet here (part_keys_bytes(k) bytes and
+    // kListSlots counters that are zero at the launch)
+    uint64_t* part_keys;
+    uint32_t* part_cnt;
 };
+
+// Workgroups of a query-list launch, the most one query is split over, and
+// the most queries of a list that is split.
+constexpr int kListGrid = 1024;
+constexpr int kListParts = 64;
+constexpr int kListSlots = kListGrid / 2;
+inline size_t part_keys_bytes(int64_t k) { return (size_t)kListGrid * (size_t)k * sizeof(uint64_t); }
 
 hipError_t launch_scan(const ScanArgs& a, int mode, int metric, hipStream_t s);
 

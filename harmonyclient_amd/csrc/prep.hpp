@@ -16,7 +16,7 @@ namespace hivf {
 // in [0, 255], and, for the int8 scan (q8 non-null), q - 128 as int8
 // (row-major, dpad32; 0 past d) with sum (q - 128)^2.  It also clears the
 // search's per-query flags and survivor counts, and (workgroup 0) the rescue
-// list counts and the per-list query counts of the first pass.
+// list and part counts and the per-list query counts of the first pass.
 struct PrepArgs {
     const float* q;
     int d, ld, dpad16, dpad32;
@@ -30,7 +30,8 @@ struct PrepArgs {
     int32_t* fb;
     int32_t* fb2;
     uint32_t* scnt;
-    uint32_t* fbc;   // [4]
+    uint32_t* fbc;   // [fbc_words]
+    int fbc_words;
     uint32_t* lcnt;  // [nlist]
     int nlist;
     float f16_scale;  // > 0: qbf holds FP16 of q times this (the FP16 shadow's queries)
@@ -104,7 +105,7 @@ __device__ inline void prep_query(const PrepArgs& a, const int qi, const int lan
         if (lane == 0) a.qn8[qi] = s8;
     }
     if (qi == 0) {
-        if (lane < 4) a.fbc[lane] = 0;
+        for (int l = lane; l < a.fbc_words; l += 64) a.fbc[l] = 0;
         for (int l = lane; l < a.nlist; l += 64) a.lcnt[l] = 0;
     }
 }

@@ -28,7 +28,6 @@ namespace {
 constexpr int kNT = 256;
 constexpr int kNW = kNT / kWave;
 constexpr int kBuf = 2048;
-constexpr int kListGrid = 1024;  // workgroups of a query-list launch
 
 
 __device__ inline void load_query(float4* qs, const float4* q, int nquad) {
@@ -166,8 +165,14 @@ static_assert(kMaxK + kRoundTiles * kNT <= kBuf, "a round's keys fit beside the 
 // lists x 100 rows of 128 dims 103 -> 65 us, of 4096 on skewed lists 221 -> 172, of
 // 2000 with 420 dims 190 -> 163 (the rows come from L2 at 17 to 21 TB/s).  More
 // than 8 row loads in flight per wave is slower (16: 305 us at 420 dims).
+//
+// With nparts > 1 the workgroup takes every nparts-th round of the query's
+// tiles (each part starts at the near lists, so its running k-th is as tight
+// as one workgroup's after the same number of rounds) and leaves its top k in
+// slot's part of part_keys; the last part to end merges them.
 template <int MODE, int METRIC>
-__device__ void scan_one(const ScanArgs& a, const int qi) {
+__device__ void scan_one(const ScanArgs& a, const int qi, const int part = 0, const int nparts = 1,
+                         const uint32_t slot = 0) {
     __shared__ LdsTopK<kNT, kBuf> top;
     __shared__ ProbeMap pm;
     __shared__ unsigned long long s_stats[3];
@@ -197,7 +202,7 @@ __device__ void scan_one(const ScanArgs& a, const int qi) {
         const int m = min(kProbeChunk, P - j0);
         const int total = pm.before[m];
         int j = 0;  // this wave's probe: before[j] <= its tile < before[j + 1]
-        for (int g0 = 0; g0 < total; g0 += kNW * kRound) {
+        for (int g0 = part * kNW * kRound; g0 < total; g0 += nparts * kNW * kRound) {
             for (int u = 0; u < kRound; ++u) {
                 const int g = g0 + u * kNW + wave;
                 if (g >= total) break;
@@ -263,6 +268,35 @@ __device__ void scan_one(const ScanArgs& a, const int qi) {
         }
     } else {
         top.finish(a.k);
+        if (nparts > 1) {
+            __shared__ uint32_t s_before;
+            uint64_t* mine = a.part_keys + ((size_t)slot * nparts + part) * a.k;
+            for (int i = tid; i < a.k; i += kNT) mine[i] = i < top.cnt ? top.buf[i] : ~0ull;
+            __threadfence();
+            __syncthreads();
+            if (tid == 0) s_before = atomicAdd(&a.part_cnt[slot], 1u);
+            __syncthreads();
+            if (s_before + 1 != (uint32_t)nparts) return;
+            __threadfence();
+            top.init();
+            thr = top.thr;
+            const uint64_t* all = a.part_keys + (size_t)slot * nparts * a.k;
+            const int nk = nparts * a.k;
+            for (int i0 = 0; i0 < nk; i0 += kRoundTiles * kNT) {
+                uint64_t key[kRoundTiles];
+#pragma unroll
+                for (int u = 0; u < kRoundTiles; ++u) {
+                    const int i = i0 + u * kNT + tid;
+                    key[u] = i < nk ? all[i] : ~0ull;
+                }
+#pragma unroll
+                for (int u = 0; u < kRoundTiles; ++u) top.offer(key[u], thr);
+                __syncthreads();
+                top.maybe_compact(a.k, kRoundTiles * kNT);
+                thr = top.thr;
+            }
+            top.finish(a.k);
+        }
         const int cnt = top.cnt;
         for (int i = tid; i < a.k; i += kNT) {
             float dv = sentinel<METRIC>();
@@ -280,11 +314,21 @@ __device__ void scan_one(const ScanArgs& a, const int qi) {
 }
 
 // One workgroup per query (all, or those flagged in `only`), or, with a
-// query list, a grid that walks the list.
+// query list, a grid that walks the list.  A list too short for the grid has
+// its queries split: one query's 62k rows of 128 dims on one workgroup hold a
+// search for 0.9 ms, 43 such queries for 1.9 ms, against 0.42 ms split.
 template <int MODE, int METRIC>
 __global__ __launch_bounds__(kNT) void scan_kernel(ScanArgs a) {
     if (a.qlist) {
         const uint32_t nl = *a.qcount;
+        if constexpr (MODE != kScanWarmup) {
+            const uint32_t np = a.part_keys && nl ? min(gridDim.x / nl, (uint32_t)kListParts) : 1u;
+            if (np > 1) {
+                const uint32_t slot = blockIdx.x / np;
+                if (slot < nl) scan_one<MODE, METRIC>(a, a.qlist[slot], (int)(blockIdx.x % np), (int)np, slot);
+                return;
+            }
+        }
         for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
             __syncthreads();  // the previous query's LDS reads are done
             scan_one<MODE, METRIC>(a, a.qlist[i]);
@@ -357,7 +401,9 @@ __global__ __launch_bounds__(kNT) void coarse_kernel(CoarseArgs a) {
 template <int MODE>
 hipError_t launch_scan_mode(const ScanArgs& a, int metric, hipStream_t s) {
     size_t lds = (size_t)a.lists.nquad * sizeof(float4);
-    const dim3 grid((unsigned)(a.qlist ? std::min(a.nq, kListGrid) : a.nq));
+    // (a list of few queries gets workgroups to split them over)
+    const int64_t want = a.part_keys ? (int64_t)a.nq * 16 : a.nq;
+    const dim3 grid((unsigned)(a.qlist ? std::min<int64_t>(want, kListGrid) : a.nq));
     if (metric == kL2)
         hipLaunchKernelGGL((scan_kernel<MODE, kL2>), grid, dim3(kNT), lds, s, a);
     else
