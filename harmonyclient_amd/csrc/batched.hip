@@ -2856,27 +2856,24 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 
     // pass 1: every query under the requested bound
     const bool learned = p.tau_source == HIVF_TAU_LEARNED;
-    int rc = learned ? run_tau_model(h, q, n, P, npq, tau, s) : warmup(tau, nullptr, nullptr, nullptr);
+    // (radii of rows that are not finite bound nothing)
+    const TauCap tc{h->d_probes.p, h->d_size.p, h->d_tile_off.p, B.i8 ? static_cast<const float2*>(B.rbound8) : nullptr,
+                    static_cast<const float2*>(B.lbound), (int)k};
+    int rc = learned ? run_tau_model(h, q, n, P, npq, tau, s, h->lists_uint8 || h->lists_sane ? &tc : nullptr)
+                     : warmup(tau, nullptr, nullptr, nullptr);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
     rc = pass(nullptr, nullptr, nullptr, tau, fb, rtau, learned, 4, true, rt_items);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[4], s));
-    // Under the learned bound, flagged queries are few (the model is trained
-    // and its offset tuned for a small miss rate): where one query's exact
-    // rescan is small (at most 2^24 list elements at the mean list size:
-    // 1M x 128 at nprobe 128) they go straight to the exact per-query rescan
-    // below, one launch, where the pair-parallel pass and its selection would
-    // cost three launches in every search that flags none.  Larger probe sets
-    // (the pair-parallel pass reads an integer list's int8 rows, a quarter of
-    // the rescan's bytes), and every warm-up-bound search (overflowing
-    // survivor buffers can flag many queries), take pass 2 first.
-    const double rescan_elems = (double)h->ntotal / (double)std::max<int64_t>(1, nlist) * (double)P * (double)h->d;
-    const bool pair_rescue = !learned || rescan_elems > (double)(1 << 24);
     // pass 2: the flagged queries, each (query, probed list, tile group) a
     // workgroup task, bounded by the k-th of the rows pass 1 kept or, for a
-    // learned-bound miss, the widened learned bound
-    if (pair_rescue) {
+    // learned-bound miss, the widened learned bound.  (Searches under the
+    // learned bound at nprobe 64 on 1M x 128 used to go straight to the exact
+    // rescan, which reads FP32 rows without a bound: 1 miss of 10k queries 609
+    // us with it, 514 with this pass, 16 of them 833 and 556; without any, the
+    // pass is three empty launches.)
+    {
         PairScanArgs ra;
         ra.lists = h->lists();
         ra.q = q;
@@ -2908,7 +2905,6 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         HIP_TRY(h, select(nullptr, fbl, fbc, tau2, fb2, rtau2, true, 5, false, true));
     }
     // last resort: exact per-query rescan of what pass 2 could not finish
-    // (or of every flagged query, bounded by pass 1's rescan bound)
     ScanArgs f{};
     f.lists = h->lists();
     f.q = q;
@@ -2919,13 +2915,13 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     f.nprobe = P;
     f.k = (int)k;
     pruning_blocks(h->d, 0, &f.block_dims, &f.nblocks);
-    f.tau = pair_rescue ? rtau2 : rtau;
+    f.tau = rtau2;
     f.row_limit = INT_MAX;
     f.warm_lists = INT_MAX;
     f.out_d = D;
     f.out_i = I;
-    f.qlist = pair_rescue ? fbl2 : fbl;
-    f.qcount = pair_rescue ? fbc + 1 : fbc;
+    f.qlist = fbl2;
+    f.qcount = fbc + 1;
     f.part_keys = (uint64_t*)at(o_part);
     f.part_cnt = fbc + 4;
     HIP_TRY(h, launch_scan(f, kScanPruned, h->metric, s));
@@ -2944,7 +2940,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         st->survivors = (int64_t)c[3];
         st->fallback_queries = (int64_t)c[4];  // rescanned by the second batched pass
         st->scan_launches = 2;
-        st->exact_rescans = (int64_t)(pair_rescue ? c[5] : c[4]);
+        st->exact_rescans = (int64_t)c[5];
         st->overflow_queries = (int64_t)c[6];
         st->batch_queries = qg * 32;
         st->batch_rows = rt * 32;

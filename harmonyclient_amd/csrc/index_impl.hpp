@@ -221,9 +221,19 @@ inline float elapsed_ms(hipEvent_t a, hipEvent_t b) {
     if (hipEventElapsedTime(&ms, a, b) != hipSuccess) return 0.0f;
     return ms;
 }
-// Learned bound: tau[q] from the attached model (mlp.hip).
+// What bounds a learned bound from above (mlp.hip): the probed lists' sizes and
+// radii, per 32-row tile in order of increasing radius (tile_r) or per list.
+struct TauCap {
+    const int32_t* probes;  // [n x P]
+    const int32_t* size;
+    const int32_t* tile_off;
+    const float2* tile_r;
+    const float2* list_r;
+    int k;
+};
+// Learned bound: tau[q] from the attached model (mlp.hip), at most the cap's.
 int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_t* npq, float* tau,
-                  hipStream_t s);
+                  hipStream_t s, const TauCap* cap = nullptr);
 // Defined in batched.hip.
 int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
                 const hivf_search_params& p, float* D, int64_t* I, hivf_search_stats* st,

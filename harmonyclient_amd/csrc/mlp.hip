@@ -265,6 +265,38 @@ __global__ void tau_out_kernel(const float* __restrict__ yhat, int n, float offs
     if (i < n) tau[i] = scale * fmaxf(expm1f(yhat[i] + offset), 0.0f);
 }
 
+// An upper bound of a query's k-th distance from its coarse distances: the k
+// rows nearest to their centroids in its nearest lists lie within sqrt(cd) + r
+// of it (widened as the plan's radius filter).  Infinite with fewer than k rows
+// probed.  A prediction above it admits rows for nothing: some queries kept
+// more than the 16384 survivors of the default buffer (up to 1487 of 10k on 1M
+// x 128, depending on the data), and their rescans and selections held the
+// search for 0.3 to 10 ms.
+__device__ float radius_cap(const TauCap& c, const float* cd, const int32_t* probes, int Pq) {
+    float m = 0.0f;
+    int need = c.k;
+    for (int j = 0; j < Pq && need > 0; ++j) {
+        const int l = probes[j];
+        if (l < 0) break;
+        const int rows = min(c.size[l], need);
+        if (rows <= 0) continue;
+        const float r = c.tile_r ? c.tile_r[2 * (int64_t)c.tile_off[l] + (rows - 1) / 32].y : c.list_r[l].y;
+        const float u = sqrtf(fmaxf(cd[j], 0.0f) * (1.0f + 1e-4f)) + r;
+        if (!(cd[j] < FLT_MAX) || !(u < 1e18f)) return INFINITY;
+        m = fmaxf(m, u);
+        need -= rows;
+    }
+    return need > 0 ? INFINITY : m * m * (1.0f + 1e-4f);
+}
+
+__global__ void tau_cap_kernel(TauCap c, const float* __restrict__ cd, int P, const int32_t* __restrict__ npq, int n,
+                               float* __restrict__ tau) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= n) return;
+    const size_t o = (size_t)i * P;
+    tau[i] = fminf(tau[i], radius_cap(c, cd + o, c.probes + o, npq ? min(npq[i], P) : P));
+}
+
 unsigned blocks(int64_t n, int t = 256) { return (unsigned)((n + t - 1) / t); }
 
 // The whole inference for a search in one launch: features, standardisation,
@@ -294,6 +326,7 @@ struct FusedArgs {
     float offset;
     float scale;
     float* tau;
+    TauCap cap;  // probes null: none
 };
 
 // LDS: weights max([33][H], [H/2][H]), features [8R][33], activations
@@ -315,6 +348,14 @@ __global__ __launch_bounds__(256) void tau_mlp_kernel(FusedArgs a) {
     const int tid = threadIdx.x;
     const int q0 = blockIdx.x * kRows;
     const int half_n = Hh * H;                 // floats of one half of W2
+    // (the last wave's, beside the loads of the weights; read at the end)
+    __shared__ float s_cap[kRows];
+    if (tid >= 192 && tid - 192 < kRows) {
+        const int q = min(q0 + tid - 192, a.n - 1);
+        const size_t o = (size_t)q * a.P;
+        s_cap[tid - 192] = a.cap.probes ? radius_cap(a.cap, a.cd + o, a.cap.probes + o, a.npq ? min(a.npq[q], a.P) : a.P)
+                                        : INFINITY;
+    }
     float wr[kHalfRegs];
     auto fetch = [&](int hf) {
 #pragma unroll
@@ -432,7 +473,7 @@ __global__ __launch_bounds__(256) void tau_mlp_kernel(FusedArgs a) {
 #pragma unroll 8
         for (int k = 0; k < H; ++k) y = __builtin_fmaf(Hs[tid * ldh + k], w3[k], y);
         y += a.prm[a.off_b3];
-        a.tau[q0 + tid] = a.scale * fmaxf(expm1f(y + a.offset), 0.0f);
+        a.tau[q0 + tid] = fminf(a.scale * fmaxf(expm1f(y + a.offset), 0.0f), s_cap[tid]);
     }
 }
 
@@ -556,7 +597,8 @@ hipError_t hivf_tau_model::predict(hipStream_t s, const float* F, int64_t n, flo
 }
 
 namespace hivf {
-int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_t* npq, float* tau, hipStream_t s) {
+int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_t* npq, float* tau, hipStream_t s,
+                  const TauCap* cap) {
     (void)q;
     if (!h->tau_model) return h->fail(HIVF_ESTATE, "learned bound requested but no model is attached");
     TauModel& m = *h->tau_model;
@@ -564,13 +606,13 @@ int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_
     if (m.hid <= kFusedHid && m.hid % 8 == 0) {
         FusedArgs fa{h->d_cd.p, P,        npq,      h->batched_qnorm, (int)n,   m.params, m.hid,
                      m.off_W1,  m.off_b1, m.off_W2, m.off_b2,         m.off_w3, m.off_b3, m.off_mu,
-                     m.off_sd,  m.host_offset, m.host_scale, tau};
+                     m.off_sd,  m.host_offset, m.host_scale, tau,             cap ? *cap : TauCap{}};
         // 8 R rows per workgroup, about two workgroups per compute unit (a
         // second wave per SIMD hides the layer loops' LDS waits: 22 us for
         // 10k queries at R = 3, 25 us at one workgroup per CU, R = 5)
         const int64_t cus = std::max(1, h->cus);
         int R = (int)std::min<int64_t>(kFusedMaxR, std::max<int64_t>(1, (n + 16 * cus - 1) / (16 * cus)));
-        while (R > 1 && fused_lds_bytes(m.hid, R) > 65536) --R;  // 64 KiB per workgroup
+        while (R > 1 && fused_lds_bytes(m.hid, R) > 65536 - 256) --R;  // 64 KiB per workgroup, with the caps
         const dim3 grid(blocks(n, 8 * R));
         const size_t lds = fused_lds_bytes(m.hid, R);
         switch (R) {
@@ -590,6 +632,10 @@ int run_tau_model(hivf_index* h, const float4* q, int64_t n, int P, const int32_
     hipLaunchKernelGGL(features_kernel, dim3(blocks(n)), dim3(256), 0, s, h->d_cd.p, P, npq, h->batched_qnorm, (int)n,
                        h->d_feat.p);
     HIP_TRY(h, m.predict(s, h->d_feat.p, n, tau, m.params));
+    if (cap) {
+        hipLaunchKernelGGL(tau_cap_kernel, dim3(blocks(n)), dim3(256), 0, s, *cap, h->d_cd.p, P, npq, (int)n, tau);
+        HIP_TRY(h, hipGetLastError());
+    }
     return HIVF_OK;
 }
 
