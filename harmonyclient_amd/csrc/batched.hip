@@ -1558,8 +1558,7 @@ dim3 resident_grid(K kernel, int variant, int cus, dim3 want) {
 }
 
 struct SelArgs {
-    const int32_t* active;      // only these queries (null = all)
-    const int32_t* qlist;       // or: only the queries of this list (count in *qcount)
+    const int32_t* qlist;       // only the queries of this list (count in *qcount; null = all)
     const uint32_t* qcount;
     uint32_t* scnt;             // survivor counts; cleared once a query is selected
     const uint64_t* sbuf;
@@ -1585,14 +1584,11 @@ struct SelArgs {
     int metric;                 // of the keys' ranks (IP: the exact FP32 scans only)
     float* out_d;
     int64_t* out_i;
-    int32_t* fallback;          // [nq] flags
     float* rescan_tau;          // [nq] bound for the rescan of flagged queries
     unsigned long long* stats;  // [3] survivors, [fb_slot] flagged queries, [6] overflows of the first pass
     int fb_slot;
     int32_t* flist;             // flagged queries are appended here (count in *fcount)
     uint32_t* fcount;
-    uint32_t* lcnt;             // per-list query counts, cleared for the next pass (workgroup 0)
-    int nlist;
 };
 
 __device__ void select_one(const SelArgs& a, const int qi) {
@@ -1709,7 +1705,6 @@ __device__ void select_one(const SelArgs& a, const int qi) {
     const bool tau_ok = top.cnt >= a.k && key_rank(top.buf[a.k - 1]) <= tau;
     if (overflow || (a.check_tau && !tau_ok)) {
         if (tid == 0) {
-            a.fallback[qi] = 1;
             a.rescan_tau[qi] = top.cnt >= a.k ? key_rank(top.buf[a.k - 1]) : FLT_MAX;
             a.flist[atomicAdd(a.fcount, 1u)] = qi;
             if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
@@ -1730,22 +1725,6 @@ __device__ void select_one(const SelArgs& a, const int qi) {
     }
 }
 
-// One workgroup per query (all, or those flagged in `active`), or, with a
-// query list, a grid that walks the list.
-__global__ __launch_bounds__(kNT) void select_kernel(SelArgs a) {
-    if (a.qlist) {
-        const uint32_t nl = *a.qcount;
-        for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
-            __syncthreads();  // the previous query's LDS reads are done
-            select_one(a, a.qlist[i]);
-        }
-        return;
-    }
-    const int qi = blockIdx.x;
-    if (a.active && !a.active[qi]) return;  // whole workgroup, before any barrier
-    select_one(a, qi);
-}
-
 // One-wave form of the selection, for queries whose survivor keys already
 // hold exact distances (every query of an int8 scan; integer queries of an
 // exact BF16 scan): the wave finds a bound V >= the k-th smallest distance
@@ -1760,8 +1739,8 @@ __global__ __launch_bounds__(kNT) void select_kernel(SelArgs a) {
 constexpr int kSelSort = 512;   // candidates one wave sorts in LDS
 constexpr int kSelThin = 128;   // more admissible keys than this (and k): thinned by the histograms first
 
-// REG: at most 64 * kSelRegSlots survivors, held in registers (one read of
-// the keys); otherwise the keys are read once per pass.
+// At most 64 * kSelRegSlots survivors, held in registers (one read of the
+// keys).
 constexpr int kSelRegSlots = 16;
 // slots whose keys are loaded together with the survivor count, before it
 // is known (positions past survivor_cap read the last slot instead), so the
@@ -1771,34 +1750,26 @@ constexpr int kSelSpecSlots = 8;
 // The first kSelSpecSlots slots of this lane's keys are in kr already
 // (loaded before n was known); tau and ids8 (the keys' positions are int8
 // shadow rows) were loaded with the survivor count.
-template <bool REG>
-__device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overflow, uint32_t* hs, uint64_t* kk,
-                                int lane, int32_t* hard, uint32_t* nhard, float tau, bool ids8,
+__device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, uint64_t* kk, int lane,
+                                int32_t* hard, uint32_t* nhard, float tau, bool ids8,
                                 uint64_t (&kr)[kSelRegSlots]) {
     auto hand_over = [&]() {
         if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
     };
     const uint64_t* sb = a.sbuf + (size_t)qi * a.cap;
-    if constexpr (REG) {
 #pragma unroll
-        for (int t = 0; t < kSelRegSlots; ++t) {
-            const uint32_t i = (uint32_t)t * 64 + lane;
-            if (t < kSelSpecSlots)
-                kr[t] = i < n ? kr[t] : ~0ull;
-            else
-                kr[t] = i < n ? sb[i] : ~0ull;
-        }
+    for (int t = 0; t < kSelRegSlots; ++t) {
+        const uint32_t i = (uint32_t)t * 64 + lane;
+        if (t < kSelSpecSlots)
+            kr[t] = i < n ? kr[t] : ~0ull;
+        else
+            kr[t] = i < n ? sb[i] : ~0ull;
     }
     // f(key) over this lane's survivors
     auto each = [&](auto&& f) {
-        if constexpr (REG) {
 #pragma unroll
-            for (int t = 0; t < kSelRegSlots; ++t)
-                if ((uint32_t)t * 64 + lane < n) f(kr[t]);
-        } else {
-#pragma unroll 4
-            for (uint32_t i = lane; i < n; i += 64) f(sb[i]);
-        }
+        for (int t = 0; t < kSelRegSlots; ++t)
+            if ((uint32_t)t * 64 + lane < n) f(kr[t]);
     };
     // distances <= tau (the learned bound's check), the range of the
     // admissible ones (rank < FLT_MAX: the heap's strict admission)
@@ -1822,10 +1793,10 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
     // candidate bins: all admissible keys when there are few, else the bins
     // up to the k-th (two histogram passes cost less than sorting a few
     // hundred keys more)
-    int b1 = 255, sb2 = 255;
-    float w1 = 0.0f, inv1 = 0.0f, lo2 = 0.0f, inv2 = 0.0f;
+    int b1 = 1023;
+    float w1 = 0.0f, inv1 = 0.0f;
     const bool thin = fin > (uint32_t)max(kSelThin, a.k);
-    if (REG && thin) {
+    if (thin) {
         // (at most 1024 keys) one 1024-bin histogram, in the sort buffer
         // (free until the compaction): the k-th's bin holds few keys at
         // this resolution, and the candidates are the bins up to it
@@ -1840,65 +1811,21 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
         __builtin_amdgcn_wave_barrier();
         b1 = wave_find_bin1024(h1k, (uint32_t)a.k, lane);
         __builtin_amdgcn_wave_barrier();  // the histogram's reads are done before the compaction's writes
-    } else if (thin) {
-        for (int i = lane; i < 256; i += 64) hs[i] = 0;
-        __builtin_amdgcn_wave_barrier();
-        w1 = (mx - mn) * (1.0f / 256.0f);
-        inv1 = w1 > 0.0f ? 1.0f / w1 : 0.0f;
-        each([&](uint64_t key) {
-            if (key < key_limit()) atomicAdd(&hs[lin_bin(key_rank(key), mn, inv1)], 1u);
-        });
-        __builtin_amdgcn_wave_barrier();
-        uint32_t need = (uint32_t)a.k;
-        b1 = wave_find_bin(hs, &need, lane);
-        // keys in the bins up to the k-th's; when they fit one small sort
-        // the k-th's bin is not split (sb2 = 255 takes all of it)
-        const uint32_t upto = (uint32_t)a.k - need + hs[b1];
-        if (upto > (uint32_t)max(kSelThin, a.k)) {
-            __builtin_amdgcn_wave_barrier();
-            for (int i = lane; i < 256; i += 64) hs[i] = 0;
-            __builtin_amdgcn_wave_barrier();
-            lo2 = mn + (float)b1 * w1;
-            inv2 = w1 > 0.0f ? 256.0f / w1 : 0.0f;
-            each([&](uint64_t key) {
-                if (key < key_limit()) {
-                    const float r = key_rank(key);
-                    if (lin_bin(r, mn, inv1) == b1) atomicAdd(&hs[lin_bin(r, lo2, inv2)], 1u);
-                }
-            });
-            __builtin_amdgcn_wave_barrier();
-            sb2 = wave_find_bin(hs, &need, lane);
-        }
     }
     // compaction (ballots) of the candidates' keys, then re-keyed by
     // (distance, id)
     uint32_t nc = 0;
     auto group = [&](uint64_t key) {
         bool take = key < key_limit();
-        if (take && thin) {
-            const float r = key_rank(key);
-            if (REG) {
-                take = lin_bin1024(r, mn, inv1) <= b1;
-            } else {
-                const int bb = lin_bin(r, mn, inv1);
-                take = bb < b1 || (bb == b1 && lin_bin(r, lo2, inv2) <= sb2);
-            }
-        }
+        if (take && thin) take = lin_bin1024(key_rank(key), mn, inv1) <= b1;
         const uint64_t mk = __ballot(take);
         const uint32_t pos = nc + lanes_below(mk);
         nc += (uint32_t)__popcll(mk);
         if (take && pos < (uint32_t)kSelSort) kk[pos] = key;
     };
-    if constexpr (REG) {
 #pragma unroll
-        for (int t = 0; t < kSelRegSlots; ++t)
-            if ((uint32_t)t * 64 < n) group(kr[t]);
-    } else {
-        for (uint32_t base = 0; base < n; base += 64) {
-            const uint32_t i = base + lane;
-            group(i < n ? sb[i] : ~0ull);
-        }
-    }
+    for (int t = 0; t < kSelRegSlots; ++t)
+        if ((uint32_t)t * 64 < n) group(kr[t]);
     if (nc > (uint32_t)kSelSort) {
         hand_over();
         return;
@@ -1925,13 +1852,11 @@ __device__ void select_wave_one(const SelArgs& a, int qi, uint32_t n, bool overf
     __builtin_amdgcn_wave_barrier();
     wave_sort(kk, n2, lane);
     if (lane == 0 && a.stats) atomicAdd(&a.stats[3], (unsigned long long)fin);  // (padding keys not counted)
-    if (overflow || (a.check_tau && le < (uint32_t)a.k)) {
+    if (a.check_tau && le < (uint32_t)a.k) {
         if (lane == 0) {
-            a.fallback[qi] = 1;
             a.rescan_tau[qi] = nc >= (uint32_t)a.k ? key_rank(kk[a.k - 1]) : FLT_MAX;
             a.flist[atomicAdd(a.fcount, 1u)] = qi;
             if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
-            if (a.stats && overflow && a.fb_slot == 4) atomicAdd(&a.stats[6], 1ull);  // first pass
         }
         return;
     }
@@ -1969,14 +1894,13 @@ __device__ float chain_of(const float4* q, const float4* tp, int nquad) {
     return rank_of<METRIC>(acc);
 }
 
-template <bool REG>
-__device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool overflow, uint64_t* kk, int lane,
+__device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, uint64_t* kk, int lane,
                                     int32_t* hard, uint32_t* nhard, float tau, bool ids8,
                                     uint64_t (&kr)[kSelRegSlots]) {
     const uint64_t* sb = a.sbuf + (size_t)qi * a.cap;
     const float qn = a.qnorm[qi];
-    float xn[REG ? kSelRegSlots : 1];
-    if constexpr (REG) {
+    float xn[kSelRegSlots];
+    {
 #pragma unroll
         for (int t = kSelSpecSlots; t < kSelRegSlots; ++t) {
             const uint32_t i = (uint32_t)t * 64 + lane;
@@ -1994,27 +1918,9 @@ __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool o
     // f(key, v, E) over this lane's survivors, a group of 64 at a time (every
     // lane calls it; a lane without one passes kNoKey)
     auto each = [&](auto&& f) {
-        if constexpr (REG) {
 #pragma unroll
-            for (int t = 0; t < kSelRegSlots; ++t)
-                if ((uint32_t)t * 64 < n) f(kr[t], key_rank(kr[t]), __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs));
-        } else {
-            constexpr int kB = 4;  // groups whose keys and norms are in flight together
-            for (uint32_t b0 = 0; b0 < n; b0 += 64 * kB) {
-                uint64_t k[kB];
-                float x[kB];
-#pragma unroll
-                for (int t = 0; t < kB; ++t) {
-                    const uint32_t i = b0 + t * 64 + lane;
-                    k[t] = sb[i < n ? i : 0];
-                    if (i >= n) k[t] = kNoKey;
-                }
-#pragma unroll
-                for (int t = 0; t < kB; ++t) x[t] = a.norms[k[t] != kNoKey ? (uint32_t)k[t] : 0u];
-#pragma unroll
-                for (int t = 0; t < kB; ++t) f(k[t], key_rank(k[t]), __builtin_fmaf(a.mcoef, qn + x[t], a.mabs));
-            }
-        }
+        for (int t = 0; t < kSelRegSlots; ++t)
+            if ((uint32_t)t * 64 < n) f(kr[t], key_rank(kr[t]), __builtin_fmaf(a.mcoef, qn + xn[t], a.mabs));
     };
     each([&](uint64_t key, float v, float e) {
         const float u = v + e;
@@ -2090,13 +1996,11 @@ __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool o
     if (lane == 0 && a.stats) atomicAdd(&a.stats[3], (unsigned long long)real);
     const uint64_t kth = (uint32_t)a.k <= n2 ? kk[a.k - 1] : ~0ull;
     const bool full = kth < key_limit();
-    if (overflow || (a.check_tau && !(full && key_rank(kth) <= tau))) {
+    if (a.check_tau && !(full && key_rank(kth) <= tau)) {
         if (lane == 0) {
-            a.fallback[qi] = 1;
             a.rescan_tau[qi] = full ? key_rank(kth) : FLT_MAX;
             a.flist[atomicAdd(a.fcount, 1u)] = qi;
             if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
-            if (a.stats && overflow && a.fb_slot == 4) atomicAdd(&a.stats[6], 1ull);  // first pass
         }
         return;
     }
@@ -2109,11 +2013,9 @@ __device__ void select_wave_inexact(const SelArgs& a, int qi, uint32_t n, bool o
 }
 
 template <bool APPROX>
-__device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t* kk, int lane, int32_t* hard,
-                                uint32_t* nhard) {
+__device__ void select_wave_any(const SelArgs& a, int qi, uint64_t* kk, int lane, int32_t* hard, uint32_t* nhard) {
     // everything the selection reads first, loaded together: the count,
-    // the flags, the bound and (when the buffer holds them) the first
-    // kSelSpecSlots slots of keys, whatever the count turns out to be
+    // the flags, the bound and the first slots' keys
     const uint32_t total = a.scnt[qi];
     const uint32_t all_int = *a.all_int;
     const int32_t qint = a.qint[qi];
@@ -2122,63 +2024,248 @@ __device__ void select_wave_any(const SelArgs& a, int qi, uint32_t* hs, uint64_t
     uint64_t kr[kSelRegSlots];
 #pragma unroll
     for (int t = 0; t < kSelSpecSlots; ++t) kr[t] = sb[min((uint32_t)t * 64 + lane, a.cap - 1)];
+    const bool ids8 = a.i8 && all_int;
+    const bool exact = a.keys_exact || ids8 || (a.exact_ok && qint);
+    if (total > min(64u * kSelRegSlots, a.cap) || a.k > kSelSort / 2 || (!exact && !APPROX) ||
+        (APPROX && !(a.qnorm[qi] < a.qn_max))) {
+        if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
+        return;
+    }
+    if (APPROX && !exact)
+        select_wave_inexact(a, qi, total, kk, lane, hard, nhard, tau, ids8, kr);
+    else
+        select_wave_one(a, qi, total, kk, lane, hard, nhard, tau, ids8, kr);
+}
+
+// One wave per query, for batches whose waves alone fill the chip.  APPROX:
+// approximate keys are selected here too (those of the split scans and of the
+// FP16 shadow, whose error bounds leave few more than k rows to rescore; the
+// BF16 shadow's leaves most survivors, which select_one rescores faster: 2000
+// queries of 420 dims 0.29 ms against 0.41).
+template <bool APPROX>
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void select_wave_kernel(SelArgs a, int nq, int32_t* hard, uint32_t* nhard) {
+    constexpr int kW = kNT / 64;
+    __shared__ __align__(16) uint64_t keys[kW][kSelSort];
+    const int wv = threadIdx.x / 64, lane = threadIdx.x % 64;
+    const int qi = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kW + wv);
+    if (qi >= nq) return;
+    select_wave_any<APPROX>(a, qi, keys[wv], lane, hard, nhard);
+}
+
+// The wave form's selection by a workgroup: 2048 survivors in registers (more
+// are read once per pass), one histogram for all, a candidate per thread.  For
+// the queries the wave form hands over, and for every query of a batch too
+// small to fill the chip with a wave each, where a wave's chain of loads (keys,
+// norms, ids, rows) is what the selection takes.  With the handed-over queries
+// taken by waves (256-bin histograms, three passes over their keys): 4096 warm-up
+// bounded queries on skewed lists 560 us, now 456; 1000 plain queries 483, now
+// 411; 2000 of 420 dims 959, now 902; a learned-bound search with 18 queries of
+// 16384 survivors 925, now 724.  False, with nothing changed: select_one's.
+constexpr int kSelWgSlots = 8;
+
+template <bool APPROX>
+__device__ bool select_wg(const SelArgs& a, const int qi) {
+    constexpr int kW = kNT / 64;
+    constexpr uint32_t kSpan = kSelWgSlots * kNT;
+    __shared__ __align__(16) uint64_t kk[kSelSort];
+    __shared__ __align__(16) uint32_t hist[1024];
+    __shared__ float s_mn[kW], s_mx[kW];
+    __shared__ uint32_t s_fin[kW], s_real[kW];
+    __shared__ uint32_t s_nc;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid / 64;
+    const uint32_t total = a.scnt[qi];
+    const uint32_t all_int = *a.all_int;
+    const int32_t qint = a.qint[qi];
+    const float tau = a.tau[qi];
+    const float qn = APPROX ? a.qnorm[qi] : 0.0f;
+    const uint64_t* sb = a.sbuf + (size_t)qi * a.cap;
     const bool overflow = total > a.cap;
     const uint32_t n = overflow ? a.cap : total;
     const bool ids8 = a.i8 && all_int;
     const bool exact = a.keys_exact || ids8 || (a.exact_ok && qint);
-    if (APPROX && !(a.qnorm[qi] < a.qn_max)) {  // (NaN too)
-        if (lane == 0) {
-            a.fallback[qi] = 1;
+    const bool approx = APPROX && !exact;
+    if (approx && !(qn < a.qn_max)) {  // (NaN too) no bound on its keys' error: the exact rescan
+        __syncthreads();  // the count is read
+        if (tid == 0) {
             a.rescan_tau[qi] = FLT_MAX;
             a.flist[atomicAdd(a.fcount, 1u)] = qi;
             a.scnt[qi] = 0;
             if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
         }
-        return;
+        return true;
     }
-    if (a.k > kSelSort / 2 || (!exact && !APPROX)) {
-        if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
-        return;
-    }
-    if (APPROX && !exact) {
-        if (n <= 64u * kSelRegSlots)
-            select_wave_inexact<true>(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
-        else
-            select_wave_inexact<false>(a, qi, n, overflow, kk, lane, hard, nhard, tau, ids8, kr);
-    } else if (n <= 64u * kSelRegSlots)
-        select_wave_one<true>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
-    else
-        select_wave_one<false>(a, qi, n, overflow, hs, kk, lane, hard, nhard, tau, ids8, kr);
-}
-
-// One wave per query: all queries (nq, or those flagged in `active`), or a
-// walk over the query list.  APPROX: approximate keys are selected here too
-// (those of the split scans and of the FP16 shadow, whose error bounds leave
-// few more than k rows to rescore; the BF16 shadow's leaves most survivors,
-// which the workgroup form rescores faster: 2000 queries of 420 dims 0.29 ms
-// against 0.41).  A query whose scaled values could overflow FP16 has no
-// bound on its error: it goes to the exact rescan.
-template <bool APPROX>
-__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void select_wave_kernel(SelArgs a, int nq, int32_t* hard, uint32_t* nhard) {
-    constexpr int kW = kNT / 64;
-    __shared__ uint32_t hist[kW][256];
-    __shared__ __align__(16) uint64_t keys[kW][kSelSort];
-    const int wv = threadIdx.x / 64, lane = threadIdx.x % 64;
-    if (blockIdx.x == 0)  // the pass's plan is done with them
-        for (int l = threadIdx.x; l < a.nlist; l += kNT) a.lcnt[l] = 0;
-    if (a.qlist) {
-        const uint32_t nl = *a.qcount;
-        for (uint32_t w = blockIdx.x * kW + wv; w < nl; w += gridDim.x * kW) {
-            __builtin_amdgcn_wave_barrier();  // the previous query's LDS reads are done
-            select_wave_any<APPROX>(a, __builtin_amdgcn_readfirstlane(a.qlist[w]), hist[wv], keys[wv], lane, hard, nhard);
+    if (a.k > kSelSort / 2 || (!exact && !APPROX)) return false;
+    uint64_t kr[kSelWgSlots];
+    float er[APPROX ? kSelWgSlots : 1];  // the keys' error bounds
+    auto load = [&](uint32_t base) {
+#pragma unroll
+        for (int t = 0; t < kSelWgSlots; ++t) {
+            const uint32_t i = base + (uint32_t)t * kNT + tid;
+            kr[t] = kNoKey;
+            if (base + (uint32_t)t * kNT < n) kr[t] = sb[min(i, n - 1)];
+            if (i >= n) kr[t] = kNoKey;
         }
-        return;
+        if constexpr (APPROX) {
+            if (!approx) return;
+#pragma unroll
+            for (int t = 0; t < kSelWgSlots; ++t)
+                if (base + (uint32_t)t * kNT < n) er[t] = a.norms[kr[t] != kNoKey ? (uint32_t)kr[t] : 0u];
+#pragma unroll
+            for (int t = 0; t < kSelWgSlots; ++t) er[t] = __builtin_fmaf(a.mcoef, qn + er[t], a.mabs);
+        }
+    };
+    if (n <= kSpan) load(0);
+    // f(key, rank, error) over the thread's survivors, every lane of a wave together
+    auto each = [&](auto&& f) {
+        for (uint32_t base = 0; base < n; base += kSpan) {
+            if (n > kSpan) load(base);
+#pragma unroll
+            for (int t = 0; t < kSelWgSlots; ++t)
+                if (base + (uint32_t)t * kNT < n) f(kr[t], key_rank(kr[t]), approx ? er[APPROX ? t : 0] : 0.0f);
+        }
+    };
+    // the range of the admissible keys' (upper bounds of) ranks
+    float mn = INFINITY, mx = -INFINITY;
+    uint32_t fin = 0, real = 0;
+    each([&](uint64_t key, float v, float e) {
+        const float u = v + e;
+        real += key != kNoKey;
+        if (key != kNoKey && u < FLT_MAX) {
+            mn = fminf(mn, u);
+            mx = fmaxf(mx, u);
+            ++fin;
+        }
+    });
+    mn = wave_min(mn);
+    mx = wave_max(mx);
+    for (int off = 32; off > 0; off >>= 1) {
+        fin += __shfl_xor(fin, off);
+        real += __shfl_xor(real, off);
     }
-    const int qi = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kW + wv);
-    if (qi >= nq || (a.active && !a.active[qi])) return;
-    select_wave_any<APPROX>(a, qi, hist[wv], keys[wv], lane, hard, nhard);
+    if (lane == 0) {
+        s_mn[wv] = mn;
+        s_mx[wv] = mx;
+        s_fin[wv] = fin;
+        s_real[wv] = real;
+    }
+    for (int i = tid; i < 1024; i += kNT) hist[i] = 0;
+    if (tid == 0) s_nc = 0;
+    __syncthreads();
+    fin = real = 0;
+#pragma unroll
+    for (int w = 0; w < kW; ++w) {
+        mn = fminf(mn, s_mn[w]);
+        mx = fmaxf(mx, s_mx[w]);
+        fin += s_fin[w];
+        real += s_real[w];
+    }
+    // candidates: every key, or those up to the bin of the k-th of 1024;
+    // approximate ones by lower bound against the bin's upper edge (widened
+    // past the binning's rounding)
+    const bool thin = approx ? fin >= (uint32_t)a.k : fin > (uint32_t)max(kSelThin, a.k);
+    const float w1 = (mx - mn) * (1.0f / 1024.0f);
+    const float inv1 = w1 > 0.0f ? 1.0f / w1 : 0.0f;
+    int b1 = 1023;
+    float U = INFINITY;
+    if (thin) {
+        each([&](uint64_t key, float v, float e) {
+            if (key != kNoKey && v + e < FLT_MAX) atomicAdd(&hist[lin_bin1024(v + e, mn, inv1)], 1u);
+        });
+        __syncthreads();
+        b1 = wave_find_bin1024(hist, (uint32_t)a.k, lane);
+        const float edge = inv1 > 0.0f && b1 < 1023 ? mn + (float)(b1 + 1) * w1 : mx;
+        U = fminf(mx, edge + 0x1p-16f * (fabsf(mn) + fabsf(mx) + w1));
+    }
+    each([&](uint64_t key, float v, float e) {
+        bool take = key != kNoKey;
+        if (approx) take = take && !(v - e > U);
+        else take = key < key_limit() && (!thin || lin_bin1024(v, mn, inv1) <= b1);
+        const uint64_t mk = __ballot(take);
+        if (mk == 0) return;
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&s_nc, (uint32_t)__popcll(mk));
+        at = __builtin_amdgcn_readfirstlane(at) + lanes_below(mk);
+        if (take && at < (uint32_t)kSelSort) kk[at] = key;
+    });
+    __syncthreads();
+    const uint32_t nc = s_nc;
+    if (nc > (uint32_t)kSelSort) return false;
+    if (tid == 0) a.scnt[qi] = 0;  // read by every thread at the start
+    uint32_t n2 = 64;
+    while (n2 < nc) n2 <<= 1;
+    // final keys: the canonical distance (rescored where approximate) and the id
+    const uint32_t* ids = ids8 ? a.ids8 : a.ids;
+    for (uint32_t i = tid; i < n2; i += kNT) {
+        uint64_t key = ~0ull;
+        if (i < nc) {
+            const uint32_t pos = (uint32_t)kk[i];
+            const uint32_t id = ids[pos];
+            float r = key_rank(kk[i]);
+            if (approx) {
+                const float4* tp = a.codes + (size_t)(pos / 64) * a.nquad * 64 + (pos % 64);
+                const float4* q = a.q + (size_t)qi * a.nquad;
+                r = a.metric == kL2 ? chain_of<kL2>(q, tp, a.nquad) : chain_of<kIP>(q, tp, a.nquad);
+            }
+            if (r < FLT_MAX) key = make_key(r, id);  // the heap's strict admission
+        }
+        kk[i] = key;
+    }
+    __syncthreads();
+    if (n2 > 128) {
+        lds_sort<kNT>(kk, (int)n2);
+    } else {
+        if (wv == 0) wave_sort(kk, n2, lane);
+        __syncthreads();
+    }
+    if (tid == 0 && a.stats) atomicAdd(&a.stats[3], (unsigned long long)(approx ? real : fin));  // (padding keys not counted)
+    const uint64_t kth = (uint32_t)a.k <= n2 ? kk[a.k - 1] : ~0ull;
+    const bool full = kth < key_limit();
+    if (overflow || (a.check_tau && !(full && key_rank(kth) <= tau))) {
+        if (tid == 0) {
+            a.rescan_tau[qi] = full ? key_rank(kth) : FLT_MAX;
+            a.flist[atomicAdd(a.fcount, 1u)] = qi;
+            if (a.stats) atomicAdd(&a.stats[a.fb_slot], 1ull);
+            if (a.stats && overflow && a.fb_slot == 4) atomicAdd(&a.stats[6], 1ull);  // first pass
+        }
+        return true;
+    }
+    for (int i = tid; i < a.k; i += kNT) {
+        const uint64_t key = (uint32_t)i < n2 ? kk[i] : ~0ull;
+        const bool ok = key < key_limit();
+        a.out_d[(size_t)qi * a.k + i] = ok ? dist_of_rank(a.metric, key_rank(key)) : a.metric == kL2 ? FLT_MAX : -FLT_MAX;
+        a.out_i[(size_t)qi * a.k + i] = ok ? (int64_t)(uint32_t)key : -1;
+    }
+    return true;
 }
 
+// One workgroup per query, or, with a query list, a grid that walks the list.
+template <bool APPROX>
+__global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void select_kernel(SelArgs a) {
+    const uint32_t nl = a.qlist ? *a.qcount : gridDim.x;
+    for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
+        __syncthreads();  // the previous query's LDS reads are done
+        const int qi = __builtin_amdgcn_readfirstlane(a.qlist ? a.qlist[i] : (int32_t)i);
+        if (!select_wg<APPROX>(a, qi)) select_one(a, qi);
+    }
+}
+
+// Batches of at most this many queries are selected by a workgroup each (a
+// wave each, then a workgroup): searches of 1000 plain queries 424 and 411 us,
+// 1200 of 300 dims 625 and 562, 3000 of an integer list 235 and 234, 4000 real
+// 406 and 413, 10k under the learned bound 473 and 522.
+constexpr int kSelWgQueries = 3072;
+
+// All queries' selection: `hard` and *nhard (zero) take the queries that the
+// wave form hands over.
+template <bool APPROX>
+void launch_select(SelArgs a, int64_t n, size_t lds, int32_t* hard, uint32_t* nhard, hipStream_t s) {
+    if (n > kSelWgQueries) {
+        hipLaunchKernelGGL(select_wave_kernel<APPROX>, dim3((unsigned)((n + 3) / 4)), dim3(kNT), 0, s, a, (int)n, hard, nhard);
+        a.qlist = hard;
+        a.qcount = nhard;
+    }
+    hipLaunchKernelGGL(select_kernel<APPROX>, dim3((unsigned)(a.qlist ? std::min<int64_t>(n, 1024) : n)), dim3(kNT), lds, s, a);
+}
 
 // Rescue pass over the listed queries.  Its bound: the k-th distance among
 // the rows the first pass kept (an upper bound of D_k when there were k of
@@ -2193,8 +2280,10 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(4))) void s
 // row, with the canonical FP32 chain.  Rows within the bound are appended to
 // the query's survivor buffer with one counted atomic per wave and tile.
 // The keys hold canonical distances, so the one-wave selection applies as
-// is.  Pairs that the list's radius interval excludes are skipped, as in the
-// plan.
+// is (in a launch of its own: with the workgroup that ends a query's last pair
+// selecting, the fence that each pair then needs took 471 queries from 1.7 to
+// 5.9 ms).  Pairs that the list's radius interval excludes are skipped, as in
+// the plan.
 constexpr float kRescueGrow = 1.25f;
 constexpr int kRescueNT = 1024;
 
@@ -2672,18 +2761,11 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         return HIVF_OK;
     };
 
-    // Top-k of every query's survivors (all queries, or the listed ones):
-    // one wave per query where the keys are exact, the rest (listed by the
-    // wave kernel) one workgroup per query.  Queries that cannot be finished
-    // exactly are flagged in fb_out, with a rescan bound in rtau_out, and
-    // appended to the pass's rescue list.
-    auto select = [&](const int32_t* active, const int32_t* qlist, const uint32_t* qcount, const float* tau_in,
-                      int32_t* fb_out, float* rtau_out, bool check_tau, int fb_slot, bool first,
-                      bool keys_exact) -> hipError_t {
-        SelArgs sa;
-        sa.active = active;
-        sa.qlist = qlist;
-        sa.qcount = qcount;
+    // What a selection needs: the first pass's of every query, or the rescue
+    // pass's.  Queries that cannot be finished exactly are appended to the
+    // pass's rescue list, with a rescan bound in rtau_out.
+    auto sel_args = [&](const float* tau_in, float* rtau_out, bool check_tau, bool first) {
+        SelArgs sa{};
         sa.scnt = scnt;
         sa.sbuf = sbuf;
         sa.cap = cap;
@@ -2697,7 +2779,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.exact_ok = exact_bf16;
         sa.i8 = i8;
         sa.all_int = all_int;
-        sa.keys_exact = keys_exact ? 1 : 0;
+        sa.keys_exact = first ? 0 : 1;
         sa.tau = tau_in;
         sa.check_tau = check_tau ? 1 : 0;
         sa.ids = h->d_ids.p;
@@ -2709,41 +2791,24 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.metric = kL2;
         sa.out_d = D;
         sa.out_i = I;
-        sa.fallback = fb_out;
         sa.rescan_tau = rtau_out;
         sa.stats = timing ? h->d_stats.p : nullptr;
-        sa.fb_slot = fb_slot;
+        sa.fb_slot = first ? 4 : 5;
         sa.flist = first ? fbl : fbl2;
         sa.fcount = fbc + (first ? 0 : 1);
-        sa.lcnt = lcnt;
-        sa.nlist = (int)nlist;
-        uint32_t* nhard = fbc + (first ? 2 : 3);
-        const int64_t wgs = (n + 3) / 4;
-        const dim3 sgrid((unsigned)(qlist ? std::min<int64_t>(wgs, 1024) : wgs));
-        if (f16) hipLaunchKernelGGL(select_wave_kernel<true>, sgrid, dim3(kNT), 0, s, sa, (int)n, shard, nhard);
-        else hipLaunchKernelGGL(select_wave_kernel<false>, sgrid, dim3(kNT), 0, s, sa, (int)n, shard, nhard);
-        sa.active = nullptr;
-        sa.qlist = shard;
-        sa.qcount = nhard;
-        hipLaunchKernelGGL(select_kernel, dim3((unsigned)std::min<int64_t>(n, 1024)), dim3(kNT),
-                           h->nquad * sizeof(float4), s, sa);
-        return hipGetLastError();
+        return sa;
     };
 
-    // One pass: invert the probes of the active queries, batched scan under
-    // tau_in, select.  Queries it cannot finish exactly are flagged in
-    // fb_out with a rescan bound in rtau_out.
-    auto pass = [&](const int32_t* active, const int32_t* qlist, const uint32_t* qcount, const float* tau_in,
-                    int32_t* fb_out, float* rtau_out, bool check_tau,
-                    int fb_slot, bool first, int rt) -> int {
-        unsigned long long* cand = (timing && first) ? h->d_stats.p : nullptr;
+    // First pass: invert the probes, batched scan under tau, select.
+    auto pass = [&](bool check_tau, int rt) -> int {
+        unsigned long long* cand = timing ? h->d_stats.p : nullptr;
         PairFilter pf;
         pf.cd = h->d_cd.p;
-        pf.tau = tau_in;
+        pf.tau = tau;
         pf.lbound = static_cast<const float2*>(B.lbound);
-        HIP_TRY(h, launch_plan(pl, h->d_probes.p, h->d_cd.p, h->d_size.p, PairSet{npq, active, qlist, qcount, (int)n, P}, pf,
+        HIP_TRY(h, launch_plan(pl, h->d_probes.p, h->d_cd.p, h->d_size.p, PairSet{npq, nullptr, nullptr, nullptr, (int)n, P}, pf,
                                qc, (uint32_t)rt, qint, (int)n, all_int, cand, s));
-        if (timing && first) HIP_TRY(h, hipEventRecord(h->ev[6], s));
+        if (timing) HIP_TRY(h, hipEventRecord(h->ev[6], s));
         BatchArgs ba;
         ba.items = items;
         ba.meta = meta;
@@ -2757,7 +2822,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         ba.norms = h->d_norms.p;
         ba.list_tile_off = h->d_tile_off.p;
         ba.list_size = h->d_size.p;
-        ba.tau = tau_in;
+        ba.tau = tau;
         ba.nkc = nkc;
         ba.aug = B.aug;
         ba.dpad16 = (int)dpad16;
@@ -2848,8 +2913,11 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
             hipLaunchKernelGGL((batched_scan_kernel<32, 1, false>), grid, dim3(kNT), 0, s, ba);
         }
         HIP_TRY(h, hipGetLastError());
-        if (timing && first) HIP_TRY(h, hipEventRecord(h->ev[3], s));
-        HIP_TRY(h, select(active, qlist, qcount, tau_in, fb_out, rtau_out, check_tau, fb_slot, first, false));
+        if (timing) HIP_TRY(h, hipEventRecord(h->ev[3], s));
+        const SelArgs sa = sel_args(tau, rtau, check_tau, true);
+        const size_t lds = h->nquad * sizeof(float4);
+        if (f16) launch_select<true>(sa, n, lds, shard, fbc + 2, s);
+        else launch_select<false>(sa, n, lds, shard, fbc + 2, s);
         HIP_TRY(h, hipGetLastError());
         return HIVF_OK;
     };
@@ -2863,7 +2931,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                      : warmup(tau, nullptr, nullptr, nullptr);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
-    rc = pass(nullptr, nullptr, nullptr, tau, fb, rtau, learned, 4, true, rt_items);
+    rc = pass(learned, rt_items);
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[4], s));
     // pass 2: the flagged queries, each (query, probed list, tile group) a
@@ -2901,8 +2969,12 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         ra.nkc8 = B.nkc8;
         hipLaunchKernelGGL(pair_scan_kernel, dim3((unsigned)std::min<int64_t>(n * P, 2048)), dim3(kRescueNT),
                            h->nquad * sizeof(float4), s, ra);
+        SelArgs sa = sel_args(tau2, rtau2, true, false);
+        sa.qlist = fbl;
+        sa.qcount = fbc;
+        hipLaunchKernelGGL(select_kernel<false>, dim3((unsigned)std::min<int64_t>(n, 1024)), dim3(kNT),
+                           h->nquad * sizeof(float4), s, sa);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, select(nullptr, fbl, fbc, tau2, fb2, rtau2, true, 5, false, true));
     }
     // last resort: exact per-query rescan of what pass 2 could not finish
     ScanArgs f{};
@@ -3168,20 +3240,12 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         sa.metric = h->metric;
         sa.out_d = D + q0 * k;
         sa.out_i = I + q0 * k;
-        sa.fallback = fb;
         sa.rescan_tau = (float*)at(o_rtau);
         sa.flist = (int32_t*)at(o_fbl);
         sa.fcount = fbc;
-        sa.lcnt = lcnt;
-        sa.nlist = 0;  // (cleared with the chunk's counters)
         int32_t* hard = (int32_t*)at(o_hard);
-        const dim3 sgrid((unsigned)((m + 3) / 4));
-        if (split) hipLaunchKernelGGL(select_wave_kernel<true>, sgrid, dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
-        else hipLaunchKernelGGL(select_wave_kernel<false>, sgrid, dim3(kNT), 0, s, sa, (int)m, hard, fbc + 2);
-        sa.qlist = hard;
-        sa.qcount = fbc + 2;
-        hipLaunchKernelGGL(select_kernel, dim3((unsigned)std::min<int64_t>(m, 1024)), dim3(kNT),
-                           split ? h->nquad * sizeof(float4) : 0, s, sa);
+        if (split) launch_select<true>(sa, m, h->nquad * sizeof(float4), hard, fbc + 2, s);
+        else launch_select<false>(sa, m, 0, hard, fbc + 2, s);
         HIP_TRY(h, hipGetLastError());
         // survivors past the buffer: the query's lists scanned by the per-query kernel
         ScanArgs f = w;
