@@ -2502,6 +2502,7 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
 #include "flat.hpp"
 #include "split.hpp"
+#include "warm.hpp"
 
 namespace hivf {
 
@@ -2737,9 +2738,42 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         if (!prepped) hipLaunchKernelGGL(prep_kernel, dim3((unsigned)n), dim3(64), 0, s, pa);
     }
 
-    // Warm-up bound (src/Index.cpp:999-1051) of all queries, or of the
-    // flagged ones only.
-    auto warmup = [&](float* out, const int32_t* qlist, const uint32_t* qcount, const float* cap_by) -> int {
+    // Warm-up bound (src/Index.cpp:999-1051): from the shadow where it is int8
+    // or FP16 and the rows fit, else by the per-query FP32 scan.
+    auto warmup = [&]() -> int {
+        const int W = p.warmup_list_size > 0 ? p.warmup_list_size : (int)k, L = std::min(P, p.warmup_lists > 0 ? p.warmup_lists : 10);
+        if ((i8 || f16) && warm_fits(L, W)) {
+            WarmArgs w{};
+            w.lists = h->lists();
+            w.q = q;
+            w.probes = h->d_probes.p;
+            w.P = P;
+            w.npq = npq;
+            w.L = L;
+            w.W = W;
+            w.k = (int)k;
+            w.qint = qint;
+            w.x8 = static_cast<const i32x4*>(B.x8);
+            w.xn8 = static_cast<const int32_t*>(B.xn8);
+            w.q8 = q8;
+            w.qn8 = qn8;
+            w.dpad32 = dpad32;
+            w.xbf = static_cast<const uint16_t*>(B.bf16);
+            w.qbf = qbf;
+            w.norms = h->d_norms.p;
+            w.qnorm = qnorm;
+            w.nkc = nkc;
+            w.dpad16 = (int)dpad16;
+            w.dot_scale = f16 ? -2.0f / (B.f16_scale * B.f16_scale) : 0.0f;
+            w.mcoef = mcoef;
+            w.mabs = mabs;
+            w.out = tau;
+            if (!i8) hipLaunchKernelGGL(warm_kernel<0>, dim3((unsigned)n), dim3(kNT), 0, s, w);
+            else if (B.nkc8 == 4) hipLaunchKernelGGL(warm_kernel<4>, dim3((unsigned)n), dim3(kNT), 0, s, w);
+            else hipLaunchKernelGGL(warm_kernel<8>, dim3((unsigned)n), dim3(kNT), 0, s, w);
+            HIP_TRY(h, hipGetLastError());
+            return HIVF_OK;
+        }
         ScanArgs w{};
         w.lists = h->lists();
         w.q = q;
@@ -2751,12 +2785,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         w.k = (int)k;
         w.block_dims = (int)h->d;
         w.nblocks = 1;
-        w.row_limit = p.warmup_list_size > 0 ? p.warmup_list_size : (int)k;
-        w.warm_lists = p.warmup_lists > 0 ? p.warmup_lists : 10;
-        w.out_tau = out;
-        w.tau_cap = cap_by;
-        w.qlist = qlist;
-        w.qcount = qcount;
+        w.row_limit = W;
+        w.warm_lists = L;
+        w.out_tau = tau;
         HIP_TRY(h, launch_scan(w, kScanWarmup, h->metric, s));
         return HIVF_OK;
     };
@@ -2928,7 +2959,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     const TauCap tc{h->d_probes.p, h->d_size.p, h->d_tile_off.p, B.i8 ? static_cast<const float2*>(B.rbound8) : nullptr,
                     static_cast<const float2*>(B.lbound), (int)k};
     int rc = learned ? run_tau_model(h, q, n, P, npq, tau, s, h->lists_uint8 || h->lists_sane ? &tc : nullptr)
-                     : warmup(tau, nullptr, nullptr, nullptr);
+                     : warmup();
     if (rc) return rc;
     if (timing) HIP_TRY(h, hipEventRecord(h->ev[2], s));
     rc = pass(learned, rt_items);

@@ -263,7 +263,6 @@ __device__ void scan_one(const ScanArgs& a, const int qi, const int part = 0, co
             const int cnt = top.cnt;
             float v = sentinel<METRIC>();
             if (cnt >= a.k) v = dist_of_rank(METRIC, ord2f(wave_kth_rank(top.buf, cnt, a.k, lane)));
-            if (a.tau_cap) v = fminf(v, a.tau_cap[qi]);
             if (lane == 0) a.out_tau[qi] = v;
         }
     } else {

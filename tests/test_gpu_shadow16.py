@@ -48,3 +48,35 @@ def test_batched_real(rows, d, nlist, n, P, k, scale, offset, spread):
             D, I, _ = idx.search(n, xq, k, params=hx.make_params(nprobe=P, algo=hx.ALGO_BATCHED, tau=tau, batch_rows=rpi))
             assert np.array_equal(I, OI), f"{(I != OI).sum()} ids differ"
             assert np.array_equal(D.view(np.uint32), OD.view(np.uint32))
+
+
+@pytest.mark.parametrize("data", ["int", "mixed", "real", "dup"])
+@pytest.mark.parametrize("d", [3, 128, 200, 420])
+@pytest.mark.parametrize("L,W,k", [(0, 0, 1), (0, 0, 50), (3, 33, 100), (1, 64, 65), (5, 1000, 200), (12, 340, 400), (40, 70, 30)])
+def test_warmup_from_the_shadow(d, data, L, W, k):
+    """The bound from the shadow's first rows: lists shorter and longer than
+    the rows taken, counts around whole tiles, fewer rows than k (no bound),
+    more than the kernel holds (the FP32 scan's bound), queries that are not
+    integer among integer ones."""
+    print(f"[case] warm {data} d={d} L={L} W={W} k={k}", flush=True)
+    rows, nlist, n, P = 5000, 20, 70, 12
+    r = np.random.default_rng(d + k)
+    xb, xq = (r.normal(0, 40, (m, d)) + 100 for m in (rows, n))
+    if data != "real":
+        xb, xq = (np.clip(np.rint(x), 0, 255) for x in (xb, xq))
+    if data == "mixed":
+        xq[::5] += 0.25
+    if data == "dup":
+        xb = xb[r.integers(0, 30, rows)]
+    xb, xq = xb.astype(np.float32), xq.astype(np.float32)
+    cent = xb[r.permutation(rows)[:nlist]].copy() if data != "dup" else np.clip(np.rint(r.normal(0, 40, (nlist, d)) + 100), 0, 255).astype(np.float32)
+    ix = oracle.Index.build(1, xb, cent)
+    idx = hx.Index(d, nlist, 1, 1)
+    idx.set_centroids(cent)
+    idx.add(rows, xb)
+    OD, OI, _ = ix.search(xq, P, k)
+    D, I, st = idx.search(n, xq, k, params=hx.make_params(nprobe=P, algo=hx.ALGO_BATCHED, tau=hx.TAU_WARMUP, warmup_lists=L,
+                                                          warmup_list_size=W))
+    assert np.array_equal(I, OI), f"{(I != OI).sum()} ids differ"
+    assert np.array_equal(D.view(np.uint32), OD.view(np.uint32))
+    assert st.exact_rescans == 0
