@@ -2501,6 +2501,7 @@ size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 }  // namespace hivf
 
 #include "flat.hpp"
+#include "shadow.hpp"
 #include "split.hpp"
 #include "warm.hpp"
 
@@ -2634,6 +2635,10 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     if (qg > qg_max) qg = 1;
     if (qg == 3) qg = 2;
     if (i8) qg = B.nkc8 == 4 ? std::min(qg, 2) : 1;  // the int8 kernel takes 32 or (d <= 128) 64 queries per item
+    // past 128 dims the FP16 shadow is scanned by workgroups, unless the caller
+    // or the tuning names the wave form's shape
+    const bool shadow_wg = f16 && nkc > 8 && p.batch_queries <= 0 && h->tune.qg <= 0;
+    if (shadow_wg) qg = kShadowItem / 32;
     int rt = p.batch_rows > 0 ? std::max(1, p.batch_rows / 32) : h->tune.item_tiles;
     // Rows per item: the caller's or the tuned size as it is; the default is at
     // most 1024, cut (cut_rt) where the (query, list) pairs are too few to fill
@@ -2642,10 +2647,12 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     // 135, 130 us; 300 x 16 (d = 200) 239, 213, 210, 212; 4000 x 32 433, 423,
     // 430, 448; 2000 x 50 (d = 420) 1024, 1020, 1052, 1141.  Int8 shadow 37 x
     // 24 132, 127, 120, 112; 1000 x 32 337, 271, 254, 261; 4000 x 32 433, 387,
-    // 377, 403; 10k x 64 (its scan) 430, 408, 459 at 256.
+    // 377, 403; 10k x 64 (its scan) 430, 408, 459 at 256.  Workgroup items repay
+    // their staged queries with more rows: 1024, 512, 256 rows 711, 741, 864 us at 2000
+    // x 50 (d = 420), 233, 249, 254 at 800 x 32 (d = 200).
     const bool cut_rt = rt <= 0;
     if (rt <= 0) rt = 32;
-    const int rt_items = !cut_rt ? rt : n * P <= 2048 ? 4 : n * P <= 65536 ? 8 : 16;
+    const int rt_items = !cut_rt ? rt : n * P <= 2048 ? 4 : shadow_wg ? 32 : n * P <= 65536 ? 8 : 16;
     int waves = p.batch_waves > 0 ? p.batch_waves : h->tune.waves_per_cu;
     if (waves <= 0) waves = 16;
     const uint32_t qc = 32u * qg;
@@ -2898,7 +2905,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                 hipLaunchKernelGGL((batched_scan_i8_kernel<8, 1>),
                                    resident_grid((batched_scan_i8_kernel<8, 1>), 2, B.cus, grid), dim3(kNT), 0, s, b8);
         }
-        if (f16) {
+        if (shadow_wg) {
+            hipLaunchKernelGGL(shadow_wg_kernel, dim3((unsigned)(B.cus * 2)), dim3(kNT), (size_t)shadow_chunks(nkc) * 2048, s, ba);
+        } else if (f16) {
             if (nkc <= 8 && qg == 4)
                 hipLaunchKernelGGL((batched_scan_kernel<8, 4, false, true>),
                                    resident_grid((batched_scan_kernel<8, 4, false, true>), 3, B.cus, grid), dim3(kNT), 0, s, ba);
