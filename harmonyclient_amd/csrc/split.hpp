@@ -125,26 +125,29 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
         const bool live = slot < nq;
         const int qid = a.lq[w.q0 + min(slot, nq - 1)];
         float4 raw[NKC][2];
-        float4 xv[4];
         // a tile's rows (lane: row slot, quads 4 kc + 2 half and the next) and
         // norms; quads past the row's end are the next tile's (or the arena's
         // zeroed tail), finite values that meet zeros of the queries' pieces
-        auto load = [&](int T) {
+        // (No branch around a load: with one, every product waits for all loads
+        // in flight.  Past nkc the last chunk meets zeros.  A chunk's next rows
+        // are loaded once it is split: with the whole tile's after the products,
+        // 40 registers spilled, and 2000 pruned queries took 379 us, now 334; 1000
+        // plain 406, now 392.)
+        const uint32_t lo = half * 128 + slot;
+        auto tile = [&](int T) {
             const int g = __builtin_amdgcn_readfirstlane(T0 + T);
-            const float4* p = a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32;
-            const uint32_t lo = half * 128 + slot;
-#pragma unroll
-            for (int kc = 0; kc < NKC; ++kc) {
-                if (kc < nkc) {
-                    raw[kc][0] = (p + kc * 256)[lo];
-                    raw[kc][1] = (p + kc * 256 + 64)[lo];
-                }
-            }
-            const float* np = a.norms + (size_t)g * 32;
-#pragma unroll
-            for (int r4 = 0; r4 < 4; ++r4) xv[r4] = *reinterpret_cast<const float4*>(np + r4 * 8 + half * 4);
+            return a.lists.codes + (size_t)(g >> 1) * nquad * 64 + (g & 1) * 32;
         };
-        load(w.t0);
+        auto load = [&](const float4* p, int kc) {
+            const float4* c = p + min(kc, nkc - 1) * 256;
+            raw[kc][0] = c[lo];
+            raw[kc][1] = (c + 64)[lo];
+        };
+        {
+            const float4* p = tile(w.t0);
+#pragma unroll
+            for (int kc = 0; kc < NKC; ++kc) load(p, kc);
+        }
         bf16x8 bh[NKC], bl[NKC];
         {
             const bf16x8* hp = reinterpret_cast<const bf16x8*>(a.qh + (size_t)qid * a.dpad16 + half * 8);
@@ -183,6 +186,20 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
         };
         for (int T = w.t0; T < te; ++T) {
             floatx16 acc = {};
+            float4 xv[4];
+            const float* np = a.norms + (size_t)__builtin_amdgcn_readfirstlane(T0 + T) * 32;
+#pragma unroll
+            for (int r4 = 0; r4 < 4; ++r4) xv[r4] = *reinterpret_cast<const float4*>(np + r4 * 8 + half * 4);
+            const float4* next = tile(min(T + 1, te - 1));
+#pragma unroll
+            for (int kc = 0; kc < NKC; ++kc) {
+                bf16x8 h, l;
+                split8<XLO>(raw[kc][0], raw[kc][1], h, l);
+                load(next, kc);
+                if constexpr (XLO) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, bh[kc], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bl[kc], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bh[kc], acc, 0, 0, 0);
+            }
             float xn[16];
 #pragma unroll
             for (int r4 = 0; r4 < 4; ++r4) {
@@ -191,16 +208,6 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
                 xn[r4 * 4 + 2] = xv[r4].z;
                 xn[r4 * 4 + 3] = xv[r4].w;
             }
-#pragma unroll
-            for (int kc = 0; kc < NKC; ++kc) {
-                if (kc >= nkc) break;
-                bf16x8 h, l;
-                split8<XLO>(raw[kc][0], raw[kc][1], h, l);
-                if constexpr (XLO) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, bh[kc], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bl[kc], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bh[kc], acc, 0, 0, 0);
-            }
-            load(min(T + 1, te - 1));
             const uint32_t m = split_pass<METRIC>(acc, xn, qn, rtau, a.coef, tile_rows_ok(rows - T * 32, half));
             if (__ballot(m != 0) == 0) continue;
             const uint32_t cg = (uint32_t)__builtin_popcount(m);
@@ -222,15 +229,16 @@ __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(2))) void s
 
 // d <= 512: a workgroup of 8 waves per item.  The queries' pieces of all dim
 // chunks are staged in LDS once per item (2 KB per 16 dims, up to 64 KB) and
-// read by every wave; the waves stride the item's tiles, 4 chunks of rows
-// loaded while the 4 before are split and multiplied.
-constexpr int kSplitWgNT = 512;
+// read by every wave; the waves stride the item's tiles, 2 chunks of rows
+// loaded while the 2 before are split and multiplied (4: registers spill, 500 inner
+// products of 201 dims 183 us against 181, 1000 of 150 dims 291 against 276).
+constexpr int kSplitWgNT = 512, kSplitChunks = 2;
 
 template <int METRIC, bool XLO>
 __global__ __launch_bounds__(kSplitWgNT) __attribute__((amdgpu_waves_per_eu(4))) void split_wg_kernel(SplitArgs a) {
-    extern __shared__ bf16x8 sb[];  // [hi, lo][nkc][64 lanes]
+    extern __shared__ bf16x8 sb[];  // [hi, lo][kC nch][64 lanes], zeros past nkc
     __shared__ uint32_t s_it;
-    constexpr int kW = kSplitWgNT / 64, kC = 4;
+    constexpr int kW = kSplitWgNT / 64, kC = kSplitChunks;
     const int tid = threadIdx.x, lane = tid & 63, half = lane >> 5, slot = lane & 31;
     const int wv = __builtin_amdgcn_readfirstlane(tid / 64);
     const int nquad = a.lists.nquad, nkc = a.nkc;
@@ -259,10 +267,11 @@ __global__ __launch_bounds__(kSplitWgNT) __attribute__((amdgpu_waves_per_eu(4)))
         const int rows = a.lists.list_size[list];
         const int T0 = a.lists.list_tile_off[list] * 2;
         const int te = min((rows + 31) >> 5, w.t0 + (w.nq >> 16));
-        for (int e = tid; e < 2 * nkc * 64; e += kSplitWgNT) {
-            const int l = e & 63, kc = (e >> 6) % nkc, lo = (e >> 6) / nkc;
+        for (int e = tid; e < 2 * nch * kC * 64; e += kSplitWgNT) {
+            const int l = e & 63, lo = (e >> 6) >= nch * kC, kc = (e >> 6) - lo * nch * kC;
             const int q = a.lq[w.q0 + min(l & 31, nq - 1)];
-            sb[e] = *reinterpret_cast<const bf16x8*>((lo ? a.ql : a.qh) + (size_t)q * a.dpad16 + kc * 16 + (l >> 5) * 8);
+            const bf16x8 z = {};
+            sb[e] = kc < nkc ? *reinterpret_cast<const bf16x8*>((lo ? a.ql : a.qh) + (size_t)q * a.dpad16 + kc * 16 + (l >> 5) * 8) : z;
         }
         const int qid = a.lq[w.q0 + min(slot, nq - 1)];
         const float qn = a.qn[qid];
@@ -281,11 +290,9 @@ __global__ __launch_bounds__(kSplitWgNT) __attribute__((amdgpu_waves_per_eu(4)))
             const uint32_t lo = half * 128 + slot;
 #pragma unroll
             for (int c = 0; c < kC; ++c) {
-                const int kc = ch * kC + c;
-                if (kc < nkc) {
-                    raw[c][0] = (p + kc * 256)[lo];
-                    raw[c][1] = (p + kc * 256 + 64)[lo];
-                }
+                const int kc = min(ch * kC + c, nkc - 1);  // (no branch, as above)
+                raw[c][0] = (p + kc * 256)[lo];
+                raw[c][1] = (p + kc * 256 + 64)[lo];
             }
         };
         if (w.t0 + wv < te) load(ra, w.t0 + wv, 0);
@@ -299,14 +306,12 @@ __global__ __launch_bounds__(kSplitWgNT) __attribute__((amdgpu_waves_per_eu(4)))
 #pragma unroll
                 for (int c = 0; c < kC; ++c) {
                     const int kc = ch * kC + c;
-                    if (kc < nkc) {
-                        const bf16x8 bh = sb[(size_t)kc * 64 + lane], bl = sb[(size_t)(nkc + kc) * 64 + lane];
-                        bf16x8 h, l;
-                        split8<XLO>(raw[c][0], raw[c][1], h, l);
-                        if constexpr (XLO) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, bh, acc, 0, 0, 0);
-                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bl, acc, 0, 0, 0);
-                        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bh, acc, 0, 0, 0);
-                    }
+                    const bf16x8 bh = sb[(size_t)kc * 64 + lane], bl = sb[(size_t)(nch * kC + kc) * 64 + lane];
+                    bf16x8 h, l;
+                    split8<XLO>(raw[c][0], raw[c][1], h, l);
+                    if constexpr (XLO) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l, bh, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bl, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h, bh, acc, 0, 0, 0);
                 }
             };
             for (int ch = 0; ch < nch; ch += 2) {
@@ -371,7 +376,7 @@ void launch_split(const SplitArgs& a, bool l2, bool xlo, int cus, hipStream_t s)
         else if (a.nkc <= 8)
             hipLaunchKernelGGL((split_wave_kernel<M, 8, X>), dim3(cus * 2), dim3(kNT), 0, s, a);
         else
-            hipLaunchKernelGGL((split_wg_kernel<M, X>), dim3(cus * 2), dim3(kSplitWgNT), (size_t)a.nkc * 2048, s, a);
+            hipLaunchKernelGGL((split_wg_kernel<M, X>), dim3(cus * 2), dim3(kSplitWgNT), (size_t)((a.nkc + 2 * kSplitChunks - 1) / (2 * kSplitChunks) * 2 * kSplitChunks) * 2048, s, a);
     };
     using std::integral_constant;
     if (l2 && xlo) go(integral_constant<int, kL2>{}, integral_constant<bool, true>{});
