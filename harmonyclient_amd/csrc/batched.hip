@@ -3041,9 +3041,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     HIP_TRY(h, launch_scan(f, kScanPruned, h->metric, s));
     if (timing) {
         HIP_TRY(h, hipEventRecord(h->ev[5], s));
-        HIP_TRY(h, hipEventSynchronize(h->ev[5]));
-        unsigned long long c[8];
-        HIP_TRY(h, hipMemcpy(c, h->d_stats.p, sizeof(c), hipMemcpyDeviceToHost));
+        unsigned long long c[9];
+        rc = read_counts(h, all_int, c, s);
+        if (rc) return rc;
         std::memset(st, 0, sizeof(*st));
         st->coarse_ms = elapsed_ms(h->ev[0], h->ev[1]);
         st->tau_ms = elapsed_ms(h->ev[1], h->ev[2]);
@@ -3060,8 +3060,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         st->batch_rows = rt * 32;
         st->batch_waves = waves;
         st->plan_ms = elapsed_ms(h->ev[2], h->ev[6]);
-        uint32_t ai = 0;
-        HIP_TRY(h, hipMemcpy(&ai, all_int, sizeof(ai), hipMemcpyDeviceToHost));
+        const uint32_t ai = (uint32_t)c[8];
         st->scan_kind = (i8 && ai) ? 2 : ((B.aug && exact_bf16 && ai) ? 1 : 0);
         st->blocks_total = (int64_t)c[1];    // 32-row tiles of the first pass's work items
         st->blocks_skipped = (int64_t)c[2];  // of which skipped by the radius bound

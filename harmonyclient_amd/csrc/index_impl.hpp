@@ -74,6 +74,20 @@ struct PinnedRing {
     void release();
 };
 
+// Pinned host memory of a handle, grown as needed up to kMax, that kernels
+// write to directly.
+struct PinnedBuf {
+    static constexpr size_t kMax = 4u << 20;
+    char* p = nullptr;
+    size_t bytes = 0;
+    PinnedBuf() = default;
+    PinnedBuf(const PinnedBuf&) = delete;
+    PinnedBuf& operator=(const PinnedBuf&) = delete;
+    ~PinnedBuf() { release(); }
+    bool ensure(size_t need);  // false: above kMax, or no memory
+    void release();
+};
+
 // State of the MFMA coarse quantizer: the 3-piece BF16 centroid shadow and
 // per-search scratch.
 struct CoarseState {
@@ -127,6 +141,8 @@ struct hivf_index {
     hivf::DevBuf<float4> d_q;
     hivf::DevBuf<float> d_stage;  // unpadded host queries on their way to d_q
     hivf::PinnedRing ring;        // large uploads of rows
+    hivf::PinnedBuf io;           // queries and results of small host searches
+    hivf::PinnedBuf counts;       // a search's counters on their way to the host
     hivf::DevBuf<float> d_cd;
     hivf::DevBuf<int32_t> d_probes;
     hivf::DevBuf<int32_t> d_npq;
@@ -244,6 +260,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
              const hivf_search_params& p, float* D, int64_t* I, unsigned long long* stats, hipEvent_t tau_done,
              hipStream_t s);
+// Waits for the stream and reads the search's counters (d_stats) and, with
+// all_int, that flag into c[8].
+int read_counts(hivf_index* h, const uint32_t* all_int, unsigned long long (&c)[9], hipStream_t s);
 struct PrepArgs;  // prep.hpp
 // MFMA coarse quantizer (coarse.hip); HIVF_EUNSUPPORTED when d > 512.  With
 // prep, its query-preparation launch also runs the batched search's.
