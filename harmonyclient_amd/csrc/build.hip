@@ -207,42 +207,57 @@ __global__ void zero_u32_kernel(uint32_t* p, int64_t n) {
 // the mean rounded to FP32.  One 64-thread workgroup per centroid and 64
 // dims, a thread per dim.  The additions stay in row order (the result does
 // not depend on the schedule), so a long list is a serial chain; what bounded
-// it was a load waited for per row.  The rows are loaded kMeanRows at a time, the
-// next ones while the current are added: 131k x 96 rows over 512 centroids 479
-// -> 121 us, the longest list's chain.
-constexpr int kMeanRows = 32;
+// it was a load waited for per row, then per 32 rows.  Now kMeanRows x kMeanBufs
+// rows are in flight, their numbers loaded 64 at a time a round ahead: 131k x 96
+// rows over 512 centroids, a load per row 479 us, 32 rows ahead 105, now 58.
+constexpr int kMeanRows = 32, kMeanBufs = 4, kMeanRound = kMeanRows * kMeanBufs;
 
 __global__ __launch_bounds__(64) void centroid_mean_kernel(const float* __restrict__ x, int64_t ldx, int d,
                                                            const int32_t* __restrict__ members,
                                                            const int64_t* __restrict__ off,
                                                            float* __restrict__ cent) {
-    const int l = blockIdx.x;
+    const int l = blockIdx.x, lane = threadIdx.x;
     const int64_t m0 = off[l], m1 = off[l + 1];
     if (m1 == m0) return;  // keeps its value
-    const int j = blockIdx.y * 64 + threadIdx.x, jc = min(j, d - 1);
-    float a[kMeanRows], b[kMeanRows];
-    auto load = [&](float (&v)[kMeanRows], int64_t m) {  // (rows past the end: the last one again, not added)
+    const int j = blockIdx.y * 64 + lane, jc = min(j, d - 1);
+    float v[kMeanBufs][kMeanRows];
+    int32_t row[kMeanRound / 64], next[kMeanRound / 64];
+    // the rows of round m (past the end: the last one again, not added)
+    auto rows = [&](int32_t (&r)[kMeanRound / 64], int64_t m) {
 #pragma unroll
-        for (int t = 0; t < kMeanRows; ++t) v[t] = x[(int64_t)members[min(m + t, m1 - 1)] * ldx + jc];
+        for (int i = 0; i < kMeanRound / 64; ++i) r[i] = members[min(m + i * 64 + lane, m1 - 1)];
     };
-    double acc = 0.0;
-    auto add = [&](const float (&v)[kMeanRows], int64_t m) {
-        if (m + kMeanRows <= m1) {
+    auto load = [&](int u) {
 #pragma unroll
-            for (int t = 0; t < kMeanRows; ++t) acc += (double)v[t];
-        } else {
-#pragma unroll
-            for (int t = 0; t < kMeanRows; ++t)
-                if (m + t < m1) acc += (double)v[t];
+        for (int t = 0; t < kMeanRows; ++t) {
+            const int at = u * kMeanRows + t;
+            v[u][t] = x[(int64_t)__builtin_amdgcn_readlane(row[at / 64], at % 64) * ldx + jc];
         }
     };
-    load(a, m0);
-    for (int64_t m = m0; m < m1; m += 2 * kMeanRows) {
-        load(b, m + kMeanRows);
-        add(a, m);
-        if (m + kMeanRows >= m1) break;
-        load(a, m + 2 * kMeanRows);
-        add(b, m + kMeanRows);
+    double acc = 0.0;
+    rows(row, m0);
+    rows(next, m0 + kMeanRound);
+#pragma unroll
+    for (int u = 0; u < kMeanBufs; ++u) load(u);
+    for (int64_t m = m0; m < m1; m += kMeanRound) {
+#pragma unroll
+        for (int i = 0; i < kMeanRound / 64; ++i) row[i] = next[i];
+        rows(next, m + 2 * kMeanRound);
+#pragma unroll
+        for (int u = 0; u < kMeanBufs; ++u) {
+            const int64_t mu = m + u * kMeanRows;
+            if (mu + kMeanRows <= m1) {
+#pragma unroll
+                for (int t = 0; t < kMeanRows; ++t) acc += (double)v[u][t];
+            } else {
+#pragma unroll
+                for (int t = 0; t < kMeanRows; ++t)
+                    if (mu + t < m1) acc += (double)v[u][t];
+            }
+            __builtin_amdgcn_sched_barrier(0);  // (the loads stay ahead of the next additions)
+            load(u);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (j < d) cent[(size_t)l * d + j] = (float)(acc / (double)(m1 - m0));
 }
