@@ -751,16 +751,18 @@ __global__ __launch_bounds__(kNT) void coarse_pick_wave_kernel(CoarsePickArgs a,
 // the exact chain.  The other rows (and any whose norms could overflow) go
 // through hard[] to the per-query kernel.
 //
-// What bounds it: the MFMA chain (6 products per 16 dims) and about 13 vector
+// What bounds it: the MFMA chain (3 products per 16 dims) and about 9 vector
 // operations per (row, centroid).  A workgroup holds 256 (d <= 128) rows'
 // BF16 pieces in registers as B operands for the whole scan and streams the
 // centroid shadow through LDS, 8 dim chunks of a 32-centroid tile at a time
-// (24 KB, double buffered, read by all four waves), so the vector memory path
+// (16 KB, double buffered, read by all four waves), so the vector memory path
 // carries a quarter of what each wave reading the shadow itself would take.
-// Measured: 500k x 128 rows, 1024 centroids 0.82 ms (0.96 PFLOP/s issued, of
-// 1.18 that a large BF16 product reaches) against 13.4 ms for one workgroup
-// per row streaming every centroid; 131k x 96, 512 centroids 0.097 ms
-// against 1.54; a few rows in a thousand are handed over (5 us).
+// Measured: 131k x 96 rows over 512 centroids 1.54 ms for one workgroup per row
+// streaming every centroid; 92 us with the search's six products of three and
+// two pieces, 78 with three of two and two (their bound is three times as wide),
+// 71 with the row's part of the lower bound added after the scan (4 vector
+// operations less per pair); add of 500k x 128 over 1024 with its first search
+// 9.46 -> 9.13 ms by the last two.  A few rows in a thousand are handed over (5 us).
 struct AssignArgs {
     const float4* x;      // rows [n x nquad]
     int64_t n;
@@ -779,7 +781,7 @@ struct AssignArgs {
 };
 
 constexpr int kStageKc = 8;                           // 16-dim chunks of a stage
-constexpr int kStageFrags = 3 * kStageKc;             // 1 KiB fragments of a stage
+constexpr int kStageFrags = 2 * kStageKc;             // 1 KiB fragments of a stage (two of the three pieces)
 constexpr int kStageRegs = kStageFrags * 64 / kNT;    // 16-byte loads per thread and stage
 
 // NS stages of 8 dim chunks per tile (d <= 128 NS), QG groups of 32 rows per wave.
@@ -873,17 +875,13 @@ void assign_kernel(AssignArgs a) {
 #pragma unroll
             for (int kc = 0; kc < kStageKc; ++kc) {
                 if (ks * kStageKc + kc < nkc) {
-                    const bf16x8 a0 = A[(size_t)kc * 64], a1 = A[(size_t)(kStageKc + kc) * 64],
-                                 a2 = A[(size_t)(2 * kStageKc + kc) * 64];
+                    const bf16x8 a0 = A[(size_t)kc * 64], a1 = A[(size_t)(kStageKc + kc) * 64];
                     auto mm = [&](const bf16x8& av, const bf16x8 (&b)[QG][NS * kStageKc]) {
 #pragma unroll
                         for (int g = 0; g < QG; ++g)
                             acc[g] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, b[g][ks * kStageKc + kc], acc[g], 0, 0, 0);
                     };
-                    mm(a2, lr);
-                    mm(a1, lr);
                     mm(a0, lr);
-                    mm(a2, hr);
                     mm(a1, hr);
                     mm(a0, hr);
                 }
@@ -896,21 +894,17 @@ void assign_kernel(AssignArgs a) {
             }
             __syncthreads();
         }
-        const bool tail = T * 32 + 32 > a.nlist;
+        // lower bounds less the row's part, which is added after the scan
 #pragma unroll
         for (int r4 = 0; r4 < 4; ++r4) {
             const float cn[4] = {cv[r4].x, cv[r4].y, cv[r4].z, cv[r4].w};
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int c = T * 32 + r4 * 8 + half * 4 + e;
+                const float part = c < a.nlist ? __builtin_fmaf(METRIC == kL2 ? 1.0f - a.coef : -a.coef, cn[e], -kEabs) : INFINITY;
 #pragma unroll
-                for (int g = 0; g < QG; ++g) {
-                    const float dot = acc[g][r4 * 4 + e], s = qn[g] + cn[e];
-                    const float rank = METRIC == kL2 ? s - 2.0f * dot : -dot;
-                    float lb = rank - (a.coef * s + kEabs);
-                    if (tail && c >= a.nlist) lb = INFINITY;
-                    insert(g, lb, c);
-                }
+                for (int g = 0; g < QG; ++g)
+                    insert(g, __builtin_fmaf(METRIC == kL2 ? -2.0f : -1.0f, acc[g][r4 * 4 + e], part), c);
             }
         }
     }
@@ -923,7 +917,8 @@ void assign_kernel(AssignArgs a) {
         insert(g, o2, oc2);
         insert(g, o3, -1);
         const int k1 = __shfl(c1[g], slot), k2 = __shfl(c2[g], slot);
-        const float b1 = __shfl(l1[g], slot), b2 = __shfl(l2[g], slot), b3 = __shfl(l3[g], slot);
+        const float rowp = (METRIC == kL2 ? 1.0f - a.coef : -a.coef) * qn[g];
+        const float b1 = __shfl(l1[g], slot) + rowp, b2 = __shfl(l2[g], slot) + rowp, b3 = __shfl(l3[g], slot) + rowp;
         const int64_t r = r0 + g * 32 + slot;
         const bool live = r < a.n;
         // U: the first one's upper bound (lower bound + 2 E), widened past
@@ -981,6 +976,18 @@ float coarse_coef(int64_t d) {
     auto gamma = [&](double m) { return m * e / (1.0 - m * e); };
     const double c = std::ldexp(1.0, -16) * (1 + u) + 2 * gamma(6.0 * d) * (1 + 2 * u) * (1 + 2 * u) + 5 * e +
                      2 * gamma(d + 2.0);
+    return (float)(c * 1.01);
+}
+
+// The same for the assignment's three products of two pieces each: the pieces'
+// residuals and the dropped lo.lo product are 3 2^-16 (1 + u)^2 ||q|| ||c||, the
+// accumulation is of 3 d products.  The bound is three times as wide, and a row
+// still has two candidates at most nearly always.
+float assign_coef(int64_t d) {
+    const double u = 1.0 / 256.0, e = 1.0 / 16777216.0;
+    auto gamma = [&](double m) { return m * e / (1.0 - m * e); };
+    const double c = 3 * std::ldexp(1.0, -16) * (1 + u) * (1 + u) + 2 * gamma(3.0 * d) * (1 + 2 * u) * (1 + 2 * u) +
+                     5 * e + 2 * gamma(d + 2.0);
     return (float)(c * 1.01);
 }
 
@@ -1045,7 +1052,7 @@ int run_assign(hivf_index* h, const float4* x, int64_t n, bool need_dist, hipStr
     a.cn = h->d_cent_norm.p;
     a.crow = h->d_cent_rows.p;
     a.nlist = (int)h->nlist;
-    a.coef = coarse_coef(h->d);
+    a.coef = assign_coef(h->d);
     a.cn_max = h->d_cent_max.p;
     a.need_dist = need_dist ? 1 : 0;
     a.out_d = h->d_cd.p;
