@@ -51,43 +51,78 @@ struct GemmArgs {
     int ldm;
 };
 
-// C = epilogue(A' B'): 64 x 64 output tile per 256-thread workgroup, 4 x 4
-// per thread, K in chunks of 16 staged in LDS; fixed summation order.
+// C = epilogue(A' B'): 32 x 64 output tile per 256-thread workgroup, 2 x 4
+// per thread, K in chunks of 16 staged in LDS, the next chunk's loads in flight
+// beside the products; fixed summation order (k ascending from zero).  What
+// bounds it is latency, 8 chunks of load, barrier and product: 8192 rows by 128 x
+// 128, 64 x 64 tiles on 128 workgroups with the loads waited for 29 us, now 18.
 __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
-    __shared__ float As[16][65];
-    __shared__ float Bs[16][65];
+    __shared__ __align__(16) float As[16][36];
+    __shared__ __align__(16) float Bs[16][68];
     const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int m0 = blockIdx.x * 64, n0 = blockIdx.y * 64;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < g.K; k0 += 16) {
-        // consecutive threads along the operand's contiguous index
+    const int m0 = blockIdx.x * 32, n0 = blockIdx.y * 64;
+    float ra[2], rb[4];
+    // consecutive threads along the operand's contiguous index
+    auto placeA = [&](int t, int& k, int& r) {
+        const int e = t * 256 + threadIdx.x;
+        k = g.transA ? e / 32 : e % 16;
+        r = g.transA ? e % 32 : e / 16;
+    };
+    auto placeB = [&](int t, int& k, int& r) {
+        const int e = t * 256 + threadIdx.x;
+        k = g.transB ? e % 16 : e / 64;
+        r = g.transB ? e / 16 : e % 64;
+    };
+    auto fetch = [&](int k0) {  // (positions outside read the nearest inside and count zero)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            int k, r;
+            placeA(t, k, r);
+            const int kc = min(k0 + k, g.K - 1), m = min(m0 + r, g.M - 1);
+            const float v = g.A[g.transA ? (size_t)kc * g.lda + m : (size_t)m * g.lda + kc];
+            ra[t] = m0 + r < g.M && k0 + k < g.K ? v : 0.0f;
+        }
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int e = t * 256 + threadIdx.x;
-            const int ka = g.transA ? e / 64 : e % 16, ra = g.transA ? e % 64 : e / 16;
-            const int kb = g.transB ? e % 16 : e / 64, rb = g.transB ? e / 16 : e % 64;
-            const int m = m0 + ra, n = n0 + rb;
-            As[ka][ra] = (m < g.M && k0 + ka < g.K) ? g.A[g.transA ? (size_t)(k0 + ka) * g.lda + m : (size_t)m * g.lda + k0 + ka] : 0.0f;
-            Bs[kb][rb] = (n < g.N && k0 + kb < g.K) ? g.B[g.transB ? (size_t)n * g.ldb + k0 + kb : (size_t)(k0 + kb) * g.ldb + n] : 0.0f;
+            int k, r;
+            placeB(t, k, r);
+            const int kc = min(k0 + k, g.K - 1), n = min(n0 + r, g.N - 1);
+            const float v = g.B[g.transB ? (size_t)n * g.ldb + kc : (size_t)kc * g.ldb + n];
+            rb[t] = n0 + r < g.N && k0 + k < g.K ? v : 0.0f;
+        }
+    };
+    float acc[2][4] = {};
+    fetch(0);
+    for (int k0 = 0; k0 < g.K; k0 += 16) {
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            int k, r;
+            placeA(t, k, r);
+            As[k][r] = ra[t];
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            int k, r;
+            placeB(t, k, r);
+            Bs[k][r] = rb[t];
         }
         __syncthreads();
+        if (k0 + 16 < g.K) fetch(k0 + 16);
 #pragma unroll
         for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
+            const float2 av = *reinterpret_cast<const float2*>(&As[kk][ty * 2]);
+            const float4 bv = *reinterpret_cast<const float4*>(&Bs[kk][tx * 4]);
+            const float a[2] = {av.x, av.y}, b[4] = {bv.x, bv.y, bv.z, bv.w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
+            for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
         }
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int m = m0 + ty * 4 + i;
+    for (int i = 0; i < 2; ++i) {
+        int m = m0 + ty * 2 + i;
         if (m >= g.M) continue;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -116,7 +151,8 @@ __global__ void dz2_kernel(const float* __restrict__ dy, const float* __restrict
 // as products with K = rows they filled 2 to 4 workgroups (1.6 ms each for
 // 8192 rows), and the bias sums one or two.  Cut into chunks they fill the
 // chip, and each FP32 chain is a chunk long instead of all rows: a gradient
-// over 8192 rows at 128 hidden units 5.47 -> 0.23 ms, its error against 64
+// over 8192 rows at 128 hidden units 5.47 -> 0.23 ms (0.21 with the next rows'
+// loads beside the products: 28 us of this kernel became 21), its error against 64
 // bits 2.5e-6 -> 1.5e-7 of the gradient's norm.  blockIdx.y:
 // the 64 x 64 tiles of W2's gradient (the first row of tiles also sums b2's),
 // then W1's (and b1's), then 64-column pieces of w3's (the first also b3's).
@@ -160,14 +196,27 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a) {
     const float* B = second ? a.dZ2 : a.dZ1;
     const int M = second ? a.hid : a.in;
     float acc[4][4] = {}, bias[4] = {};
+    // (the next 16 rows' loads in flight beside the products)
+    float ra[4], rb[4];
+    const int c = tid % 64, mc = min(m0 + c, M - 1), nc = min(n0 + c, a.hid - 1);
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int k = k0 + t * 4 + tid / 64, kc = min(k, r1 - 1);
+            const float x = A[(size_t)kc * M + mc], y = B[(size_t)kc * a.hid + nc];
+            ra[t] = m0 + c < M && k < r1 ? x : 0.0f;
+            rb[t] = n0 + c < a.hid && k < r1 ? y : 0.0f;
+        }
+    };
+    fetch(r0);
     for (int k0 = r0; k0 < r1; k0 += 16) {
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            const int e = t * 256 + tid, kk = e / 64, c = e % 64, k = k0 + kk;
-            As[kk][c] = (m0 + c < M && k < r1) ? A[(size_t)k * M + m0 + c] : 0.0f;
-            Bs[kk][c] = (n0 + c < a.hid && k < r1) ? B[(size_t)k * a.hid + n0 + c] : 0.0f;
+            As[t * 4 + tid / 64][c] = ra[t];
+            Bs[t * 4 + tid / 64][c] = rb[t];
         }
         __syncthreads();
+        if (k0 + 16 < r1) fetch(k0 + 16);
 #pragma unroll
         for (int kk = 0; kk < 16; ++kk) {
             const float4 av = *reinterpret_cast<const float4*>(&As[kk][ty * 4]);
@@ -504,7 +553,7 @@ namespace hivf {
 static hipError_t gemm(hipStream_t s, const float* A, int lda, int tA, const float* B, int ldb, int tB, float* C,
                        int ldc, int M, int N, int K, const float* bias, int relu, const float* mask, int ldm) {
     GemmArgs g{A, lda, tA, B, ldb, tB, C, ldc, M, N, K, bias, relu, mask, ldm};
-    hipLaunchKernelGGL(gemm_kernel, dim3(blocks(M, 64), blocks(N, 64)), dim3(256), 0, s, g);
+    hipLaunchKernelGGL(gemm_kernel, dim3(blocks(M, 32), blocks(N, 64)), dim3(256), 0, s, g);
     return hipGetLastError();
 }
 
