@@ -438,6 +438,16 @@ __global__ void fill_kernel(const int32_t* __restrict__ probes, const float* __r
 // Lists up to this many use the LDS-histogram planning kernels below.
 constexpr int kLdsLists = 8192;
 constexpr int kPlanEntries = 4096;  // (query, probe) entries per planning workgroup
+// Fewer where so few workgroups would leave each a chain of loads that the chip
+// waits for (their counts cost 4 bytes per class and list to write and scan):
+// 1024, 2048, 4096 entries, whole search: 500 x 20 (nlist 400) 174, 174, 179 us;
+// 3000 x 24 (512) 211, 212, 220; 2000 x 48 (1024) 326, 326, 330; 4096 x 64 321, 310,
+// 313; 10k x 64 509, 486, 472.
+inline int plan_entries(int64_t entries) { return entries <= 1 << 17 ? 1024 : entries <= 1 << 18 ? 2048 : kPlanEntries; }
+// Most planning workgroups of any pass of up to this many entries.
+inline int64_t plan_wgs(int64_t entries) {
+    return std::max((std::min<int64_t>(entries, 1 << 17) + 1023) / 1024, (entries + kPlanEntries - 1) / kPlanEntries);
+}
 
 // count_kernel with a per-workgroup LDS histogram: one global atomic per
 // (workgroup, list) instead of one per entry.
@@ -675,12 +685,12 @@ __device__ inline int entry_class(const Entry& x) {
 template <int C>
 __global__ __launch_bounds__(256) void count_wg_kernel(const int32_t* __restrict__ probes, PairSet ps,
                                                        const int32_t* __restrict__ list_size, int nlist,
-                                                       PairFilter pf, uint32_t* __restrict__ hwg,
+                                                       PairFilter pf, int per, uint32_t* __restrict__ hwg,
                                                        unsigned long long* cand) {
     __shared__ uint32_t hc[kWgSlots];  // [class][list]
     __shared__ unsigned long long s_c;
-    const int64_t e0 = (int64_t)blockIdx.x * kPlanEntries;
-    const int64_t e1 = min(ps.size(), e0 + kPlanEntries);
+    const int64_t e0 = (int64_t)blockIdx.x * per;
+    const int64_t e1 = min(ps.size(), e0 + per);
     const int nb = C * nlist;
     uint32_t* on = hwg + (size_t)blockIdx.x * nb;  // this workgroup's counts
     if (e0 >= e1) {  // whole workgroup: no entries, zero counts
@@ -909,7 +919,7 @@ __global__ void items_par_kernel(ItemArgs a) {
 template <int C>
 __global__ __launch_bounds__(256) void fill_wg_kernel(const int32_t* __restrict__ probes,
                                                       const float* __restrict__ cd, PairSet ps, int nlist,
-                                                      PairFilter pf, const uint32_t* __restrict__ hwg,
+                                                      PairFilter pf, int per, const uint32_t* __restrict__ hwg,
                                                       const uint32_t* __restrict__ qoff, int32_t* __restrict__ lq,
                                                       float* __restrict__ lqd, unsigned nfill, ItemArgs ia) {
     __shared__ uint32_t rc[kWgSlots];  // [class][list] next position; item offsets in the item workgroups
@@ -935,8 +945,8 @@ __global__ __launch_bounds__(256) void fill_wg_kernel(const int32_t* __restrict_
         }
         return;
     }
-    const int64_t e0 = (int64_t)blockIdx.x * kPlanEntries;
-    const int64_t e1 = min(ps.size(), e0 + kPlanEntries);
+    const int64_t e0 = (int64_t)blockIdx.x * per;
+    const int64_t e1 = min(ps.size(), e0 + per);
     if (e0 >= e1) return;  // whole workgroup
     const int nb = C * nlist;
     const uint32_t* on = hwg + (size_t)blockIdx.x * nb;
@@ -2441,7 +2451,7 @@ struct PlanBufs {
 
 // Words of a planning workgroup's per-(class, list) counts buffer.
 size_t plan_hwg_bytes(int64_t nlist, int64_t entries) {
-    return nlist * 2 <= kWgSlots ? (size_t)((entries + kPlanEntries - 1) / kPlanEntries + 1) * kWgSlots * 4 : 0;
+    return nlist * 2 <= kWgSlots ? (size_t)(plan_wgs(entries) + 1) * kWgSlots * 4 : 0;
 }
 
 // Inverts the pass's probes into work items of qc queries and rt 32-row tiles
@@ -2455,20 +2465,22 @@ hipError_t launch_plan(const PlanBufs& b, const int32_t* probes, const float* cd
     const unsigned gnp = (unsigned)((np + 255) / 256);
     const bool lds = nlist <= kLdsLists;
     const unsigned gpe = (unsigned)((np + kPlanEntries - 1) / kPlanEntries);
-    const int wgc = nlist * 8 <= kWgSlots ? 8 : nlist * 4 <= kWgSlots ? 4 : nlist * 2 <= kWgSlots ? 2 : 0;
+    // (classes by reach need radius intervals)
+    const int wgc = !pf.lbound && nlist * 2 <= kWgSlots ? 2 : nlist * 8 <= kWgSlots ? 8 : nlist * 4 <= kWgSlots ? 4 : nlist * 2 <= kWgSlots ? 2 : 0;
     const ItemArgs ia{b.lcnt, wgc ? b.lnear : nullptr, b.qoff, b.ioff, b.meta, list_size, nlist, qc, rt,
                       b.max_items, b.items};
     const unsigned iwg = (unsigned)((b.max_items + 255) / 256);
     if (wgc) {
-        const unsigned nwg = std::max(1u, gpe);
+        const int per = plan_entries(np);
+        const unsigned nwg = std::max(1u, (unsigned)((np + per - 1) / per));
         const dim3 g1(nwg), gs((unsigned)((nlist + 63) / 64)), gf(nwg + iwg);
         auto classes = [&](auto c) {
             constexpr int C = decltype(c)::value;
-            hipLaunchKernelGGL(count_wg_kernel<C>, g1, dim3(256), 0, s, probes, ps, list_size, nlist, pf, b.hwg, cand);
+            hipLaunchKernelGGL(count_wg_kernel<C>, g1, dim3(256), 0, s, probes, ps, list_size, nlist, pf, per, b.hwg, cand);
             hipLaunchKernelGGL(wg_scan_kernel<C>, gs, dim3(1024), 0, s, b.hwg, (int)nwg, nlist, b.lcnt, b.lnear);
             hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, b.lcnt, b.lnear, list_size, nlist, qc, rt,
                                b.qoff, b.lcur, b.lend, b.ioff, b.meta, qint, nint, all_int);
-            hipLaunchKernelGGL(fill_wg_kernel<C>, gf, dim3(256), 0, s, probes, cd, ps, nlist, pf, b.hwg, b.qoff, b.lq,
+            hipLaunchKernelGGL(fill_wg_kernel<C>, gf, dim3(256), 0, s, probes, cd, ps, nlist, pf, per, b.hwg, b.qoff, b.lq,
                                b.lqd, nwg, ia);
         };
         if (wgc == 8)
