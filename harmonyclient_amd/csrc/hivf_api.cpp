@@ -894,8 +894,8 @@ int hivf_index_search(hivf_index* h, int64_t n, const float* x, int64_t k, float
     // Small searches go through pinned memory: the queries' upload does not wait,
     // and the selections store their results there, so that the one wait is for
     // the counters: one query 159 us, now 94; 37 batched 255 and 168; 1000 plain
-    // (1.7 MB) 394 and 343, 3000 batched (3.4 MB) 561 and 473.  Larger ones copy from
-    // device buffers.
+    // (1.7 MB) 394 and 343.  Larger ones copy from device buffers (3.4 MB: 561 us, 473
+    // through pinned memory, whose making would cost the first search 1.4 ms).
     const size_t qb = ((size_t)n * h->d * sizeof(float) + 15) & ~(size_t)15, ib = (size_t)n * k * sizeof(int64_t),
                  db = (size_t)n * k * sizeof(float);
     if (qb + ib + db <= hivf::PinnedBuf::kMax && h->io.ensure(qb + ib + db)) {

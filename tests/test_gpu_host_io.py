@@ -1,4 +1,4 @@
-"""Host searches around the size that pinned buffers serve (4 MiB of queries
+"""Host searches around the size that pinned buffers serve (2 MiB of queries
 and results), growing and shrinking from call to call, against the device
 search of the same queries; counters as many as with device buffers."""
 import numpy as np
@@ -19,7 +19,7 @@ def test_sizes(algo, metric, d):
     idx = hx.Index(d, nlist, P, metric)
     idx.set_centroids(xb[:nlist].copy())
     idx.add(rows, xb)
-    edge = (4 << 20) // (4 * d + 12 * k)
+    edge = (2 << 20) // (4 * d + 12 * k)
     prm = hx.make_params(nprobe=P, algo=algo)
     for n in (1, edge - 1, 3, edge, edge + 1, 7, 2 * edge, 1):
         print(f"[case] n={n} d={d} algo={algo}", flush=True)
