@@ -134,10 +134,11 @@ __device__ __forceinline__ void flat_tiles(const FlatArgs& a, int tile, int left
     }
 }
 
-// Rank bound of a query: the warm-up bound, or below every rank for an absent one.
+// Rank bound of a query: the warm-up bound, or for an absent one NaN, which no
+// rank is within (an inner product of +inf ranks at -inf).
 template <int METRIC>
 __device__ inline float flat_rank_bound(const FlatArgs& a, int qi) {
-    return qi < 0 ? -INFINITY : METRIC == kL2 ? a.tau[qi] : -a.tau[qi];
+    return qi < 0 ? __builtin_nanf("") : METRIC == kL2 ? a.tau[qi] : -a.tau[qi];
 }
 
 // Queries of a list-major item, and how many of them share a pass over its
