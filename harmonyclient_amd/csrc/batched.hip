@@ -1580,7 +1580,8 @@ struct SelArgs {
     const float* norms;         // [rows] squared row norms
     float mcoef;                // margin of inexact keys: mcoef (||q||^2 + ||x||^2) + mabs
     float mabs;
-    float qn_max;               // APPROX: a query whose norm is not below it is flagged for the exact rescan
+    float qn_max;               // APPROX: a query whose norm is not below it is flagged for the exact rescan,
+    const int32_t* qover;       // and so is a query flagged here (FP16 shadow; null: none)
     int exact_ok;               // BF16 keys exact for integer queries
     int i8;                     // the int8 scan ran when *all_int
     const uint32_t* all_int;
@@ -2039,7 +2040,7 @@ __device__ void select_wave_any(const SelArgs& a, int qi, uint64_t* kk, int lane
     const bool ids8 = a.i8 && all_int;
     const bool exact = a.keys_exact || ids8 || (a.exact_ok && qint);
     if (total > min(64u * kSelRegSlots, a.cap) || a.k > kSelSort / 2 || (!exact && !APPROX) ||
-        (APPROX && !(a.qnorm[qi] < a.qn_max))) {
+        (APPROX && (!(a.qnorm[qi] < a.qn_max) || (a.qover && a.qover[qi])))) {
         if (lane == 0) hard[atomicAdd(nhard, 1u)] = qi;
         return;
     }
@@ -2096,7 +2097,7 @@ __device__ bool select_wg(const SelArgs& a, const int qi) {
     const bool ids8 = a.i8 && all_int;
     const bool exact = a.keys_exact || ids8 || (a.exact_ok && qint);
     const bool approx = APPROX && !exact;
-    if (approx && !(qn < a.qn_max)) {  // (NaN too) no bound on its keys' error: the exact rescan
+    if (approx && (!(qn < a.qn_max) || (a.qover && a.qover[qi]))) {  // (NaN too) no bound on its keys' error: the exact rescan
         __syncthreads();  // the count is read
         if (tid == 0) {
             a.rescan_tau[qi] = FLT_MAX;
@@ -2633,8 +2634,11 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     }
     const float mcoef = f16 ? margin_coef_f16(h->d) : margin_coef(h->d);
     const float mabs = f16 ? margin_abs_f16(h->d, B.f16_scale) : 0.0f;
-    // (a query's scaled values stay finite in FP16 below this norm)
-    const float qn_max = f16 ? std::min(1e37f, (60000.0f / B.f16_scale) * (60000.0f / B.f16_scale)) : INFINITY;
+    // (the ranks of norms this large could overflow; the components that leave
+    // FP16's range are flagged one query at a time.  Until then any query whose norm
+    // passed FP16's largest value was flagged: dense data of many dims, all of whose
+    // components are near the largest, took the rescans for every query)
+    const float qn_max = f16 ? 1e37f : INFINITY;
     // the int8 scan serves integer lists unless the caller asks for the BF16
     // shadow (HIVF_PREC_BF16); results are the same either way
     const int i8 = (B.i8 && p.precision != HIVF_PREC_BF16) ? 1 : 0;
@@ -2693,8 +2697,8 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                  o_hwg = take(plan_hwg_bytes(nlist, n * P)),
                  o_ioff = take((nlist + 1) * 8), o_lnear = take(nlist * 4), o_meta = take(kMetaWords * 4), o_lq = take((size_t)n * P * 4),
                  o_items = take((size_t)max_items * sizeof(BatchItem)), o_scnt = take(n * 4),
-                 o_sbuf = take((size_t)n * cap * 8), o_fb = take(n * 4), o_tau = take(n * 4),
-                 o_rtau = take(n * 4), o_tau2 = take(n * 4), o_rtau2 = take(n * 4), o_fb2 = take(n * 4),
+                 o_sbuf = take((size_t)n * cap * 8), o_qover = take(n * 4), o_tau = take(n * 4),
+                 o_rtau = take(n * 4), o_tau2 = take(n * 4), o_rtau2 = take(n * 4),
                  o_fbl = take(n * 4), o_fbl2 = take(n * 4), o_fbc = take(kFbcWords * 4), o_part = take(part_keys_bytes(k)), o_shard = take(n * 4),
                  o_allint = take(4), o_q8 = take(i8 ? (size_t)n * B.nkc8 * 32 : 0),
                  o_qn8 = take(i8 ? (size_t)n * 4 : 0);
@@ -2725,7 +2729,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     BatchItem* items = (BatchItem*)at(o_items);
     uint32_t* scnt = (uint32_t*)at(o_scnt);
     uint64_t* sbuf = (uint64_t*)at(o_sbuf);
-    int32_t* fb = (int32_t*)at(o_fb);
+    int32_t* qover = (int32_t*)at(o_qover);
     float* tau = (float*)at(o_tau);
     float* rtau = (float*)at(o_rtau);
     h->batched_qnorm = qnorm;
@@ -2736,7 +2740,6 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     const int dpad32 = B.nkc8 * 32;
     float* tau2 = (float*)at(o_tau2);
     float* rtau2 = (float*)at(o_rtau2);
-    int32_t* fb2 = (int32_t*)at(o_fb2);
     const PlanBufs pl{(int)nlist, lcnt, lcur, lend, qoff, hwg, ioff, lnear, meta, lq, lqd, items, max_items};
     // the BF16 scans are exact for integer queries and lists when d <= 129
     const int exact_bf16 = (h->lists_uint8 && h->d <= 129) ? 1 : 0;
@@ -2751,7 +2754,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         // the coarse step, whose query-preparation launch also prepares the
         // queries for the scan (else prep_kernel does)
         PrepArgs pa{reinterpret_cast<const float*>(q), (int)h->d, (int)h->d_pad, (int)dpad16, dpad32, qbf, qbf2,
-                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, fb, fb2, scnt, fbc, kFbcWords, lcnt, (int)nlist, B.f16_scale};
+                    qaug, qnorm, qint, i8 ? q8 : nullptr, qn8, qover, scnt, fbc, kFbcWords, lcnt, (int)nlist, B.f16_scale};
         bool prepped = false;
         const int rc0 = run_coarse(h, q, n, P, s, &pa, &prepped);
         if (rc0) return rc0;
@@ -2826,8 +2829,9 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         sa.norms = h->d_norms.p;
         sa.mcoef = mcoef;
         sa.mabs = mabs;
-        // (a query flagged for its norm goes through the exact rescans)
+        // (a query flagged for its norm or its range goes through the exact rescans)
         sa.qn_max = first ? qn_max : INFINITY;
+        sa.qover = first && f16 ? qover : nullptr;
         sa.exact_ok = exact_bf16;
         sa.i8 = i8;
         sa.all_int = all_int;

@@ -15,7 +15,7 @@ namespace hivf {
 // squared norm with its 3-piece augmentation, whether the query is integer
 // in [0, 255], and, for the int8 scan (q8 non-null), q - 128 as int8
 // (row-major, dpad32; 0 past d) with sum (q - 128)^2.  It also clears the
-// search's per-query flags and survivor counts, and (workgroup 0) the rescue
+// search's survivor counts and (workgroup 0) the rescue
 // list and part counts and the per-list query counts of the first pass.
 struct PrepArgs {
     const float* q;
@@ -27,8 +27,7 @@ struct PrepArgs {
     int32_t* qint;
     int8_t* q8;      // null: no int8 scan
     int32_t* qn8;
-    int32_t* fb;
-    int32_t* fb2;
+    int32_t* qover;   // FP16 form: 1 when a component leaves FP16's range
     uint32_t* scnt;
     uint32_t* fbc;   // [fbc_words]
     int fbc_words;
@@ -56,9 +55,11 @@ __device__ inline void prep_query(const PrepArgs& a, const int qi, const int lan
     const bool regs = a.dpad16 <= 64 * kQRegs && a.dpad32 <= 64 * kQRegs;
     double s = 0.0;
     int ok = 1;
+    bool over = false;
     auto one = [&](int c, float v) {
         a.qbf[(size_t)qi * a.dpad16 + c] =
             a.f16_scale > 0.0f ? __builtin_bit_cast(uint16_t, (_Float16)(v * a.f16_scale)) : f2bf(v);
+        over = over || !(fabsf(v * a.f16_scale) <= 65504.0f);  // (NaN too)
         a.qbf2[(size_t)qi * a.dpad16 + c] = f2bf(-2.0f * v);  // = -2 bf16(v) exactly
         s += (double)v * (double)v;
         ok &= (v == rintf(v)) && v >= 0.0f && v <= 255.0f;
@@ -74,6 +75,7 @@ __device__ inline void prep_query(const PrepArgs& a, const int qi, const int lan
         s += __shfl_down(s, off);
         ok &= __shfl_down(ok, off);
     }
+    const uint64_t any_over = __ballot(over);
     if (lane == 0) {
         const float n = (float)s;
         a.qnorm[qi] = n;
@@ -81,8 +83,7 @@ __device__ inline void prep_query(const PrepArgs& a, const int qi, const int lan
         uint16_t v[8] = {kBf16One, kBf16One, kBf16One, 0, 0, 0, 0, 0};
         split3(n, v + 3);
         for (int e = 0; e < 8; ++e) a.qaug[(size_t)qi * 8 + e] = v[e];
-        a.fb[qi] = 0;
-        a.fb2[qi] = 0;
+        a.qover[qi] = a.f16_scale > 0.0f && any_over ? 1 : 0;
         a.scnt[qi] = 0;
     }
     if (a.q8) {
