@@ -2440,6 +2440,17 @@ float margin_abs_f16(int64_t d, float scale) {
     return (float)(1.01 * 2 * (double)d * delta * delta * (16384.0 + 1.0)) + 1e-30f;
 }
 
+// Rows (ids other than the padding's) whose squared norm is below lim.
+__global__ __launch_bounds__(256) void count_below_kernel(const float* __restrict__ norms,
+                                                          const uint32_t* __restrict__ ids, int64_t n, float lim,
+                                                          unsigned long long* __restrict__ out) {
+    unsigned long long c = 0;
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
+        c += ids[i] != kNoId && norms[i] < lim;
+    for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
+    if ((threadIdx.x & 63) == 0 && c) atomicAdd(out, c);
+}
+
 // Buffers of the planning (carved from the scratch) and its work-item bound.
 struct PlanBufs {
     int nlist;
@@ -2540,6 +2551,38 @@ void BatchedState::release() {
     valid = false;
 }
 
+// Real-valued lists hold their shadow in FP16, scaled by a power of two so that
+// the largest value lies in [2^13, 2^14): three bits more than BF16, so the
+// margin is an eighth and little more than k survivors of a query need
+// rescoring.  0 (BF16): integer lists, values whose squares leave FP32's range,
+// and lists most of whose rows are so far below the largest value that FP16's
+// absolute part makes their margin wider than BF16's, which is relative (200k x
+// 96, 1000 queries of 24 lists, one component of one row at 1e8 times the rest's:
+// 2.81 ms in FP16, 0.29 in BF16; 0.19 in FP16 without it).
+static int f16_scale_of(hivf_index* h, float* scale, hipStream_t s) {
+    *scale = 0.0f;
+    const float mx = h->lists_absmax;
+    if (h->lists_uint8 || !h->lists_sane || !(mx == 0.0f || (mx >= 0x1p-40f && mx < 0x1p50f))) return HIVF_OK;
+    const float sc = mx > 0.0f ? std::ldexp(1.0f, 13 - std::ilogb(mx)) : 1.0f;
+    if (mx > 0.0f && h->tiles > 0) {
+        // where a row meets a query of its own norm
+        const float lim = margin_abs_f16(h->d, sc) / (2.0f * (margin_coef(h->d) - margin_coef_f16(h->d)));
+        DevBuf<unsigned long long> cnt;
+        unsigned long long below = 0;
+        HIP_TRY(h, cnt.ensure(1));
+        HIP_TRY(h, hipMemcpyAsync(cnt.p, &below, sizeof(below), hipMemcpyHostToDevice, s));
+        const int64_t rows = h->tiles * kTileRows;
+        hipLaunchKernelGGL(count_below_kernel, dim3((unsigned)std::min<int64_t>((rows + 255) / 256, 1024)), dim3(256), 0,
+                           s, h->d_norms.p, h->d_ids.p, rows, lim, cnt.p);
+        HIP_TRY(h, hipGetLastError());
+        HIP_TRY(h, hipMemcpyAsync(&below, cnt.p, sizeof(below), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipStreamSynchronize(s));
+        if (below > (unsigned long long)h->ntotal / 2) return HIVF_OK;
+    }
+    *scale = sc;
+    return HIVF_OK;
+}
+
 int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
                 const hivf_search_params& p, float* D, int64_t* I, hivf_search_stats* st, hipStream_t s,
                 bool timing) {
@@ -2550,16 +2593,11 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     if (nkc > 32) return h->fail(HIVF_EUNSUPPORTED, "batched scan: d <= 512");
     if (n * P >= INT32_MAX) return h->fail(HIVF_EUNSUPPORTED, "batched scan: queries x nprobe < 2^31");
     const int64_t tiles32 = h->tiles * 2;
-    // Real-valued lists hold their shadow in FP16, scaled by a power of two so
-    // that the largest value lies in [2^13, 2^14): three bits more than BF16,
-    // so the margin is an eighth and little more than k survivors of a query
-    // need rescoring.  (Values whose squares leave FP32's range keep BF16.)
-    const bool f16 = !h->lists_uint8 && h->lists_sane && (h->lists_absmax == 0.0f ||
-                     (h->lists_absmax >= 0x1p-40f && h->lists_absmax < 0x1p50f));
     if (!B.valid) {
         B.release();
         B.nkc = nkc;
-        B.f16_scale = !f16 ? 0.0f : h->lists_absmax > 0.0f ? std::ldexp(1.0f, 13 - std::ilogb(h->lists_absmax)) : 1.0f;
+        const int rc = f16_scale_of(h, &B.f16_scale, s);
+        if (rc) return rc;
         // integer lists: the int8 arena (d <= 256, distances below 2^24);
         // otherwise the BF16 norm chunk where it is exact (d <= 129)
         B.i8 = (h->lists_uint8 && h->d <= 256) ? 1 : 0;
@@ -2632,6 +2670,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         B.cus = prop.multiProcessorCount;
         B.valid = true;
     }
+    const bool f16 = B.f16_scale > 0.0f;
     const float mcoef = f16 ? margin_coef_f16(h->d) : margin_coef(h->d);
     const float mabs = f16 ? margin_abs_f16(h->d, B.f16_scale) : 0.0f;
     // (the ranks of norms this large could overflow; the components that leave
