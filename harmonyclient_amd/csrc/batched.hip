@@ -2567,15 +2567,14 @@ static int f16_scale_of(hivf_index* h, float* scale, hipStream_t s) {
     if (mx > 0.0f && h->tiles > 0) {
         // where a row meets a query of its own norm
         const float lim = margin_abs_f16(h->d, sc) / (2.0f * (margin_coef(h->d) - margin_coef_f16(h->d)));
-        DevBuf<unsigned long long> cnt;
         unsigned long long below = 0;
-        HIP_TRY(h, cnt.ensure(1));
-        HIP_TRY(h, hipMemcpyAsync(cnt.p, &below, sizeof(below), hipMemcpyHostToDevice, s));
+        HIP_TRY(h, h->d_vote.ensure(2));
+        HIP_TRY(h, hipMemcpyAsync(h->d_vote.p, &below, sizeof(below), hipMemcpyHostToDevice, s));
         const int64_t rows = h->tiles * kTileRows;
         hipLaunchKernelGGL(count_below_kernel, dim3((unsigned)std::min<int64_t>((rows + 255) / 256, 1024)), dim3(256), 0,
-                           s, h->d_norms.p, h->d_ids.p, rows, lim, cnt.p);
+                           s, h->d_norms.p, h->d_ids.p, rows, lim, h->d_vote.p);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, hipMemcpyAsync(&below, cnt.p, sizeof(below), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipMemcpyAsync(&below, h->d_vote.p, sizeof(below), hipMemcpyDeviceToHost, s));
         HIP_TRY(h, hipStreamSynchronize(s));
         if (below > (unsigned long long)h->ntotal / 2) return HIVF_OK;
     }
@@ -3148,6 +3147,38 @@ static bool flat_shared(int64_t n, int P, int64_t nlist, double tiles_per_list, 
     return n * P >= 2 * nlist && pair_tiles * (double)d >= (d <= 128 ? 2.2e6 : 4.0e6);
 }
 
+// Whether the split scan's error bound is narrow against the lists' spread, for
+// most of a sample of their rows (asked once per lists).  A
+// query's bound and a row's together are 4 coef ||x||^2 where their norms are
+// alike: past the distances between the rows of a list everything probed
+// survives, and the selection and the overflowed queries' rescans cost more than
+// the FP32 scan.  Rows of unit spread per dimension around an offset, split and
+// FP32 scan, at 4 coef ||x||^2 / ||x - c||^2 = r: 500k x 128, 1000 queries of 32
+// lists: r 0.2 331 and 482 us, 2.0 544 and 536, 8 2412 and 543, 200 4374 and 543;
+// 300k x 200: 0.25 399 and 425, 2.7 805 and 473.  Inner products spread by about
+// ||x|| ||x - c|| / sqrt(d), r = 4 coef ||x|| sqrt(d) / ||x - c||: 1.7 1379 and
+// 3212, 5.2 13,840 and 3205.
+static int split_fits(hivf_index* h, hipStream_t s, bool* fits) {
+    BatchedState& B = h->batched;
+    if (B.split_ok < 0 && h->tiles > 0) {
+        unsigned long long v[2] = {0, 0};  // rows asked, rows whose bound is wide
+        HIP_TRY(h, h->d_vote.ensure(2));
+        HIP_TRY(h, hipMemcpyAsync(h->d_vote.p, v, sizeof(v), hipMemcpyHostToDevice, s));
+        const float c = 4.0f * split_coef(h->d);
+        const bool l2 = h->metric == HIVF_METRIC_L2;
+        const float w = l2 ? c : c * c * (float)h->d / (2.5f * 2.5f);
+        const int64_t step = std::max<int64_t>(1, h->tiles / 1024);
+        hipLaunchKernelGGL(wide_rows_kernel, dim3((unsigned)((h->tiles / step + 4) / 4)), dim3(256), 0, s, h->lists(),
+                           h->d_norms.p, h->d_cent_rows.p, (int)h->nlist, h->tiles, step, w, h->d_vote.p);
+        HIP_TRY(h, hipGetLastError());
+        HIP_TRY(h, hipMemcpyAsync(v, h->d_vote.p, sizeof(v), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipStreamSynchronize(s));
+        B.split_ok = v[1] * 2 > v[0] ? 0 : 1;
+    }
+    *fits = B.split_ok != 0;
+    return HIVF_OK;
+}
+
 // Batches of plain and pruned searches by the exact FP32 scans (flat.hpp).
 // HIVF_EUNSUPPORTED, with nothing launched: the per-query kernel serves them.
 int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
@@ -3165,9 +3196,13 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     if (!flat_pays(n, P, tiles_per_list)) return HIVF_EUNSUPPORTED;
     const int nkc = (int)((h->d + 15) / 16);
     const bool small_d = nkc <= 8;
-    // the split scan, unless norms could overflow its ranks or the caller
-    // wants the pruning's statistics, which the FP32 scan counts
-    const bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
+    // the split scan, unless norms could overflow its ranks, the caller wants the
+    // pruning's statistics, which the FP32 scan counts, or its bound is wide
+    bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
+    if (can_split && flat_shared(n, P, nlist, tiles_per_list, h->d, true)) {
+        const int rc = split_fits(h, s, &can_split);
+        if (rc) return rc;
+    }
     const bool shared = flat_shared(n, P, nlist, tiles_per_list, h->d, can_split);
     const bool split = shared && can_split;
     const uint32_t qc = split ? kSplitItem : kFlatItem;

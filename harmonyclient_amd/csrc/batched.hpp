@@ -49,7 +49,12 @@ struct BatchedState {
 
     int cus = 0;            // compute units of the device
 
-    void invalidate() { valid = false; }
+    int split_ok = -1;      // the split scan's error bound is narrow for these lists (-1: not asked yet)
+
+    void invalidate() {
+        valid = false;
+        split_ok = -1;
+    }
     void release();
     ~BatchedState() { release(); }
 };

@@ -143,6 +143,7 @@ struct hivf_index {
     hivf::PinnedRing ring;        // large uploads of rows
     hivf::PinnedBuf io;           // queries and results of small host searches
     hivf::PinnedBuf counts;       // a search's counters on their way to the host
+    hivf::DevBuf<unsigned long long> d_vote; // counts of rows by which a form of the lists is chosen
     hivf::DevBuf<float> d_cd;
     hivf::DevBuf<int32_t> d_probes;
     hivf::DevBuf<int32_t> d_npq;

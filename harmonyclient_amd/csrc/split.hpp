@@ -363,6 +363,33 @@ float split_coef(int64_t d) {
                            8 * e + 2 * gamma(d + 2.0)));
 }
 
+// Every step-th tile (a wave each, a row per lane): rows with w ||x||^2 above
+// their squared distance to the list's centroid into out[1], all rows asked into
+// out[0] (those on their centroid tell nothing).
+__global__ __launch_bounds__(256) void wide_rows_kernel(DevLists lists, const float* __restrict__ norms,
+                                                        const float4* __restrict__ cent, int nlist, int64_t tiles,
+                                                        int64_t step, float w, unsigned long long* __restrict__ out) {
+    const int lane = threadIdx.x & 63;
+    const int64_t T = ((int64_t)blockIdx.x * 4 + threadIdx.x / 64) * step;
+    if (T >= tiles) return;  // whole wave
+    int l = 0, hi = nlist;   // the last list that starts at T or before
+    while (hi - l > 1) {
+        const int mid = (l + hi) / 2;
+        if (lists.list_tile_off[mid] <= T) l = mid;
+        else hi = mid;
+    }
+    const int rows = lists.list_size[l] - (int)(T - lists.list_tile_off[l]) * 64;
+    float dist = 0.0f;
+    for (int j = 0; j < lists.nquad; ++j)
+        dist = accum<kL2>(dist, cent[(size_t)l * lists.nquad + j], lists.codes[((size_t)T * lists.nquad + j) * 64 + lane]);
+    const bool on = lane < rows && dist > 0.0f && dist < FLT_MAX;
+    const uint64_t asked = __ballot(on), wide = __ballot(on && w * norms[T * 64 + lane] > dist);
+    if (lane == 0) {
+        atomicAdd(&out[0], (unsigned long long)__popcll(asked));
+        atomicAdd(&out[1], (unsigned long long)__popcll(wide));
+    }
+}
+
 // 32-row tiles per item (near-query items: half) of the two forms.
 constexpr int kSplitTiles = 8;
 constexpr int kSplitWgTiles = 32;
