@@ -40,7 +40,6 @@ struct ScanArgs {
     int64_t* out_i;           // [nq x k]
     float* out_tau;           // warm-up: [nq]
     unsigned long long* stats;// optional: candidates, blocks_total, blocks_skipped
-    const int32_t* only;      // optional [nq] flags: scan only the flagged queries
     const int32_t* qlist;     // optional: scan only these queries (count in *qcount)
     const uint32_t* qcount;
     // optional, with qlist: short lists' queries are split over several

@@ -16,6 +16,7 @@
 // read with broadcast loads.  A distance is one sequential FMA chain over
 // the dims, the same arithmetic as the oracle, so results are bit-identical.
 #include <algorithm>
+#include <type_traits>
 
 #include "common.hpp"
 #include "kernels.hpp"
@@ -36,6 +37,24 @@ __device__ inline void load_query(float4* qs, const float4* q, int nquad) {
 
 __device__ inline float quad_comp(float4 v, int c) {
     return c == 0 ? v.x : c == 1 ? v.y : c == 2 ? v.z : v.w;
+}
+
+// Quads [j, je) of the canonical chain of one row, 8 loads in flight.  (Loaded
+// into registers first, and fenced: from an unrolled loop of load and FMA the
+// compiler waits for each load in some inlined copies.  The rescan of 1988 listed
+// queries, 32 lists of 488 rows x 128 dims each: 1.97 ms so, 1.25 now.)
+template <int METRIC>
+__device__ inline float accum_quads(float acc, const float4* qs, const float4* tp, int j, int je) {
+    for (; j + 8 <= je; j += 8) {
+        float4 x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = tp[(size_t)(j + u) * kWave];
+        __builtin_amdgcn_sched_barrier(0x104);  // (scalar operations and LDS reads may cross)
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc = accum<METRIC>(acc, qs[j + u], x[u]);
+    }
+    for (; j < je; ++j) acc = accum<METRIC>(acc, qs[j], tp[(size_t)j * kWave]);
+    return acc;
 }
 
 // Dims [d0, d1) of the canonical chain of one row: a partial first quad,
@@ -60,8 +79,10 @@ __device__ inline float accum_dims(float acc, const float4* qs, const float4* tp
         ++j;
     }
     const int jend = d1 >> 2;
-#pragma unroll 8
-    for (; j < jend; ++j) acc = accum<METRIC>(acc, qs[j], tp[(size_t)j * kWave]);
+    if (j < jend) {
+        acc = accum_quads<METRIC>(acc, qs, tp, j, jend);
+        j = jend;
+    }
     const int r = d1 & 3;
     if (r && 4 * j >= d0 && 4 * j < d1) {
         const float4 q = qs[j], x = tp[(size_t)j * kWave];
@@ -156,6 +177,10 @@ __device__ inline uint32_t wave_kth_rank(const uint64_t* keys, int n, int kth, i
 // Tiles a wave takes between two barriers of the workgroup: the top-k's
 // buffer holds k <= 1024 kept keys and 4 x 256 more.  (The pruned scan takes
 // one: its bound follows the running k-th.)
+// Past k = 512, two: with four the kept keys leave no room for a second round,
+// and the buffer is sorted after nearly every one (64 queries of 32 lists, k =
+// 1000, four, two and one: 635, 397 and 379 us; the warm-up of 10 lists 322, 260
+// and 278; k = 512: 316, 325 and 342).
 constexpr int kRoundTiles = 4;
 static_assert(kMaxK + kRoundTiles * kNT <= kBuf, "a round's keys fit beside the kept ones");
 
@@ -196,14 +221,14 @@ __device__ void scan_one(const ScanArgs& a, const int qi, const int part = 0, co
     unsigned long long my_cand = 0, my_skip = 0;
     uint64_t thr = top.thr;
 
-    constexpr int kRound = MODE == kScanPruned ? 1 : kRoundTiles;
+    const int round = MODE == kScanPruned ? 1 : a.k <= kBuf / 4 ? kRoundTiles : 2;
     for (int j0 = 0; j0 < P; j0 += kProbeChunk) {
         stage_probes(a, probes, j0, min(kProbeChunk, P - j0), pm);
         const int m = min(kProbeChunk, P - j0);
         const int total = pm.before[m];
         int j = 0;  // this wave's probe: before[j] <= its tile < before[j + 1]
-        for (int g0 = part * kNW * kRound; g0 < total; g0 += nparts * kNW * kRound) {
-            for (int u = 0; u < kRound; ++u) {
+        for (int g0 = part * kNW * round; g0 < total; g0 += nparts * kNW * round) {
+            for (int u = 0; u < round; ++u) {
                 const int g = g0 + u * kNW + wave;
                 if (g >= total) break;
                 while (pm.before[j + 1] <= g) ++j;
@@ -229,17 +254,13 @@ __device__ void scan_one(const ScanArgs& a, const int qi, const int part = 0, co
                         }
                     }
                 } else {
-                    if (valid) {
-#pragma unroll 8
-                        for (int jj = 0; jj < nquad; ++jj)
-                            acc = accum<METRIC>(acc, qs[jj], tp[(size_t)jj * kWave]);
-                    }
+                    if (valid) acc = accum_quads<METRIC>(acc, qs, tp, 0, nquad);
                 }
                 if (valid) my_cand++;
                 if (keep) top.offer(make_key(rank_of<METRIC>(acc), id), thr);
             }
             __syncthreads();
-            top.maybe_compact(a.k, kNT * kRound);
+            top.maybe_compact(a.k, kNT * round);
             thr = top.thr;
         }
         __syncthreads();  // the map's last reads are done
@@ -312,31 +333,24 @@ __device__ void scan_one(const ScanArgs& a, const int qi, const int part = 0, co
     }
 }
 
-// One workgroup per query (all, or those flagged in `only`), or, with a
-// query list, a grid that walks the list.  A list too short for the grid has
-// its queries split: one query's 62k rows of 128 dims on one workgroup hold a
-// search for 0.9 ms, 43 such queries for 1.9 ms, against 0.42 ms split.
-template <int MODE, int METRIC>
+// One workgroup per query, or (LIST) a grid that walks the query list.  A list
+// too short for the grid has its queries split: one query's 62k rows of 128 dims
+// on one workgroup hold a search for 0.9 ms, 43 such queries for 1.9 ms, against
+// 0.42 ms split.  (A kernel of its own with one call of scan_one: with several
+// in one kernel the compiler waited for each row load of some of them.)
+template <int MODE, int METRIC, bool LIST>
 __global__ __launch_bounds__(kNT) void scan_kernel(ScanArgs a) {
-    if (a.qlist) {
+    if constexpr (!LIST) {
+        scan_one<MODE, METRIC>(a, blockIdx.x);
+    } else {
         const uint32_t nl = *a.qcount;
-        if constexpr (MODE != kScanWarmup) {
-            const uint32_t np = a.part_keys && nl ? min(gridDim.x / nl, (uint32_t)kListParts) : 1u;
-            if (np > 1) {
-                const uint32_t slot = blockIdx.x / np;
-                if (slot < nl) scan_one<MODE, METRIC>(a, a.qlist[slot], (int)(blockIdx.x % np), (int)np, slot);
-                return;
-            }
-        }
-        for (uint32_t i = blockIdx.x; i < nl; i += gridDim.x) {
+        const uint32_t np = MODE != kScanWarmup && a.part_keys && nl ? max(1u, min(gridDim.x / nl, (uint32_t)kListParts)) : 1u;
+        // (of a split list each workgroup takes one query: the step ends the loop)
+        for (uint32_t i = blockIdx.x / np; i < nl; i += gridDim.x) {
             __syncthreads();  // the previous query's LDS reads are done
-            scan_one<MODE, METRIC>(a, a.qlist[i]);
+            scan_one<MODE, METRIC>(a, __builtin_amdgcn_readfirstlane(a.qlist[i]), (int)(blockIdx.x % np), (int)np, i);
         }
-        return;
     }
-    const int qi = blockIdx.x;
-    if (a.only && !a.only[qi]) return;  // whole workgroup, before any barrier
-    scan_one<MODE, METRIC>(a, qi);
 }
 
 template <int METRIC>
@@ -403,10 +417,17 @@ hipError_t launch_scan_mode(const ScanArgs& a, int metric, hipStream_t s) {
     // (a list of few queries gets workgroups to split them over)
     const int64_t want = a.part_keys ? (int64_t)a.nq * 16 : a.nq;
     const dim3 grid((unsigned)(a.qlist ? std::min<int64_t>(want, kListGrid) : a.nq));
-    if (metric == kL2)
-        hipLaunchKernelGGL((scan_kernel<MODE, kL2>), grid, dim3(kNT), lds, s, a);
+    auto go = [&](auto list) {
+        constexpr bool L = decltype(list)::value;
+        if (metric == kL2)
+            hipLaunchKernelGGL((scan_kernel<MODE, kL2, L>), grid, dim3(kNT), lds, s, a);
+        else
+            hipLaunchKernelGGL((scan_kernel<MODE, kIP, L>), grid, dim3(kNT), lds, s, a);
+    };
+    if (a.qlist)
+        go(std::true_type{});
     else
-        hipLaunchKernelGGL((scan_kernel<MODE, kIP>), grid, dim3(kNT), lds, s, a);
+        go(std::false_type{});
     return hipGetLastError();
 }
 
