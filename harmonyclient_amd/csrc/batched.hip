@@ -27,7 +27,9 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <functional>
 #include <type_traits>
+#include <vector>
 
 #include "bf16.hpp"
 #include "index_impl.hpp"
@@ -2551,6 +2553,31 @@ void BatchedState::release() {
     valid = false;
 }
 
+// Most work items of n queries with P probes each, qc queries and rn tiles or
+// more per item.  A list of t chunks of rn tiles that c queries probe has at most
+// ceil(c / qc) t <= (c / qc + 1) t items, and a query probes a list once: the sum
+// is largest where every query probes the P lists of the most chunks.  (Counted as
+// if every list were as long as the longest, one list of 700k rows among 4096
+// took a table of 14 M items for 2000 queries of 32 lists, 100 k now, and the
+// launch over it 40 us, now 13.)
+static int64_t item_bound(const hivf_index* h, BatchedState::ItemBound& b, int rn, int64_t n, int P, int64_t qc) {
+    if (b.rn != rn) {
+        std::vector<int32_t> t((size_t)h->nlist);
+        b.all = 0;
+        for (int64_t l = 0; l < h->nlist; ++l) {
+            t[l] = (2 * (h->tile_off[l + 1] - h->tile_off[l]) + rn - 1) / rn;
+            b.all += t[l];
+        }
+        const int64_t m = std::min<int64_t>(h->nlist, kMaxK);  // (the most probes)
+        std::partial_sort(t.begin(), t.begin() + m, t.end(), std::greater<int32_t>());
+        b.top.assign(1, 0);
+        for (int64_t i = 0; i < m; ++i) b.top.push_back(b.top.back() + t[i]);
+        b.rn = rn;
+    }
+    const int64_t top = b.top[std::min<size_t>(P, b.top.size() - 1)];
+    return std::max<int64_t>(1, b.all + (n * top + qc - 1) / qc);
+}
+
 // Real-valued lists hold their shadow in FP16, scaled by a power of two so that
 // the largest value lies in [2^13, 2^14): three bits more than BF16, so the
 // margin is an eighth and little more than k survivors of a query need
@@ -2713,13 +2740,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
     if (waves <= 0) waves = 16;
     const uint32_t qc = 32u * qg;
     const int64_t nlist = h->nlist;
-    // upper bound of work items: sum over lists of ceil(c/QC) * ceil(t32/RT)
-    int64_t max_t32 = 1;
-    for (int64_t l = 0; l < nlist; ++l)
-        max_t32 = std::max<int64_t>(max_t32, 2 * (h->tile_off[l + 1] - h->tile_off[l]));
-    // (near-query items hold rt / kNearSplit tiles: bound every item by that)
-    const int64_t rtn = std::max(1, rt_items / (int)kNearSplit);
-    const int64_t max_items = (n * P / qc + nlist) * ((max_t32 + rtn - 1) / rtn);
+    const int64_t max_items = item_bound(h, B.bound, (int)near_tiles((uint32_t)rt_items), n, P, qc);
 
     // scratch layout
     size_t off = 0;
@@ -3214,11 +3235,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     // stay within 512 MB
     const uint32_t cap = (uint32_t)std::max<int64_t>(16384, 16 * k);
     const int64_t chunk = std::min<int64_t>(n, ((int64_t)64 << 20) / cap);
-    int64_t max_t32 = 1;
-    for (int64_t l = 0; l < nlist; ++l)
-        max_t32 = std::max<int64_t>(max_t32, 2 * (h->tile_off[l + 1] - h->tile_off[l]));
-    const int64_t rtn = near_tiles(rt);
-    const int64_t max_items = shared ? (chunk * P / qc + nlist) * ((max_t32 + rtn - 1) / rtn) : 0;
+    const int64_t max_items = shared ? item_bound(h, h->batched.flat_bound, (int)near_tiles(rt), chunk, P, qc) : 0;
     if (chunk * P >= INT32_MAX || max_items >= INT32_MAX) return HIVF_EUNSUPPORTED;
     if (split && P == 1) {  // (otherwise the coarse step split the queries)
         const int rc = split_queries(h, q, n, s, nullptr);

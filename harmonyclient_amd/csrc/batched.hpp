@@ -5,6 +5,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <vector>
 
 namespace hivf {
 
@@ -49,11 +50,21 @@ struct BatchedState {
 
     int cus = 0;            // compute units of the device
 
+    // What bounds the work items of a plan whose items hold rn tiles or more
+    // (item_bound): the lists' chunks of rn tiles, all and the largest added up.
+    struct ItemBound {
+        int rn = 0;  // 0: to be made
+        int64_t all = 0;
+        std::vector<int64_t> top;  // [p]: of the p lists with the most
+    };
+    ItemBound bound, flat_bound;
+
     int split_ok = -1;      // the split scan's error bound is narrow for these lists (-1: not asked yet)
 
     void invalidate() {
         valid = false;
         split_ok = -1;
+        bound.rn = flat_bound.rn = 0;
     }
     void release();
     ~BatchedState() { release(); }
