@@ -33,9 +33,13 @@ namespace {
 
 constexpr int kNT = 256;
 constexpr int kCandChunk = 2048;   // centroids examined per candidate round
-// 32-centroid tiles per wave task (one where the chunk count is not known at
-// compile time: too few waves otherwise)
-constexpr int tiles_per_task(int nkc) { return nkc == 8 ? 2 : 1; }
+// Chunk counts with a kernel of their own (the others' loop takes 8 at a time:
+// at 8 to 48 dims it multiplied four times what there is; 10k queries x 5000
+// centroids of 16 dims 402 us for the whole coarse step, now 300), and the
+// 32-centroid tiles of a wave's task: two with those (8 and 16 dims: the same
+// with four, 5 % slower with one), else one (too few waves otherwise).
+constexpr bool own_kernel(int nkc) { return (nkc >= 1 && nkc <= 4) || nkc == 8; }
+constexpr int tiles_per_task(int nkc) { return own_kernel(nkc) ? 2 : 1; }
 constexpr int64_t kMaxRankFloats = 64ll << 20;  // approximate-rank buffer
 // absolute part of the error bound: BF16 / FP32 values below the normal
 // range may be flushed to zero by the matrix cores
@@ -1142,23 +1146,26 @@ int run_coarse_mfma(hivf_index* h, const float4* q, int64_t n, int64_t P, hipStr
         const size_t lds = (size_t)h->nquad * sizeof(float4);
         const dim3 wgrid((unsigned)((m + 3) / 4));
         const dim3 hgrid((unsigned)std::min<int64_t>(m, 1024));
-        if (h->metric == HIVF_METRIC_L2) {
-            if (nkc == 8) hipLaunchKernelGGL((coarse_dot_kernel<kL2, 8>), grid, dim3(kNT), 0, s, da);
-            else hipLaunchKernelGGL((coarse_dot_kernel<kL2, 0>), grid, dim3(kNT), 0, s, da);
+        auto go = [&](auto metric) {
+            constexpr int M = decltype(metric)::value;
+            switch (nkc) {
+                case 1: hipLaunchKernelGGL((coarse_dot_kernel<M, 1>), grid, dim3(kNT), 0, s, da); break;
+                case 2: hipLaunchKernelGGL((coarse_dot_kernel<M, 2>), grid, dim3(kNT), 0, s, da); break;
+                case 3: hipLaunchKernelGGL((coarse_dot_kernel<M, 3>), grid, dim3(kNT), 0, s, da); break;
+                case 4: hipLaunchKernelGGL((coarse_dot_kernel<M, 4>), grid, dim3(kNT), 0, s, da); break;
+                case 8: hipLaunchKernelGGL((coarse_dot_kernel<M, 8>), grid, dim3(kNT), 0, s, da); break;
+                default: hipLaunchKernelGGL((coarse_dot_kernel<M, 0>), grid, dim3(kNT), 0, s, da);
+            }
             if (h->nlist <= 64 * kRegSlots)
-                hipLaunchKernelGGL((coarse_pick_wave_kernel<kL2, true>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
+                hipLaunchKernelGGL((coarse_pick_wave_kernel<M, true>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
             else
-                hipLaunchKernelGGL((coarse_pick_wave_kernel<kL2, false>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
-            hipLaunchKernelGGL((coarse_pick_kernel<kL2>), hgrid, dim3(kNT), lds, s, pa);
-        } else {
-            if (nkc == 8) hipLaunchKernelGGL((coarse_dot_kernel<kIP, 8>), grid, dim3(kNT), 0, s, da);
-            else hipLaunchKernelGGL((coarse_dot_kernel<kIP, 0>), grid, dim3(kNT), 0, s, da);
-            if (h->nlist <= 64 * kRegSlots)
-                hipLaunchKernelGGL((coarse_pick_wave_kernel<kIP, true>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
-            else
-                hipLaunchKernelGGL((coarse_pick_wave_kernel<kIP, false>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
-            hipLaunchKernelGGL((coarse_pick_kernel<kIP>), hgrid, dim3(kNT), lds, s, pa);
-        }
+                hipLaunchKernelGGL((coarse_pick_wave_kernel<M, false>), wgrid, dim3(kNT), 4 * lds, s, pa, (int)m);
+            hipLaunchKernelGGL((coarse_pick_kernel<M>), hgrid, dim3(kNT), lds, s, pa);
+        };
+        if (h->metric == HIVF_METRIC_L2)
+            go(std::integral_constant<int, kL2>{});
+        else
+            go(std::integral_constant<int, kIP>{});
         HIP_TRY(h, hipGetLastError());
     }
     return HIVF_OK;
