@@ -123,7 +123,10 @@ bool hivf::PinnedBuf::ensure(size_t need) {
     if (need <= bytes) return true;
     if (need > kMax) return false;
     release();
-    const size_t want = std::max<size_t>(need, 4096);
+    // (powers of two: of batches that grow from call to call hardly any makes it
+    // anew: 215 host searches of 1 to 1499 queries 213 ms at exact sizes, now 149)
+    size_t want = 4096;
+    while (want < need) want *= 2;
     if (hipHostMalloc(reinterpret_cast<void**>(&p), want) != hipSuccess) {
         (void)hipGetLastError();
         p = nullptr;
