@@ -1215,6 +1215,7 @@ int hivf_index_autotune(hivf_index* h, int64_t n, const float* x_dev, int64_t k,
     if (base) p = *base;
     p.algo = HIVF_ALGO_BATCHED;
     p.use_graph = 0;
+    p.batch_queries = p.batch_rows = p.batch_waves = 0;  // (set per candidate)
     if (reps < 1) reps = 3;
     DevBuf<float> D;
     DevBuf<int64_t> I;
@@ -1250,7 +1251,9 @@ int hivf_index_autotune(hivf_index* h, int64_t n, const float* x_dev, int64_t k,
     // integer data runs the int8 scan, whose items hold 32 queries, or 64
     // when d <= 128
     if (h->batched.valid && h->batched.i8) qg_max = h->batched.nkc8 == 4 ? 2 : 1;
-    double best = 1e30;
+    // The default is the shape to beat: it has forms that no shape names (the
+    // workgroup scan past 128 dims, items of fewer rows for small batches).
+    double best = dflt;
     int bq = 0, br = 0, bw = 0, tried = 0;
     for (int q = 32; q <= 32 * qg_max; q *= 2)
         for (int rows : {256, 512, 1024, 2048})
@@ -1273,6 +1276,17 @@ int hivf_index_autotune(hivf_index* h, int64_t n, const float* x_dev, int64_t k,
     h->tune.item_tiles = br / 32;
     h->tune.waves_per_cu = bw;
     h->drop_graph();  // a captured search holds the old default shape
+    if (bq == 0) {  // the default's shape, as a search's statistics report it
+        hivf_search_stats st;
+        rc = hivf_index_search_device(h, n, x_dev, k, D.p, I.p, &p, &st, h->stream);
+        if (rc) {
+            h->tune = saved;
+            return rc;
+        }
+        bq = (int)st.batch_queries;
+        br = (int)st.batch_rows;
+        bw = (int)st.batch_waves;
+    }
     std::memset(out, 0, sizeof(*out));
     out->batch_queries = bq;
     out->batch_rows = br;

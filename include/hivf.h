@@ -216,9 +216,11 @@ int hivf_merge_topk_device(int metric, int64_t n, int64_t parts, int64_t k_in, c
 
 /* ---- tile-shape autotuner ----------------------------------------------
  * No counterpart in the reference.  Times the batched scan on n device
- * queries for every candidate (queries per item, rows per item, waves per
- * CU), keeps the fastest as this index's default (used when a search leaves
- * those parameters 0) and reports it. */
+ * queries for the built-in default and every candidate (queries per item, rows
+ * per item, waves per CU), keeps the fastest as this index's default (used when
+ * a search leaves those parameters 0) and reports it.  Where no candidate beats
+ * the built-in default, that stays (ms == ms_default; its searches' reported
+ * shape is given, but no shape names all it does: a saved table holds 0 then). */
 typedef struct {
     int32_t batch_queries;
     int32_t batch_rows;
