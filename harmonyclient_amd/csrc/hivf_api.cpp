@@ -272,6 +272,10 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
         int64_t n_l = size[l];
         float* base = codes.data() + (size_t)tile_off[l] * tile_floats;
         std::vector<float> tmp((size_t)std::max<int64_t>(n_l, 1) * h->d);
+        // (in registers: written per value, the lists' neighbouring entries sent
+        // their cache line from thread to thread: 300k x 20 29 ms, now 3.4)
+        float mx = 0.0f;
+        bool u8 = true, ok = true;
         for (int64_t r = 0; r < n_l; ++r) {
             int64_t id;
             const float* src = row(l, r, &id);
@@ -281,13 +285,17 @@ int upload_lists(hivf_index* h, const std::vector<int64_t>& list_off, RowFn row)
             ids[slot] = (uint32_t)id;
             double s = 0.0;  // norms in FP64, rounded once
             for (int64_t c = 0; c < h->d; ++c) {
-                s += (double)src[c] * (double)src[c];
-                amax[l] = std::max(amax[l], std::fabs(src[c]));
-                if (!(src[c] >= 0.0f && src[c] <= 255.0f && src[c] == std::rint(src[c]))) small[l] = 0;
+                const float v = src[c];
+                s += (double)v * (double)v;
+                mx = std::max(mx, std::fabs(v));
+                u8 = u8 && v >= 0.0f && v <= 255.0f && v == std::rint(v);
             }
             norms[slot] = (float)s;
-            if (!(norms[slot] < 1e37f)) sane[l] = 0;
+            ok = ok && norms[slot] < 1e37f;
         }
+        amax[l] = mx;
+        small[l] = u8 ? 1 : 0;
+        sane[l] = ok ? 1 : 0;
         tile_rows(tmp.data(), n_l, h->d, nquad, base);
     });
     if (bad) return h->fail(HIVF_EINVAL, "ids must lie in [0, 2^32 - 2]");
