@@ -3145,27 +3145,41 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 }
 
 
-// Whether a batch repays the exact FP32 scans' launches (bound, plan,
-// selection).  The per-query kernel takes a workgroup 64 x 4 rows at a time
-// through a query's lists: one query of 100 tiles 224 us against 59, of 20
-// tiles 71 against 46, of 6 tiles (one list) 19 against 34; 16 queries of 6
-// tiles 65 against 47.
-static bool flat_pays(int64_t n, int P, double tiles_per_list) {
-    return P * tiles_per_list >= 12.0 || (double)n * P * tiles_per_list >= 90.0;
-}
-// Whether its queries share lists enough for a list-major form (else a
+// The form of a plain or pruned search, by n queries, P probes each, the mean rows
+// of a list and d dims.  Measured over 11 list sizes of 16 to 2000 rows (256
+// lists), 1 to 4000 queries, 1 to 64 probes, 32, 128 and 300 dims; figures are the
+// whole search's in us.
+//
+// Whether the queries share lists enough for a list-major form (else a
 // workgroup per query and list, which reads every pair's rows through the
-// caches).  The split scan and its plan repay themselves from about 500 MB of
-// such reads on: 256 queries of 16 lists in 512 (6.1 tiles, 128 dims) 148 us
-// against 179, 128 of them 141 against 127; 512 of 32 lists in 1024 (1.5 tiles,
-// 96 dims) 153 against 166, 256 of them 151 against 119; past 128 dims from 1 GB:
-// 128 of 20 lists (7.8 tiles, 201 dims) 245 against 255, 64 of them 243 against
-// 178.  The FP32 scan from about 40,000 tiles: 256 queries of 20 lists 270
-// against 401, 512 of 32 lists of 1.5 tiles 221 against 181.
-static bool flat_shared(int64_t n, int P, int64_t nlist, double tiles_per_list, int64_t d, bool split) {
-    const double pair_tiles = (double)n * P * tiles_per_list;
-    if (!split) return n * P >= 6 * nlist && pair_tiles >= 40000.0;
-    return n * P >= 2 * nlist && pair_tiles * (double)d >= (d <= 128 ? 2.2e6 : 4.0e6);
+// caches): the plan repays itself from about 1.4e8 components on (256 queries of 16
+// lists of 390 rows in 512, 128 dims: 148 against 179, 128 of them 141 against 127),
+// 3.2e8 past 128 dims (128 of 20 lists of 500 rows, 201 dims, 2.6e8: 245 against
+// 255), where one probe also means that the split scan prepares its own queries
+// (1000 on lists of 2000 rows, 300 dims: 27 % slower), and for the FP32 scan (1000
+// of 16 lists of 256 rows, 32 dims, 1.3e8: 40 % slower).
+static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, int64_t d, bool split) {
+    const double comps = (double)n * P * rows * (double)d;
+    if (!split) return n * P >= 6 * nlist && comps >= 3.2e8;
+    return n * P >= 2 * nlist && comps >= (d <= 128 ? 1.4e8 : P == 1 ? 1.28e9 : 3.2e8);
+}
+// Whether a batch repays these scans' launches (bound, plan, selection), or each
+// query's lists are scanned by a workgroup (64 x 4 rows at a time).  Plain: from
+// about 1100 rows per query (100 queries of 16 lists of 64 rows 1.15 times as slow,
+// of 100 rows 0.75), or in list-major form from 3.2e8 components (4000 of 4 lists of
+// 100 rows, 300 dims: 1.07, of 128 rows 0.92); lists of fewer rows leave half of a
+// tile's lanes empty (4000 of 16 lists of 64 rows, 128 dims: 1.09).  The pruned scan
+// skips most of its rows' dims, better with more queries at once: up to 100 queries
+// (32 with statistics, whose scan is FP32) from 1600 rows (16 queries of 16 lists of 100
+// rows 0.97), else in list-major form where comps x rows, at most 1000 of them, pass
+// 3.2e11 (1000 of 16 lists, 128 dims, of 256 rows 1.16, of 400 0.82; 4000 of 16 lists of 64
+// rows 1.3; with statistics 1000 of 32 lists of 64 rows 4.6).  A rule on tiles for both
+// took 794 of these 3234 searches to a form slower than the per-query kernel.
+static bool flat_pays(int64_t n, int P, double rows, int64_t d, bool pruned, bool stats, bool shared) {
+    const double comps = (double)n * P * rows * (double)d, per_query = P * rows;
+    const bool large = shared && rows >= 100.0 && comps >= (P == 1 && d > 128 ? 1.28e9 : 3.2e8);
+    if (!pruned) return per_query >= 1100.0 || large;
+    return (n <= (stats ? 32 : 100) && per_query >= 1600.0) || (large && comps * std::min(rows, 1000.0) >= 3.2e11);
 }
 
 // Whether the split scan's error bound is narrow against the lists' spread, for
@@ -3213,18 +3227,18 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         block_dims = std::max(h->nquad / 4, 1) * 4;
         nblocks = h->nquad >= 8 ? 4 : 1;
     }
-    const double tiles_per_list = (double)h->tiles / (double)nlist;
-    if (!flat_pays(n, P, tiles_per_list)) return HIVF_EUNSUPPORTED;
+    const double tiles_per_list = (double)h->tiles / (double)nlist, rows = (double)h->ntotal / (double)nlist;
     const int nkc = (int)((h->d + 15) / 16);
     const bool small_d = nkc <= 8;
     // the split scan, unless norms could overflow its ranks, the caller wants the
     // pruning's statistics, which the FP32 scan counts, or its bound is wide
     bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
-    if (can_split && flat_shared(n, P, nlist, tiles_per_list, h->d, true)) {
+    if (can_split && flat_shared(n, P, nlist, rows, h->d, true)) {
         const int rc = split_fits(h, s, &can_split);
         if (rc) return rc;
     }
-    const bool shared = flat_shared(n, P, nlist, tiles_per_list, h->d, can_split);
+    const bool shared = flat_shared(n, P, nlist, rows, h->d, can_split);
+    if (!flat_pays(n, P, rows, h->d, pruned, stats != nullptr, shared)) return HIVF_EUNSUPPORTED;
     const bool split = shared && can_split;
     const uint32_t qc = split ? kSplitItem : kFlatItem;
     // (fewer tiles per item do not pay even where the items are few: 256
@@ -3282,7 +3296,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     // least).  Fewer lists with more rows bound most queries better and a few
     // much worse: 1000 queries (k 100) keep 617 rows on average and 5.4 k at
     // most from 10 x 100, 398 and 13 k from 3 x 300
-    const double mean_rows = std::max(1.0, (double)h->ntotal / (double)nlist);
+    const double mean_rows = std::max(1.0, rows);
     const int warm_lists = (int)std::min<double>(std::max({10.0, (double)p.warmup_lists, 2.0 * (double)k / mean_rows}), 1024.0);
     const int warm_rows = (int)std::max<int64_t>({k, (int64_t)p.warmup_list_size, (int64_t)kTileRows});
     for (int64_t q0 = 0; q0 < n; q0 += chunk) {
