@@ -3170,8 +3170,9 @@ static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, int64_t d,
 // 100 rows, 300 dims: 1.07, of 128 rows 0.92); lists of fewer rows leave half of a
 // tile's lanes empty (4000 of 16 lists of 64 rows, 128 dims: 1.09).  The pruned scan
 // skips most of its rows' dims, better with more queries at once: up to 100 queries
-// (32 with statistics, whose scan is FP32) from 1600 rows (16 queries of 16 lists of 100
-// rows 0.97), else in list-major form where comps x rows, at most 1000 of them, pass
+// (32 with statistics, whose scan is FP32) from 3200 rows, past 128 dims 1600 (one
+// query of 4 lists of 400 rows of 32 dims 73 and 55 us, of 128 62 and 57, of 300 66 and
+// 91), else in list-major form where comps x rows, at most 1000 of them, pass
 // 3.2e11 (1000 of 16 lists, 128 dims, of 256 rows 1.16, of 400 0.82; 4000 of 16 lists of 64
 // rows 1.3; with statistics 1000 of 32 lists of 64 rows 4.6).  A rule on tiles for both
 // took 794 of these 3234 searches to a form slower than the per-query kernel.
@@ -3179,7 +3180,7 @@ static bool flat_pays(int64_t n, int P, double rows, int64_t d, bool pruned, boo
     const double comps = (double)n * P * rows * (double)d, per_query = P * rows;
     const bool large = shared && rows >= 100.0 && comps >= (P == 1 && d > 128 ? 1.28e9 : 3.2e8);
     if (!pruned) return per_query >= 1100.0 || large;
-    return (n <= (stats ? 32 : 100) && per_query >= 1600.0) || (large && comps * std::min(rows, 1000.0) >= 3.2e11);
+    return (n <= (stats ? 32 : 100) && per_query >= (d <= 128 ? 3200.0 : 1600.0)) || (large && comps * std::min(rows, 1000.0) >= 3.2e11);
 }
 
 // Whether the split scan's error bound is narrow against the lists' spread, for
