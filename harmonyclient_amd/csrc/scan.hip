@@ -42,7 +42,11 @@ __device__ inline float quad_comp(float4 v, int c) {
 // Quads [j, je) of the canonical chain of one row, 8 loads in flight.  (Loaded
 // into registers first, and fenced: from an unrolled loop of load and FMA the
 // compiler waits for each load in some inlined copies.  The rescan of 1988 listed
-// queries, 32 lists of 488 rows x 128 dims each: 1.97 ms so, 1.25 now.)
+// queries, 32 lists of 488 rows x 128 dims each: 1.97 ms so, 1.25 now.)  The last 1 to
+// 7 quads likewise, four and up to three (the last one's address again where there
+// are fewer), not each after the other: 200 queries of 4 lists of 1500 rows, 60 dims,
+// plain 137 us and pruned 138, now 108 and 124; pruned blocks of 24 dims, 96 dims 158
+// and 122.
 template <int METRIC>
 __device__ inline float accum_quads(float acc, const float4* qs, const float4* tp, int j, int je) {
     for (; j + 8 <= je; j += 8) {
@@ -53,7 +57,24 @@ __device__ inline float accum_quads(float acc, const float4* qs, const float4* t
 #pragma unroll
         for (int u = 0; u < 8; ++u) acc = accum<METRIC>(acc, qs[j + u], x[u]);
     }
-    for (; j < je; ++j) acc = accum<METRIC>(acc, qs[j], tp[(size_t)j * kWave]);
+    if (j + 4 <= je) {
+        float4 x[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) x[u] = tp[(size_t)(j + u) * kWave];
+        __builtin_amdgcn_sched_barrier(0x104);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) acc = accum<METRIC>(acc, qs[j + u], x[u]);
+        j += 4;
+    }
+    if (j < je) {
+        float4 x[3];
+#pragma unroll
+        for (int u = 0; u < 3; ++u) x[u] = tp[(size_t)min(j + u, je - 1) * kWave];
+        __builtin_amdgcn_sched_barrier(0x104);
+#pragma unroll
+        for (int u = 0; u < 3; ++u)
+            if (j + u < je) acc = accum<METRIC>(acc, qs[j + u], x[u]);
+    }
     return acc;
 }
 
