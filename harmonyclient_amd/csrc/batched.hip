@@ -3146,41 +3146,56 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 
 
 // The form of a plain or pruned search, by n queries, P probes each, the mean rows
-// of a list and d dims.  Measured over 11 list sizes of 16 to 2000 rows (256
-// lists), 1 to 4000 queries, 1 to 64 probes, 32, 128 and 300 dims; figures are the
-// whole search's in us.
+// of a list and d dims; list-major forms also by the queries that a list gets on
+// average.  Measured over 16 to 1000 lists of 60 to 3000 rows, 30 to 4000 queries, 1
+// to 64 probes, 32 to 420 dims, each search in every form (5280 searches): these rules'
+// choice takes 2.5 % longer than the best on average.  Figures are the whole
+// search's in us.
 //
 // Whether the queries share lists enough for a list-major form (else a
 // workgroup per query and list, which reads every pair's rows through the
-// caches): the plan repays itself from about 1.4e8 components on (256 queries of 16
-// lists of 390 rows in 512, 128 dims: 148 against 179, 128 of them 141 against 127),
-// 3.2e8 past 128 dims (128 of 20 lists of 500 rows, 201 dims, 2.6e8: 245 against
-// 255), where one probe also means that the split scan prepares its own queries
-// (1000 on lists of 2000 rows, 300 dims: 27 % slower), and for the FP32 scan (1000
-// of 16 lists of 256 rows, 32 dims, 1.3e8: 40 % slower).
-static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, int64_t d, bool split) {
-    const double comps = (double)n * P * rows * (double)d;
-    if (!split) return n * P >= 6 * nlist && comps >= 3.2e8;
-    return n * P >= 2 * nlist && comps >= (d <= 128 ? 1.4e8 : P == 1 ? 1.28e9 : 3.2e8);
+// caches).  The plan repays itself from about 2.5e8 components on (1000 queries of 2
+// lists of 1000 rows in 256, 128 dims: 132 against 172; below it, at 2e8, 1.15 times as
+// slow on average).  Past 128 dims a workgroup's waves split the lists' rows, 1024 at a
+// time: 4.5e8 components there (1000 of 2 of 3000 rows in 64, 201 dims: 261 against 457),
+// and past 256 dims, where a tile's rows are long, 6.4e8, 12 queries a list and 128
+// items to fill the chip (250 queries of 2 of 3000 rows in 16, 420 dims, are 48 items:
+// 480 against 235; 1000 of 4 of 1000 rows in 64 are 128: 385 against 652).  With one
+// probe the split scan prepares its own queries, and the per-query kernel reads
+// few rows twice: from 3.2e8 (4000 of lists of 1000 rows in 16, 201 dims, 8e8: 234 against
+// 525) and not past 256 dims (4000 of 3000 rows in 256, 420 dims: 3549 against 2794).  The
+// pruned scan skips most of its rows' dims and wants more queries a list: 1000 of 4 lists
+// of 1000 rows in 1000, 201 dims, 345 against 273.  For the FP32 scan: 1000 of 16 lists of 256
+// rows, 32 dims, 1.3e8, are 40 % slower.
+static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, int64_t d, bool split, bool pruned) {
+    const double comps = (double)n * P * rows * (double)d, per_list = (double)n * P / (double)nlist;
+    if (!split) return per_list >= 6.0 && comps >= 3.2e8;
+    if (d <= 128) return per_list >= 2.0 && comps >= 2.5e8;
+    if (P == 1) return d <= 256 && per_list >= 2.0 && comps >= 3.2e8;
+    if (d <= 256) return per_list >= (pruned ? 6.0 : 2.0) && comps >= 4.5e8;
+    const double items = (double)nlist * std::ceil(rows / (kSplitWgTiles * 32.0)) * std::ceil(per_list / kSplitItem);
+    return per_list >= (pruned ? 20.0 : 12.0) && items >= (pruned ? 256.0 : 128.0) && comps >= 6.4e8;
 }
 // Whether a batch repays these scans' launches (bound, plan, selection), or each
 // query's lists are scanned by a workgroup (64 x 4 rows at a time).  Plain: from
 // about 1100 rows per query (100 queries of 16 lists of 64 rows 1.15 times as slow,
-// of 100 rows 0.75), or in list-major form from 3.2e8 components (4000 of 4 lists of
+// of 100 rows 0.75), with one list each only while the queries leave the chip idle
+// (1000 of a list of 3000 rows in 16, 201 dims: 298 against 179, 300 of them, 32
+// dims, 59 against 73), or in list-major form from 3.2e8 components (4000 of 4 lists of
 // 100 rows, 300 dims: 1.07, of 128 rows 0.92); lists of fewer rows leave half of a
 // tile's lanes empty (4000 of 16 lists of 64 rows, 128 dims: 1.09).  The pruned scan
-// skips most of its rows' dims, better with more queries at once: up to 100 queries
+// gains with more queries at once: up to 100 queries
 // (32 with statistics, whose scan is FP32) from 3200 rows, past 128 dims 1600 (one
 // query of 4 lists of 400 rows of 32 dims 73 and 55 us, of 128 62 and 57, of 300 66 and
 // 91), else in list-major form where comps x rows, at most 1000 of them, pass
-// 3.2e11 (1000 of 16 lists, 128 dims, of 256 rows 1.16, of 400 0.82; 4000 of 16 lists of 64
-// rows 1.3; with statistics 1000 of 32 lists of 64 rows 4.6).  A rule on tiles for both
-// took 794 of these 3234 searches to a form slower than the per-query kernel.
+// 3.2e11, past 256 dims 4.8e11 (1000 of 16 lists, 128 dims, of 256 rows 1.16, of 400 0.82; 4000
+// of 16 lists of 64 rows 1.3; with statistics 1000 of 32 lists of 64 rows 4.6).
 static bool flat_pays(int64_t n, int P, double rows, int64_t d, bool pruned, bool stats, bool shared) {
     const double comps = (double)n * P * rows * (double)d, per_query = P * rows;
-    const bool large = shared && rows >= 100.0 && comps >= (P == 1 && d > 128 ? 1.28e9 : 3.2e8);
-    if (!pruned) return per_query >= 1100.0 || large;
-    return (n <= (stats ? 32 : 100) && per_query >= (d <= 128 ? 3200.0 : 1600.0)) || (large && comps * std::min(rows, 1000.0) >= 3.2e11);
+    const bool large = shared && rows >= 100.0 && comps >= 3.2e8;
+    if (!pruned) return (per_query >= 1100.0 && (P > 1 || n <= 512 || shared)) || large;
+    return (n <= (stats ? 32 : 100) && per_query >= (d <= 128 ? 3200.0 : 1600.0)) ||
+           (large && comps * std::min(rows, 1000.0) >= (d <= 256 ? 3.2e11 : 4.8e11));
 }
 
 // Whether the split scan's error bound is narrow against the lists' spread, for
@@ -3234,11 +3249,11 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     // the split scan, unless norms could overflow its ranks, the caller wants the
     // pruning's statistics, which the FP32 scan counts, or its bound is wide
     bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
-    if (can_split && flat_shared(n, P, nlist, rows, h->d, true)) {
+    if (can_split && flat_shared(n, P, nlist, rows, h->d, true, pruned)) {
         const int rc = split_fits(h, s, &can_split);
         if (rc) return rc;
     }
-    const bool shared = flat_shared(n, P, nlist, rows, h->d, can_split);
+    const bool shared = flat_shared(n, P, nlist, rows, h->d, can_split, pruned);
     if (!flat_pays(n, P, rows, h->d, pruned, stats != nullptr, shared)) return HIVF_EUNSUPPORTED;
     const bool split = shared && can_split;
     const uint32_t qc = split ? kSplitItem : kFlatItem;
