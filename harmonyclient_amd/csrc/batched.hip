@@ -3212,19 +3212,29 @@ static bool flat_pays(int64_t n, int P, double rows, int64_t d, bool pruned, boo
 static int split_fits(hivf_index* h, hipStream_t s, bool* fits) {
     BatchedState& B = h->batched;
     if (B.split_ok < 0 && h->tiles > 0) {
-        unsigned long long v[2] = {0, 0};  // rows asked, rows whose bound is wide
-        HIP_TRY(h, h->d_vote.ensure(2));
-        HIP_TRY(h, hipMemcpyAsync(h->d_vote.p, v, sizeof(v), hipMemcpyHostToDevice, s));
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        HIP_TRY(h, hipStreamIsCapturing(s, &cap));
+        if (cap != hipStreamCaptureStatusNone) {  // (nothing can be waited for: either form gives the same result)
+            *fits = true;
+            return HIVF_OK;
+        }
         const float c = 4.0f * split_coef(h->d);
         const bool l2 = h->metric == HIVF_METRIC_L2;
         const float w = l2 ? c : c * c * (float)h->d / (2.5f * 2.5f);
-        const int64_t step = std::max<int64_t>(1, h->tiles / 1024);
-        hipLaunchKernelGGL(wide_rows_kernel, dim3((unsigned)((h->tiles / step + 4) / 4)), dim3(256), 0, s, h->lists(),
-                           h->d_norms.p, h->d_cent_rows.p, (int)h->nlist, h->tiles, step, w, h->d_vote.p);
+        const int64_t step = (h->tiles + kWideTiles - 1) / kWideTiles;
+        const int blocks = (int)((h->tiles + 4 * step - 1) / (4 * step));
+        unsigned long long v[kWideTiles / 4 + 1], asked = 0, wide = 0;
+        HIP_TRY(h, h->d_vote.ensure(sizeof(v) / sizeof(v[0])));
+        hipLaunchKernelGGL(wide_rows_kernel, dim3(blocks), dim3(256), 0, s, h->lists(), h->d_norms.p, h->d_cent_rows.p,
+                           (int)h->nlist, h->tiles, step, w, h->d_vote.p);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, hipMemcpyAsync(v, h->d_vote.p, sizeof(v), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipMemcpyAsync(v, h->d_vote.p, blocks * sizeof(v[0]), hipMemcpyDeviceToHost, s));
         HIP_TRY(h, hipStreamSynchronize(s));
-        B.split_ok = v[1] * 2 > v[0] ? 0 : 1;
+        for (int i = 0; i < blocks; ++i) {
+            asked += v[i] >> 32;
+            wide += (uint32_t)v[i];
+        }
+        B.split_ok = wide * 2 > asked ? 0 : 1;
     }
     *fits = B.split_ok != 0;
     return HIVF_OK;

@@ -363,31 +363,38 @@ float split_coef(int64_t d) {
                            8 * e + 2 * gamma(d + 2.0)));
 }
 
-// Every step-th tile (a wave each, a row per lane): rows with w ||x||^2 above
-// their squared distance to the list's centroid into out[1], all rows asked into
-// out[0] (those on their centroid tell nothing).
+// Every step-th tile (a wave each, a row per lane): the workgroup's rows with
+// w ||x||^2 above their squared distance to the list's centroid, and (high word) all
+// rows asked, into its word of out (those on their centroid tell nothing).
+// At most kWideTiles tiles: a list's first search waits for them (1024 of 128 dims with
+// an atomic per tile 44 us).
+constexpr int kWideTiles = 256;
 __global__ __launch_bounds__(256) void wide_rows_kernel(DevLists lists, const float* __restrict__ norms,
                                                         const float4* __restrict__ cent, int nlist, int64_t tiles,
                                                         int64_t step, float w, unsigned long long* __restrict__ out) {
-    const int lane = threadIdx.x & 63;
-    const int64_t T = ((int64_t)blockIdx.x * 4 + threadIdx.x / 64) * step;
-    if (T >= tiles) return;  // whole wave
-    int l = 0, hi = nlist;   // the last list that starts at T or before
-    while (hi - l > 1) {
-        const int mid = (l + hi) / 2;
-        if (lists.list_tile_off[mid] <= T) l = mid;
-        else hi = mid;
+    __shared__ unsigned long long votes[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x / 64;
+    const int64_t T = ((int64_t)blockIdx.x * 4 + wave) * step;
+    unsigned long long v = 0;
+    if (T < tiles) {            // whole wave
+        int l = 0, hi = nlist;  // the last list that starts at T or before
+        while (hi - l > 1) {
+            const int mid = (l + hi) / 2;
+            if (lists.list_tile_off[mid] <= T) l = mid;
+            else hi = mid;
+        }
+        const int rows = lists.list_size[l] - (int)(T - lists.list_tile_off[l]) * 64;
+        float dist = 0.0f;
+        const float4 *c = cent + (size_t)l * lists.nquad, *x = lists.codes + (size_t)T * lists.nquad * 64 + lane;
+#pragma unroll 8
+        for (int j = 0; j < lists.nquad; ++j) dist = accum<kL2>(dist, c[j], x[(size_t)j * 64]);
+        const bool on = lane < rows && dist > 0.0f && dist < FLT_MAX;
+        v = (unsigned long long)__popcll(__ballot(on)) << 32 |
+            (unsigned)__popcll(__ballot(on && w * norms[T * 64 + lane] > dist));
     }
-    const int rows = lists.list_size[l] - (int)(T - lists.list_tile_off[l]) * 64;
-    float dist = 0.0f;
-    for (int j = 0; j < lists.nquad; ++j)
-        dist = accum<kL2>(dist, cent[(size_t)l * lists.nquad + j], lists.codes[((size_t)T * lists.nquad + j) * 64 + lane]);
-    const bool on = lane < rows && dist > 0.0f && dist < FLT_MAX;
-    const uint64_t asked = __ballot(on), wide = __ballot(on && w * norms[T * 64 + lane] > dist);
-    if (lane == 0) {
-        atomicAdd(&out[0], (unsigned long long)__popcll(asked));
-        atomicAdd(&out[1], (unsigned long long)__popcll(wide));
-    }
+    if (lane == 0) votes[wave] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = votes[0] + votes[1] + votes[2] + votes[3];
 }
 
 // 32-row tiles per item (near-query items: half) of the two forms.
