@@ -395,7 +395,7 @@ int upload_rows(hivf_index* h, int64_t n, const float* x, float* dst, hipStream_
     const int want = (int)std::min<int64_t>({PinnedRing::kThreads, parallel_threads(), chunks});
     try {
         for (int t = 1; t < want; ++t) th.emplace_back(work, t);
-    } catch (const std::system_error&) {  // fewer threads share the chunks
+    } catch (...) {  // fewer threads share the chunks (no thread, or no memory for one)
     }
     work(0);
     for (auto& t : th) t.join();
