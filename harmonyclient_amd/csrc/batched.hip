@@ -208,8 +208,6 @@ __global__ void prep_kernel(PrepArgs a) {
     prep_query(a, (int)blockIdx.x, (int)threadIdx.x, qv);
 }
 
-// Queries per list (only the `active` ones when non-null); optionally the
-// candidate count sum_q C_q into *cand.
 // List-level radius bound on a (query, list) pair: every row x of the list
 // (centroid c) has ||x - c|| in [Rmin, Rmax], so | ||q - c|| - ||x - c|| | >
 // sqrt(tau) for all of them when ||q - c|| lies farther than sqrt(tau) from
@@ -233,9 +231,10 @@ __device__ inline bool pair_may_pass(const PairFilter& f, int64_t i, int q, int 
     return !(dlo - rb.y > sq) && !(rb.x - dhi > sq);
 }
 
+// Queries per list; optionally the candidate count sum_q C_q into *cand.
 __global__ void count_kernel(const int32_t* __restrict__ probes, int nq, int P, const int32_t* __restrict__ npq,
-                             const int32_t* __restrict__ active, const int32_t* __restrict__ list_size,
-                             PairFilter pf, uint32_t* __restrict__ lcnt, unsigned long long* cand) {
+                             const int32_t* __restrict__ list_size, PairFilter pf, uint32_t* __restrict__ lcnt,
+                             unsigned long long* cand) {
     __shared__ unsigned long long s_c;
     if (threadIdx.x == 0) s_c = 0;
     __syncthreads();
@@ -244,7 +243,7 @@ __global__ void count_kernel(const int32_t* __restrict__ probes, int nq, int P, 
         int q = (int)(i / P), j = (int)(i % P);
         int Pq = npq ? min(npq[q], P) : P;
         int l = probes[i];
-        if (j < Pq && l >= 0 && (!active || active[q])) {
+        if (j < Pq && l >= 0) {
             // the candidate count is every probed row (the algorithmic work)
             if (cand) atomicAdd(&s_c, (unsigned long long)list_size[l]);
             if (pair_may_pass(pf, i, q, l)) atomicAdd(&lcnt[l], 1u);
@@ -422,15 +421,14 @@ __global__ __launch_bounds__(1024) void plan_kernel(const uint32_t* __restrict__
 constexpr int kNearProbes = 2;
 
 __global__ void fill_kernel(const int32_t* __restrict__ probes, const float* __restrict__ cd, int nq, int P,
-                            const int32_t* __restrict__ npq, const int32_t* __restrict__ active,
-                            PairFilter pf, uint32_t* __restrict__ lcur, uint32_t* __restrict__ lend,
+                            const int32_t* __restrict__ npq, PairFilter pf, uint32_t* __restrict__ lcur, uint32_t* __restrict__ lend,
                             int32_t* __restrict__ lq, float* __restrict__ lqd) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)nq * P) return;
     int q = (int)(i / P), j = (int)(i % P);
     int Pq = npq ? min(npq[q], P) : P;
     int l = probes[i];
-    if (j < Pq && l >= 0 && (!active || active[q]) && pair_may_pass(pf, i, q, l)) {
+    if (j < Pq && l >= 0 && pair_may_pass(pf, i, q, l)) {
         const uint32_t pos = j < kNearProbes ? atomicAdd(&lcur[l], 1u) : atomicSub(&lend[l], 1u) - 1u;
         lq[pos] = q;
         lqd[pos] = cd[i];
@@ -451,35 +449,16 @@ inline int64_t plan_wgs(int64_t entries) {
     return std::max((std::min<int64_t>(entries, 1 << 17) + 1023) / 1024, (entries + kPlanEntries - 1) / kPlanEntries);
 }
 
-// count_kernel with a per-workgroup LDS histogram: one global atomic per
-// (workgroup, list) instead of one per entry.
-// The (query, probe) entries of a pass: every query's (those flagged in
-// `active` when non-null), or, with a query list, the listed queries' only.
-// Entry e is probe slot j of query q, at index gi = q * P + j of the probe
-// table; q < 0 for an entry outside the pass.
+// The (query, probe) entries of a pass: entry e is probe slot e % P of query e / P.
 struct PairSet {
     const int32_t* npq;
-    const int32_t* active;
-    const int32_t* qlist;
-    const uint32_t* qcount;
     int nq, P;
-    __device__ int64_t size() const { return qlist ? (int64_t)*qcount * P : (int64_t)nq * P; }
-    __device__ int query(int64_t e, int& j, int64_t& gi) const {
-        const int w = (int)(e / P);
-        j = (int)(e % P);
-        const int q = qlist ? qlist[w] : w;
-        gi = (int64_t)q * P + j;
-        const int Pq = npq ? min(npq[q], P) : P;
-        return j < Pq && (qlist || !active || active[q]) ? q : -1;
-    }
+    __device__ int64_t size() const { return (int64_t)nq * P; }
 };
 
-// Entry e of a pass, evaluated with unconditional loads (every index is
-// valid whether or not the entry is in the pass), so that the unrolled loops
-// below overlap the latencies of a thread's consecutive entries: the query
-// q, probe slot j, its probe-table index i and list l; `in` = part of the
-// pass; `pass` = in and the list-level radius bound keeps it; dc = the
-// query's coarse distance to the list.
+// One entry: query q, probe slot j, its probe-table index i and list l; `in` =
+// among the query's probes; `pass` = in and the list-level radius bound keeps it; dc =
+// the query's coarse distance to the list.
 struct Entry {
     int q, j, l;
     int64_t i;
@@ -497,39 +476,9 @@ __device__ inline float reach_frac(float dlo, float sq, float2 rb) {
     return fminf(fmaxf(fr, 0.0f), 1.0f);  // (fmaxf takes 0 for NaN)
 }
 
-__device__ inline Entry entry_at(const PairSet& ps, const PairFilter& f, const int32_t* __restrict__ probes,
-                                 int64_t e) {
-    Entry x;
-    const int w = (int)(e / ps.P);
-    x.j = (int)(e % ps.P);
-    x.q = ps.qlist ? ps.qlist[w] : w;
-    x.i = (int64_t)x.q * ps.P + x.j;
-    const int Pq = ps.npq ? min(ps.npq[x.q], ps.P) : ps.P;
-    const bool act = ps.qlist || !ps.active || ps.active[x.q];
-    x.l = probes[x.i];
-    x.in = x.j < Pq && act && x.l >= 0;
-    if (!f.cd) {
-        x.pass = x.in;
-        x.dc = 0.0f;
-        x.fr = 0.0f;
-        return x;
-    }
-    // pair_may_pass, branch-free
-    const float t = f.tau[x.q];
-    const float dc = f.cd[x.i];
-    const float2 rb = f.lbound[max(x.l, 0)];
-    const float dlo = sqrtf(fmaxf(dc, 0.0f) * (1.0f - 1e-4f));
-    const float dhi = sqrtf(dc * (1.0f + 1e-4f));
-    const float sq = sqrtf(t * (1.0f + 1e-4f));
-    x.dc = dc;
-    x.pass = x.in && t >= 0.0f && !(dlo - rb.y > sq) && !(rb.x - dhi > sq);
-    x.fr = reach_frac(dlo, sq, rb);
-    return x;
-}
-
-// The entries e0 + tid + 256 u (u < kEntryBatch) of a pass over every query
-// (no query list, no flags), evaluated together: all their loads are issued
-// before any is used.  f(x) is called for each entry below e1.
+// The entries e0 + tid + 256 u (u < kEntryBatch) of a pass, evaluated together: all
+// their loads are issued before any is used (every index is valid).  f(x) is called for each
+// entry below e1.
 constexpr int kEntryBatch = 8;
 
 template <bool NPQ, bool CD, class F>
@@ -580,25 +529,22 @@ __device__ inline void entry_batches(const PairSet& ps, const PairFilter& pf, co
         entry_batch<NPQ, CD>(ps, pf, probes, e, e1, f);
 }
 
-// Every entry of [e0, e1) owned by this thread (stride 256), batched when
-// the pass covers every query.
+// Every entry of [e0, e1) owned by this thread (stride 256).
 template <class F>
 __device__ inline void for_entries(const PairSet& ps, const PairFilter& pf, const int32_t* __restrict__ probes,
                                    int64_t e0, int64_t e1, F&& f) {
-    if (!ps.qlist && !ps.active) {
-        if (ps.npq && pf.cd)
-            entry_batches<true, true>(ps, pf, probes, e0, e1, f);
-        else if (ps.npq)
-            entry_batches<true, false>(ps, pf, probes, e0, e1, f);
-        else if (pf.cd)
-            entry_batches<false, true>(ps, pf, probes, e0, e1, f);
-        else
-            entry_batches<false, false>(ps, pf, probes, e0, e1, f);
-    } else {
-        for (int64_t e = e0 + threadIdx.x; e < e1; e += 256) f(entry_at(ps, pf, probes, e));
-    }
+    if (ps.npq && pf.cd)
+        entry_batches<true, true>(ps, pf, probes, e0, e1, f);
+    else if (ps.npq)
+        entry_batches<true, false>(ps, pf, probes, e0, e1, f);
+    else if (pf.cd)
+        entry_batches<false, true>(ps, pf, probes, e0, e1, f);
+    else
+        entry_batches<false, false>(ps, pf, probes, e0, e1, f);
 }
 
+// count_kernel with a per-workgroup LDS histogram: one global atomic per
+// (workgroup, list) instead of one per entry.
 __global__ __launch_bounds__(256) void count_lds_kernel(const int32_t* __restrict__ probes, PairSet ps,
                                                         const int32_t* __restrict__ list_size, int nlist,
                                                         PairFilter pf, uint32_t* __restrict__ lcnt,
@@ -1065,7 +1011,7 @@ __device__ __forceinline__ floatx16 mfma16(const bf16x8& x, const bf16x8& y, con
 template <int NKC, int QG, bool FAST, bool F16>
 __device__ __forceinline__ void batched_scan_body(const BatchArgs& a) {
     // exactly one of the scan kernels works on a batch; none when there is
-    // no work (a rescue pass with nothing flagged)
+    // no work (no query reaches a list)
     if (batch_kind(a) != (FAST ? 1 : 0) || a.meta[0] == 0) return;
     // one-query-group waves stage their survivors per query slot in LDS
     // (kStage keys per slot): the keys of many tiles go out with one counted
@@ -1303,7 +1249,7 @@ constexpr bool kI8RunsBf16 = NKC8 == 4 && QG == 2;  // d <= 128, 64-query items
 template <int NKC8, int QG>
 __global__ __launch_bounds__(kNT) __attribute__((amdgpu_waves_per_eu(NKC8 == 4 ? (QG == 1 ? 3 : 2) : 1)))
 void batched_scan_i8_kernel(BatchArgs a) {
-    if (a.meta[0] == 0) return;  // no work (a rescue pass with nothing flagged)
+    if (a.meta[0] == 0) return;  // no work (no query reaches a list)
     if (batch_kind(a) != 2) {
         // Not every query integer: the 64-query form runs the BF16 form
         // itself (its arena order, its bound intervals), which saves the
@@ -1596,7 +1542,7 @@ struct SelArgs {
     const float4* q;            // padded queries
     int nquad;
     int k;
-    int metric;                 // of the keys' ranks (IP: the exact FP32 scans only)
+    int metric;                 // of the keys' ranks (IP: plain searches only)
     float* out_d;
     int64_t* out_i;
     float* rescan_tau;          // [nq] bound for the rescan of flagged queries
@@ -2294,8 +2240,8 @@ void launch_select(SelArgs a, int64_t n, size_t lds, int32_t* hard, uint32_t* nh
 // distance as the int8 scan); otherwise 64 rows of the FP32 arena, lane per
 // row, with the canonical FP32 chain.  Rows within the bound are appended to
 // the query's survivor buffer with one counted atomic per wave and tile.
-// The keys hold canonical distances, so the one-wave selection applies as
-// is (in a launch of its own: with the workgroup that ends a query's last pair
+// The keys hold canonical distances, so the selection takes them as they
+// are (in a launch of its own: with the workgroup that ends a query's last pair
 // selecting, the fence that each pair then needs took 471 queries from 1.7 to
 // 5.9 ms).  Pairs that the list's radius interval excludes are skipped, as in
 // the plan.
@@ -2509,7 +2455,7 @@ hipError_t launch_plan(const PlanBufs& b, const int32_t* probes, const float* cd
         hipLaunchKernelGGL(count_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, probes, ps, list_size, nlist,
                            pf, b.lcnt, cand);
     else
-        hipLaunchKernelGGL(count_kernel, dim3(gnp), dim3(256), 0, s, probes, ps.nq, ps.P, ps.npq, ps.active, list_size,
+        hipLaunchKernelGGL(count_kernel, dim3(gnp), dim3(256), 0, s, probes, ps.nq, ps.P, ps.npq, list_size,
                            pf, b.lcnt, cand);
     hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(1024), 0, s, b.lcnt, (const uint32_t*)nullptr, list_size, nlist, qc,
                        rt, b.qoff, b.lcur, b.lend, b.ioff, b.meta, qint, nint, all_int);
@@ -2517,7 +2463,7 @@ hipError_t launch_plan(const PlanBufs& b, const int32_t* probes, const float* cd
         hipLaunchKernelGGL(fill_lds_kernel, dim3(std::max(1u, gpe)), dim3(256), 0, s, probes, cd, ps, nlist, pf,
                            b.lcur, b.lend, b.lq, b.lqd);
     else
-        hipLaunchKernelGGL(fill_kernel, dim3(gnp), dim3(256), 0, s, probes, cd, ps.nq, ps.P, ps.npq, ps.active, pf,
+        hipLaunchKernelGGL(fill_kernel, dim3(gnp), dim3(256), 0, s, probes, cd, ps.nq, ps.P, ps.npq, pf,
                            b.lcur, b.lend, b.lq, b.lqd);
     hipLaunchKernelGGL(items_par_kernel, dim3(iwg), dim3(256), 0, s, ia);
     return hipGetLastError();
@@ -2921,7 +2867,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
         pf.cd = h->d_cd.p;
         pf.tau = tau;
         pf.lbound = static_cast<const float2*>(B.lbound);
-        HIP_TRY(h, launch_plan(pl, h->d_probes.p, h->d_cd.p, h->d_size.p, PairSet{npq, nullptr, nullptr, nullptr, (int)n, P}, pf,
+        HIP_TRY(h, launch_plan(pl, h->d_probes.p, h->d_cd.p, h->d_size.p, PairSet{npq, (int)n, P}, pf,
                                qc, (uint32_t)rt, qint, (int)n, all_int, cand, s));
         if (timing) HIP_TRY(h, hipEventRecord(h->ev[6], s));
         BatchArgs ba;
@@ -3240,7 +3186,8 @@ static int split_fits(hivf_index* h, hipStream_t s, bool* fits) {
     return HIVF_OK;
 }
 
-// Batches of plain and pruned searches by the exact FP32 scans (flat.hpp).
+// Batches of plain and pruned searches by the split scan (split.hpp) or the FP32
+// scans (flat.hpp): results are the FP32 chain's either way.
 // HIVF_EUNSUPPORTED, with nothing launched: the per-query kernel serves them.
 int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
              const hivf_search_params& p, float* D, int64_t* I, unsigned long long* stats, hipEvent_t tau_done,
@@ -3288,7 +3235,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         return o;
     };
     const size_t entries = shared ? (size_t)chunk * P : 0;
-    const size_t o_sbuf = take((size_t)chunk * cap * 8), o_scnt = take(chunk * 4), o_fb = take(chunk * 4),
+    const size_t o_sbuf = take((size_t)chunk * cap * 8), o_scnt = take(chunk * 4),
                  o_fbl = take(chunk * 4), o_hard = take(chunk * 4), o_tau = take(chunk * 4), o_rtau = take(chunk * 4),
                  o_fbc = take(kFbcWords * 4), o_part = take(part_keys_bytes(k)), o_allint = take(4), o_lcnt = take(nlist * 4), o_lcur = take(nlist * 4),
                  o_lend = take(nlist * 4), o_qoff = take((nlist + 1) * 4), o_ioff = take((nlist + 1) * 8),
@@ -3309,7 +3256,6 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     }
     auto at = [&](size_t o) { return static_cast<void*>(static_cast<char*>(B.scratch) + o); };
     uint32_t* scnt = (uint32_t*)at(o_scnt);
-    int32_t* fb = (int32_t*)at(o_fb);
     uint32_t* lcnt = (uint32_t*)at(o_lcnt);
     uint32_t* fbc = (uint32_t*)at(o_fbc);
     uint32_t* all_int = (uint32_t*)at(o_allint);
@@ -3340,7 +3286,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         const int32_t* probes = h->d_probes.p + q0 * P;
         const int32_t* npqc = npq ? npq + q0 : nullptr;
         hipLaunchKernelGGL(flat_clear_kernel, dim3((unsigned)((std::max<int64_t>(std::max(m, nlist), kFbcWords) + 255) / 256)),
-                           dim3(256), 0, s, scnt, fb, (int)m, lcnt, (int)nlist, fbc, kFbcWords, all_int);
+                           dim3(256), 0, s, scnt, (int)m, lcnt, (int)nlist, fbc, kFbcWords, all_int);
         ScanArgs w{};
         w.lists = h->lists();
         w.q = q + q0 * h->nquad;
@@ -3373,8 +3319,8 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         const int64_t dpad16 = (int64_t)nkc * 16;
         if (shared) {
             PairFilter pf{};  // (no radius intervals here: every pair is scanned)
-            HIP_TRY(h, launch_plan(pl, probes, h->d_cd.p + q0 * P, h->d_size.p, PairSet{npqc, nullptr, nullptr, nullptr, (int)m, P},
-                                   pf, qc, rt, fb, 0, all_int, stats, s));
+            HIP_TRY(h, launch_plan(pl, probes, h->d_cd.p + q0 * P, h->d_size.p, PairSet{npqc, (int)m, P},
+                                   pf, qc, rt, nullptr, 0, all_int, stats, s));
         }
         if (split) {
             SplitArgs b{};
@@ -3418,7 +3364,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         sa.scnt = scnt;
         sa.sbuf = a.sbuf;
         sa.cap = cap;
-        sa.qint = split ? C.qint.p + q0 : fb;  // (fb: read, not used)
+        sa.qint = split ? C.qint.p + q0 : probes;  // (probes: read, not used)
         sa.all_int = all_int;
         // (the FP32 scans' keys are final; the split scan's are where every
         // product and sum is an integer below 2^24)

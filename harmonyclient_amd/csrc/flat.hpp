@@ -237,13 +237,10 @@ __global__ __launch_bounds__(kNT) void flat_pair_kernel(FlatArgs a) {
 }
 
 // Counters of one chunk of queries, cleared before it.
-__global__ void flat_clear_kernel(uint32_t* scnt, int32_t* fb, int n, uint32_t* lcnt, int nlist, uint32_t* fbc,
+__global__ void flat_clear_kernel(uint32_t* scnt, int n, uint32_t* lcnt, int nlist, uint32_t* fbc,
                                   int fbc_words, uint32_t* all_int) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        scnt[i] = 0;
-        fb[i] = 0;
-    }
+    if (i < n) scnt[i] = 0;
     if (i < nlist) lcnt[i] = 0;
     if (i < fbc_words) fbc[i] = 0;
     if (i == 0) *all_int = 0;

@@ -256,7 +256,7 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
                 const hivf_search_params& p, float* D, int64_t* I, hivf_search_stats* st,
                 hipStream_t s, bool timing);
 // Plain or pruned search of n staged queries whose probes are in d_probes, by
-// the batch's exact FP32 scans (batched.hip); stats: d_stats or null; tau_done:
+// the batch's scans (batched.hip); stats: d_stats or null; tau_done:
 // recorded after the first bound, or null.
 int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const int32_t* npq,
              const hivf_search_params& p, float* D, int64_t* I, unsigned long long* stats, hipEvent_t tau_done,

@@ -38,7 +38,6 @@ constexpr int kFeatCoarse = 32;
 struct GemmArgs {
     const float* A;
     int lda;
-    int transA;  // A'(m, k) = transA ? A[k * lda + m] : A[m * lda + k]
     const float* B;
     int ldb;
     int transB;  // B'(k, n) = transB ? B[n * ldb + k] : B[k * ldb + n]
@@ -51,7 +50,7 @@ struct GemmArgs {
     int ldm;
 };
 
-// C = epilogue(A' B'): 32 x 64 output tile per 256-thread workgroup, 2 x 4
+// C = epilogue(A B'): 32 x 64 output tile per 256-thread workgroup, 2 x 4
 // per thread, K in chunks of 16 staged in LDS, the next chunk's loads in flight
 // beside the products; fixed summation order (k ascending from zero).  What
 // bounds it is latency, 8 chunks of load, barrier and product: 8192 rows by 128 x
@@ -65,8 +64,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
     // consecutive threads along the operand's contiguous index
     auto placeA = [&](int t, int& k, int& r) {
         const int e = t * 256 + threadIdx.x;
-        k = g.transA ? e / 32 : e % 16;
-        r = g.transA ? e % 32 : e / 16;
+        k = e % 16;
+        r = e / 16;
     };
     auto placeB = [&](int t, int& k, int& r) {
         const int e = t * 256 + threadIdx.x;
@@ -79,7 +78,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(GemmArgs g) {
             int k, r;
             placeA(t, k, r);
             const int kc = min(k0 + k, g.K - 1), m = min(m0 + r, g.M - 1);
-            const float v = g.A[g.transA ? (size_t)kc * g.lda + m : (size_t)m * g.lda + kc];
+            const float v = g.A[(size_t)m * g.lda + kc];
             ra[t] = m0 + r < g.M && k0 + k < g.K ? v : 0.0f;
         }
 #pragma unroll
@@ -550,9 +549,9 @@ hipError_t hivf_tau_model::ensure_work(int64_t rows) {
 }
 
 namespace hivf {
-static hipError_t gemm(hipStream_t s, const float* A, int lda, int tA, const float* B, int ldb, int tB, float* C,
+static hipError_t gemm(hipStream_t s, const float* A, int lda, const float* B, int ldb, int tB, float* C,
                        int ldc, int M, int N, int K, const float* bias, int relu, const float* mask, int ldm) {
-    GemmArgs g{A, lda, tA, B, ldb, tB, C, ldc, M, N, K, bias, relu, mask, ldm};
+    GemmArgs g{A, lda, B, ldb, tB, C, ldc, M, N, K, bias, relu, mask, ldm};
     hipLaunchKernelGGL(gemm_kernel, dim3(blocks(M, 32), blocks(N, 64)), dim3(256), 0, s, g);
     return hipGetLastError();
 }
@@ -566,10 +565,10 @@ hipError_t hivf_tau_model::forward(hipStream_t s, const float* Xs, int rows, flo
     const float *W1 = P + off_W1, *b1 = P + off_b1, *W2 = P + off_W2, *b2 = P + off_b2, *w3 = P + off_w3,
                 *b3 = P + off_b3;
     hipError_t e;
-    if ((e = gemm(s, Xs, in, 0, W1, hid, 0, H1, hid, rows, hid, in, b1, 1, nullptr, 0)) != hipSuccess) return e;
-    if ((e = gemm(s, H1, hid, 0, W2, hid, 0, H2, hid, rows, hid, hid, b2, 1, nullptr, 0)) != hipSuccess) return e;
+    if ((e = gemm(s, Xs, in, W1, hid, 0, H1, hid, rows, hid, in, b1, 1, nullptr, 0)) != hipSuccess) return e;
+    if ((e = gemm(s, H1, hid, W2, hid, 0, H2, hid, rows, hid, hid, b2, 1, nullptr, 0)) != hipSuccess) return e;
     if (!yhat) return hipSuccess;  // (the backward alone needs no output)
-    return gemm(s, H2, hid, 0, w3, 1, 0, yhat, 1, rows, 1, hid, b3, 0, nullptr, 0);
+    return gemm(s, H2, hid, w3, 1, 0, yhat, 1, rows, 1, hid, b3, 0, nullptr, 0);
 }
 
 // Gradient of sum_i dy[i] yhat[i] w.r.t. the trained parameters into G (all
@@ -594,7 +593,7 @@ hipError_t hivf_tau_model::backward(hipStream_t s, const float* Xs, int rows, co
     const int64_t nz = (int64_t)rows * hid;
     hipLaunchKernelGGL(dz2_kernel, dim3(blocks(nz)), dim3(256), 0, s, dy, w3, H2, nz, hid, dZ2);
     // dZ1 = (dZ2 W2^T) * [H1 > 0]
-    if ((e = gemm(s, dZ2, hid, 0, W2, hid, 1, dZ1, hid, rows, hid, hid, nullptr, 0, H1, hid)) != hipSuccess) return e;
+    if ((e = gemm(s, dZ2, hid, W2, hid, 1, dZ1, hid, rows, hid, hid, nullptr, 0, H1, hid)) != hipSuccess) return e;
     const WgradArgs wa{Xs, H1, H2, dZ1, dZ2, dy, rows, (int)chunk, in, hid, off_W1, off_b1, off_W2, off_b2, off_w3,
                        off_b3, n_trained, part};
     const unsigned ht = blocks(hid, 64), it = blocks(in, 64);
