@@ -465,7 +465,7 @@ int check_params(hivf_index* h, int64_t k, const hivf_search_params& p) {
     if (p.precision != HIVF_PREC_FP32 && p.precision != HIVF_PREC_BF16)
         return h->fail(HIVF_EINVAL, "unknown precision");
     if (p.precision == HIVF_PREC_BF16 && p.algo != HIVF_ALGO_BATCHED)
-        return h->fail(HIVF_EUNSUPPORTED, "the per-query scans compute in FP32; BF16 is a batched-scan option");
+        return h->fail(HIVF_EUNSUPPORTED, "plain and pruned searches take no precision; BF16 is a batched-scan option");
     return HIVF_OK;
 }
 

@@ -38,9 +38,14 @@ extern "C" {
 #define HIVF_EUNSUPPORTED (-5)/* combination not implemented */
 #define HIVF_EIO (-6)         /* file read/write failed */
 
-/* Scan algorithm. */
-#define HIVF_ALGO_PLAIN 0   /* per-query scan, full distances (src/Index.cpp:1420-1554) */
-#define HIVF_ALGO_PRUNED 1  /* per-query scan, dimension-block pruning (src/node.cpp:606-678) */
+/* Scan algorithm.  Plain and pruned searches return the canonical FP32 chain's ids
+ * and distance bits; batches large enough are scanned list by list, the rows there
+ * ruled out by a bound whose error is proven (two BF16 pieces per value), the rest
+ * scored with the FP32 chain.  The pruned scan's block counts exist only in its
+ * FP32 form: a pruned search that asks for statistics takes that form, and may
+ * take longer than the same search without. */
+#define HIVF_ALGO_PLAIN 0   /* full distances (src/Index.cpp:1420-1554) */
+#define HIVF_ALGO_PRUNED 1  /* dimension-block pruning (src/node.cpp:606-678) */
 #define HIVF_ALGO_BATCHED 2 /* list-major batched scan with MFMA contractions */
 
 /* Source of the per-query pruning bound. */
@@ -51,11 +56,11 @@ extern "C" {
 /* Arithmetic of the batched scan's contractions.  Results are the FP32
  * path's either way (ids and distance bits); only the speed differs.
  * FP32: the batched scan picks its form -- exact int8 MFMA when every list
- * value and every query is an integer in [0, 255] and d <= 256, else the
- * BF16 shadow with a proven error margin and exact FP32 rescoring of the
- * candidates inside it.  The per-query scans always compute in FP32.
- * BF16: the batched scan uses the BF16 shadow even where the int8 form
- * applies (EUNSUPPORTED for the per-query scans). */
+ * value and every query is an integer in [0, 255] and d <= 256, else a 16-bit
+ * shadow (FP16 scaled by a power of two, or BF16) with a proven error margin and
+ * exact FP32 rescoring of the candidates inside it.
+ * BF16: the batched scan uses the shadow even where the int8 form applies
+ * (EUNSUPPORTED for plain and pruned searches, whose results are FP32's always). */
 #define HIVF_PREC_FP32 0
 #define HIVF_PREC_BF16 1
 
@@ -104,7 +109,7 @@ typedef struct {
     int64_t batch_rows;
     int64_t batch_waves;
     double plan_ms;        /* batched scan: probe inversion and work-item planning */
-    int64_t scan_kind;     /* batched scan that ran: 0 BF16 with error margin, 1 BF16 exact,
+    int64_t scan_kind;     /* batched scan that ran: 0 16-bit shadow with error margin, 1 BF16 exact,
                               2 int8 (integer data) */
     int64_t overflow_queries; /* batched scan: of fallback_queries, those whose survivors
                                  overflowed survivor_cap (the rest: learned bound too low) */
