@@ -17,7 +17,7 @@ import numpy as np
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
-HBM_PEAK_GBS = 8000.0          # MI355X HBM3E
+FP32_VECTOR_PEAK_TFLOPS = 157.3 # MI355X FP32 vector
 BF16_DENSE_PEAK_TFLOPS = 2500.0  # MI355X dense BF16 MFMA
 INT8_DENSE_PEAK_TOPS = 5000.0    # MI355X dense int8 MFMA
 METRIC = "QPS at fixed recall@100, 1M×128 IVF: tuned GPU vs plain GPU vs CPU"
@@ -448,15 +448,17 @@ def main():
     rec = recall(ref_I[:rs], GT)
 
     # Roofline of each path's dominant kernel, from HIP events on the stream
-    # the kernel runs on.  Per-query scans stream 4 d bytes per candidate
-    # (HBM-bound); the batched scan contracts 2 d flops per candidate on
-    # BF16 MFMA.  Candidates = sum over queries of the probed list lengths.
+    # the kernel runs on.  Every path's scan of a batch is list-major (a row read
+    # serves many queries) and does 2 d operations per candidate: the batched scan on
+    # int8 or 16-bit MFMA, the plain scan as three BF16 products per FP32 one, the
+    # pruned scan, timed with its block counts, on FP32 vector units.
+    # Candidates = sum over queries of the probed list lengths.
     def roof(name, stats):
         """`frac` is the EFFECTIVE fraction: algorithmic work of every probed
         row (also the tiles, pairs or dimension blocks the bounds let the
         kernel skip) over the kernel's time.  `frac_issued` counts only the
-        work the kernel issued: the MFMA tiles it ran (batched), or the
-        dimension blocks it loaded (per-query scans)."""
+        work the kernel issued: the MFMA tiles it ran (batched), the three
+        products (plain), or the dimension blocks it did not skip (pruned)."""
         scan_ms = float(np.mean([s.scan_ms for s in stats]))
         cand = float(np.mean([s.candidates for s in stats]))
         tiles_run = float(np.mean([s.blocks_total - s.blocks_skipped for s in stats]))
@@ -485,16 +487,21 @@ def main():
                     "issued_flops_per_launch": issued,
                     "traffic": traffic_of(name, "batched_scan_kernel"), "kernel": "batched_scan_kernel",
                     "kernel_ms": round(scan_ms, 4), "alg_flops_per_launch": ops, "precision": "bf16 -> f32"}
-        alg = cand * w.d * 4
-        gbs = alg / sec / 1e9
-        nblk = float(np.mean([s.blocks_total for s in stats])) / max(cand, 1.0)  # blocks per candidate
-        loaded = alg * (tiles_run / max(float(np.mean([s.blocks_total for s in stats])), 1.0)) if nblk > 1 else alg
-        return {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": round(gbs / HBM_PEAK_GBS, 4), "frac_kind": "effective",
-                "frac_issued": round(loaded / sec / 1e9 / HBM_PEAK_GBS, 4), "loaded_bytes_per_launch": loaded,
-                "traffic": traffic_of(name, "scan_kernel"),
-                "kernel": "scan_kernel", "kernel_ms": round(scan_ms, 4),
-                "alg_bytes_per_launch": alg}
+        ops = 2.0 * w.d * cand
+        rate = ops / sec / 1e12
+        out = {"bound": "mfma", "achieved": round(rate, 2), "peak": BF16_DENSE_PEAK_TFLOPS, "unit": "TFLOP/s",
+               "frac": round(rate / BF16_DENSE_PEAK_TFLOPS, 4), "frac_kind": "effective",
+               "kernel_ms": round(scan_ms, 4), "alg_flops_per_launch": ops}
+        if name.startswith("pruned"):
+            total = max(float(np.mean([s.blocks_total for s in stats])), 1.0)
+            out.update(bound="valu", peak=FP32_VECTOR_PEAK_TFLOPS, frac=round(rate / FP32_VECTOR_PEAK_TFLOPS, 4),
+                       issued_flops_per_launch=ops * tiles_run / total, kernel="flat_scan_kernel", precision="f32")
+        else:
+            out.update(issued_flops_per_launch=3.0 * ops, precision="2 x bf16 -> f32",
+                       kernel="split_wave_kernel" if w.d <= 128 else "split_wg_kernel")
+        out["frac_issued"] = round(out["issued_flops_per_launch"] / sec / 1e12 / out["peak"], 4)
+        out["traffic"] = traffic_of(name, out["kernel"])
+        return out
 
     traffic = read_traffic(w.name)
 

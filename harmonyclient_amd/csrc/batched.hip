@@ -2388,15 +2388,25 @@ float margin_abs_f16(int64_t d, float scale) {
     return (float)(1.01 * 2 * (double)d * delta * delta * (16384.0 + 1.0)) + 1e-30f;
 }
 
-// Rows (ids other than the padding's) whose squared norm is below lim.
+// Words of the counts by which a form of the lists is chosen.
+constexpr int kVoteWords = 256;
+
+// Rows (ids other than the padding's) whose squared norm is below lim, each
+// workgroup's into its word of out.
 __global__ __launch_bounds__(256) void count_below_kernel(const float* __restrict__ norms,
                                                           const uint32_t* __restrict__ ids, int64_t n, float lim,
                                                           unsigned long long* __restrict__ out) {
-    unsigned long long c = 0;
+    __shared__ unsigned int sum;
+    if (threadIdx.x == 0) sum = 0;
+    __syncthreads();
+    unsigned int c = 0;  // (a workgroup has at most 2^31 / 64 rows)
+#pragma unroll 4
     for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256)
         c += ids[i] != kNoId && norms[i] < lim;
     for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off);
-    if ((threadIdx.x & 63) == 0 && c) atomicAdd(out, c);
+    if ((threadIdx.x & 63) == 0) atomicAdd(&sum, c);
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = sum;
 }
 
 // Buffers of the planning (carved from the scratch) and its work-item bound.
@@ -2540,15 +2550,16 @@ static int f16_scale_of(hivf_index* h, float* scale, hipStream_t s) {
     if (mx > 0.0f && h->tiles > 0) {
         // where a row meets a query of its own norm
         const float lim = margin_abs_f16(h->d, sc) / (2.0f * (margin_coef(h->d) - margin_coef_f16(h->d)));
-        unsigned long long below = 0;
-        HIP_TRY(h, h->d_vote.ensure(2));
-        HIP_TRY(h, hipMemcpyAsync(h->d_vote.p, &below, sizeof(below), hipMemcpyHostToDevice, s));
+        unsigned long long v[kVoteWords], below = 0;
+        HIP_TRY(h, h->d_vote.ensure(kVoteWords));
         const int64_t rows = h->tiles * kTileRows;
-        hipLaunchKernelGGL(count_below_kernel, dim3((unsigned)std::min<int64_t>((rows + 255) / 256, 1024)), dim3(256), 0,
-                           s, h->d_norms.p, h->d_ids.p, rows, lim, h->d_vote.p);
+        const int blocks = (int)std::min<int64_t>((rows + 1023) / 1024, kVoteWords);
+        hipLaunchKernelGGL(count_below_kernel, dim3(blocks), dim3(256), 0, s, h->d_norms.p, h->d_ids.p, rows, lim,
+                           h->d_vote.p);
         HIP_TRY(h, hipGetLastError());
-        HIP_TRY(h, hipMemcpyAsync(&below, h->d_vote.p, sizeof(below), hipMemcpyDeviceToHost, s));
+        HIP_TRY(h, hipMemcpyAsync(v, h->d_vote.p, blocks * sizeof(v[0]), hipMemcpyDeviceToHost, s));
         HIP_TRY(h, hipStreamSynchronize(s));
+        for (int i = 0; i < blocks; ++i) below += v[i];
         if (below > (unsigned long long)h->ntotal / 2) return HIVF_OK;
     }
     *scale = sc;
@@ -3169,8 +3180,9 @@ static int split_fits(hivf_index* h, hipStream_t s, bool* fits) {
         const float w = l2 ? c : c * c * (float)h->d / (2.5f * 2.5f);
         const int64_t step = (h->tiles + kWideTiles - 1) / kWideTiles;
         const int blocks = (int)((h->tiles + 4 * step - 1) / (4 * step));
-        unsigned long long v[kWideTiles / 4 + 1], asked = 0, wide = 0;
-        HIP_TRY(h, h->d_vote.ensure(sizeof(v) / sizeof(v[0])));
+        unsigned long long v[kVoteWords], asked = 0, wide = 0;
+        static_assert(kWideTiles / 4 <= kVoteWords, "a word per workgroup");
+        HIP_TRY(h, h->d_vote.ensure(kVoteWords));
         hipLaunchKernelGGL(wide_rows_kernel, dim3(blocks), dim3(256), 0, s, h->lists(), h->d_norms.p, h->d_cent_rows.p,
                            (int)h->nlist, h->tiles, step, w, h->d_vote.p);
         HIP_TRY(h, hipGetLastError());
