@@ -450,14 +450,15 @@ def main():
     # Roofline of each path's dominant kernel, from HIP events on the stream
     # the kernel runs on.  Every path's scan of a batch is list-major (a row read
     # serves many queries) and does 2 d operations per candidate: the batched scan on
-    # int8 or 16-bit MFMA, the plain scan as three BF16 products per FP32 one, the
-    # pruned scan, timed with its block counts, on FP32 vector units.
+    # int8 or 16-bit MFMA, the plain scan as three BF16 products per FP32 one (two where
+    # the rows are small integers, exact in one BF16 piece), the pruned scan, timed with
+    # its block counts, on FP32 vector units.
     # Candidates = sum over queries of the probed list lengths.
     def roof(name, stats):
         """`frac` is the EFFECTIVE fraction: algorithmic work of every probed
         row (also the tiles, pairs or dimension blocks the bounds let the
         kernel skip) over the kernel's time.  `frac_issued` counts only the
-        work the kernel issued: the MFMA tiles it ran (batched), the three
+        work the kernel issued: the MFMA tiles it ran (batched), its
         products (plain), or the dimension blocks it did not skip (pruned)."""
         scan_ms = float(np.mean([s.scan_ms for s in stats]))
         cand = float(np.mean([s.candidates for s in stats]))
@@ -468,6 +469,7 @@ def main():
             # probed row)
             ops = 2.0 * w.d * cand
             rate = ops / sec / 1e12
+            kern = "batched_scan_kernel" if w.d <= 128 else "shadow_wg_kernel"
             qslots = stats[-1].batch_queries  # query slots of an item (MFMA columns issued)
             if stats[-1].scan_kind == 2:
                 dpad = 128 if w.d <= 128 else 256
@@ -479,14 +481,12 @@ def main():
                         "issued_ops_per_launch": issued,
                         "traffic": traffic_of(name, kern), "kernel": kern,
                         "kernel_ms": round(scan_ms, 4), "alg_ops_per_launch": ops, "precision": "int8 x int8 -> int32"}
-            dpad = (w.d + 15) // 16 * 16
-            issued = tiles_run * 32 * qslots * 2 * dpad
+            # (only the int8 scan counts its tiles)
             return {"bound": "mfma", "achieved": round(rate, 2), "peak": BF16_DENSE_PEAK_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(rate / BF16_DENSE_PEAK_TFLOPS, 4),
-                    "frac_kind": "effective", "frac_issued": round(issued / sec / 1e12 / BF16_DENSE_PEAK_TFLOPS, 4),
-                    "issued_flops_per_launch": issued,
-                    "traffic": traffic_of(name, "batched_scan_kernel"), "kernel": "batched_scan_kernel",
-                    "kernel_ms": round(scan_ms, 4), "alg_flops_per_launch": ops, "precision": "bf16 -> f32"}
+                    "frac_kind": "effective", "frac_issued": None, "issued_flops_per_launch": None,
+                    "traffic": traffic_of(name, kern), "kernel": kern,
+                    "kernel_ms": round(scan_ms, 4), "alg_flops_per_launch": ops, "precision": "f16 or bf16 -> f32"}
         ops = 2.0 * w.d * cand
         rate = ops / sec / 1e12
         out = {"bound": "mfma", "achieved": round(rate, 2), "peak": BF16_DENSE_PEAK_TFLOPS, "unit": "TFLOP/s",
@@ -497,7 +497,9 @@ def main():
             out.update(bound="valu", peak=FP32_VECTOR_PEAK_TFLOPS, frac=round(rate / FP32_VECTOR_PEAK_TFLOPS, 4),
                        issued_flops_per_launch=ops * tiles_run / total, kernel="flat_scan_kernel", precision="f32")
         else:
-            out.update(issued_flops_per_launch=3.0 * ops, precision="2 x bf16 -> f32",
+            x = xb[:1000]
+            pieces = 2.0 if ((x == np.rint(x)) & (x >= 0) & (x <= 255)).all() else 3.0
+            out.update(issued_flops_per_launch=pieces * ops, precision="2 x bf16 -> f32",
                        kernel="split_wave_kernel" if w.d <= 128 else "split_wg_kernel")
         out["frac_issued"] = round(out["issued_flops_per_launch"] / sec / 1e12 / out["peak"], 4)
         out["traffic"] = traffic_of(name, out["kernel"])
