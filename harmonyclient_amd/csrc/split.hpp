@@ -11,8 +11,8 @@
 // cycles, where the FP32 chain needs 2048 vector cycles for the same.  1000 plain
 // queries of 32 lists (500k x 128): 98 us against 336 for the FP32 scan, their host
 // search 0.70 -> 0.49 ms with it (0.35 now); 2000 pruned queries of 48 lists 173 us,
-// the search 0.96 -> 0.43 ms (0.26 now); 500 inner-product queries of 201 dims 46 us
-// against 152.
+// the search without statistics 0.96 -> 0.43 ms (0.26 now); 500 inner-product
+// queries of 201 dims 46 us against 152.
 #pragma once
 
 namespace hivf {
