@@ -3102,57 +3102,73 @@ int run_batched(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, con
 }
 
 
-// The form of a plain or pruned search, by n queries, P probes each, the mean rows
-// of a list and d dims; list-major forms also by the queries that a list gets on
-// average.  Measured over 16 to 1000 lists of 60 to 3000 rows, 30 to 4000 queries, 1
-// to 64 probes, 32 to 420 dims, each search in every form (5280 searches): these rules'
-// choice takes 2.5 % longer than the best on average.  Figures are the whole
-// search's in us.
+// Rows of the list that a row of the index lies in, on average and in whole tiles:
+// queries spread like the rows probe lists of that many, more than the mean list
+// where lists differ.
+static double probed_rows(hivf_index* h) {
+    BatchedState& B = h->batched;
+    if (B.probed_rows < 0.0) {
+        double sq = 0.0;
+        for (int64_t l = 0; l < h->nlist; ++l) {
+            const double t = 64.0 * (double)(h->tile_off[l + 1] - h->tile_off[l]);
+            sq += t * t;
+        }
+        B.probed_rows = h->tiles > 0 ? sq / (64.0 * (double)h->tiles) : 64.0;
+    }
+    return B.probed_rows;
+}
+
+// The form of a plain or pruned search, by n queries, P probes each, the rows of a
+// probed list and d dims; list-major forms also by the queries that a probed list
+// gets.  Measured, each search in every form: 13,700 searches of 16 to 2000 lists of 60
+// to 3000 rows, 1 to 4000 queries, 1 to 64 probes, 32 to 420 dims, on Gaussian, anisotropic
+// and clustered data, whose lists differ in size by their builds, and on equal lists set by
+// the caller, far apart from one another and in no order, where the pruned
+// per-query scan skips most and the first bounds are loose.  These rules' choice takes 4 %
+// (plain), 7 and 5 % (pruned, without and with statistics) longer than the best on built lists, 1
+// to 5 % on the others; by the mean list, and for pruned searches by lines drawn on
+// the equal lists, it was 10 to 84 %.  Figures are the whole search's in us.
 //
 // Whether the queries share lists enough for a list-major form (else a
 // workgroup per query and list, which reads every pair's rows through the
-// caches).  The plan repays itself from about 2.5e8 components on (1000 queries of 2
-// lists of 1000 rows in 256, 128 dims: 132 against 172; below it, at 2e8, 1.15 times as
-// slow on average).  Past 128 dims a workgroup's waves split the lists' rows, 1024 at a
-// time: 4.5e8 components there (1000 of 2 of 3000 rows in 64, 201 dims: 261 against 457),
-// and past 256 dims, where a tile's rows are long, 6.4e8, 12 queries a list and 128
-// items to fill the chip (250 queries of 2 of 3000 rows in 16, 420 dims, are 48 items:
-// 480 against 235; 1000 of 4 of 1000 rows in 64 are 128: 385 against 652).  With one
-// probe the split scan prepares its own queries, and the per-query kernel reads
-// few rows twice: from 3.2e8 (4000 of lists of 1000 rows in 16, 201 dims, 8e8: 234 against
-// 525) and not past 256 dims (4000 of 3000 rows in 256, 420 dims: 3549 against 2794).  The
-// pruned scan skips most of its rows' dims and wants more queries a list: 1000 of 4 lists
-// of 1000 rows in 1000, 201 dims, 345 against 273.  For the FP32 scan: 1000 of 16 lists of 256
-// rows, 32 dims, 1.3e8, are 40 % slower.
-static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, int64_t d, bool split, bool pruned) {
-    const double comps = (double)n * P * rows * (double)d, per_list = (double)n * P / (double)nlist;
+// caches).  The plan repays itself from about 2.5e8 components on, pruned 3.2e8 (1.6e8 to
+// 2.5e8: 1.05 to 1.3 times as slow; 1000 queries of 2 lists of 1000 rows in 256, 128 dims, 2.6e8: 132 against
+// 172, 600 of 4 lists in 2000, 3e8: 240 against 220), with one probe, whose few pairs the
+// other forms spread worst, from 1.6e8 (600 of one of 1800 in 16, 1.4e8: 97 against 81, 4000 of one of 1600 in 256, 8.4e8: 185 against
+// 552).  Past 256 dims a tile's rows are long: 6.4e8, and 128
+// items of 1024 rows to fill the chip (250 queries of 2 lists of 3000 rows in 16, 420 dims, are 48
+// items: 480 against 235; 4000 of one of 1600 in 256, 300 dims: 335 against 1095).  The pruned scan, which
+// skips rows' dims, wants more work past 128 dims (4.5e8) and twice the items and queries a list past
+// 256 (1000 of 2 lists of 3000 rows, 420 dims, 841 against 533).  The FP32 scan: pruned, whose
+// tests skip dims, from 1.6e8 on long lists (100 queries of 64 lists of 1000 rows, 32 dims: 192 against
+// 358; 1000 of 16 of 60 rows 190 against 78), plain from 3.2e8 and 6 queries a list (1000 of 16 lists
+// of 256 rows, 32 dims, 1.3e8, are 40 % slower).
+static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, double per_list, int64_t d, bool split, bool pruned) {
+    const double comps = (double)n * P * rows * (double)d;
+    if (!split && pruned)
+        return per_list >= 2.0 && rows >= 60.0 && comps >= 1.6e8 && comps * std::min(rows, 1000.0) >= 1.6e11;
     if (!split) return per_list >= 6.0 && comps >= 3.2e8;
-    if (d <= 128) return per_list >= 2.0 && comps >= 2.5e8;
-    if (P == 1) return d <= 256 && per_list >= 2.0 && comps >= 3.2e8;
-    if (d <= 256) return per_list >= (pruned ? 6.0 : 2.0) && comps >= 4.5e8;
+    if (d <= 128) return per_list >= 2.0 && comps >= (P == 1 ? 1.6e8 : pruned ? 3.2e8 : 2.5e8);
+    if (d <= 256) return per_list >= 2.0 && comps >= (pruned ? 4.5e8 : 3.2e8);
     const double items = (double)nlist * std::ceil(rows / (kSplitWgTiles * 32.0)) * std::ceil(per_list / kSplitItem);
-    return per_list >= (pruned ? 20.0 : 12.0) && items >= (pruned ? 256.0 : 128.0) && comps >= 6.4e8;
+    return per_list >= (pruned ? 8.0 : 4.0) && items >= (pruned ? 256.0 : 128.0) && comps >= 6.4e8;
 }
 // Whether a batch repays these scans' launches (bound, plan, selection), or each
-// query's lists are scanned by a workgroup (64 x 4 rows at a time).  Plain: from
-// about 1100 rows per query (100 queries of 16 lists of 64 rows 1.15 times as slow,
-// of 100 rows 0.75), with one list each only while the queries leave the chip idle
-// (1000 of a list of 3000 rows in 16, 201 dims: 298 against 179, 300 of them, 32
-// dims, 59 against 73), or in list-major form from 3.2e8 components (4000 of 4 lists of
-// 100 rows, 300 dims: 1.07, of 128 rows 0.92); lists of fewer rows leave half of a
-// tile's lanes empty (4000 of 16 lists of 64 rows, 128 dims: 1.09).  The pruned scan
-// gains with more queries at once: up to 100 queries
-// (32 with statistics, whose scan is FP32) from 3200 rows, past 128 dims 1600 (one
-// query of 4 lists of 400 rows of 32 dims 73 and 55 us, of 128 62 and 57, of 300 66 and
-// 91), else in list-major form where comps x rows, at most 1000 of them, pass
-// 3.2e11, past 256 dims 4.8e11 (1000 of 16 lists, 128 dims, of 256 rows 1.16, of 400 0.82; 4000
-// of 16 lists of 64 rows 1.3; with statistics 1000 of 32 lists of 64 rows 4.6).
-static bool flat_pays(int64_t n, int P, double rows, int64_t d, bool pruned, bool stats, bool shared) {
-    const double comps = (double)n * P * rows * (double)d, per_query = P * rows;
-    const bool large = shared && rows >= 100.0 && comps >= 3.2e8;
-    if (!pruned) return (per_query >= 1100.0 && (P > 1 || n <= 512 || shared)) || large;
-    return (n <= (stats ? 32 : 100) && per_query >= (d <= 128 ? 3200.0 : 1600.0)) ||
-           (large && comps * std::min(rows, 1000.0) >= (d <= 256 ? 3.2e11 : 4.8e11));
+// query's lists are scanned by a workgroup (64 x 4 rows at a time): from
+// about 1100 rows per query, in whole tiles where lists fill half of theirs (700 to 1000
+// rows 1.05 to 1.2 times as slow, 1000 to 1300 0.8 to 0.9; 4000 of 32 lists of 16 rows 1.5). In pair
+// form only while the queries leave the chip idle: with one list each up to 1024 (600 of 1800
+// rows, 128 dims, 81 against 106), past 256 dims 512 (1000 of 3000 rows, 300 dims: 445 against 304),
+// pruned up to 512 (600 of 16 lists of 200 rows, 300 dims, equal lists far apart, 390 against 203). Or
+// in list-major form on lists of 100 rows (4000 of 4 lists of 100 rows, 300 dims: 1.07, of 128
+// rows 0.92; of 64 rows half of a tile's lanes are empty).  Where a pruned search takes the FP32
+// scan, in pair form up to 100 queries and 2000 pairs (100 of 64 lists of 60 rows: 246 against 98).
+static bool flat_pays(int64_t n, int P, double rows, double tile_rows, int64_t d, bool pruned, bool split, bool shared) {
+    const double comps = (double)n * P * rows * (double)d;
+    const bool many = P * (2.0 * rows >= tile_rows ? tile_rows : rows) >= 1100.0;
+    if (pruned && !split) return shared || (many && n <= 100 && n * P <= 2000);
+    const bool idle = P == 1 ? n <= (d <= 256 ? 1024 : 512) : !pruned || n <= 512;
+    return (many && (shared || idle)) || (shared && rows >= 100.0 && comps >= 3.2e8);
 }
 
 // Whether the split scan's error bound is narrow against the lists' spread, for
@@ -3212,18 +3228,20 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         block_dims = std::max(h->nquad / 4, 1) * 4;
         nblocks = h->nquad >= 8 ? 4 : 1;
     }
-    const double tiles_per_list = (double)h->tiles / (double)nlist, rows = (double)h->ntotal / (double)nlist;
+    const double tiles_per_list = (double)h->tiles / (double)nlist;
+    const double tile_rows = probed_rows(h), rows = std::max(tile_rows * (double)h->ntotal / (64.0 * (double)std::max<int64_t>(h->tiles, 1)), 1.0);
+    const double per_list = (double)n * P * rows / (double)std::max<int64_t>(h->ntotal, 1);
     const int nkc = (int)((h->d + 15) / 16);
     const bool small_d = nkc <= 8;
     // the split scan, unless norms could overflow its ranks, the caller wants the
     // pruning's statistics, which the FP32 scan counts, or its bound is wide
     bool can_split = nkc <= 32 && h->lists_sane && !(pruned && stats);
-    if (can_split && flat_shared(n, P, nlist, rows, h->d, true, pruned)) {
+    if (can_split && flat_shared(n, P, nlist, rows, per_list, h->d, true, pruned)) {
         const int rc = split_fits(h, s, &can_split);
         if (rc) return rc;
     }
-    const bool shared = flat_shared(n, P, nlist, rows, h->d, can_split, pruned);
-    if (!flat_pays(n, P, rows, h->d, pruned, stats != nullptr, shared)) return HIVF_EUNSUPPORTED;
+    const bool shared = flat_shared(n, P, nlist, rows, per_list, h->d, can_split, pruned);
+    if (!flat_pays(n, P, rows, tile_rows, h->d, pruned, can_split, shared)) return HIVF_EUNSUPPORTED;
     const bool split = shared && can_split;
     const uint32_t qc = split ? kSplitItem : kFlatItem;
     // (fewer tiles per item do not pay even where the items are few: 256
@@ -3282,7 +3300,7 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
     // pruned search's own lists and rows where they are more rows (those lists, and
     // not that many rows of ten: 5000 queries with one list of up to 5000 rows took 2.31
     // ms, now 0.49)
-    const double mean_rows = std::max(1.0, rows);
+    const double mean_rows = std::max(1.0, (double)h->ntotal / (double)nlist);
     int warm_lists = (int)std::min<double>(std::max(10.0, 2.0 * (double)k / mean_rows), 1024.0);
     int warm_rows = (int)std::max<int64_t>(k, kTileRows);
     if (pruned) {

@@ -60,10 +60,12 @@ struct BatchedState {
     ItemBound bound, flat_bound;
 
     int split_ok = -1;      // the split scan's error bound is narrow for these lists (-1: not asked yet)
+    double probed_rows = -1.0;  // rows of the list that a row lies in, on average and in whole tiles (-1: not summed yet)
 
     void invalidate() {
         valid = false;
         split_ok = -1;
+        probed_rows = -1.0;
         bound.rn = flat_bound.rn = 0;
     }
     void release();
