@@ -757,25 +757,25 @@ int hivf_tau_model_set_params(hivf_tau_model* m, const float* in) {
 
 }  // extern "C"
 
-// Host copies of a call, waited for.  (Up to 64 KB beside the stream's other
-// work; past it hipMemcpyAsync takes longer with pageable memory, most of all
-// with addresses it has not copied before: the forward of 1000 rows by 128 hidden
-// units 122 us, so 80; the gradient over them 208 and 119.)
+// Host copies of a call, waited for.  Results past 64 KB by hipMemcpy (the gradient
+// of 128 hidden units, 84 KB: over 1000 rows 117 us by hipMemcpyAsync, so 101; 8192 rows
+// 202 and 190), rows only past 640 KB: below it the wait costs more than the copy (1600
+// rows 118 us, so 104).
 namespace {
-constexpr size_t kAsyncBytes = 64 << 10;
+constexpr size_t kAsyncIn = 640 << 10, kAsyncOut = 64 << 10;
 
 hipError_t copy_in(float* dst, const float* src, size_t floats, hipStream_t s) {
     const size_t bytes = floats * sizeof(float);
-    return bytes <= kAsyncBytes ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s)
-                                : hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    return bytes <= kAsyncIn ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s)
+                             : hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
 }
 
 hipError_t copy_out(float* dst, const float* src, size_t floats, hipStream_t s) {
     const size_t bytes = floats * sizeof(float);
     hipError_t e = hipSuccess;
-    if (bytes <= kAsyncBytes) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
+    if (bytes <= kAsyncOut) e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
-    if (e == hipSuccess && bytes > kAsyncBytes) e = hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
+    if (e == hipSuccess && bytes > kAsyncOut) e = hipMemcpy(dst, src, bytes, hipMemcpyDeviceToHost);
     return e;
 }
 }  // namespace
