@@ -3133,30 +3133,33 @@ static double probed_rows(hivf_index* h) {
 
 // The form of a plain or pruned search, by n queries, P probes each, the rows of a
 // probed list and d dims; list-major forms also by the queries that a probed list
-// gets.  Measured, each search in every form: 13,700 searches of 16 to 2000 lists of 60
-// to 3000 rows, 1 to 4000 queries, 1 to 64 probes, 32 to 420 dims, on Gaussian, anisotropic
-// and clustered data, whose lists differ in size by their builds, and on equal lists set by
-// the caller, far apart from one another and in no order, where the pruned
-// per-query scan skips most and the first bounds are loose.  These rules' choice takes 4 %
-// (plain), 7 and 5 % (pruned, without and with statistics) longer than the best on built lists, 1
-// to 5 % on the others; by the mean list, and for pruned searches by lines drawn on
-// the equal lists, it was 10 to 84 %.  Figures are the whole search's in us.
+// gets. Measured, each search in every form: 13,700 searches of 16 to 2000 lists of 60
+// to 3000 rows, 1 to 4000 queries, 1 to 64 probes, 32 to 420 dims, on Gaussian,
+// anisotropic and clustered data, whose lists differ in size by their builds, and on
+// equal lists set by the caller, far apart from one another and in no order, where the
+// pruned per-query scan skips most and the first bounds are loose. These rules' choice
+// takes 4 % (plain), 7 and 5 % (pruned, without and with statistics) longer than the
+// best on built lists, 1 to 5 % on the others; by the mean list, and for pruned
+// searches by lines drawn on the equal lists, it was 10 to 84 %. Figures are the whole
+// search's in us.
 //
-// Whether the queries share lists enough for a list-major form (else a
-// workgroup per query and list, which reads every pair's rows through the
-// caches).  The plan repays itself from about 2.5e8 components on, pruned 3.2e8 (1.6e8 to
-// 2.5e8: 1.05 to 1.3 times as slow; 1000 queries of 2 lists of 1000 rows in 256, 128 dims, 2.6e8: 132 against
-// 172, 600 of 4 lists in 2000, 3e8: 240 against 220), with one probe, whose few pairs the
-// other forms spread worst, from 1.6e8 (600 of one of 1800 in 16, 1.4e8: 97 against 81, 4000 of one of 1600 in 256, 8.4e8: 185 against
-// 552).  Past 256 dims a tile's rows are long: 6.4e8, and 128
-// items of 1024 rows to fill the chip (250 queries of 2 lists of 3000 rows in 16, 420 dims, are 48
-// items: 480 against 235; 4000 of one of 1600 in 256, 300 dims: 335 against 1095).  The pruned scan, which
-// skips rows' dims, wants more work past 128 dims (4.5e8) and twice the items and queries a list past
-// 256 (1000 of 2 lists of 3000 rows, 420 dims, 841 against 533).  The FP32 scan: pruned, whose
-// tests skip dims, from 1.6e8 on long lists (100 queries of 64 lists of 1000 rows, 32 dims: 192 against
-// 358; 1000 of 16 of 60 rows 190 against 78), plain from 3.2e8 and 6 queries a list (1000 of 16 lists
-// of 256 rows, 32 dims, 1.3e8, are 40 % slower).
-static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, double per_list, int64_t d, bool split, bool pruned) {
+// Whether the queries share lists enough for a list-major form (else a workgroup per
+// query and list, which reads every pair's rows through the caches). The plan repays
+// itself from about 2.5e8 components on, pruned 3.2e8 (1.6e8 to 2.5e8: 1.05 to 1.3
+// times as slow as pairs; 1000 queries of 2 lists of 1000 rows in 256, 128 dims,
+// 2.6e8: 132 against 172), with one probe, whose few pairs the other forms spread
+// worst, from 1.6e8 (600 of one list of 1800 rows in 16, 1.4e8: 97 against 81; 4000 of
+// one of 1600 in 256, 8.4e8: 185 against 552). Past 256 dims a tile's rows are long:
+// 6.4e8, and 128 items of 1024 rows to fill the chip (250 queries of 2 lists of 3000
+// rows in 16, 420 dims, are 48 items: 480 against 235; 4000 of one of 1600 in 256, 300
+// dims: 335 against 1095). The pruned scan, which skips rows' dims, wants more work
+// past 128 dims (4.5e8) and twice the items and queries a list past 256 (1000 of 2
+// lists of 3000 rows, 420 dims: 841 against 533). The FP32 scan: pruned, whose tests
+// skip dims, from 1.6e8 on long lists (100 queries of 64 lists of 1000 rows, 32 dims:
+// 192 against 358; of 60 rows 189 against 98), plain from 3.2e8 and 6 queries a list
+// (1000 of 16 lists of 256 rows, 32 dims, 1.3e8, are 40 % slower).
+static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, double per_list, int64_t d, bool split,
+                        bool pruned) {
     const double comps = (double)n * P * rows * (double)d;
     if (!split && pruned)
         return per_list >= 2.0 && rows >= 60.0 && comps >= 1.6e8 && comps * std::min(rows, 1000.0) >= 1.6e11;
@@ -3167,16 +3170,19 @@ static bool flat_shared(int64_t n, int P, int64_t nlist, double rows, double per
     return per_list >= (pruned ? 8.0 : 4.0) && items >= (pruned ? 256.0 : 128.0) && comps >= 6.4e8;
 }
 // Whether a batch repays these scans' launches (bound, plan, selection), or each
-// query's lists are scanned by a workgroup (64 x 4 rows at a time): from
-// about 1100 rows per query, in whole tiles where lists fill half of theirs (700 to 1000
-// rows 1.05 to 1.2 times as slow, 1000 to 1300 0.8 to 0.9; 4000 of 32 lists of 16 rows 1.5). In pair
-// form only while the queries leave the chip idle: with one list each up to 1024 (600 of 1800
-// rows, 128 dims, 81 against 106), past 256 dims 512 (1000 of 3000 rows, 300 dims: 445 against 304),
-// pruned up to 512 (600 of 16 lists of 200 rows, 300 dims, equal lists far apart, 390 against 203). Or
-// in list-major form on lists of 100 rows (4000 of 4 lists of 100 rows, 300 dims: 1.07, of 128
-// rows 0.92; of 64 rows half of a tile's lanes are empty).  Where a pruned search takes the FP32
-// scan, in pair form up to 100 queries and 2000 pairs (100 of 64 lists of 60 rows: 246 against 98).
-static bool flat_pays(int64_t n, int P, double rows, double tile_rows, int64_t d, bool pruned, bool split, bool shared) {
+// query's lists are scanned by a workgroup (64 x 4 rows at a time): from about 1100
+// rows per query, in whole tiles where lists fill half of theirs (700 to 1000 rows
+// 1.05 to 1.2 times as slow, 1000 to 1300 0.8 to 0.9; 4000 of 32 lists of 16 rows
+// 1.5). In pair form only while the queries leave the chip idle: with one list each up
+// to 1024 (600 of 1800 rows, 128 dims, 81 against 106), past 256 dims 512 (1000 of
+// 3000 rows, 300 dims: 445 against 304), pruned up to 512 (600 of 16 lists of 200
+// rows, 300 dims, equal lists far apart, 390 against 203). Or in list-major form on
+// lists of 100 rows (4000 of 4 lists of 100 rows, 300 dims: 1.07, of 128 rows 0.92; of
+// 64 rows half of a tile's lanes are empty). Where a pruned search takes the FP32
+// scan, in pair form up to 100 queries and 2000 pairs (100 of 64 lists of 60 rows: 246
+// against 98).
+static bool flat_pays(int64_t n, int P, double rows, double tile_rows, int64_t d, bool pruned, bool split,
+                      bool shared) {
     const double comps = (double)n * P * rows * (double)d;
     const bool many = P * (2.0 * rows >= tile_rows ? tile_rows : rows) >= 1100.0;
     if (pruned && !split) return shared || (many && n <= 100 && n * P <= 2000);
@@ -3242,7 +3248,8 @@ int run_flat(hivf_index* h, const float4* q, int64_t n, int64_t k, int P, const 
         nblocks = h->nquad >= 8 ? 4 : 1;
     }
     const double tiles_per_list = (double)h->tiles / (double)nlist;
-    const double tile_rows = probed_rows(h), rows = std::max(tile_rows * (double)h->ntotal / (64.0 * (double)std::max<int64_t>(h->tiles, 1)), 1.0);
+    const double tile_rows = probed_rows(h);
+    const double rows = std::max(tile_rows * (double)h->ntotal / (64.0 * (double)std::max<int64_t>(h->tiles, 1)), 1.0);
     const double per_list = (double)n * P * rows / (double)std::max<int64_t>(h->ntotal, 1);
     const int nkc = (int)((h->d + 15) / 16);
     const bool small_d = nkc <= 8;
