@@ -757,17 +757,16 @@ int hivf_tau_model_set_params(hivf_tau_model* m, const float* in) {
 
 }  // extern "C"
 
-// Host copies of a call, waited for.  Results past 64 KB by hipMemcpy (the gradient
-// of 128 hidden units, 84 KB: over 1000 rows 117 us by hipMemcpyAsync, so 101; 8192 rows
-// 202 and 190), rows only past 640 KB: below it the wait costs more than the copy (1600
-// rows 118 us, so 104).
+// Results of a call, waited for.  Past 64 KB by hipMemcpy (the gradient of 128 hidden
+// units, 84 KB: over 1000 rows 117 us by hipMemcpyAsync, so 101; 8192 rows 202 and
+// 190).  The rows go by hipMemcpyAsync at any size: the wait costs more than the copy
+// (the gradient of 64 units over 1600 rows 118 us with hipMemcpy, so 104, over 5620 rows
+// 154 and 145).
 namespace {
-constexpr size_t kAsyncIn = 640 << 10, kAsyncOut = 64 << 10;
+constexpr size_t kAsyncOut = 64 << 10;
 
 hipError_t copy_in(float* dst, const float* src, size_t floats, hipStream_t s) {
-    const size_t bytes = floats * sizeof(float);
-    return bytes <= kAsyncIn ? hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s)
-                             : hipMemcpy(dst, src, bytes, hipMemcpyHostToDevice);
+    return hipMemcpyAsync(dst, src, floats * sizeof(float), hipMemcpyHostToDevice, s);
 }
 
 hipError_t copy_out(float* dst, const float* src, size_t floats, hipStream_t s) {
